@@ -23,6 +23,9 @@ const char *const kMatmulTemplate =
 const char *const kMatmulDmaTemplate =
 #include "matmul_dma.hip.inc"
     ;
+const char *const kMatmulWaveTemplate =
+#include "matmul_wave.hip.inc"
+    ;
 const char *const kMatmulF32Template =
 #include "matmul_f32_mfma.hip.inc"
     ;
@@ -188,7 +191,7 @@ bool match_matmul(const KernelGraph &g, MatmulMatch *mm, int *reject_line) {
     if (e <= 0 || K > 2147483647LL / e) MM_REJECT();
     K *= e;
   }
-  if (K < 16) MM_REJECT();
+  if (K < 8) MM_REJECT();
   const KNode &mul = g.n(R.src[0]);
   if (mul.op != POLY_OP_MUL || mul.dt != DT_F32) MM_REJECT();
   Operand A, B;
@@ -652,6 +655,118 @@ static void f32_variants(int64_t M, int64_t N, const F32Shape &chosen, const std
   if (out->variants.size() < 2) out->variants.clear();
 }
 
+// Products of few or ragged tiles: kernels/matmul_wave.hip, the depth dealt to the waves of
+// a workgroup.  Where it is taken, and on which tile (all times: one launch, operands in the
+// memory-side cache, the other templates in brackets):
+//   16-bit  outputs of at most 64 tiles of 64x64, on which the template that loads through
+//           LDS leaves most of the chip idle at half a microsecond per K tile (12x768x3072:
+//           5.4 us [31.0]; 128x768x3072: 6.1 [12.2]; from 72 tiles on it is behind:
+//           345x768x3072: 13.2 [10.8], 128x3072x768: 5.0 [4.5]), and up to 16 rows always
+//           (12x50257x768: 15.7 [25.7]); and operands that the LDS templates cannot take
+//           where they lie (a depth of no whole K tiles, rows that no 16-byte load divides)
+//           below 2^30 multiply-adds, from where copies of them in planes pay
+//           (7473x219x188: 6.9 [17.7]; 410x7104x318: 13.5 [39.1]; 3001x2999x1003: 86 [53])
+//   fp32    up to 640 tiles of 32x64 (12x768x3072: 8.1 us [265]; 128x3072x768: 10.1 [22.3];
+//           1024^3: 21.6 [30.2]; 4096x512x784, 1024 tiles: 50.1 [38.9])
+//   (16-bit products from a depth of 8192 on are left to the templates that deal it to
+//   several workgroups; fp32 ones from 4096 on are dealt to eight here, which one tile of a
+//   few gains most from: 100x50x4096 7.1 -> 5.7 us [277], 300x200x4096 15.2 -> 17 [24.2],
+//   512x784x4096 36.6 -> 47.8 [68.7])
+// The smallest tile that does not need more workgroups than the chip runs at once: few rows
+// want many narrow workgroups (128x768x768 fp32: 16x32 4.9 us, 32x64 9.8), many rows tiles
+// that read each operand fewer times.
+static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, bool whole_tiles, RenderedKernel *out) {
+  const int64_t K = mm.K, M = mm.M, N = mm.N, Z = mm.Z;
+  if (getenv("POLY_HIP_NO_WAVE_MM")) return false;
+  const bool f32 = mm.A.dt == DT_F32;
+  const int kv = f32 ? 4 : 8;
+  auto tiles_of = [&](int tm, int tn) { return (double)((M + 16 * tm - 1) / (16 * tm)) * (double)((N + 16 * tn - 1) / (16 * tn)) * (double)Z; };
+  struct Form { int tm, tn, waves, depth; };
+  Form f{1, 2, 8, 6};
+  int S = 1;      // workgroups sharing the depth of a tile
+  if (f32) {
+    if (tiles_of(2, 4) > 640) return false;
+    if (tiles_of(1, 1) <= 192) f = Form{1, 1, 8, 6};
+    else if (tiles_of(1, 2) <= 288) f = Form{1, 2, 4, 6};
+    else f = Form{2, 4, 4, 6};
+    if (tiles_of(2, 4) > 256 && tiles_of(4, 4) <= 256 && M >= 64 && N >= 64) f = Form{4, 4, 4, 6};
+    if (K >= 4096) {
+      f = tiles_of(2, 4) >= 26 ? Form{2, 4, 4, 6} : Form{1, 2, 4, 6};
+      for (S = 8; S > 1 && K % (S * kv) != 0;) S /= 2;
+    }
+  } else {
+    const bool few = M <= 16 || N <= 16 || tiles_of(4, 4) <= 64;
+    if (!few && (whole_tiles || (double)M * (double)N * (double)K * (double)Z >= 1073741824.0)) return false;
+    if (tiles_of(1, 2) > 640 && M > 16) f = Form{2, 2, 8, 6};
+    if (f.tm == 2 && tiles_of(2, 2) > 640) f = Form{2, 4, 4, 6};
+    if (f.tn == 4 && tiles_of(2, 4) > 640) f = Form{4, 4, 4, 4};
+  }
+  if (K >= 8192) return false;
+  if (K <= 256 && f.waves > 4) f.waves = 4;
+  if (const char *ov = measurement_env("POLY_HIP_MM_WAVE")) {   // "TM,TN,WAVES,DEPTH": tuning experiments
+    if (sscanf(ov, "%d,%d,%d,%d,%d", &f.tm, &f.tn, &f.waves, &f.depth, &S) < 4) return false;
+  }
+  if (S > 1 && (K % (S * kv) != 0 || !ep.scratch_type.empty() || Z * S > 65535)) S = 1;
+  // an operand is read along K where its steps are contiguous there, along its rows otherwise
+  // (runs of as many rows as the tile has blocks)
+  auto layout = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a, int64_t rows, int run, bool *kc) {
+    if (ks.s_lo == 1 && (ks.kb >= K || ks.kb % kv == 0)) { *kc = true; return true; }
+    *kc = false;
+    return (is_a ? dims.back().ca : dims.back().cb) == 1 && rows >= run && (dims.size() == 1 || dims.back().extent % run == 0);
+  };
+  bool a_kc, b_kc;
+  if (!layout(mm.ka, mm.md, true, M, f.tm, &a_kc) || !layout(mm.kb, mm.nd, false, N, f.tn, &b_kc)) return false;
+  const int64_t tiles = ((M + 16 * f.tm - 1) / (16 * f.tm)) * ((N + 16 * f.tn - 1) / (16 * f.tn));
+  if (Z > 65535 || M > 2147483647LL / 2 || N > 2147483647LL / 2 || K > 2147483647LL / 2 || tiles > 2147483647LL / 2) return false;
+  std::string cfg;
+  cfg += strf("#define POLY_TIN %s\n#define POLY_F32 %d\n", dt_cname(mm.A.dt), f32 ? 1 : 0);
+  if (!f32) cfg += strf("#define POLY_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_%s(a, b, c, 0, 0, 0)\n", mm.A.dt == DT_BF16 ? "bf16" : "f16");
+  else cfg += "#define POLY_MFMA(a, b, c) (c)\n";
+  cfg += strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_K %lld\n#define POLY_Z %lld\n", (long long)M, (long long)N, (long long)K, (long long)Z);
+  cfg += strf("#define POLY_TM %d\n#define POLY_TN %d\n#define POLY_WAVES %d\n#define POLY_DEPTH %d\n", f.tm, f.tn, f.waves, f.depth);
+  cfg += strf("#define POLY_A_KC %d\n#define POLY_B_KC %d\n#define POLY_A_PTR %s\n#define POLY_B_PTR %s\n", a_kc ? 1 : 0, b_kc ? 1 : 0, ep.a_ptr.c_str(), ep.b_ptr.c_str());
+  cfg += offset_fn("poly_a_row", mm.md, true, 0) + offset_fn("poly_b_row", mm.nd, false, 0);
+  if (mm.zd.empty()) {
+    cfg += strf("__device__ __forceinline__ int poly_a_z(int) { return %lld; }\n", (long long)mm.a_c0);
+    cfg += strf("__device__ __forceinline__ int poly_b_z(int) { return %lld; }\n", (long long)mm.b_c0);
+  } else {
+    cfg += offset_fn("poly_a_z", mm.zd, true, mm.a_c0) + offset_fn("poly_b_z", mm.zd, false, mm.b_c0);
+  }
+  cfg += matmul_k_fn("poly_a_k", mm.ka, K) + matmul_k_fn("poly_b_k", mm.kb, K);
+  const std::string shape = strf("#define POLY_SIGNATURE %s%s\n#define POLY_KSPLIT %d\n#define POLY_PARTIALS poly_scratch\n", ep.signature.c_str(), S > 1 ? ", float* poly_scratch" : "", S) + ep.code;
+  cfg += shape;
+  if (S > 1) cfg += "#define POLY_EPILOGUE(acc, m, n, z) POLY_PARTIALS[(((size_t)poly_ks * POLY_Z + (z)) * POLY_M + (m)) * POLY_N + (n)] = (acc)\n";
+  else cfg += strf("#define POLY_EPILOGUE(acc, m, n, z) %s\n", ep.call.c_str());
+  if (S == 1 && !ep.mid_value_call.empty())
+    cfg += strf("#define POLY_EP_MID_VALUE(acc, m, n, z) %s\n#define POLY_EP_MID_PTR(m, n, z) %s\n", ep.mid_value_call.c_str(), ep.mid_ptr_call.c_str());
+  *out = RenderedKernel();
+  out->source = std::string(hip_prelude()) + cfg + kMatmulWaveTemplate;
+  out->entry = "poly_k";
+  out->launch.grid[0] = (unsigned)tiles;
+  out->launch.grid[1] = (unsigned)(Z * S);
+  out->launch.block[0] = (unsigned)(64 * f.waves);
+  if (S > 1) {
+    // the template becomes a first stage; the kernel proper adds the partial results up
+    out->pres.push_back({out->source, out->entry, out->launch});
+    out->scratch_bytes = (size_t)S * (size_t)Z * (size_t)M * (size_t)N * sizeof(float);
+    out->source = std::string(hip_prelude()) + strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_Z %lld\n", (long long)M, (long long)N, (long long)Z) + shape +
+                  strf("#define POLY_EPILOGUE(acc, m, n, z) %s\n", ep.call.c_str()) + kSplitKCombine;
+    out->launch = LaunchSpec();
+    out->launch.grid[0] = (unsigned)(((double)Z * M * N + 255) / 256);
+    out->launch.block[0] = 256;
+  }
+  out->klass = KernelClass::MATMUL_MFMA;
+  out->reads_b_ahead = true;
+  out->strategy = strf("mfma %s M=%lld N=%lld K=%lld Z=%lld tile %dx%d, depth dealt to %d waves, A:%s B:%s", f32 ? "16x16x4 f32" : mm.A.dt == DT_BF16 ? "16x16x32 bf16" : "16x16x32 f16",
+                       (long long)M, (long long)N, (long long)K, (long long)Z, 16 * f.tm, 16 * f.tn, f.waves, a_kc ? "k-major" : "m-major", b_kc ? "k-major" : "n-major");
+  if (S > 1) out->strategy += strf(", K dealt to %d workgroups per tile, partial results added by a second kernel", S);
+  out->n_params = ep.n_params;
+  out->n_vars = 0;
+  out->flops = 2.0 * (double)M * (double)N * (double)K * (double)Z;
+  out->bytes = ep.bytes;
+  return true;
+}
+
 // fp32 operands: kernels/matmul_f32_mfma.hip (v_mfma_f32_32x32x2_f32, exact fp32 products).
 static bool render_matmul_f32(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKernel *out) {
   const int64_t K = mm.K, M = mm.M, N = mm.N, Z = mm.Z;
@@ -747,6 +862,7 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   const KSplit &ka = mm.ka, &kb = mm.kb;
   const std::vector<Dim> &md = mm.md, &nd = mm.nd, &zd = mm.zd;
   if (M > 2147483647LL || N > 2147483647LL || Z > 65535) return reject(__LINE__);
+  if (A.dt == DT_F32 && render_matmul_wave(mm, ep, false, out)) return true;
   if (A.dt == DT_F32) return ep.mid_value_call.empty() ? render_matmul_f32(mm, ep, out) : false;     // (no second output in the fp32 template)
   int BK = 64;
   if (const char *e = measurement_env("POLY_HIP_MM_BK")) BK = atoi(e) == 32 ? 32 : 64;
@@ -758,7 +874,9 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     return reject(__LINE__);
   };
   bool a_kc, b_kc;
-  if (!layout(ka, md, true, M, &a_kc) || !layout(kb, nd, false, N, &b_kc)) return reject(__LINE__);
+  const bool whole_tiles = layout(ka, md, true, M, &a_kc) && layout(kb, nd, false, N, &b_kc);
+  if (render_matmul_wave(mm, ep, whole_tiles, out)) return true;
+  if (!whole_tiles) return reject(__LINE__);
 
   // tile shape: 4 waves; narrow outputs get a narrow tile
   // Candidates: (BM, BN, waves M x N, workgroups resident per CU, throughput of one CU
