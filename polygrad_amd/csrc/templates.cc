@@ -1002,7 +1002,7 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     // grid run ahead through it, so that the others wait for HBM once and not at every K tile
     int touch_wgs = 0;
     if (use_dma && ep.b_from_hbm && S == 1 && Z == 1 && zd.empty() && nd.size() == 1 && kb.kb >= K && !getenv("POLY_HIP_NO_PREFETCH") &&
-        ((b_kc && kb.s_lo == 1 && nd[0].cb == K) || (!b_kc && nd[0].cb == 1 && kb.s_lo == N)) && K * N * 2 >= (128 << 10) && tiles >= 64) {
+        ((b_kc && kb.s_lo == 1 && nd[0].cb == K) || (!b_kc && nd[0].cb == 1 && kb.s_lo == N)) && K * N * 2 >= (128 << 10) && tiles >= 8) {
       touch_wgs = K * N * 2 >= (2 << 20) ? 64 : 32;
       cfg += strf("#define POLY_TOUCH_WGS %d\n#define POLY_TOUCH_FIRST %lld\n#define POLY_TOUCH_LINES %lldll\n", touch_wgs,
                   (long long)(mm.b_c0 & ~1ll), (long long)((K * N * 2 - 64) / 64));
@@ -1112,7 +1112,21 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     Dma probe{0, 0, 0, 0, 0};
     auto count = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * Z * S; };   // workgroups of the launch
     const int64_t t = count(BM, BN);
-    if (dma_for(BM, BN, &probe)) {
+    // A launch that 128x128 tiles leave a fifth to three quarters of the chip of: 64x64 tiles
+    // while every one of them has a CU (six stages of 64; from 192 tiles on four, for two to
+    // a CU), 64x128 tiles while each has one, or two share one.  What such a launch waits
+    // for is the latency of its loads: more of them in flight on more CUs.  1035 rows:
+    // 768x3072 24.5 -> 12.2 us, 768x768 11.0 -> 4.8, 2304x768 10.1 -> 9.7, 3072x768
+    // 12.0 -> 10.9; 2048x768x3072 21.5 -> 16.3; 1024^3 9.1 -> 5.8; 2048x3072x768, 768 tiles
+    // of 64x128, is the same either way (17.5 and 17.2).
+    Dma small{0, 0, 0, 0, 0};
+    const int64_t t64 = count(64, 64), t128 = count(64, 128);
+    if (S == 1 && K >= 256 && !getenv("POLY_HIP_NO_SMALL_TILES")) {
+      if (t64 <= 256) small = t64 > 192 ? Dma{64, 4, 2, 2, 2} : Dma{64, 6, 1, 2, 2};
+      else if (t128 <= 448) small = t128 > 256 ? Dma{64, 3, 2, 2, 2} : Dma{64, 4, 1, 2, 2};
+    }
+    if (small.bk && dma_for(64, t64 <= 256 ? 64 : 128, &small)) { BM = 64; BN = t64 <= 256 ? 64 : 128; WVM = WVN = 2; chosen = small; }
+    else if (dma_for(BM, BN, &probe)) {
       Dma p2{0, 0, 0, 0, 0}, p3{0, 0, 0, 0, 0}, wide{64, 3, 1, 2, 4};
       // Three quarters of a round of 128x256 tiles and more on a deep K, A along k and B along
       // n (8192 x 768 x 3072 of the GPT-2 layer, 192 tiles): the tile stays, on 8 waves of

@@ -1,6 +1,8 @@
-"""Products of few or ragged output tiles (kernels/matmul_wave.hip): every extent at, below
+"""Products of few or ragged output tiles.  kernels/matmul_wave.hip: every extent at, below
 and above the edges of its tiles, the depth below one step, at whole steps of all waves and
 with a remainder, operands along the depth and along their rows, the three input types.
+kernels/matmul_dma.hip on tiles of 64 rows: ragged rows and columns, a depth of the fewest
+and of many K tiles, every layout, two, three, four and six stages.
 Against the product in float64, element by element, within the rounding of K fp32 additions
 and products (K * 2^-24 * sum of |a b|; the products of 16-bit values are exact)."""
 import ctypes as C
@@ -20,6 +22,11 @@ EDGES = [(12, 33, 8, "bfloat16", "nn"), (16, 32, 256, "bfloat16", "nn"), (17, 31
          (1500, 1283, 101, "bfloat16", "nt"), (2, 5, 9, "float32", "nn"), (15, 16, 128, "float32", "nt"), (143, 40, 791, "float32", "nn"),
          (33, 129, 784, "float32", "nt"), (200, 300, 4096, "float32", "tn"), (130, 770, 515, "float32", "nn"), (64, 96, 4100, "float32", "nn"), (600, 650, 67, "float32", "nt")]
 
+LDS_TILES = [(333, 840, 256, "bfloat16", "nn", "64x64x64"), (345, 768, 3072, "bfloat16", "nn", "64x64x64"), (1000, 904, 256, "bfloat16", "nt", "64x64x64"),
+             (1000, 904, 320, "float16", "tn", "64x64x64"), (1111, 1000, 1536, "bfloat16", "nt", "64x128x64"), (1112, 1000, 256, "bfloat16", "tn", "64x128x64"),
+             (1035, 3000, 768, "bfloat16", "nn", "64x128x64")]
+ALL = [(c, "depth dealt to") for c in EDGES] + [(c[:5], "tile " + c[5]) for c in LDS_TILES]
+
 
 def _name(c):
     return "-".join(str(v) for v in c)
@@ -30,22 +37,22 @@ def _case(m, n, k, dtype, layout):
 
 
 @pytest.mark.skipif(not os.path.exists(hostcheck.CLANG), reason="no host clang with AddressSanitizer")
-@pytest.mark.parametrize("c", EDGES, ids=_name)
-def test_stays_in_bounds(c, hiplib, monkeypatch):
+@pytest.mark.parametrize("c,how", ALL, ids=lambda v: _name(v) if isinstance(v, tuple) else "")
+def test_stays_in_bounds(c, how, hiplib, monkeypatch):
     monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
     pf = cases._matmul_schedule(_case(*c)).plan()
     s = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents
-    assert "depth dealt to" in _ffi.take_string(hiplib.poly_hip_describe(s.items[0].root, 0))
+    assert how in _ffi.take_string(hiplib.poly_hip_describe(s.items[0].root, 0))
     assert hostcheck.check_schedule(hiplib, pf.schedule) >= 1
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("c", EDGES, ids=_name)
-def test_against_float64(c):
+@pytest.mark.parametrize("c,how", ALL, ids=lambda v: _name(v) if isinstance(v, tuple) else "")
+def test_against_float64(c, how):
     import torch
     m, n, k, dtype, layout = c
     state = cases.prepare(_case(*c), 5)
-    assert "depth dealt to" in state["plan"].kernel_info()[0]["desc"]
+    assert how in state["plan"].kernel_info()[0]["desc"]
     got = cases.run(state)["C"]
     state["plan"].sync()
     by_name = {s.name: state["data"][s.index] for s in state["plan"].external_slots()}
