@@ -77,6 +77,11 @@ int poly_hip_sync(void);
 /* The HIP stream (hipStream_t) all launches go to; callers that own device
  * memory on another stream order against it with events. */
 void *poly_hip_stream(void);
+/* Orders that stream after everything queued so far on `stream` (a hipStream_t of the same
+ * device, NULL for the default stream) without blocking the host; costs nothing on the
+ * device when `stream` has no work left.  0 = ok.  No counterpart in the reference, whose
+ * runtime has no streams. */
+int poly_hip_order_after(void *stream);
 
 /* poly_cuda_compile / launch / program_destroy (runtime_cuda.c:288-406, 418-424).
  * Compiles HIP C with hiprtc for gfx950; identical sources share one module. */
@@ -115,7 +120,7 @@ int poly_hip_check_index_simplification(PolyUOp *scheduled_root, int samples);
  * intermediates that are dead share memory, only the intermediates that their
  * producers leave holes in are cleared per run (poly_hip_unwritten_slots), launches are
  * asynchronous on one stream and the launch sequence is replayed from a
- * hipGraph when the bound pointers repeat (in that graph, small launches that are
+ * hipGraph when the bound pointers repeat, unless there are only a few (in that graph, small launches that are
  * chains of dependent steps may run on side branches beside the others, ordered by
  * the buffers they share: poly_hip_plan_side_launches). */
 typedef struct PolyHipPlan PolyHipPlan;

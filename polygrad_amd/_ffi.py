@@ -85,6 +85,7 @@ SYMBOLS = {
     "poly_hip_memset": (C.c_int, [C.c_void_p, C.c_int, C.c_size_t]),
     "poly_hip_sync": (C.c_int, []),
     "poly_hip_stream": (C.c_void_p, []),
+    "poly_hip_order_after": (C.c_int, [C.c_void_p]),
     "poly_hip_compile": (C.c_void_p, [C.c_char_p, C.c_char_p]),
     "poly_hip_launch": (C.c_int, [C.c_void_p, C.POINTER(C.c_void_p), C.c_int] + [C.c_uint] * 7),
     "poly_hip_program_destroy": (None, [C.c_void_p]),

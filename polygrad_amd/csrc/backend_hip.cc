@@ -329,6 +329,7 @@ int poly_hip_copy_dtoh(void *dst, const void *src, size_t n) { return runtime_co
 int poly_hip_copy_dtod(void *dst, const void *src, size_t n) { return runtime_copy(dst, src, n, 2); }
 int poly_hip_memset(void *p, int value, size_t n) { return runtime_memset(p, value, n); }
 int poly_hip_sync(void) { return runtime_sync(); }
+int poly_hip_order_after(void *stream) { return runtime_order_after(stream); }
 void *poly_hip_stream(void) { return runtime_stream(); }
 
 struct PolyHipProgram { Program *p; };

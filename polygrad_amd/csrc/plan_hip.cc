@@ -115,6 +115,11 @@ struct PolyHipPlan {
   std::vector<std::vector<int>> touch_at;
   Program *touch = nullptr;
   bool use_graph = true;
+  // Kernel launches of one pass.  A plan of a few of them is launched kernel by kernel: a
+  // graph of one to three nodes takes the host 16 us to launch, each kernel 2.5-3 us
+  // (a row sum: 16.6 against 3.2 us of host time, 3 launches of a LayerNorm 17.9 against
+  // 8.0; 22 launches of an MLP step 27 against 73).
+  int n_launches = 0;
   bool tuned = false;            // candidates of the tunable kernels have been timed (or there are none)
   // The launch sequence is captured once (`captured`, with the kernel node of every launch
   // in `launches`); a binding the plan has not seen gets a graph instantiated from it whose
@@ -779,6 +784,11 @@ PolyHipPlan *poly_hip_compile_schedule(PolyCtx *ctx, const PolySchedule *s) {
       if (!plan->touch) return nullptr;
     }
   }
+  for (int u = 0; u < n_units; u++) {
+    const HipRunner *r = plan->units[(size_t)u].runner;
+    plan->n_launches += (int)(plan->fills_before[(size_t)u].size() + plan->touch_at[(size_t)u].size() + (r->skip_pres ? 0 : r->pres.size()) + 1 +
+                              (r->guards.empty() ? 0 : r->guards.size() + 1));
+  }
   plan->kargs.resize((size_t)n_units);
   plan->var_vals.resize((size_t)n_units);
   for (int u = 0; u < n_units; u++) {
@@ -959,7 +969,8 @@ int poly_hip_plan_run(PolyHipPlan *plan, void **slot_data, int n_slots, const Po
     plan->tuned = true;
   }
   hipStream_t stream = (hipStream_t)runtime_stream();
-  if (!plan->use_graph || getenv("POLY_HIP_NO_GRAPH")) return enqueue_all(plan);
+  constexpr int kFewLaunches = 6;
+  if (!plan->use_graph || (plan->n_launches <= kFewLaunches && !plan->forked) || getenv("POLY_HIP_NO_GRAPH")) return enqueue_all(plan);
   plan->tick++;
   (void)key;
   for (GraphEntry &g : plan->graphs)

@@ -25,6 +25,8 @@ void runtime_free(void *p);
 int runtime_copy(void *dst, const void *src, size_t n, int kind);
 int runtime_memset(void *p, int value, size_t n);
 int runtime_sync();
+// The backend's stream waits for what `stream` has queued so far; the host does not.
+int runtime_order_after(void *stream);
 // Can a kernel dereference `p`?  False for pageable host memory (malloc, numpy arrays, the
 // host-side constant registry of the frontend) and for addresses HIP does not know.
 bool runtime_device_can_read(const void *p);

@@ -53,7 +53,8 @@ class HipPlan:
         self.slots = [Slot(i, s.buf_slots[i], (names[i] if names and i < len(names) else "") or "")
                       for i in range(s.n_buf_slots)]
         self.n_kernels = self.lib.poly_hip_plan_n_kernels(self.handle)
-        self._ext_stream = None
+        self._slot_nbytes = [s.nbytes for s in self.slots]
+        self._ptr_type = C.c_void_p * len(self.slots)
 
     @classmethod
     def from_file(cls, path):
@@ -74,34 +75,31 @@ class HipPlan:
     def external_slots(self):
         return [s for s in self.slots if not s.is_intermediate]
 
-    def _order_after_torch(self):
+    def _order_after_torch(self, device):
         """The backend launches on its own non-blocking stream: make that stream wait
-        for whatever torch has queued so far (fills, copies, random init of the tensors
-        handed in), without blocking the host."""
-        import torch
-        if self._ext_stream is None:
-            self._ext_stream = torch.cuda.ExternalStream(self.lib.poly_hip_stream())
-        self._ext_stream.wait_stream(torch.cuda.current_stream())
+        for whatever torch has queued so far on the current stream of `device` (fills, copies,
+        random init of the tensors handed in), without blocking the host."""
+        from torch import _C as torch_c
+        if self.lib.poly_hip_order_after(torch_c._cuda_getCurrentRawStream(device)) != 0:
+            raise RuntimeError("poly_hip_order_after failed (see stderr)")
 
     def _ptr_array(self, slot_data):
-        n = len(self.slots)
-        arr = (C.c_void_p * n)()
-        if any(v is not None and not isinstance(v, int) for v in slot_data):
-            self._order_after_torch()
-        for i in range(n):
-            v = slot_data[i] if i < len(slot_data) else None
-            if v is None:
-                arr[i] = None
-            elif isinstance(v, int):
-                arr[i] = v
-            else:  # torch tensor
-                if not v.is_cuda or not v.is_contiguous():
-                    raise ValueError(f"slot {i}: need a contiguous CUDA tensor")
-                if v.numel() * v.element_size() < self.slots[i].nbytes:
-                    raise ValueError(f"slot {i}: tensor has {v.numel() * v.element_size()} bytes, "
-                                     f"slot needs {self.slots[i].nbytes}")
-                arr[i] = v.data_ptr()
-        return arr
+        ptrs = [None] * len(self.slots)
+        device = -1
+        for i, (v, nbytes) in enumerate(zip(slot_data, self._slot_nbytes)):
+            if v is None or isinstance(v, int):
+                ptrs[i] = v
+                continue
+            # torch tensor
+            if not (v.is_cuda and v.is_contiguous()):
+                raise ValueError(f"slot {i}: need a contiguous CUDA tensor")
+            if v.nbytes < nbytes:
+                raise ValueError(f"slot {i}: tensor has {v.nbytes} bytes, slot needs {nbytes}")
+            ptrs[i] = v.data_ptr()
+            device = v.get_device()
+        if device >= 0:
+            self._order_after_torch(device)
+        return self._ptr_type(*ptrs)
 
     def run(self, slot_data, sync=True, var_bindings=None):
         """Enqueues one pass of the plan.  slot_data[i]: tensor / device pointer for
