@@ -30,6 +30,9 @@ namespace {
 const char *const kAttentionTemplate =
 #include "attention_mfma.hip.inc"
     ;
+const char *const kAttentionRowsTemplate =
+#include "attention_rows.hip.inc"
+    ;
 
 int fa_item = -1;     // the schedule item a group is being grown from (for the message below)
 bool fa_reject(int line) {
@@ -1480,19 +1483,34 @@ static std::string attention_order(int64_t MB, int64_t Z) {
   return t + "};\n";
 }
 
+// The most keys a workgroup of kernels/attention_rows.hip holds the scores of (eight waves, 16
+// 16-key blocks and two query blocks each: 128 registers of a lane for fp32).
+constexpr int64_t kAttentionRowsKeys = 1024;
+
 static bool match_attention(const Sched &sc, int s_item, const std::vector<char> &taken, FusedGroup *out) {
   const PolySchedule *s = sc.s;
   const KernelGraph &gS = sc.graphs[(size_t)s_item];
   MatmulMatch mS;
   if (!match_matmul(gS, &mS, nullptr)) return false;   // not a matmul: not a candidate, no diagnostics
-  if (mS.K != 64 || mS.M % 128 != 0 || mS.N % 64 != 0 || mS.Z > (1 << 20)) FA_REJECT();
+  if (mS.K != 64 || mS.Z > (1 << 20)) FA_REJECT();
   if (mS.ka.kb < mS.K || mS.kb.kb < mS.K || mS.ka.s_lo != 1 || mS.kb.s_lo != 1) FA_REJECT();   // features contiguous
   if (mS.nd_full.size() != 1 || mS.nd_full[0].cut != 1) FA_REJECT();                         // keys: one plain range
   const int n_master = mS.nd_full[0].ord;
   const StoreInfo &stS = gS.stores[0];
   const DT tin = mS.A.dt;
-  if (tin != DT_BF16 && tin != DT_F16) FA_REJECT();
+  const bool f32 = tin == DT_F32;
+  if (tin != DT_BF16 && tin != DT_F16 && !f32) FA_REJECT();
   if (gS.n(stS.value).dt != tin) FA_REJECT();
+  // Blocks of 128 queries and 64 keys of a 16-bit type: kernels/attention_mfma.hip.  What they
+  // do not divide, and fp32: kernels/attention_rows.hip, which keeps the scores of its queries
+  // in registers.  That one also takes few scores in whole blocks, where the other has too few
+  // workgroups and each walks its keys in order (bf16, us, attention_mfma in brackets; 12 heads
+  // of 128 keys 4.0 [12.3], 512: 12.2 [23.2]; 48 of 128: 5.5 [14.2], 384, near the
+  // line: 20.1 [22.6]; 96 of 512, three times the scores of the line: 43.8 [28.1]).
+  const bool whole_blocks = !f32 && mS.M % 128 == 0 && mS.N % 64 == 0;
+  const bool rows_possible = mS.N <= kAttentionRowsKeys && mS.M <= (1 << 24) && !getenv("POLY_HIP_NO_ATTENTION_ROWS");
+  bool rows_form = rows_possible && (!whole_blocks || (mS.Z * mS.M * mS.N <= (int64_t)1 << 23 && !getenv("POLY_HIP_EXACT_ATTENTION")));
+  if (!rows_form && !whole_blocks) FA_REJECT();
   std::vector<int64_t> mext(gS.ranges.size());
   for (size_t i = 0; i < gS.ranges.size(); i++) mext[i] = gS.ranges[i].extent;
   RangeMap idS;
@@ -1672,6 +1690,8 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
         mP.preset.count(mn) && mP.preset[mn] == "mx" && mP.preset.count(den) && mP.preset[den] == "sum" && mP.preset[xn] == "x")
       p_is_term_over_sum = true;
   }
+  if (!p_is_term_over_sum) rows_form = false;      // (the rows form divides terms by the sum itself)
+  if (!rows_form && !whole_blocks) FA_REJECT();
   const int sl_p = sc.slot(i_p, sc.graphs[(size_t)i_p].param_slot(sc.graphs[(size_t)i_p].stores[0].param));
   if (!only_group_reads(cur, {i_max, i_sum, i_p}) || !only_group_reads(sl_max, {i_sum, i_p}) || !only_group_reads(sl_sum, {i_p})) FA_REJECT();
   if (sc.readers[(size_t)sl_p].size() != 1 || !s->buf_slots[sl_p].is_intermediate || sc.writers[(size_t)sl_p].size() != 1) FA_REJECT();
@@ -1682,7 +1702,7 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
   if (taken[(size_t)i_pv]) FA_REJECT();
   const KernelGraph &gP = sc.graphs[(size_t)i_pv];
   MatmulMatch mV;
-  if (!match_matmul(gP, &mV, nullptr)) FA_REJECT();
+  if (!match_matmul(gP, &mV, nullptr, 1)) FA_REJECT();
   if (mV.A.dt != tin || sc.slot(i_pv, mV.A.param) != sl_p || sc.slot(i_pv, mV.B.param) == sl_p) FA_REJECT();
   if (mV.M != mS.M || mV.Z != mS.Z || mV.K != mS.N || mV.N != 64) FA_REJECT();
   if (mV.ka.kb < mV.K || mV.kb.kb < mV.K) FA_REJECT();
@@ -1821,12 +1841,13 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
   // The softmax terms use the bare exp2 instruction: a term below 2^-126 of the row's
   // largest (which is exactly 1, so the sum is at least 1) cannot change the fp32 sum, and
   // the probability it would give is below the smallest normal 16-bit float.
-  const bool online = p_is_term_over_sum && !getenv("POLY_HIP_EXACT_ATTENTION");
+  // (fp32 probabilities have that range, and keep the exp2 of the unfused kernels.)
+  const bool online = !rows_form && p_is_term_over_sum && !getenv("POLY_HIP_EXACT_ATTENTION");
   auto value_fn = [&](const Member &m, const char *name, const char *ret, const char *lead_args, int node,
                       const std::map<int, std::string> &extra_preset) {
     const KernelGraph &g = sc.graphs[(size_t)m.item];
     Emitter em(g);
-    em.raw_exp2 = (m.item == i_sum || m.item == i_p);
+    em.raw_exp2 = !f32 && (m.item == i_sum || m.item == i_p);
     em.pow2_mul16_exact = online;
     Scope S0;
     S0.indent = 1;
@@ -1840,9 +1861,10 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
     cfg += strf("  return %s;\n}\n", v.c_str());
   };
   cfg += strf("#define POLY_TIN %s\n", tn);
-  cfg += strf("#define POLY_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_%s(a, b, c, 0, 0, 0)\n", tin == DT_BF16 ? "bf16" : "f16");
+  if (f32) cfg += "#define POLY_MFMA(a, b, c) (c)\n";
+  else cfg += strf("#define POLY_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_%s_%s(a, b, c, 0, 0, 0)\n", rows_form ? "16x16x32" : "32x32x16", tin == DT_BF16 ? "bf16" : "f16");
   cfg += strf("#define POLY_FA_M %lld\n#define POLY_FA_N %lld\n#define POLY_FA_Z %lld\n", (long long)mS.M, (long long)mS.N, (long long)mS.Z);
-  cfg += attention_order(mS.M / 128, mS.Z);
+  if (!rows_form) cfg += attention_order(mS.M / 128, mS.Z);
   auto operand_arg = [&](int o) { return arg_of(folded[o].item >= 0 ? folded[o].src_slot : op_slot[o]); };
   cfg += strf("#define POLY_Q_PTR fa%d\n#define POLY_K_PTR fa%d\n#define POLY_V_PTR fa%d\n", operand_arg(0), operand_arg(1), operand_arg(2));
   // position in the operand's own buffer -> position in the buffer it was copied from
@@ -1909,7 +1931,7 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
   // b * N + 64 kb, column c0 + 64 h?  Then that product can say how large the keys of every
   // block are (key_bounds; find_fused_groups asks it to).
   FusedGroup::KeyBounds kbnd;
-  if (k_pitch >= 64 && mS.N % 64 == 0 && mS.N / 64 <= 64 && mS.K == 64) {
+  if (!rows_form && k_pitch >= 64 && mS.N % 64 == 0 && mS.N / 64 <= 64 && mS.K == 64) {
     const int64_t T = mS.N, NKB = T / 64, c0 = eval_src(1, raw_off(1, 0, 0)) % k_pitch;
     // z counts (b, h) with either of the two running fastest
     const bool heads_fastest = mS.Z > 1 && eval_src(1, raw_off(1, 1, 0)) % k_pitch != c0;
@@ -2170,18 +2192,35 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
       }
     }
   }
-  rk.source = std::string(hip_prelude()) + cfg + kAttentionTemplate;
-  const std::string fa_cfg = cfg;
   rk.entry = "poly_k";
-  rk.launch.grid[0] = (unsigned)((mS.M / 128) * mS.Z);
-  rk.launch.block[0] = 256;
   rk.klass = KernelClass::ATTENTION;
-  rk.strategy = strf("fused attention (%zu kernels): mfma 32x32x16 %s Z=%lld M=%lld N=%lld D=64, %s", all.size() + copy_items.size(),
-                     tin == DT_BF16 ? "bf16" : "f16", (long long)mS.Z, (long long)mS.M, (long long)mS.N,
-                     cfg.find("#define POLY_FA_ONLINE 1") != std::string::npos ? "one pass, online softmax" : "two passes over keys, exact roundings");
-  if (mask_table) rk.strategy += ", mask tiles classified by a first kernel";
-  if (out->key_bounds.used) rk.strategy += ", products of masked key blocks bounded by the block maxima the keys' product leaves";
-  if (matmul_tuning_enabled()) {
+  const std::string fa_cfg = cfg;
+  if (rows_form) {
+    // As many waves as there are units of keys to deal, up to four a wave before there are
+    // eight (36 heads of 345 keys: 16.3 us on four waves, 18.4 on eight); two blocks of queries
+    // to a workgroup, which halves the reads of K and V, once that leaves every CU two
+    // workgroups (36 heads of 839 keys on eight waves: 61.7, 78.7 with one; 16 of 249, 128
+    // workgroups: 8.4, 6.0 with one).
+    const int64_t units = f32 ? (mS.N + 15) / 16 : (mS.N + 31) / 32;
+    int waves = units <= 1 ? 1 : units <= 2 ? 2 : units <= 16 ? 4 : 8;
+    int qt = mS.Z * ((mS.M + 31) / 32) >= 512 ? 2 : 1;
+    if (const char *ov = measurement_env("POLY_HIP_FA_ROWS")) sscanf(ov, "%d,%d", &waves, &qt);   // "WAVES,QT": tuning experiments
+    rk.source = std::string(hip_prelude()) + strf("#define POLY_F32 %d\n#define POLY_FA_WAVES %d\n#define POLY_FA_QT %d\n#define POLY_FA_PASS_ZEROS %d\n", f32 ? 1 : 0, waves, qt, whole_blocks ? 1 : 0) + cfg + kAttentionRowsTemplate;
+    rk.launch.grid[0] = (unsigned)(((mS.M + 16 * qt - 1) / (16 * qt)) * mS.Z);
+    rk.launch.block[0] = (unsigned)(64 * waves);
+    rk.strategy = strf("fused attention (%zu kernels): mfma %s Z=%lld M=%lld N=%lld D=64, one pass, scores of %d queries in registers, keys dealt to %d waves, exact roundings", all.size() + copy_items.size(),
+                       f32 ? "16x16x4 f32" : tin == DT_BF16 ? "16x16x32 bf16" : "16x16x32 f16", (long long)mS.Z, (long long)mS.M, (long long)mS.N, 16 * qt, waves);
+  } else {
+    rk.source = std::string(hip_prelude()) + cfg + kAttentionTemplate;
+    rk.launch.grid[0] = (unsigned)((mS.M / 128) * mS.Z);
+    rk.launch.block[0] = 256;
+    rk.strategy = strf("fused attention (%zu kernels): mfma 32x32x16 %s Z=%lld M=%lld N=%lld D=64, %s", all.size() + copy_items.size(),
+                       tin == DT_BF16 ? "bf16" : "f16", (long long)mS.Z, (long long)mS.M, (long long)mS.N,
+                       cfg.find("#define POLY_FA_ONLINE 1") != std::string::npos ? "one pass, online softmax" : "two passes over keys, exact roundings");
+    if (mask_table) rk.strategy += ", mask tiles classified by a first kernel";
+    if (out->key_bounds.used) rk.strategy += ", products of masked key blocks bounded by the block maxima the keys' product leaves";
+  }
+  if (matmul_tuning_enabled() && !rows_form) {
     // the register budget (waves per SIMD) changes the schedule of the instructions, not
     // one value: candidates of the search that POLY_BEAM switches on
     rk.variants.push_back({"default", rk.source, rk.strategy, rk.launch});

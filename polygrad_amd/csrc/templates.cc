@@ -174,7 +174,7 @@ static bool reject(int line) {
 
 }  // namespace
 
-bool match_matmul(const KernelGraph &g, MatmulMatch *mm, int *reject_line) {
+bool match_matmul(const KernelGraph &g, MatmulMatch *mm, int *reject_line, int64_t min_depth) {
 #define MM_REJECT() do { if (reject_line) *reject_line = __LINE__; return false; } while (0)
   if (g.stores.size() != 1 || g.reduces.size() != 1 || !g.vars.empty()) MM_REJECT();
   const StoreInfo &st = g.stores[0];
@@ -191,7 +191,7 @@ bool match_matmul(const KernelGraph &g, MatmulMatch *mm, int *reject_line) {
     if (e <= 0 || K > 2147483647LL / e) MM_REJECT();
     K *= e;
   }
-  if (K < 8) MM_REJECT();
+  if (K < min_depth) MM_REJECT();
   const KNode &mul = g.n(R.src[0]);
   if (mul.op != POLY_OP_MUL || mul.dt != DT_F32) MM_REJECT();
   Operand A, B;

@@ -35,7 +35,7 @@ struct MatmulMatch {
   int64_t a_c0 = 0, b_c0 = 0;   // constant parts of the operand indices
 };
 
-bool match_matmul(const KernelGraph &g, MatmulMatch *mm, int *reject_line);
+bool match_matmul(const KernelGraph &g, MatmulMatch *mm, int *reject_line, int64_t min_depth = 8);
 
 // C text that splits the flattened coordinates `m`, `n`, `z` (ints in scope) into the
 // kernel's END ranges, declared as `const int r<ord>`; binds them in `em` when given.
