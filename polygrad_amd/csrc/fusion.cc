@@ -787,7 +787,9 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
     *red = g.reduces[0];
     *ord = g.range_ord.at(R.src[1]);
     for (int r : g.stores[0].ranges) if (g.ranges[(size_t)r].extent < 0 || r == *ord) return false;
-    return g.ranges[(size_t)*ord].extent >= 128;
+    // (rows shorter than a wave: lanes idle, but three launches of a chain of four go; softmax
+    // of 65536 x 33: 28.8 -> 12.8 us, of 4 x 8: 16.0 -> 6.9)
+    return g.ranges[(size_t)*ord].extent >= (allow_rows && !getenv("POLY_HIP_NO_ROW_CHAIN_SIZES") ? 8 : 128);
   };
   RowPhase A;
   if (!reduce_shape(gA, &A.red, &A.own_red_ord)) return false;
@@ -1013,6 +1015,27 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
         if ((double)s->buf_slots[sc.slot(it, (int)(&p - &sc.graphs[(size_t)it].params[0]))].numel >= rows * (double)R) maxsz = std::max(maxsz, dt_size(p.dt));
     if (maxsz == 2) G = 32;
   }
+  // A chain that keeps rows between its phases holds a row whole, one read and one write of
+  // memory: up to kept_values elements a lane, on as many lanes as that takes.  Odd rows are
+  // kept as single elements (a wave reads 256 consecutive bytes either way).  One launch for
+  // three or four: LayerNorm of 4097 x 1001 32.4 -> 11.4 us (5.8 TB/s), 2256 x 25472 462 -> 161,
+  // 8000 x 8193 443 -> 183; softmax of 127 x 10278 22.1 -> 7.1, 38497 x 614 148 -> 66.
+  // kept_values: what leaves the compiler registers for the loads in flight; 64 lanes x 16 and
+  // 256 x 32 keep four and two rows to a CU's SIMDs, 1024 x 52 is as far as it goes (above 45
+  // it spills some, and 1300 x 50257 still takes 341 us against 554 in three launches).
+  bool keeps_rows = false;
+  for (const RowPhase &p : phases) keeps_rows = keeps_rows || p.keeps_row;
+  if (getenv("POLY_HIP_NO_ROW_CHAIN_SIZES")) keeps_rows = false;
+  auto kept_values = [](int lanes) { return lanes <= 64 ? 16 : lanes == 256 ? 32 : 52; };
+  if (R <= 32) G = 32;
+  else if (keeps_rows) {
+    const bool wide = R % 8 == 0 && std::all_of(items.begin(), items.end(), [&](int it) {      // 16 bytes of 16-bit elements a lane
+      for (const auto &p : sc.graphs[(size_t)it].params) if (dt_size(p.dt) > 2 && (double)s->buf_slots[sc.slot(it, (int)(&p - &sc.graphs[(size_t)it].params[0]))].numel >= rows * (double)R) return false;
+      return true;
+    });
+    if (!wide && G == 64 && R > 64 * kept_values(64)) G = 256;
+    if (!wide && G == 256 && R > 256 * kept_values(256)) G = 1024;
+  }
   std::vector<int> arg_slots;
   arg_slots.push_back(out_slot);
   for (int sl : inputs) arg_slots.push_back(sl);
@@ -1132,7 +1155,7 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
       if (!reads_row && V >= 8 && G == 64 && R % ((int64_t)G * V) != 0 && R % ((int64_t)G * V / 2) == 0) V /= 2;
       // long rows of an extent that is no multiple of the vector width (a vocabulary of
       // 50257): vector accesses at element alignment and a scalar tail
-      if (V == 1 && !reads_row && !ph.keeps_row && !getenv("POLY_HIP_NO_RAGGED_VEC")) {
+      if (V == 1 && !reads_row && !keeps_rows && !getenv("POLY_HIP_NO_RAGGED_VEC")) {
         int vr = std::max(1, 16 / maxsz);
         while (vr > 1 && R < (int64_t)G * vr * 16) vr /= 2;
         if (vr > 1) { V = vr; ragged = true; }
@@ -1154,12 +1177,12 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
     std::vector<int> pres;
     const int nit = (int)((R + (int64_t)G * V - 1) / ((int64_t)G * V));
     // iterations as an unrolled loop over `it` (what is kept between phases is indexed by it)
-    const bool unrolled = (G <= 64 && nit <= 4) || (G == 256 && nit <= 8);
+    const bool unrolled = (G <= 64 && nit <= 4) || (G == 256 && nit <= 8) || (keeps_rows && nit * V <= kept_values(G));
     if (!unrolled) n_walked_phases++;
     {
       bool reads_row = false;
       for (auto &kv : ph.m.preset) if (kv.second.find("[it]") != std::string::npos) reads_row = true;
-      if ((reads_row || ph.keeps_row) && (!unrolled || V <= 1)) FA_REJECT();
+      if ((reads_row || ph.keeps_row) && (!unrolled || (V <= 1 && !keeps_rows))) FA_REJECT();
       if (reads_row && nit != row_nit) FA_REJECT();
       if (ph.keeps_row) {
         if (row_V && (row_V != V || row_nit != nit)) FA_REJECT();
@@ -1184,7 +1207,7 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
       return strf("(c%zu[it] = %s)", cache.size() - 1, ld.c_str());
     };
     if (ragged && unrolled) FA_REJECT();
-    if (V > 1) pres = hoist_vector_loads(g, em, roots, own_f, V, fv + "_0", &L, unrolled ? &keep : nullptr, ragged);
+    if (V > 1 || (unrolled && keeps_rows)) pres = hoist_vector_loads(g, em, roots, own_f, V, fv + "_0", &L, unrolled ? &keep : nullptr, ragged);
     // the row loop: positions fv_0 = lane * V, + G * V, ...
     // q: position in the row; the phase's own variable starts there (or, for a flat phase,
     // at the row's first element plus q)
@@ -1235,12 +1258,19 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
       if (ragged)
         loop += ragged_tail(Rn.src[0], [&](Scope *, const std::string &v2) { return strf("    acc = %s;\n", Emitter::reduce_combine(op, Rn.dt, "acc", v2).c_str()); });
       loop += strf("  acc = %s;\n", wave_reduce_call(op, Rn.dt, "acc", G == 32 ? 32 : 64).c_str());
-      if (G == 256) {
-        loop += strf("  __shared__ %s red[4];\n  __syncthreads();\n  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;\n  __syncthreads();\n",
-                     dt_cname(Rn.dt));
-        std::string e = "red[0]";
-        for (int w = 1; w < 4; w++) e = Emitter::reduce_combine(op, Rn.dt, e, strf("red[%d]", w));
-        loop += strf("  acc = %s;\n", e.c_str());
+      if (G >= 256) {
+        loop += strf("  __shared__ %s red[%d];\n  __syncthreads();\n  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;\n  __syncthreads();\n",
+                     dt_cname(Rn.dt), G / 64);
+        // (sixteen waves pairwise: one after the other the last additions, of nearly whole sums,
+        // would round twice as often as those of four waves do)
+        std::vector<std::string> e;
+        for (int w = 0; w < G / 64; w++) e.push_back(strf("red[%d]", w));
+        while (e.size() > 4) {
+          for (size_t w = 0; w < e.size() / 2; w++) e[w] = Emitter::reduce_combine(op, Rn.dt, e[2 * w], e[2 * w + 1]);
+          e.resize(e.size() / 2);
+        }
+        for (size_t w = 1; w < e.size(); w++) e[0] = Emitter::reduce_combine(op, Rn.dt, e[0], e[w]);
+        loop += strf("  acc = %s;\n", e[0].c_str());
       }
       for (int n : pres) em.clear_preset(n);
       em.preset(ph.red, "acc");
@@ -1347,7 +1377,7 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
     b += calls + "  }\n}\n";
     return b;
   };
-  const std::string body = body_for(256);
+  const std::string body = body_for(std::max(256, G));
 
   out->items = items;
   out->launch_item = last_item;
@@ -1357,8 +1387,8 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
   rk = RenderedKernel();
   rk.source = std::string(hip_prelude()) + code + body;
   rk.entry = "poly_k";
-  rk.launch.grid[0] = (unsigned)(G == 256 ? rows : G == 32 ? std::ceil(rows / 8) : std::ceil(rows / 4));
-  rk.launch.block[0] = 256;
+  rk.launch.grid[0] = (unsigned)(G >= 256 ? rows : G == 32 ? std::ceil(rows / 8) : std::ceil(rows / 4));
+  rk.launch.block[0] = (unsigned)std::max(256, G);
   rk.klass = KernelClass::ROW_REDUCE;
   rk.strategy = strf("row chain of %zu kernels (%s) G=%d R=%lld rows=%.0f", phases.size(), strat.c_str(), G, (long long)R, rows);
   if (n_cached_uses) rk.strategy += strf(", %d row loads kept in registers", n_cached_uses);
@@ -1381,7 +1411,7 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
   // workgroup, more workgroups).  Which lanes add which elements of a row, and in what
   // order, stays as it is -- the width of a row's group of lanes and of its loads would
   // change that, so they are not candidates.
-  if (matmul_tuning_enabled() && G != 256) {
+  if (matmul_tuning_enabled() && G < 256) {
     rk.variants.push_back({"default", rk.source, rk.strategy, rk.launch});
     for (int threads : {128, 64}) {
       LaunchSpec ls = rk.launch;
