@@ -1661,7 +1661,14 @@ bool try_render_matmul_generic(const KernelGraph &g, const std::string &fn, cons
     // (two pieces, hi + lo, leave an error below 2^-17 |x|: enough where the result is
     // stored as a 16-bit float, whose own rounding is 2^-9 or 2^-12 of it)
     const int pieces = ep.out_16bit && !getenv("POLY_HIP_SPLIT_THREE") ? 2 : 3;
-    const int parts[2] = {exact16(0) ? 1 : pieces, exact16(1) ? 1 : pieces};
+    // two fp16 values cast to fp32 are a plane of fp16 each, for the fp16 MFMA (one beside
+    // another operand is cut into bf16 pieces like any fp32 value)
+    auto half = [&](int side) {
+      const KNode &k = g.n(opnd[side]);
+      return k.op == POLY_OP_CAST && k.dt == DT_F32 && g.n(k.src[0]).dt == DT_F16;
+    };
+    const DT plane_dt = half(0) && half(1) && !getenv("POLY_HIP_NO_F16_PLANES") ? DT_F16 : DT_BF16;
+    const int parts[2] = {plane_dt == DT_F16 || exact16(0) ? 1 : pieces, plane_dt == DT_F16 || exact16(1) ? 1 : pieces};
     const int P = std::max(parts[0], parts[1]);
     const int64_t KP = (K + 63) / 64 * 64;
     const double elems_a = (double)Z * (double)M * parts[0] * (double)KP, elems_b = (double)Z * (double)N * parts[1] * (double)KP;
@@ -1695,7 +1702,7 @@ bool try_render_matmul_generic(const KernelGraph &g, const std::string &fn, cons
         // 16-bit buffer it is, at the same element indices)
         const bool narrow = kind[side] == 2;
         if (parts[side] != 1 || K % 64 != 0 || kr.size() > 2 || (side == 0 && shared)) continue;
-        if (!match_operand(g, opnd[side], &ip.op) || ip.op.dt != (narrow ? DT_F32 : DT_BF16)) continue;
+        if (!match_operand(g, opnd[side], &ip.op) || ip.op.dt != (narrow ? DT_F32 : plane_dt)) continue;
         if (!narrow && kind[side] != 0) continue;
         const Lin &l = g.lins[(size_t)ip.op.lin];
         if (kr.size() == 1) {
@@ -1755,25 +1762,35 @@ bool try_render_matmul_generic(const KernelGraph &g, const std::string &fn, cons
         if (narrow) ip.op.dt = DT_BF16;
         ip.ok = ok;
       }
-      RenderedKernel::Pre pre[2];
-      for (int side = 0; side < 2; side++) {
-        const char *nm = side == 0 ? "a" : "b";
-        const int64_t rows = side == 0 ? M : N;
+      // (a launch that writes the planes of the operands that need them: one kernel for both)
+      const char *const plane_t = dt_cname(plane_dt);
+      auto plane_writer = [&](bool write_a, bool write_b) {
+        const bool write[2] = {write_a, write_b};
         std::string c2;
-        c2 += strf("#define POLY_SP_ROWS %lld\n#define POLY_SP_K %lld\n#define POLY_SP_KP %lld\n#define POLY_SP_Z %lld\n", (long long)rows, (long long)K,
-                   (long long)KP, (long long)Z);
-        c2 += strf("#define POLY_SP_PARTS %d\n#define POLY_SP_WALK_K %d\n#define POLY_SP_NRAW %d\n", parts[side], walk_k[side] ? 1 : 0, std::max(1, n_loads[side]));
-        c2 += strf("#define POLY_SIGNATURE %s, __bf16* poly_scratch\n", ep.signature.c_str());
+        c2 += strf("#define POLY_SP_T %s\n#define POLY_SP_K %lld\n#define POLY_SP_KP %lld\n#define POLY_SP_Z %lld\n", plane_t, (long long)K, (long long)KP, (long long)Z);
+        c2 += strf("#define POLY_SP_A %d\n#define POLY_SP_B %d\n", write_a ? 1 : 0, write_b ? 1 : 0);
+        c2 += strf("#define POLY_SIGNATURE %s, %s* poly_scratch\n", ep.signature.c_str(), plane_t);
         c2 += code;
-        c2 += strf("#define POLY_SP_LOAD(row, k, z, raw) poly_%s_load(row, k, z, raw, %s)\n#define POLY_SP_MATH(row, k, z, raw) poly_%s_math(row, k, z, raw, %s)\n",
-                   nm, params_call.c_str(), nm, params_call.c_str());
-        c2 += strf("#define POLY_SP_OUT ((__bf16*)((char*)poly_scratch + %zuull))\n", side == 0 ? (size_t)0 : off_b);
-        pre[side].source = std::string(hip_prelude()) + c2 + kOperandSplitTemplate;
-        pre[side].entry = "poly_k";
-        pre[side].launch.grid[0] = (unsigned)((KP / 64) * ((rows + 63) / 64));
-        pre[side].launch.grid[1] = (unsigned)Z;
-        pre[side].launch.block[0] = 256;
-      }
+        RenderedKernel::Pre pre;
+        int64_t tiles = 0;
+        for (int side = 0; side < 2; side++) {
+          if (!write[side]) continue;
+          const char *nm = side == 0 ? "a" : "b", *NM = side == 0 ? "A" : "B";
+          const int64_t rows = side == 0 ? M : N;
+          c2 += strf("#define POLY_SP_%s_ROWS %lld\n#define POLY_SP_%s_PARTS %d\n#define POLY_SP_%s_WALK_K %d\n#define POLY_SP_%s_NRAW %d\n", NM, (long long)rows, NM,
+                     parts[side], NM, walk_k[side] ? 1 : 0, NM, std::max(1, n_loads[side]));
+          c2 += strf("#define POLY_SP_%s_LOAD(row, k, z, raw) poly_%s_load(row, k, z, raw, %s)\n#define POLY_SP_%s_MATH(row, k, z, raw) poly_%s_math(row, k, z, raw, %s)\n",
+                     NM, nm, params_call.c_str(), NM, nm, params_call.c_str());
+          c2 += strf("#define POLY_SP_%s_OUT ((%s*)((char*)poly_scratch + %zuull))\n", NM, plane_t, side == 0 ? (size_t)0 : off_b);
+          tiles += (KP / 64) * ((rows + 63) / 64);
+        }
+        pre.source = std::string(hip_prelude()) + c2 + kOperandSplitTemplate;
+        pre.entry = "poly_k";
+        pre.launch.grid[0] = (unsigned)tiles;
+        pre.launch.grid[1] = (unsigned)Z;
+        pre.launch.block[0] = 256;
+        return pre;
+      };
       // the product of the planes, as the 16-bit template sees it (a second time with every
       // operand as planes if the template does not take an operand where it lies)
       for (int attempt = 0; attempt < 2; attempt++) {
@@ -1783,7 +1800,7 @@ bool try_render_matmul_generic(const KernelGraph &g, const std::string &fn, cons
       }
       MatmulMatch m2;
       m2.red = red; m2.K = P * KP; m2.M = M; m2.N = N; m2.Z = Z;
-      m2.A.dt = m2.B.dt = DT_BF16;
+      m2.A.dt = m2.B.dt = plane_dt;
       m2.ka = parts[0] == P ? KSplit{P * KP, 0, 1} : KSplit{KP, 0, 1};
       m2.kb = parts[1] == P ? KSplit{P * KP, 0, 1} : KSplit{KP, 0, 1};
       m2.md.push_back(Dim{-1, M, parts[0] * KP, 0, 1});
@@ -1824,23 +1841,23 @@ bool try_render_matmul_generic(const KernelGraph &g, const std::string &fn, cons
       }
       m2.md_full = mm.md_full; m2.nd_full = mm.nd_full; m2.zd_full = mm.zd_full;
       MatmulEpilogue ep2 = ep;
-      ep2.signature += ", __bf16* poly_scratch";
-      ep2.scratch_type = "__bf16";
+      ep2.signature += strf(", %s* poly_scratch", plane_t);
+      ep2.scratch_type = plane_t;
       const size_t planes_bytes = in_place[1].ok ? (in_place[0].ok ? (size_t)256 : std::max<size_t>(off_b, 256)) : scratch_bytes;
       ep2.scratch_used = planes_bytes;
-      ep2.a_ptr = "((const __bf16*)poly_scratch)";
-      ep2.b_ptr = strf("((const __bf16*)((const char*)poly_scratch + %zuull))", off_b);
+      ep2.a_ptr = strf("((const %s*)poly_scratch)", plane_t);
+      ep2.b_ptr = strf("((const %s*)((const char*)poly_scratch + %zuull))", plane_t, off_b);
       if (in_place[0].ok) ep2.a_ptr = strf(kind[0] == 2 ? "((const __bf16*)data%d)" : "data%d", in_place[0].op.param);
       if (in_place[1].ok) ep2.b_ptr = strf(kind[1] == 2 ? "((const __bf16*)data%d)" : "data%d", in_place[1].op.param);
       RenderedKernel main;
       if (render_matmul(m2, ep2, &main)) {
         *out = main;
         // planes first, then a split product's first stage
-        if (!in_place[1].ok) out->pres.insert(out->pres.begin(), pre[1]);
-        if (!shared && !in_place[0].ok) out->pres.insert(out->pres.begin(), pre[0]);
+        const bool write_a = !shared && !in_place[0].ok, write_b = !in_place[1].ok;
+        if (write_a || write_b) out->pres.insert(out->pres.begin(), plane_writer(write_a, write_b));
         out->scratch_bytes = std::max(planes_bytes, main.scratch_bytes);
         out->flops = 2.0 * (double)M * (double)N * (double)K * (double)Z;
-        out->strategy = strf("operands as expressions, written as bf16 planes first (%d + %d planes of K=%lld, %.0f MB%s): ", parts[0], parts[1],
+        out->strategy = strf("operands as expressions, written as %s planes first (%d + %d planes of K=%lld, %.0f MB%s): ", plane_dt == DT_F16 ? "fp16" : "bf16", parts[0], parts[1],
                              (long long)KP, (double)planes_bytes / 1e6,
                              shared ? "; A is what the kernel before left as its A, rows and depth exchanged, and is not written again"
                              : in_place[0].ok && in_place[1].ok ? "; both read in place" : in_place[0].ok ? "; A read in place" : in_place[1].ok ? "; B read in place" : "") + out->strategy;
