@@ -36,7 +36,7 @@
 // loads: hence both operands in one launch, and for an operand of a single load all 16 of a
 // thread's loads in flight (four otherwise: the registers of what computes the value).
 // Measured, whole plan: bf16 1111x999x1501 27.3 us with a launch per operand and four loads in
-// flight, 21.3 so; 3001x2999x1003 53 -> 46.  fp16 operands as fp16 planes where they were one
+// flight, 21.3 so, 17.8 without launches that read the operands ahead; 3001x2999x1003 53 -> 46.  fp16 operands as fp16 planes where they were one
 // computed-operand product on the fp32 MFMA: 1111x999x1501 105 -> 25, 3001x2999x1003 411 -> 48.
 #ifdef POLY_TEMPLATE_STANDALONE
 #include <hip/hip_runtime.h>

@@ -1855,6 +1855,9 @@ bool try_render_matmul_generic(const KernelGraph &g, const std::string &fn, cons
         // planes first, then a split product's first stage
         const bool write_a = !shared && !in_place[0].ok, write_b = !in_place[1].ok;
         if (write_a || write_b) out->pres.insert(out->pres.begin(), plane_writer(write_a, write_b));
+        // (what writes the planes streams both operands once: a launch that reads them before it
+        // only costs its own time)
+        if (write_a && write_b) out->reads_b_ahead = true;
         out->scratch_bytes = std::max(planes_bytes, main.scratch_bytes);
         out->flops = 2.0 * (double)M * (double)N * (double)K * (double)Z;
         out->strategy = strf("operands as expressions, written as %s planes first (%d + %d planes of K=%lld, %.0f MB%s): ", plane_dt == DT_F16 ? "fp16" : "bf16", parts[0], parts[1],
