@@ -1093,7 +1093,11 @@ static bool try_slice_reduce(const KernelGraph &g, const std::string &fn_name, c
     if (!gen.run(&plain, &err) || plain.klass != KernelClass::THREAD_REDUCE) return false;
   }
   int parts = 1;
-  while (parts < 128 && rows * parts < 65536.0 && (int64_t)parts * 8 <= g.ranges[(size_t)longest].extent) parts *= 2;
+  // (64 Ki threads, and up to four times as many where each still has 32 terms or more: a
+  // thread's loads come one after another, and more of them in flight on a CU is what helps:
+  // 5120 sums of 4096 terms 17.0 us in 16 parts, 9.2 in 64)
+  const int64_t terms = g.ranges[(size_t)longest].extent;
+  while (parts < 128 && ((rows * parts < 65536.0 && (int64_t)parts * 8 <= terms) || (rows * parts < 262144.0 && (int64_t)parts * 64 <= terms))) parts *= 2;
   if (parts < 4) return false;
   return split_in_two(g, fn_name, opt, T, top, rows, (double)parts, longest, parts, out);
 }
