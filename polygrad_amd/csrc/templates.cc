@@ -668,14 +668,10 @@ static void f32_variants(int64_t M, int64_t N, const F32Shape &chosen, const std
 //           (7473x219x188: 6.9 [17.7]; 410x7104x318: 13.5 [39.1]; 3001x2999x1003: 86 [53])
 //   fp32    up to 640 tiles of 32x64 (12x768x3072: 8.1 us [265]; 128x3072x768: 10.1 [22.3];
 //           1024^3: 21.6 [30.2]; 4096x512x784, 1024 tiles: 50.1 [38.9])
-//   From a depth of 8192 (16-bit) or 4608 (fp32) on, products of more than 64 rows and
+//   From a depth of 4096 (fp32) or 8192 (16-bit) on, products of more than 64 rows and
 //   columns are left to the templates that deal the depth to several workgroups, which add
-//   up in a second kernel; of fewer, and in fp32 from 4096 on, that is done here
-//   (100x50x4096 fp32: 5.6 us dealt to eight, 9.5 to one [277]; 40x700x5000: 13.2 to two
-//   [380]; 512x784x4096: 38.8 on 64x64 tiles dealt to two, whose 208 workgroups are one
-//   round, 56.5 on 32x64 tiles of 8 waves, 58.8 dealt to four [68.7]).  A sum then runs over
-//   an eighth of the depth, no more than in the other template up to a depth of 4608, from
-//   where that may deal it to nine parts.
+//   up in a second kernel; of fewer, that is done here (100x50x4096 fp32: 5.6 us dealt to
+//   eight, 9.5 to one [277]; 40x700x5000: 13.2 to two [380]).
 // The smallest tile that does not need more workgroups than the chip runs at once: few rows
 // want many narrow workgroups (128x768x768 fp32: 16x32 4.9 us, 32x64 9.8), many rows tiles
 // that read each operand fewer times.
@@ -695,16 +691,9 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
     else f = Form{2, 4, 4, 6};
     if (tiles_of(2, 4) > 256 && tiles_of(4, 4) <= 256 && M >= 64 && N >= 64) f = Form{4, 4, 4, 6};
     if (K >= 4096) {
-      auto share = [&]() { for (S = 8; S > 1 && (K % (S * kv) != 0 || tiles_of(f.tm, f.tn) * S > 256);) S /= 2; };
+      if (M > 64 && N > 64) return false;
       f = tiles_of(1, 1) <= 64 ? Form{1, 1, 8, 6} : Form{1, 2, 4, 6};
-      if (M > 64 && N > 64) {
-        if (K >= 4608 || tiles_of(2, 4) > 256) return false;
-        f = Form{4, 4, 4, 4};
-        share();
-        // (four waves and no second workgroup: a quarter of the depth in one sum)
-        if (S == 1 || tiles_of(4, 4) < 64) f = Form{2, 4, 8, 6};
-      }
-      share();
+      for (S = 8; S > 1 && (K % (S * kv) != 0 || tiles_of(f.tm, f.tn) * S > 256);) S /= 2;
     }
   } else {
     const bool few = M <= 16 || N <= 16 || tiles_of(4, 4) <= 64;

@@ -20,7 +20,7 @@ import cases  # noqa: E402
 EDGES = [(12, 33, 8, "bfloat16", "nn"), (16, 32, 256, "bfloat16", "nn"), (17, 31, 255, "bfloat16", "nt"), (12, 770, 1000, "bfloat16", "nn"),
          (65, 63, 777, "bfloat16", "tn"), (37, 1280, 291, "float16", "nn"), (333, 219, 188, "bfloat16", "nn"), (900, 1410, 70, "bfloat16", "tn"),
          (1500, 1283, 101, "bfloat16", "nt"), (2, 5, 9, "float32", "nn"), (15, 16, 128, "float32", "nt"), (143, 40, 791, "float32", "nn"),
-         (33, 129, 784, "float32", "nt"), (200, 50, 4096, "float32", "tn"), (64, 700, 5000, "float32", "nn"), (200, 300, 4095, "float32", "tn"), (130, 770, 515, "float32", "nn"), (17, 96, 9000, "bfloat16", "nn"), (64, 96, 4100, "float32", "nn"), (130, 300, 4097, "float32", "nn"), (100, 66, 4604, "float32", "tn"), (384, 784, 4096, "float32", "tn"), (600, 650, 67, "float32", "nt")]
+         (33, 129, 784, "float32", "nt"), (200, 50, 4096, "float32", "tn"), (64, 700, 5000, "float32", "nn"), (200, 300, 4095, "float32", "tn"), (130, 770, 515, "float32", "nn"), (17, 96, 9000, "bfloat16", "nn"), (64, 96, 4100, "float32", "nn"), (600, 650, 67, "float32", "nt")]
 
 LDS_TILES = [(333, 840, 256, "bfloat16", "nn", "64x64x64"), (345, 768, 3072, "bfloat16", "nn", "64x64x64"), (1000, 904, 256, "bfloat16", "nt", "64x64x64"),
              (1000, 904, 320, "float16", "tn", "64x64x64"), (1111, 1000, 1536, "bfloat16", "nt", "64x128x64"), (1112, 1000, 256, "bfloat16", "tn", "64x128x64"),
