@@ -32,7 +32,7 @@
 // Measured against the tile templates (one launch, us): bf16 12 x 768 x 3072 31.0 -> 5.4,
 // 64 x 3072 x 768 12.5 -> 3.9, 7473 x 219 x 188 17.7 -> 6.9, 410 x 7104 x 318 39.1 -> 13.5;
 // fp32 128 x 3072 x 768 22.3 -> 10.1 (60 TFLOP/s of the 157 of the fp32 MFMAs),
-// 512 x 784 x 4096 69.0 -> 37.2, 33 x 129 x 784 30.6 -> 3.8.  What bounds it where there are
+// 33 x 129 x 784 30.6 -> 3.8.  What bounds it where there are
 // many rows is the address path: 16 lanes of a load along K read 16 different rows, 64 bytes
 // of each (1035 x 768 x 3072 takes 20 us where tiles in LDS take 12).
 #ifdef POLY_TEMPLATE_STANDALONE
