@@ -601,6 +601,9 @@ extern "C" __global__ void __launch_bounds__(256) poly_k(POLY_SIGNATURE) {
   float acc = part[gid];
 #pragma unroll
   for (int s = 1; s < POLY_KSPLIT; s++) acc += part[(size_t)s * POLY_Z * POLY_M * POLY_N + gid];
+#ifdef POLY_EP_MID_VALUE
+  *POLY_EP_MID_PTR(m, n, z) = POLY_EP_MID_VALUE(acc, m, n, z);
+#endif
   POLY_EPILOGUE(acc, m, n, z);
 }
 )HIP";
@@ -736,10 +739,12 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
   cfg += matmul_k_fn("poly_a_k", mm.ka, K) + matmul_k_fn("poly_b_k", mm.kb, K);
   const std::string shape = strf("#define POLY_SIGNATURE %s%s\n#define POLY_KSPLIT %d\n#define POLY_PARTIALS poly_scratch\n", ep.signature.c_str(), S > 1 ? ", float* poly_scratch" : "", S) + ep.code;
   cfg += shape;
+  // what the kernel that has an element's whole sum does with it
+  std::string finish = strf("#define POLY_EPILOGUE(acc, m, n, z) %s\n", ep.call.c_str());
+  if (!ep.mid_value_call.empty())
+    finish += strf("#define POLY_EP_MID_VALUE(acc, m, n, z) %s\n#define POLY_EP_MID_PTR(m, n, z) %s\n", ep.mid_value_call.c_str(), ep.mid_ptr_call.c_str());
   if (S > 1) cfg += "#define POLY_EPILOGUE(acc, m, n, z) POLY_PARTIALS[(((size_t)poly_ks * POLY_Z + (z)) * POLY_M + (m)) * POLY_N + (n)] = (acc)\n";
-  else cfg += strf("#define POLY_EPILOGUE(acc, m, n, z) %s\n", ep.call.c_str());
-  if (S == 1 && !ep.mid_value_call.empty())
-    cfg += strf("#define POLY_EP_MID_VALUE(acc, m, n, z) %s\n#define POLY_EP_MID_PTR(m, n, z) %s\n", ep.mid_value_call.c_str(), ep.mid_ptr_call.c_str());
+  else cfg += finish;
   *out = RenderedKernel();
   out->source = std::string(hip_prelude()) + cfg + kMatmulWaveTemplate;
   out->entry = "poly_k";
@@ -751,7 +756,7 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
     out->pres.push_back({out->source, out->entry, out->launch});
     out->scratch_bytes = (size_t)S * (size_t)Z * (size_t)M * (size_t)N * sizeof(float);
     out->source = std::string(hip_prelude()) + strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_Z %lld\n", (long long)M, (long long)N, (long long)Z) + shape +
-                  strf("#define POLY_EPILOGUE(acc, m, n, z) %s\n", ep.call.c_str()) + kSplitKCombine;
+                  finish + kSplitKCombine;
     out->launch = LaunchSpec();
     out->launch.grid[0] = (unsigned)(((double)Z * M * N + 255) / 256);
     out->launch.block[0] = 256;
