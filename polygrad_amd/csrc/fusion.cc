@@ -1868,16 +1868,16 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
   std::string cfg;
   bool failed = false;
   // one device function per kernel of the group: value of `node` with the member's presets
-  // The softmax terms use the bare exp2 instruction: a term below 2^-126 of the row's
-  // largest (which is exactly 1, so the sum is at least 1) cannot change the fp32 sum, and
-  // the probability it would give is below the smallest normal 16-bit float.
-  // (fp32 probabilities have that range, and keep the exp2 of the unfused kernels.)
+  // The softmax terms use the bare exp2 instruction, which gives 0 below 2^-126: such a term of
+  // a row whose largest is exactly 1 cannot change the fp32 sum, and the probability it would
+  // give is 0 in fp16 and below the smallest normal bf16.  bf16 and fp32 have probabilities
+  // there, if subnormal ones: where the kernels would run unfused otherwise, their exp2 stays.
   const bool online = !rows_form && p_is_term_over_sum && !getenv("POLY_HIP_EXACT_ATTENTION");
   auto value_fn = [&](const Member &m, const char *name, const char *ret, const char *lead_args, int node,
                       const std::map<int, std::string> &extra_preset) {
     const KernelGraph &g = sc.graphs[(size_t)m.item];
     Emitter em(g);
-    em.raw_exp2 = !f32 && (m.item == i_sum || m.item == i_p);
+    em.raw_exp2 = (tin == DT_F16 || (tin == DT_BF16 && whole_blocks)) && (m.item == i_sum || m.item == i_p);
     em.pow2_mul16_exact = online;
     Scope S0;
     S0.indent = 1;

@@ -5,7 +5,9 @@
 // normalise, P V) where that template's blocks of 128 queries x 64 keys do not divide the
 // problem, and for fp32 operands.  Every rounding step of the unfused kernels is kept: the
 // score as the chain stores it, the term, the probability cast to the operand type before
-// the second product; only the order of the sums differs.  The renderer prepends:
+// the second product.  What differs is the order of the sums, that a term times the sum's
+// reciprocal is divided by the sum, and, for the bf16 shapes that attention_mfma.hip could
+// take, that a term below 2^-126 is 0 as it is there.  The renderer prepends:
 //
 //   POLY_TIN, POLY_F32                 operand type, and 1 when it is float
 //   POLY_MFMA(a, b, c)                 the 16x16x32 MFMA of a 16-bit type (fp32: 16x16x4)
