@@ -10,6 +10,8 @@
 //   POLY_WAVES          waves of a workgroup: each has the whole tile and every
 //                       POLY_WAVES-th step of the depth
 //   POLY_DEPTH          steps of a wave whose loads are in flight at a time
+//   POLY_SUMS           (optional) 2: a wave adds its even and its odd steps up apart, and the
+//                       two at the end (POLY_DEPTH is even)
 //   POLY_KSPLIT         (optional) workgroups that share the depth of a tile (blockIdx.y =
 //                       z * POLY_KSPLIT + part): each leaves its sum where POLY_EPILOGUE puts
 //                       it, which may use `poly_ks`, the part
@@ -81,6 +83,9 @@ typedef unsigned int poly_u32x4 __attribute__((ext_vector_type(4)));
 #define POLY_KSPLIT 1
 #endif
 #define POLY_KPART (POLY_K / POLY_KSPLIT)   // depth of one workgroup
+#ifndef POLY_SUMS
+#define POLY_SUMS 1
+#endif
 #define POLY_BM (16 * POLY_TM)
 #define POLY_BN (16 * POLY_TN)
 
@@ -186,12 +191,14 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
   auto ka = [&](int k) { return poly_a_k(k_base + k); };
   auto kb = [&](int k) { return poly_b_k(k_base + k); };
 
-  poly_f32x4 acc[POLY_TM][POLY_TN];
+  poly_f32x4 sums[POLY_SUMS][POLY_TM][POLY_TN];
 #pragma unroll
-  for (int i = 0; i < POLY_TM; i++)
+  for (int s = 0; s < POLY_SUMS; s++)
 #pragma unroll
-    for (int j = 0; j < POLY_TN; j++) acc[i][j] = poly_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  auto multiply = [&](const OpA &a, const OpB &b) {
+    for (int i = 0; i < POLY_TM; i++)
+#pragma unroll
+      for (int j = 0; j < POLY_TN; j++) sums[s][i][j] = poly_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto multiply = [&](const OpA &a, const OpB &b, poly_f32x4 (&acc)[POLY_TM][POLY_TN]) {
 #if POLY_F32
 #pragma unroll
     for (int e = 0; e < POLY_KV; e++)
@@ -241,13 +248,21 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
 #pragma unroll 1
   for (int s = 0; s < STEADY; s += D) {
 #pragma unroll
-    for (int d = 0; d < D; d++) { multiply(ra[d], rb[d]); load(d, s + d + D); }
+    for (int d = 0; d < D; d++) { multiply(ra[d], rb[d], sums[d % POLY_SUMS]); load(d, s + d + D); }
   }
 #pragma unroll
   for (int s = STEADY; s < ALL; s++) {
-    multiply(ra[s % D], rb[s % D]);
+    multiply(ra[s % D], rb[s % D], sums[s % POLY_SUMS]);
     if (s + D < ALL) load(s % D, s + D);
   }
+  static_assert(D % POLY_SUMS == 0, "a step of the unrolled loop has its sum");
+  poly_f32x4 (&acc)[POLY_TM][POLY_TN] = sums[0];
+#if POLY_SUMS == 2
+#pragma unroll
+  for (int i = 0; i < POLY_TM; i++)
+#pragma unroll
+    for (int j = 0; j < POLY_TN; j++) acc[i][j] += sums[1][i][j];
+#endif
 
   // The partial tiles of the waves, CH blocks of rows at a time, in LDS as the MFMA leaves
   // them (lane l, register r: row 4 (l / 16) + r, column l % 16 of a block): rows 20 floats

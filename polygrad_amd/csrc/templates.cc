@@ -711,6 +711,11 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
     if (sscanf(ov, "%d,%d,%d,%d,%d", &f.tm, &f.tn, &f.waves, &f.depth, &S) < 4) return false;
   }
   if (S > 1 && (K % (S * kv) != 0 || !ep.scratch_type.empty() || Z * S > 65535)) S = 1;
+  // From a depth of 2048 on the fp32 tile template deals it to as many as seven workgroups: no
+  // fewer partial sums here, or the sums get less exact (128x768x3072 against float64: 4.97e-7 with
+  // four, 4.07e-7 there with six, 3.55e-7 with the eight of two sums a wave, whose time is within
+  // 2 %).
+  const int sums = f32 && K >= 2048 && f.waves * S < 8 && f.depth % 2 == 0 ? 2 : 1;
   // an operand is read along K where its steps are contiguous there, along its rows otherwise
   // (runs of as many rows as the tile has blocks)
   auto layout = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a, int64_t rows, int run, bool *kc) {
@@ -727,7 +732,7 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
   if (!f32) cfg += strf("#define POLY_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_%s(a, b, c, 0, 0, 0)\n", mm.A.dt == DT_BF16 ? "bf16" : "f16");
   else cfg += "#define POLY_MFMA(a, b, c) (c)\n";
   cfg += strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_K %lld\n#define POLY_Z %lld\n", (long long)M, (long long)N, (long long)K, (long long)Z);
-  cfg += strf("#define POLY_TM %d\n#define POLY_TN %d\n#define POLY_WAVES %d\n#define POLY_DEPTH %d\n", f.tm, f.tn, f.waves, f.depth);
+  cfg += strf("#define POLY_TM %d\n#define POLY_TN %d\n#define POLY_WAVES %d\n#define POLY_DEPTH %d\n#define POLY_SUMS %d\n", f.tm, f.tn, f.waves, f.depth, sums);
   cfg += strf("#define POLY_A_KC %d\n#define POLY_B_KC %d\n#define POLY_A_PTR %s\n#define POLY_B_PTR %s\n", a_kc ? 1 : 0, b_kc ? 1 : 0, ep.a_ptr.c_str(), ep.b_ptr.c_str());
   cfg += offset_fn("poly_a_row", mm.md, true, 0) + offset_fn("poly_b_row", mm.nd, false, 0);
   if (mm.zd.empty()) {
@@ -763,8 +768,8 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
   }
   out->klass = KernelClass::MATMUL_MFMA;
   out->reads_b_ahead = true;
-  out->strategy = strf("mfma %s M=%lld N=%lld K=%lld Z=%lld tile %dx%d, depth dealt to %d waves, A:%s B:%s", f32 ? "16x16x4 f32" : mm.A.dt == DT_BF16 ? "16x16x32 bf16" : "16x16x32 f16",
-                       (long long)M, (long long)N, (long long)K, (long long)Z, 16 * f.tm, 16 * f.tn, f.waves, a_kc ? "k-major" : "m-major", b_kc ? "k-major" : "n-major");
+  out->strategy = strf("mfma %s M=%lld N=%lld K=%lld Z=%lld tile %dx%d, depth dealt to %d waves%s, A:%s B:%s", f32 ? "16x16x4 f32" : mm.A.dt == DT_BF16 ? "16x16x32 bf16" : "16x16x32 f16",
+                       (long long)M, (long long)N, (long long)K, (long long)Z, 16 * f.tm, 16 * f.tn, f.waves, sums == 2 ? " of two sums each" : "", a_kc ? "k-major" : "m-major", b_kc ? "k-major" : "n-major");
   if (S > 1) out->strategy += strf(", K dealt to %d workgroups per tile, partial results added by a second kernel", S);
   out->n_params = ep.n_params;
   out->n_vars = 0;
