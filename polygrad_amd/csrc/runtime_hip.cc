@@ -21,6 +21,7 @@
 #include <fstream>
 #include <map>
 #include <memory>
+#include <mutex>
 
 namespace polyhip {
 
@@ -206,6 +207,28 @@ int runtime_sync() {
   return check(hipStreamSynchronize(rt().stream), "hipStreamSynchronize") ? 0 : -1;
 }
 
+// Events between calls of runtime_order_after: as many as there have been calls at one time.
+static std::mutex events_lock;
+static std::vector<hipEvent_t> idle_events;
+
+static hipEvent_t take_event() {
+  {
+    std::lock_guard<std::mutex> hold(events_lock);
+    if (!idle_events.empty()) {
+      hipEvent_t e = idle_events.back();
+      idle_events.pop_back();
+      return e;
+    }
+  }
+  hipEvent_t e = nullptr;
+  return check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate") ? e : nullptr;
+}
+
+static void give_back(hipEvent_t e) {
+  std::lock_guard<std::mutex> hold(events_lock);
+  idle_events.push_back(e);
+}
+
 int runtime_order_after(void *stream) {
   if (runtime_init() != 0) return -1;
   hipStream_t other = (hipStream_t)stream;
@@ -219,11 +242,11 @@ int runtime_order_after(void *stream) {
     if (e != hipErrorNotReady) return check(e, "hipStreamQuery") ? 0 : -1;
     (void)hipGetLastError();
   }
-  // (one event per thread and device context is enough: a wait takes the record that was the
-  // latest when it was enqueued)
-  static thread_local hipEvent_t event = nullptr;
-  if (!event && !check(hipEventCreateWithFlags(&event, hipEventDisableTiming), "hipEventCreate")) { event = nullptr; return -1; }
-  return check(hipEventRecord(event, other), "hipEventRecord") && check(hipStreamWaitEvent(rt().stream, event, 0), "hipStreamWaitEvent") ? 0 : -1;
+  hipEvent_t event = take_event();
+  if (!event) return -1;
+  const bool ok = check(hipEventRecord(event, other), "hipEventRecord") && check(hipStreamWaitEvent(rt().stream, event, 0), "hipStreamWaitEvent");
+  give_back(event);      // (a wait takes the record that was the latest when it was enqueued)
+  return ok ? 0 : -1;
 }
 
 struct Program {
