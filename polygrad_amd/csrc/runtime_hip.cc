@@ -207,31 +207,43 @@ int runtime_sync() {
   return check(hipStreamSynchronize(rt().stream), "hipStreamSynchronize") ? 0 : -1;
 }
 
-// Events between calls of runtime_order_after: as many as there have been calls at one time.
-static std::mutex events_lock;
-static std::vector<hipEvent_t> idle_events;
+// Makes `device` the calling thread's for as long as it lives.
+struct OnDevice {
+  int before = -1;
+  explicit OnDevice(int device) {
+    if (hipGetDevice(&before) != hipSuccess || before == device || !check(hipSetDevice(device), "hipSetDevice")) before = -1;
+  }
+  ~OnDevice() { if (before >= 0) (void)hipSetDevice(before); }
+};
 
-static hipEvent_t take_event() {
+// Events between calls of runtime_order_after, by device: as many as there have been calls at one time.
+static std::mutex events_lock;
+static std::map<int, std::vector<hipEvent_t>> idle_events;
+
+static hipEvent_t take_event(int device) {
   {
     std::lock_guard<std::mutex> hold(events_lock);
-    if (!idle_events.empty()) {
-      hipEvent_t e = idle_events.back();
-      idle_events.pop_back();
+    std::vector<hipEvent_t> &idle = idle_events[device];
+    if (!idle.empty()) {
+      hipEvent_t e = idle.back();
+      idle.pop_back();
       return e;
     }
   }
+  OnDevice on(device);
   hipEvent_t e = nullptr;
   return check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate") ? e : nullptr;
 }
 
-static void give_back(hipEvent_t e) {
+static void give_back(hipEvent_t e, int device) {
   std::lock_guard<std::mutex> hold(events_lock);
-  idle_events.push_back(e);
+  idle_events[device].push_back(e);
 }
 
 int runtime_order_after(void *stream) {
   if (runtime_init() != 0) return -1;
   hipStream_t other = (hipStream_t)stream;
+  OnDevice on(rt().device);      // (NULL is the default stream of the current device)
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (!check(hipStreamIsCapturing(other, &capturing), "hipStreamIsCapturing")) return -1;
   if (capturing == hipStreamCaptureStatusNone) {
@@ -242,10 +254,13 @@ int runtime_order_after(void *stream) {
     if (e != hipErrorNotReady) return check(e, "hipStreamQuery") ? 0 : -1;
     (void)hipGetLastError();
   }
-  hipEvent_t event = take_event();
+  // (an event can only be recorded on a stream of the device it was made on)
+  int device = rt().device;
+  if (other && !check(hipStreamGetDevice(other, &device), "hipStreamGetDevice")) return -1;
+  hipEvent_t event = take_event(device);
   if (!event) return -1;
   const bool ok = check(hipEventRecord(event, other), "hipEventRecord") && check(hipStreamWaitEvent(rt().stream, event, 0), "hipStreamWaitEvent");
-  give_back(event);      // (a wait takes the record that was the latest when it was enqueued)
+  give_back(event, device);      // (a wait takes the record that was the latest when it was enqueued)
   return ok ? 0 : -1;
 }
 
