@@ -220,8 +220,8 @@ struct OnDevice {
 static std::mutex events_lock;
 static std::map<int, std::vector<hipEvent_t>> idle_events;
 
-static hipEvent_t take_event(int device) {
-  {
+static hipEvent_t take_event(int device, bool kept_will_do) {
+  if (kept_will_do) {
     std::lock_guard<std::mutex> hold(events_lock);
     std::vector<hipEvent_t> &idle = idle_events[device];
     if (!idle.empty()) {
@@ -257,10 +257,13 @@ int runtime_order_after(void *stream) {
   // (an event can only be recorded on a stream of the device it was made on)
   int device = rt().device;
   if (other && !check(hipStreamGetDevice(other, &device), "hipStreamGetDevice")) return -1;
-  hipEvent_t event = take_event(device);
+  hipEvent_t event = take_event(device, capturing == hipStreamCaptureStatusNone);
   if (!event) return -1;
   const bool ok = check(hipEventRecord(event, other), "hipEventRecord") && check(hipStreamWaitEvent(rt().stream, event, 0), "hipStreamWaitEvent");
-  give_back(event, device);      // (a wait takes the record that was the latest when it was enqueued)
+  // A wait takes the record that was the latest when it was enqueued, so the event is free again
+  // -- unless a capture saw it, which would take whatever it is recorded on next for its own.
+  if (capturing == hipStreamCaptureStatusNone) give_back(event, device);
+  else (void)hipEventDestroy(event);
   return ok ? 0 : -1;
 }
 

@@ -1,7 +1,7 @@
 """The host side of poly_hip_order_after without a GPU: the runtime's own code against a HIP
 runtime that tests/runtime_order_main.cc acts out.  Events are kept per call in flight and not
-per thread, and belong to the device of the stream they are recorded on, whatever device the
-caller is on."""
+per thread, belong to the device of the stream they are recorded on whatever device the
+caller is on, and one that a capture has seen is not recorded on another stream."""
 import os
 import subprocess
 
@@ -23,7 +23,7 @@ def driver(tmp_path_factory):
 
 
 @pytest.mark.skipif(not os.path.exists(hostcheck.CLANG), reason="no host clang with AddressSanitizer")
-@pytest.mark.parametrize("what", ["threads", "device"])
+@pytest.mark.parametrize("what", ["threads", "device", "capture"])
 def test_order_after(driver, what):
     r = subprocess.run([driver, what], capture_output=True, text=True, timeout=60, env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"))
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr
