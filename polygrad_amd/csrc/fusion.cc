@@ -1529,7 +1529,7 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
   const StoreInfo &stS = gS.stores[0];
   const DT tin = mS.A.dt;
   const bool f32 = tin == DT_F32;
-  if (tin != DT_BF16 && tin != DT_F16 && !f32) FA_REJECT();
+  if (tin != DT_BF16 && tin != DT_F16 && (!f32 || getenv("POLY_HIP_NO_F32_MFMA"))) FA_REJECT();
   if (gS.n(stS.value).dt != tin) FA_REJECT();
   // Blocks of 128 queries and 64 keys of a 16-bit type: kernels/attention_mfma.hip.  What they
   // do not divide, and fp32: kernels/attention_rows.hip, which keeps the scores of its queries

@@ -682,6 +682,7 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
   const int64_t K = mm.K, M = mm.M, N = mm.N, Z = mm.Z;
   if (getenv("POLY_HIP_NO_WAVE_MM")) return false;
   const bool f32 = mm.A.dt == DT_F32;
+  if (f32 && getenv("POLY_HIP_NO_F32_MFMA")) return false;
   const int kv = f32 ? 4 : 8;
   auto tiles_of = [&](int tm, int tn) { return (double)((M + 16 * tm - 1) / (16 * tm)) * (double)((N + 16 * tn - 1) / (16 * tn)) * (double)Z; };
   struct Form { int tm, tn, waves, depth; };
