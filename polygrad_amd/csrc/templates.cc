@@ -711,7 +711,7 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
   if (const char *ov = measurement_env("POLY_HIP_MM_WAVE")) {   // "TM,TN,WAVES,DEPTH": tuning experiments
     if (sscanf(ov, "%d,%d,%d,%d,%d", &f.tm, &f.tn, &f.waves, &f.depth, &S) < 4) return false;
   }
-  if (S > 1 && (K % (S * kv) != 0 || !ep.scratch_type.empty() || Z * S > 65535)) S = 1;
+  if (S > 1 && (K % (S * kv) != 0 || !ep.scratch_type.empty() || Z * S > 65535 || getenv("POLY_HIP_NO_SPLIT_K"))) S = 1;
   // From a depth of 2048 on the fp32 tile template deals it to as many as seven workgroups: no
   // fewer partial sums here, or the sums get less exact (128x768x3072 against float64: 4.97e-7 with
   // four, 4.07e-7 there with six, 3.55e-7 with the eight of two sums a wave, whose time is within

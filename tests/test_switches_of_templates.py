@@ -1,5 +1,6 @@
 """Switches that take a mechanism away take it away from every template that has it:
-POLY_HIP_NO_F32_MFMA from fp32 products and fp32 attention."""
+POLY_HIP_NO_F32_MFMA from fp32 products and fp32 attention, POLY_HIP_NO_SPLIT_K from fp32
+products whose depth goes to several workgroups."""
 import ctypes as C
 
 import pytest
@@ -36,3 +37,11 @@ def test_no_f32_mfma_in_attention(hiplib, monkeypatch):
     monkeypatch.setenv("POLY_HIP_NO_F32_MFMA", "1")
     items, groups = _described(case, hiplib, monkeypatch)
     assert not any("POLY_FA_M" in g or "POLY_MFMA_F32" in g for g in groups) and not any("mfma" in i for i in items)
+
+
+@pytest.mark.parametrize("shape", [(32, 512, 4096), (300, 10, 8192)])
+def test_no_split_k(shape, hiplib, monkeypatch):
+    case = _case(*shape, "float32", "nn")
+    assert "K dealt to" in _described(case, hiplib, monkeypatch)[0][0]
+    monkeypatch.setenv("POLY_HIP_NO_SPLIT_K", "1")
+    assert "K dealt to" not in _described(case, hiplib, monkeypatch)[0][0]
