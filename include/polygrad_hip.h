@@ -179,7 +179,8 @@ int poly_hip_plan_profile(PolyHipPlan *plan, void **slot_data, int n_slots, floa
 char *poly_hip_plan_kernel_desc(const PolyHipPlan *plan, int k);
 /* Device address of an intermediate slot (tests compare intermediates). */
 void *poly_hip_plan_slot_ptr(const PolyHipPlan *plan, int slot);
-/* Enable (1, default) or disable (0) hipGraph replay for this plan. */
+/* Replay this plan from a hipGraph (1), or never (0).  A plan that neither was said of does
+ * so unless it has only a few launches, which take the host less time one by one. */
 void poly_hip_plan_set_graph(PolyHipPlan *plan, int enabled);
 size_t poly_hip_plan_workspace_bytes(const PolyHipPlan *plan);
 /* How many launches of the plan its captured graph runs on side streams beside the

@@ -115,8 +115,9 @@ struct PolyHipPlan {
   std::vector<std::vector<int>> touch_at;
   Program *touch = nullptr;
   bool use_graph = true;
-  // Kernel launches of one pass.  A plan of a few of them is launched kernel by kernel: a
-  // graph of one to three nodes takes the host 16 us to launch, each kernel 2.5-3 us
+  bool graph_asked = false;      // by poly_hip_plan_set_graph, however few launches there are
+  // Kernel launches of one pass.  A plan of a few of them is launched kernel by kernel unless
+  // a graph was asked for: one of one to three nodes takes the host 16 us to launch, each kernel 2.5-3 us
   // (a row sum: 16.6 against 3.2 us of host time, 3 launches of a LayerNorm 17.9 against
   // 8.0; 22 launches of an MLP step 27 against 73).
   int n_launches = 0;
@@ -970,7 +971,8 @@ int poly_hip_plan_run(PolyHipPlan *plan, void **slot_data, int n_slots, const Po
   }
   hipStream_t stream = (hipStream_t)runtime_stream();
   constexpr int kFewLaunches = 6;
-  if (!plan->use_graph || (plan->n_launches <= kFewLaunches && !plan->forked) || getenv("POLY_HIP_NO_GRAPH")) return enqueue_all(plan);
+  const bool few = plan->n_launches <= kFewLaunches && !plan->forked && !plan->graph_asked;
+  if (!plan->use_graph || few || getenv("POLY_HIP_NO_GRAPH")) return enqueue_all(plan);
   plan->tick++;
   (void)key;
   for (GraphEntry &g : plan->graphs)
@@ -1214,7 +1216,7 @@ void *poly_hip_plan_slot_ptr(const PolyHipPlan *plan, int slot) {
   return plan->slot_ptr[(size_t)slot];
 }
 
-void poly_hip_plan_set_graph(PolyHipPlan *plan, int enabled) { if (plan) plan->use_graph = enabled != 0; }
+void poly_hip_plan_set_graph(PolyHipPlan *plan, int enabled) { if (plan) plan->use_graph = plan->graph_asked = enabled != 0; }
 int poly_hip_plan_side_launches(const PolyHipPlan *plan) {
   int n = 0;
   if (plan) for (char c : plan->on_side) n += c != 0;

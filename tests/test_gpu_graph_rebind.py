@@ -13,7 +13,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 from polygrad_amd import HipPlan
-from polygrad_amd.inputs import block_train_slot_tensors, gpt2_slot_tensors
+from polygrad_amd.inputs import block_train_slot_tensors, gpt2_slot_tensors, random_slot_tensors
 
 PLANS = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "polygrad_amd", "plans")
 
@@ -163,3 +163,31 @@ def test_per_launch_times_add_up_to_the_step():
     assert "N=50257" in info[longest]["desc"], info[longest]["desc"]
     total = sum(acc)
     assert 0.6 * step_ms <= total <= 1.05 * step_ms, (total, step_ms)
+
+
+def test_a_plan_of_few_launches_gets_the_graph_it_asks_for():
+    """A row sum of one launch: launched directly as it comes, captured once and replayed after
+    set_graph(True), launched directly again after set_graph(False); other buffers by updating."""
+    import torch
+    plan = load("rowops_f32_8192_sum")
+    by = {s.name: s.index for s in plan.external_slots()}
+    data = random_slot_tensors(plan, seed=4)
+    more = [None if t is None else t.clone() for t in data]
+    more[by["a"]].mul_(0.5)
+    want = []
+    for d in (data, more):
+        plan.run(d)
+        want.append(d[by["sum"]].clone())
+    assert not torch.equal(*want) and plan.graph_counts() == (0, 0)
+    plan.set_graph(True)
+    for _ in range(3):
+        for d, w in zip((data, more), want):
+            d[by["sum"]].zero_()
+            plan.run(d)
+            assert torch.equal(d[by["sum"]], w)
+    assert plan.graph_counts() == (1, 1)
+    plan.set_graph(False)
+    data[by["sum"]].zero_()
+    plan.run(data)
+    assert torch.equal(data[by["sum"]], want[0]) and plan.graph_counts() == (1, 1)
+    plan.close()
