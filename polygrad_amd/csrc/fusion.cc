@@ -2224,7 +2224,8 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
   }
   rk.entry = "poly_k";
   rk.klass = KernelClass::ATTENTION;
-  const std::string fa_cfg = cfg;
+  std::string fa_cfg = cfg;      // behind the prelude, with the template
+  const char *fa_template = rows_form ? kAttentionRowsTemplate : kAttentionTemplate;
   if (rows_form) {
     // As many waves as there are units of keys to deal, up to four a wave before there are
     // eight (36 heads of 345 keys: 16.3 us on four waves, 18.4 on eight); two blocks of queries
@@ -2235,13 +2236,12 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
     int waves = units <= 1 ? 1 : units <= 2 ? 2 : units <= 16 ? 4 : 8;
     int qt = mS.Z * ((mS.M + 31) / 32) >= 512 ? 2 : 1;
     if (const char *ov = measurement_env("POLY_HIP_FA_ROWS")) sscanf(ov, "%d,%d", &waves, &qt);   // "WAVES,QT": tuning experiments
-    rk.source = std::string(hip_prelude()) + strf("#define POLY_F32 %d\n#define POLY_FA_WAVES %d\n#define POLY_FA_QT %d\n#define POLY_FA_PASS_ZEROS %d\n", f32 ? 1 : 0, waves, qt, whole_blocks ? 1 : 0) + cfg + kAttentionRowsTemplate;
+    fa_cfg = strf("#define POLY_F32 %d\n#define POLY_FA_WAVES %d\n#define POLY_FA_QT %d\n#define POLY_FA_PASS_ZEROS %d\n", f32 ? 1 : 0, waves, qt, whole_blocks ? 1 : 0) + cfg;
     rk.launch.grid[0] = (unsigned)(((mS.M + 16 * qt - 1) / (16 * qt)) * mS.Z);
     rk.launch.block[0] = (unsigned)(64 * waves);
     rk.strategy = strf("fused attention (%zu kernels): mfma %s Z=%lld M=%lld N=%lld D=64, one pass, scores of %d queries in registers, keys dealt to %d waves, exact roundings", all.size() + copy_items.size(),
                        f32 ? "16x16x4 f32" : tin == DT_BF16 ? "16x16x32 bf16" : "16x16x32 f16", (long long)mS.Z, (long long)mS.M, (long long)mS.N, 16 * qt, waves);
   } else {
-    rk.source = std::string(hip_prelude()) + cfg + kAttentionTemplate;
     rk.launch.grid[0] = (unsigned)((mS.M / 128) * mS.Z);
     rk.launch.block[0] = 256;
     rk.strategy = strf("fused attention (%zu kernels): mfma 32x32x16 %s Z=%lld M=%lld N=%lld D=64, %s", all.size() + copy_items.size(),
@@ -2250,12 +2250,13 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
     if (mask_table) rk.strategy += ", mask tiles classified by a first kernel";
     if (out->key_bounds.used) rk.strategy += ", products of masked key blocks bounded by the block maxima the keys' product leaves";
   }
-  if (matmul_tuning_enabled() && !rows_form) {
+  rk.source = std::string(hip_prelude()) + fa_cfg + fa_template;
+  if (matmul_tuning_enabled()) {
     // the register budget (waves per SIMD) changes the schedule of the instructions, not
     // one value: candidates of the search that POLY_BEAM switches on
     rk.variants.push_back({"default", rk.source, rk.strategy, rk.launch});
     for (int occ : {2, 4})
-      rk.variants.push_back({strf("attn_occ%d", occ), std::string(hip_prelude()) + strf("#define POLY_FA_OCC %d\n", occ) + fa_cfg + kAttentionTemplate,
+      rk.variants.push_back({strf("attn_occ%d", occ), std::string(hip_prelude()) + strf("#define POLY_FA_OCC %d\n", occ) + fa_cfg + fa_template,
                              rk.strategy + strf(", %d waves per SIMD", occ), rk.launch});
   }
   rk.n_params = (int)arg_slots.size();

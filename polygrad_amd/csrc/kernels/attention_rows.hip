@@ -88,7 +88,13 @@ __device__ __forceinline__ float fr_lane_xor(float v, int mask) {
   return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((int)((threadIdx.x & 63) ^ mask) * 4, __builtin_bit_cast(int, v)));
 }
 
-extern "C" __global__ void __launch_bounds__(64 * POLY_FA_WAVES) poly_k(POLY_SIGNATURE) {
+#ifdef POLY_FA_OCC   // waves per SIMD the register budget is set for (a tuning candidate: no effect on the values)
+#define FR_BUDGET __attribute__((amdgpu_waves_per_eu(POLY_FA_OCC, POLY_FA_OCC)))
+#else
+#define FR_BUDGET
+#endif
+
+extern "C" __global__ void __launch_bounds__(64 * POLY_FA_WAVES) FR_BUDGET poly_k(POLY_SIGNATURE) {
   // Workgroup ids congruent mod 8 run on one XCD (own L2): each XCD gets a contiguous run of
   // query blocks, those of one z side by side, which read the same K and V.
   constexpr int MB = (POLY_FA_M + FR_BM - 1) / FR_BM, NT = MB * POLY_FA_Z;

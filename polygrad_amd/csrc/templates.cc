@@ -724,58 +724,76 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
     *kc = false;
     return (is_a ? dims.back().ca : dims.back().cb) == 1 && rows >= run && (dims.size() == 1 || dims.back().extent % run == 0);
   };
-  bool a_kc, b_kc;
-  if (!layout(mm.ka, mm.md, true, M, f.tm, &a_kc) || !layout(mm.kb, mm.nd, false, N, f.tn, &b_kc)) return false;
-  const int64_t tiles = ((M + 16 * f.tm - 1) / (16 * f.tm)) * ((N + 16 * f.tn - 1) / (16 * f.tn));
-  if (Z > 65535 || M > 2147483647LL / 2 || N > 2147483647LL / 2 || K > 2147483647LL / 2 || tiles > 2147483647LL / 2) return false;
-  std::string cfg;
-  cfg += strf("#define POLY_TIN %s\n#define POLY_F32 %d\n", dt_cname(mm.A.dt), f32 ? 1 : 0);
-  if (!f32) cfg += strf("#define POLY_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_%s(a, b, c, 0, 0, 0)\n", mm.A.dt == DT_BF16 ? "bf16" : "f16");
-  else cfg += "#define POLY_MFMA(a, b, c) (c)\n";
-  cfg += strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_K %lld\n#define POLY_Z %lld\n", (long long)M, (long long)N, (long long)K, (long long)Z);
-  cfg += strf("#define POLY_TM %d\n#define POLY_TN %d\n#define POLY_WAVES %d\n#define POLY_DEPTH %d\n#define POLY_SUMS %d\n", f.tm, f.tn, f.waves, f.depth, sums);
-  cfg += strf("#define POLY_A_KC %d\n#define POLY_B_KC %d\n#define POLY_A_PTR %s\n#define POLY_B_PTR %s\n", a_kc ? 1 : 0, b_kc ? 1 : 0, ep.a_ptr.c_str(), ep.b_ptr.c_str());
-  cfg += offset_fn("poly_a_row", mm.md, true, 0) + offset_fn("poly_b_row", mm.nd, false, 0);
-  if (mm.zd.empty()) {
-    cfg += strf("__device__ __forceinline__ int poly_a_z(int) { return %lld; }\n", (long long)mm.a_c0);
-    cfg += strf("__device__ __forceinline__ int poly_b_z(int) { return %lld; }\n", (long long)mm.b_c0);
-  } else {
-    cfg += offset_fn("poly_a_z", mm.zd, true, mm.a_c0) + offset_fn("poly_b_z", mm.zd, false, mm.b_c0);
+  if (Z > 65535 || M > 2147483647LL / 2 || N > 2147483647LL / 2 || K > 2147483647LL / 2) return false;
+  auto render = [&](const Form &f, RenderedKernel *out) {
+    bool a_kc, b_kc;
+    if (!layout(mm.ka, mm.md, true, M, f.tm, &a_kc) || !layout(mm.kb, mm.nd, false, N, f.tn, &b_kc)) return false;
+    const int64_t tiles = ((M + 16 * f.tm - 1) / (16 * f.tm)) * ((N + 16 * f.tn - 1) / (16 * f.tn));
+    if (tiles > 2147483647LL / 2) return false;
+    std::string cfg;
+    cfg += strf("#define POLY_TIN %s\n#define POLY_F32 %d\n", dt_cname(mm.A.dt), f32 ? 1 : 0);
+    if (!f32) cfg += strf("#define POLY_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_%s(a, b, c, 0, 0, 0)\n", mm.A.dt == DT_BF16 ? "bf16" : "f16");
+    else cfg += "#define POLY_MFMA(a, b, c) (c)\n";
+    cfg += strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_K %lld\n#define POLY_Z %lld\n", (long long)M, (long long)N, (long long)K, (long long)Z);
+    cfg += strf("#define POLY_TM %d\n#define POLY_TN %d\n#define POLY_WAVES %d\n#define POLY_DEPTH %d\n#define POLY_SUMS %d\n", f.tm, f.tn, f.waves, f.depth, sums);
+    cfg += strf("#define POLY_A_KC %d\n#define POLY_B_KC %d\n#define POLY_A_PTR %s\n#define POLY_B_PTR %s\n", a_kc ? 1 : 0, b_kc ? 1 : 0, ep.a_ptr.c_str(), ep.b_ptr.c_str());
+    cfg += offset_fn("poly_a_row", mm.md, true, 0) + offset_fn("poly_b_row", mm.nd, false, 0);
+    if (mm.zd.empty()) {
+      cfg += strf("__device__ __forceinline__ int poly_a_z(int) { return %lld; }\n", (long long)mm.a_c0);
+      cfg += strf("__device__ __forceinline__ int poly_b_z(int) { return %lld; }\n", (long long)mm.b_c0);
+    } else {
+      cfg += offset_fn("poly_a_z", mm.zd, true, mm.a_c0) + offset_fn("poly_b_z", mm.zd, false, mm.b_c0);
+    }
+    cfg += matmul_k_fn("poly_a_k", mm.ka, K) + matmul_k_fn("poly_b_k", mm.kb, K);
+    const std::string shape = strf("#define POLY_SIGNATURE %s%s\n#define POLY_KSPLIT %d\n#define POLY_PARTIALS poly_scratch\n", ep.signature.c_str(), S > 1 ? ", float* poly_scratch" : "", S) + ep.code;
+    cfg += shape;
+    // what the kernel that has an element's whole sum does with it
+    std::string finish = strf("#define POLY_EPILOGUE(acc, m, n, z) %s\n", ep.call.c_str());
+    if (!ep.mid_value_call.empty())
+      finish += strf("#define POLY_EP_MID_VALUE(acc, m, n, z) %s\n#define POLY_EP_MID_PTR(m, n, z) %s\n", ep.mid_value_call.c_str(), ep.mid_ptr_call.c_str());
+    if (S > 1) cfg += "#define POLY_EPILOGUE(acc, m, n, z) POLY_PARTIALS[(((size_t)poly_ks * POLY_Z + (z)) * POLY_M + (m)) * POLY_N + (n)] = (acc)\n";
+    else cfg += finish;
+    *out = RenderedKernel();
+    out->source = std::string(hip_prelude()) + cfg + kMatmulWaveTemplate;
+    out->entry = "poly_k";
+    out->launch.grid[0] = (unsigned)tiles;
+    out->launch.grid[1] = (unsigned)(Z * S);
+    out->launch.block[0] = (unsigned)(64 * f.waves);
+    if (S > 1) {
+      // the template becomes a first stage; the kernel proper adds the partial results up
+      out->pres.push_back({out->source, out->entry, out->launch});
+      out->scratch_bytes = (size_t)S * (size_t)Z * (size_t)M * (size_t)N * sizeof(float);
+      out->source = std::string(hip_prelude()) + strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_Z %lld\n", (long long)M, (long long)N, (long long)Z) + shape +
+                    finish + kSplitKCombine;
+      out->launch = LaunchSpec();
+      out->launch.grid[0] = (unsigned)(((double)Z * M * N + 255) / 256);
+      out->launch.block[0] = 256;
+    }
+    out->klass = KernelClass::MATMUL_MFMA;
+    out->reads_b_ahead = true;
+    out->strategy = strf("mfma %s M=%lld N=%lld K=%lld Z=%lld tile %dx%d, depth dealt to %d waves%s, A:%s B:%s", f32 ? "16x16x4 f32" : mm.A.dt == DT_BF16 ? "16x16x32 bf16" : "16x16x32 f16",
+                         (long long)M, (long long)N, (long long)K, (long long)Z, 16 * f.tm, 16 * f.tn, f.waves, sums == 2 ? " of two sums each" : "", a_kc ? "k-major" : "m-major", b_kc ? "k-major" : "n-major");
+    if (S > 1) out->strategy += strf(", K dealt to %d workgroups per tile, partial results added by a second kernel", S);
+    out->n_params = ep.n_params;
+    out->n_vars = 0;
+    out->flops = 2.0 * (double)M * (double)N * (double)K * (double)Z;
+    out->bytes = ep.bytes;
+    return true;
+  };
+  if (!render(f, out)) return false;
+  // The other tiles and depths of loads as tuning candidates.  Which steps of the depth a wave
+  // adds up, and in what order, depends on the waves and sums alone, so these stay.
+  if (matmul_tuning_enabled() && S == 1) {
+    out->variants.push_back({"default", out->source, out->strategy, out->launch});
+    static const Form forms[] = {{1, 1, 0, 6}, {1, 2, 0, 6}, {2, 2, 0, 6}, {2, 4, 0, 6}, {4, 4, 0, 4}};
+    for (Form c : forms) {
+      RenderedKernel v;
+      c.waves = f.waves;
+      if ((c.tm == f.tm && c.tn == f.tn) || M <= 8 * c.tm || N <= 8 * c.tn || !render(c, &v)) continue;      // (mostly padding)
+      out->variants.push_back({strf(f32 ? "f32_%dx%dw%dx%d" : "%dx%dw%dx%dp1", 16 * c.tm, 16 * c.tn, c.waves, c.depth), v.source, v.strategy, v.launch});
+    }
+    if (out->variants.size() < 2) out->variants.clear();
   }
-  cfg += matmul_k_fn("poly_a_k", mm.ka, K) + matmul_k_fn("poly_b_k", mm.kb, K);
-  const std::string shape = strf("#define POLY_SIGNATURE %s%s\n#define POLY_KSPLIT %d\n#define POLY_PARTIALS poly_scratch\n", ep.signature.c_str(), S > 1 ? ", float* poly_scratch" : "", S) + ep.code;
-  cfg += shape;
-  // what the kernel that has an element's whole sum does with it
-  std::string finish = strf("#define POLY_EPILOGUE(acc, m, n, z) %s\n", ep.call.c_str());
-  if (!ep.mid_value_call.empty())
-    finish += strf("#define POLY_EP_MID_VALUE(acc, m, n, z) %s\n#define POLY_EP_MID_PTR(m, n, z) %s\n", ep.mid_value_call.c_str(), ep.mid_ptr_call.c_str());
-  if (S > 1) cfg += "#define POLY_EPILOGUE(acc, m, n, z) POLY_PARTIALS[(((size_t)poly_ks * POLY_Z + (z)) * POLY_M + (m)) * POLY_N + (n)] = (acc)\n";
-  else cfg += finish;
-  *out = RenderedKernel();
-  out->source = std::string(hip_prelude()) + cfg + kMatmulWaveTemplate;
-  out->entry = "poly_k";
-  out->launch.grid[0] = (unsigned)tiles;
-  out->launch.grid[1] = (unsigned)(Z * S);
-  out->launch.block[0] = (unsigned)(64 * f.waves);
-  if (S > 1) {
-    // the template becomes a first stage; the kernel proper adds the partial results up
-    out->pres.push_back({out->source, out->entry, out->launch});
-    out->scratch_bytes = (size_t)S * (size_t)Z * (size_t)M * (size_t)N * sizeof(float);
-    out->source = std::string(hip_prelude()) + strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_Z %lld\n", (long long)M, (long long)N, (long long)Z) + shape +
-                  finish + kSplitKCombine;
-    out->launch = LaunchSpec();
-    out->launch.grid[0] = (unsigned)(((double)Z * M * N + 255) / 256);
-    out->launch.block[0] = 256;
-  }
-  out->klass = KernelClass::MATMUL_MFMA;
-  out->reads_b_ahead = true;
-  out->strategy = strf("mfma %s M=%lld N=%lld K=%lld Z=%lld tile %dx%d, depth dealt to %d waves%s, A:%s B:%s", f32 ? "16x16x4 f32" : mm.A.dt == DT_BF16 ? "16x16x32 bf16" : "16x16x32 f16",
-                       (long long)M, (long long)N, (long long)K, (long long)Z, 16 * f.tm, 16 * f.tn, f.waves, sums == 2 ? " of two sums each" : "", a_kc ? "k-major" : "m-major", b_kc ? "k-major" : "n-major");
-  if (S > 1) out->strategy += strf(", K dealt to %d workgroups per tile, partial results added by a second kernel", S);
-  out->n_params = ep.n_params;
-  out->n_vars = 0;
-  out->flops = 2.0 * (double)M * (double)N * (double)K * (double)Z;
-  out->bytes = ep.bytes;
   return true;
 }
 
