@@ -1022,7 +1022,9 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
   // 8000 x 8193 443 -> 183; softmax of 127 x 10278 22.1 -> 7.1, 38497 x 614 148 -> 66.
   // kept_values: what leaves the compiler registers for the loads in flight; 64 lanes x 16 and
   // 256 x 32 keep four and two rows to a CU's SIMDs, 1024 x 52 is as far as it goes (above 45
-  // it spills some, and 1300 x 50257 still takes 341 us against 554 in three launches).
+  // it spills some, and 1300 x 50257 still takes 341 us against 554 in three launches; what is
+  // kept is each operand of a computed row, and the six kernels of a cross-entropy's gradient over
+  // 4096 x 50257, three operands, take 1080 us against 1189 in three).
   bool keeps_rows = false;
   for (const RowPhase &p : phases) keeps_rows = keeps_rows || p.keeps_row;
   if (getenv("POLY_HIP_NO_ROW_CHAIN_SIZES")) keeps_rows = false;
@@ -1513,8 +1515,9 @@ static std::string attention_order(int64_t MB, int64_t Z) {
   return t + "};\n";
 }
 
-// The most keys a workgroup of kernels/attention_rows.hip holds the scores of (eight waves, 16
-// 16-key blocks and two query blocks each: 128 registers of a lane for fp32).
+// The most keys a workgroup of kernels/attention_rows.hip holds the scores of: on eight waves
+// eight 16-key blocks each, with two blocks of queries 64 scores a lane beside the keys and
+// values in flight.  Longer rows have not been measured on it.
 constexpr int64_t kAttentionRowsKeys = 1024;
 
 static bool match_attention(const Sched &sc, int s_item, const std::vector<char> &taken, FusedGroup *out) {

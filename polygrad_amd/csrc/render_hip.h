@@ -73,8 +73,9 @@ struct RenderedKernel {
     LaunchSpec launch;
   };
   std::vector<Variant> variants;
-  // A matrix product whose own first workgroups read operand B into the memory-side cache, or
-  // whose first stage reads both operands (the plan then launches nothing ahead of it for that).
+  // A matrix product that the plan launches nothing ahead of to read operand B into the
+  // memory-side cache: its own first workgroups do that, its first stage reads both operands, or
+  // its loads are far enough ahead for what such a launch costs to be more than it gives.
   bool reads_b_ahead = false;
   // A product that leaves the largest magnitude of every 64 x 64 block of some of its output
   // columns in its scratch memory (MatmulEpilogue::block_maxima) -- and, set by the plan-level
