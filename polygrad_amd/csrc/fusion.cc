@@ -1031,6 +1031,8 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
   auto kept_values = [](int lanes) { return lanes <= 64 ? 16 : lanes == 256 ? 32 : 52; };
   if (R <= 32) G = 32;
   else if (keeps_rows) {
+    // (16-byte loads of 16-bit elements: the lanes as they were, and what 64 or 256 of them do
+    // not hold still ends the chain)
     const bool wide = R % 8 == 0 && std::all_of(items.begin(), items.end(), [&](int it) {      // 16 bytes of 16-bit elements a lane
       for (const auto &p : sc.graphs[(size_t)it].params) if (dt_size(p.dt) > 2 && (double)s->buf_slots[sc.slot(it, (int)(&p - &sc.graphs[(size_t)it].params[0]))].numel >= rows * (double)R) return false;
       return true;
