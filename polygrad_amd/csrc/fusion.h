@@ -49,4 +49,23 @@ std::vector<int> fused_groups_out_of_order(const PolySchedule *s, const std::vec
 // has been made to store the bf16 values themselves).
 std::vector<int> matmul_param_kinds_of(const PolySchedule *s, const std::vector<KernelGraph> &graphs, int item, const std::vector<int> &narrow_slots);
 
+// A schedule as it is planned: its kernels analysed, grouped, and without the copies that
+// need no launch (copies.cc).  `sched` is the schedule itself where there are none.
+struct PlannedSchedule {
+  PolySchedule sched;
+  std::vector<KernelGraph> graphs;          // of the items of `sched`
+  std::vector<FusedGroup> groups;
+  std::vector<char> unused;                 // per slot: an intermediate that no kernel touches any more
+  std::vector<int> written_early;           // the caller's buffers that are written before their copy's place
+  PlannedSchedule() = default;
+  PlannedSchedule(const PlannedSchedule &) = delete;
+  PlannedSchedule &operator=(PlannedSchedule &&) = default;
+  std::vector<PolyExecItem> items;          // what `sched` points to, where it is not the caller's
+  std::vector<std::vector<int>> args;
+  std::vector<int> order;
+};
+// Analyses and groups schedule `s` (POLY_HIP_NO_COPY_DROP in the environment, or
+// !drop_copies: every copy keeps its launch).  False with a message on a malformed kernel.
+bool plan_schedule(const PolySchedule *s, bool drop_copies, PlannedSchedule *out, std::string *err);
+
 }  // namespace polyhip

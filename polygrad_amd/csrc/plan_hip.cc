@@ -32,6 +32,65 @@
 
 using namespace polyhip;
 
+namespace polyhip {
+
+// Do the producers of `slot` write every element?  Every ungated STORE into the slot's
+// PARAM whose index is affine in its ranges with strides that nest (sorted by stride,
+// each stride is the previous stride times the previous extent, the smallest is 1)
+// writes exactly one contiguous interval of elements; the slot is covered when the union
+// of those intervals is [0, numel).  Gated stores, strided stores and indices with
+// divisions count for nothing: the answer errs towards "needs a fill".
+bool slot_fully_written(const PolySchedule *s, int slot, const std::vector<KernelGraph> &graphs) {
+  std::vector<std::pair<int64_t, int64_t>> spans;    // [first, end)
+  for (int k = 0; k < s->n_items; k++) {
+    const PolyExecItem &it = s->items[k];
+    const KernelGraph &g = graphs[(size_t)k];
+    for (const StoreInfo &st : g.stores) {
+      int p = g.param_slot(st.param);
+      if (p < 0 || p >= it.n_buf_slots || it.buf_slot_indices[p] != slot) continue;
+      if (st.gate >= 0) continue;
+      int li = g.n(g.n(st.index).src[1]).lin;
+      if (li < 0) continue;
+      const Lin &l = g.lins[(size_t)li];
+      if (!g.lin_is_affine(l)) continue;
+      std::vector<std::pair<int64_t, int64_t>> dims;   // (|stride|, extent)
+      int64_t base = l.c0;
+      bool ok = true;
+      uint64_t seen = 0;
+      for (int r : st.ranges) {
+        bool aff;
+        int64_t c = g.lin_range_coef(l, r, &aff);
+        const int64_t ext = g.ranges[(size_t)r].extent;
+        if (!aff || ext <= 0 || r >= 64) { ok = false; break; }
+        seen |= 1ull << r;
+        if (c == 0 || ext == 1) continue;              // rewrites the same elements / a single value
+        if (c < 0) { base += c * (ext - 1); c = -c; }  // walks downwards: the interval starts at its last step
+        dims.push_back({c, ext});
+      }
+      // anything else the index depends on (a variable, a range of an enclosing loop)
+      if (ok && (g.lin_deps(l) & ~seen) != 0) ok = false;
+      if (ok) for (const Term &t : l.terms) if (g.atoms[(size_t)t.atom].kind != Atom::RANGE) ok = false;
+      if (!ok) continue;
+      std::sort(dims.begin(), dims.end());
+      int64_t expect = 1;
+      for (const auto &d : dims) {
+        if (d.first != expect) { ok = false; break; }
+        expect *= d.second;
+      }
+      if (ok) spans.push_back({base, base + expect});
+    }
+  }
+  std::sort(spans.begin(), spans.end());
+  int64_t covered_to = 0;
+  for (const auto &sp : spans) {
+    if (sp.first > covered_to) break;
+    covered_to = std::max(covered_to, sp.second);
+  }
+  return covered_to >= s->buf_slots[slot].numel;
+}
+
+}  // namespace polyhip
+
 namespace {
 
 // One instantiated graph of the plan's launch sequence, bound to one set of buffers and
@@ -114,6 +173,13 @@ struct PolyHipPlan {
   // before launch u.
   std::vector<std::vector<int>> touch_at;
   Program *touch = nullptr;
+  // Buffers of the caller's that a launch writes before the schedule would (copies.cc).  Where
+  // one of them shares memory with another buffer bound beside it, `plain` runs instead: the
+  // schedule with all its copies, compiled when such a binding is first met.
+  std::vector<int> written_early;
+  std::vector<void *> last_bound;            // what `shares_memory` was worked out for
+  bool shares_memory = false;
+  PolyHipPlan *plain = nullptr;
   bool use_graph = true;
   bool graph_asked = false;      // by poly_hip_plan_set_graph, however few launches there are
   // Kernel launches of one pass.  A plan of a few of them is launched kernel by kernel unless
@@ -133,6 +199,7 @@ struct PolyHipPlan {
   uint64_t tick = 0;
   long long n_captures = 0, n_rebinds = 0;   // (how often the sequence was captured / rebound by updating nodes)
   ~PolyHipPlan() {
+    delete plain;
     for (GraphEntry &g : graphs)
       if (g.exec) (void)hipGraphExecDestroy(g.exec);
     if (captured) (void)hipGraphDestroy(captured);
@@ -149,61 +216,6 @@ struct PolyHipPlan {
 namespace {
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
-
-// Do the producers of `slot` write every element?  Every ungated STORE into the slot's
-// PARAM whose index is affine in its ranges with strides that nest (sorted by stride,
-// each stride is the previous stride times the previous extent, the smallest is 1)
-// writes exactly one contiguous interval of elements; the slot is covered when the union
-// of those intervals is [0, numel).  Gated stores, strided stores and indices with
-// divisions count for nothing: the answer errs towards "needs a fill".
-bool slot_fully_written(const PolySchedule *s, int slot, const std::vector<KernelGraph> &graphs) {
-  std::vector<std::pair<int64_t, int64_t>> spans;    // [first, end)
-  for (int k = 0; k < s->n_items; k++) {
-    const PolyExecItem &it = s->items[k];
-    const KernelGraph &g = graphs[(size_t)k];
-    for (const StoreInfo &st : g.stores) {
-      int p = g.param_slot(st.param);
-      if (p < 0 || p >= it.n_buf_slots || it.buf_slot_indices[p] != slot) continue;
-      if (st.gate >= 0) continue;
-      int li = g.n(g.n(st.index).src[1]).lin;
-      if (li < 0) continue;
-      const Lin &l = g.lins[(size_t)li];
-      if (!g.lin_is_affine(l)) continue;
-      std::vector<std::pair<int64_t, int64_t>> dims;   // (|stride|, extent)
-      int64_t base = l.c0;
-      bool ok = true;
-      uint64_t seen = 0;
-      for (int r : st.ranges) {
-        bool aff;
-        int64_t c = g.lin_range_coef(l, r, &aff);
-        const int64_t ext = g.ranges[(size_t)r].extent;
-        if (!aff || ext <= 0 || r >= 64) { ok = false; break; }
-        seen |= 1ull << r;
-        if (c == 0 || ext == 1) continue;              // rewrites the same elements / a single value
-        if (c < 0) { base += c * (ext - 1); c = -c; }  // walks downwards: the interval starts at its last step
-        dims.push_back({c, ext});
-      }
-      // anything else the index depends on (a variable, a range of an enclosing loop)
-      if (ok && (g.lin_deps(l) & ~seen) != 0) ok = false;
-      if (ok) for (const Term &t : l.terms) if (g.atoms[(size_t)t.atom].kind != Atom::RANGE) ok = false;
-      if (!ok) continue;
-      std::sort(dims.begin(), dims.end());
-      int64_t expect = 1;
-      for (const auto &d : dims) {
-        if (d.first != expect) { ok = false; break; }
-        expect *= d.second;
-      }
-      if (ok) spans.push_back({base, base + expect});
-    }
-  }
-  std::sort(spans.begin(), spans.end());
-  int64_t covered_to = 0;
-  for (const auto &sp : spans) {
-    if (sp.first > covered_to) break;
-    covered_to = std::max(covered_to, sp.second);
-  }
-  return covered_to >= s->buf_slots[slot].numel;
-}
 
 // The fill kernel over one slot (a slot whose producers leave holes reads as zero there,
 // as every intermediate does in the reference, src/exec_plan.c:946-963).
@@ -311,30 +323,68 @@ int enqueue_captured(PolyHipPlan *plan) {
 
 extern "C" {
 
+static PolyHipPlan *compile_schedule(const PolySchedule *s, bool drop_copies);
+
 PolyHipPlan *poly_hip_compile_schedule(PolyCtx *ctx, const PolySchedule *s) {
   (void)ctx;
+  return compile_schedule(s, true);
+}
+
+// The plan that runs on these buffers: `plan` itself, or the one that keeps every copy.
+static PolyHipPlan *plan_for(PolyHipPlan *plan, void **slot_data, int n_slots) {
+  if (plan->written_early.empty() || !slot_data) return plan;
+  const PolySchedule *s = plan->sched;
+  const int n = std::min(n_slots, s->n_buf_slots);
+  if (plan->last_bound.size() != (size_t)n || memcmp(plan->last_bound.data(), slot_data, (size_t)n * sizeof(void *)) != 0) {
+    plan->last_bound.assign(slot_data, slot_data + n);
+    struct Span { uintptr_t lo, hi; bool early; };
+    std::vector<Span> spans;
+    for (int i = 0; i < n; i++) {
+      if (s->buf_slots[i].is_intermediate || !slot_data[i]) continue;
+      const uintptr_t lo = (uintptr_t)slot_data[i];
+      spans.push_back({lo, lo + (uintptr_t)std::max<int64_t>(s->buf_slots[i].nbytes, 1),
+                       std::find(plan->written_early.begin(), plan->written_early.end(), i) != plan->written_early.end()});
+    }
+    std::sort(spans.begin(), spans.end(), [](const Span &a, const Span &b) { return a.lo < b.lo; });
+    plan->shares_memory = false;
+    uintptr_t any_hi = 0, early_hi = 0;      // how far the buffers before this one reach
+    for (const Span &x : spans) {
+      if (x.lo < early_hi || (x.early && x.lo < any_hi)) plan->shares_memory = true;
+      any_hi = std::max(any_hi, x.hi);
+      if (x.early) early_hi = std::max(early_hi, x.hi);
+    }
+  }
+  if (!plan->shares_memory) return plan;
+  if (!plan->plain) {
+    plan->plain = compile_schedule(s, false);
+    if (!plan->plain) return nullptr;
+  }
+  plan->plain->use_graph = plan->use_graph;
+  plan->plain->graph_asked = plan->graph_asked;
+  return plan->plain;
+}
+
+static PolyHipPlan *compile_schedule(const PolySchedule *s, bool drop_copies) {
   if (!s) return nullptr;
   if (runtime_init() != 0) return nullptr;
   std::unique_ptr<PolyHipPlan> plan(new PolyHipPlan());
   plan->sched = s;
   static int plan_counter = 0;
-  std::vector<KernelGraph> graphs((size_t)s->n_items);
-  for (int k = 0; k < s->n_items; k++) {
-    const PolyExecItem &it = s->items[k];
-    if (it.kind != POLY_EXEC_COMPUTE) {
-      log_err("compile_schedule", "non-COMPUTE item %d not supported", k);
-      return nullptr;
-    }
-    if (!graphs[(size_t)k].build(it.root)) {
-      log_err("compile_schedule", "kernel %d: %s", k, graphs[(size_t)k].error.c_str());
+  // the kernels, their groups that run as one launch, and the copies that need none
+  PlannedSchedule planned;
+  {
+    std::string err;
+    if (!plan_schedule(s, drop_copies, &planned, &err)) {
+      log_err("compile_schedule", "%s", err.c_str());
       return nullptr;
     }
   }
-  // kernel groups that run as one launch
-  std::vector<FusedGroup> groups;
-  find_fused_groups(s, graphs, &groups);
+  s = &planned.sched;
+  const std::vector<KernelGraph> &graphs = planned.graphs;
+  std::vector<FusedGroup> &groups = planned.groups;
+  plan->written_early = planned.written_early;
   std::vector<int> group_of((size_t)s->n_items, -1);
-  std::vector<char> internal((size_t)s->n_buf_slots, 0);
+  std::vector<char> internal = planned.unused;
   for (size_t gi = 0; gi < groups.size(); gi++) {
     for (int it : groups[gi].items) group_of[(size_t)it] = (int)gi;
     for (int sl : groups[gi].internal_slots) internal[(size_t)sl] = 1;
@@ -833,7 +883,6 @@ static int bind_args(PolyHipPlan *plan, void **slot_data, int n_slots, const Pol
   }
   for (size_t u = 0; u < plan->units.size(); u++) {
     const Unit &un = plan->units[u];
-    const PolyExecItem &it = s->items[un.item];
     std::vector<void *> &a = plan->kargs[u];
     for (size_t i = 0; i < un.slots.size(); i++) {
       void *p = plan->slot_ptr[(size_t)un.slots[i]];
@@ -844,7 +893,6 @@ static int bind_args(PolyHipPlan *plan, void **slot_data, int n_slots, const Pol
       a[i] = p;
       if (i < un.runner->vetted.size()) un.runner->vetted[i] = p;     // vetted above, or the plan's own arena
     }
-    (void)it;
     for (int v = 0; v < un.n_vars; v++) {
       bool found = false;
       for (const PolyVarBinding &m : plan->merged)
@@ -961,6 +1009,7 @@ static int tuned_first_run(PolyHipPlan *plan) {
 
 int poly_hip_plan_run(PolyHipPlan *plan, void **slot_data, int n_slots, const PolyVarBinding *vb, int nvb) {
   if (!plan || !plan->sched) return -1;
+  if (!(plan = plan_for(plan, slot_data, n_slots))) return -1;
   uint64_t key = 0;
   if (bind_args(plan, slot_data, n_slots, vb, nvb, &key) != 0) return -1;
   if (!plan->tuned) {
@@ -1074,12 +1123,10 @@ int poly_hip_plan_run(PolyHipPlan *plan, void **slot_data, int n_slots, const Po
 }
 
 int poly_hip_fused_groups(const PolySchedule *s, int index, char **source_out, int *n_items_out) {
-  if (!s) return -1;
-  std::vector<KernelGraph> graphs((size_t)s->n_items);
-  for (int k = 0; k < s->n_items; k++)
-    if (s->items[k].kind != POLY_EXEC_COMPUTE || !graphs[(size_t)k].build(s->items[k].root)) return -1;
-  std::vector<FusedGroup> groups;
-  find_fused_groups(s, graphs, &groups);
+  PlannedSchedule planned;
+  std::string err;
+  if (!s || !plan_schedule(s, true, &planned, &err)) return -1;
+  const std::vector<FusedGroup> &groups = planned.groups;
   if (index >= 0 && index < (int)groups.size()) {
     if (n_items_out) *n_items_out = (int)groups[(size_t)index].items.size();
     if (source_out) {
@@ -1105,12 +1152,10 @@ int poly_hip_fused_groups(const PolySchedule *s, int index, char **source_out, i
 }
 
 int poly_hip_fused_group_launch(const PolySchedule *s, int index, int *slots_out, int cap, int *launch_out) {
-  if (!s) return -1;
-  std::vector<KernelGraph> graphs((size_t)s->n_items);
-  for (int k = 0; k < s->n_items; k++)
-    if (s->items[k].kind != POLY_EXEC_COMPUTE || !graphs[(size_t)k].build(s->items[k].root)) return -1;
-  std::vector<FusedGroup> groups;
-  find_fused_groups(s, graphs, &groups);
+  PlannedSchedule planned;
+  std::string err;
+  if (!s || !plan_schedule(s, true, &planned, &err)) return -1;
+  const std::vector<FusedGroup> &groups = planned.groups;
   if (index < 0 || index >= (int)groups.size()) return -1;
   const FusedGroup &fg = groups[(size_t)index];
   for (size_t i = 0; i < fg.arg_slots.size() && (int)i < cap; i++) if (slots_out) slots_out[i] = fg.arg_slots[i];
@@ -1122,13 +1167,13 @@ int poly_hip_fused_group_launch(const PolySchedule *s, int index, int *slots_out
 }
 
 int poly_hip_unwritten_slots(const PolySchedule *s, int *slots_out, int cap) {
-  if (!s) return -1;
-  std::vector<KernelGraph> graphs((size_t)s->n_items);
-  for (int k = 0; k < s->n_items; k++)
-    if (s->items[k].kind != POLY_EXEC_COMPUTE || !graphs[(size_t)k].build(s->items[k].root)) return -1;
-  std::vector<FusedGroup> groups;
-  find_fused_groups(s, graphs, &groups);
-  std::vector<char> internal((size_t)s->n_buf_slots, 0);
+  PlannedSchedule planned;
+  std::string err;
+  if (!s || !plan_schedule(s, true, &planned, &err)) return -1;
+  const std::vector<FusedGroup> &groups = planned.groups;
+  s = &planned.sched;
+  const std::vector<KernelGraph> &graphs = planned.graphs;
+  std::vector<char> internal = planned.unused;
   for (const FusedGroup &fg : groups) for (int sl : fg.internal_slots) internal[(size_t)sl] = 1;
   int n = 0;
   for (int sl = 0; sl < s->n_buf_slots; sl++) {

@@ -1,0 +1,144 @@
+"""Kernels that copy a whole buffer cost no launch: readers of an intermediate copy read what it
+copies, and what is copied into a buffer of the caller's is written there by the kernel that makes
+it.  Which copies go, and the same bits as with all of them launched -- also where buffers of the
+caller share memory, when a buffer written early would be read late."""
+import os
+import sys
+
+import pytest
+
+from polygrad_amd import PlanFile
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "perf"))
+import cases  # noqa: E402
+
+N, K = 40, 300
+
+
+def s_i(s):
+    """The first range of the kernel that is being put together."""
+    return cases.E("RANGE", "int32", (cases.const(N),), (0, 3), N)
+
+
+def _copy(s, dst, src):
+    (i,) = s.ranges(src.numel)
+    return s.store(dst, i, src[i], i)
+
+
+def _sums(s, x, dst, value=lambda v: v):
+    (i,) = s.ranges(N)
+    k = s.rrange(K)
+    return s.store(dst, i, value(s.reduce("ADD", x[i * K + k], k)), i)
+
+
+def _scaled(s, x, dst, by, at=lambda i: i):
+    (i,) = s.ranges(N)
+    return s.store(dst, i, x[at(i)] * by, i)
+
+
+def _schedule(what):
+    """(schedule, copies that need no launch)"""
+    s = cases.Schedule()
+    x, p, out = s.buf("x", N * K), s.buf("p", N), s.buf("out", N)
+    if what == "intermediate":
+        c = _copy(s, s.tmp(N), _sums(s, x, s.tmp(N)))
+        _sums(s, x, out, lambda v: v + c[s_i(s) * -1 + (N - 1)])
+        return s, 1
+    if what == "copy of a copy":
+        c = _copy(s, s.tmp(N), _copy(s, s.tmp(N), _sums(s, x, s.tmp(N))))
+        _sums(s, x, out, lambda v: v + c[s_i(s) * -1 + (N - 1)])
+        return s, 2
+    if what == "update in place":
+        (i,) = s.ranges(N)
+        k = s.rrange(K)
+        new = s.store(s.tmp(N), i, p[i] - s.reduce("ADD", x[i * K + k], k) * 0.01, i)
+        _copy(s, p, new)
+        _sums(s, x, out, lambda v: v + p[s_i(s) * -1 + (N - 1)])
+        return s, 1
+    if what == "update reads other elements":
+        (i,) = s.ranges(N)
+        k = s.rrange(K)
+        new = s.store(s.tmp(N), i, p[i * -1 + (N - 1)] - s.reduce("ADD", x[i * K + k], k) * 0.01, i)
+        _copy(s, p, new)
+        return s, 0
+    if what == "old value read behind the update":
+        (i,) = s.ranges(N)
+        k = s.rrange(K)
+        new = s.store(s.tmp(N), i, p[i] - s.reduce("ADD", x[i * K + k], k) * 0.01, i)
+        _sums(s, x, out, lambda v: v + p[s_i(s) * -1 + (N - 1)])
+        _copy(s, p, new)
+        return s, 0
+    if what == "copied in another order":
+        t = _sums(s, x, s.tmp(N))
+        c = _scaled(s, t, s.tmp(N), 1.0, lambda i: i * -1 + (N - 1))
+        _sums(s, x, out, lambda v: v + c[s_i(s)])
+        return s, 0
+    if what == "part of a buffer":
+        t = _sums(s, x, s.tmp(N))
+        c = s.tmp(N)
+        (i,) = s.ranges(N // 2)
+        s.store(c, i, t[i], i)
+        _sums(s, x, out, lambda v: v + c[s_i(s) * -1 + (N - 1)])
+        return s, 0
+    if what == "written twice":
+        t = _sums(s, x, s.tmp(N))
+        c = _copy(s, s.tmp(N), t)
+        _sums(s, x, t, lambda v: v * 2.0)
+        _sums(s, x, out, lambda v: v + c[s_i(s) * -1 + (N - 1)])
+        return s, 0
+    assert what == "copy of an input"
+    c = _copy(s, s.tmp(N), p)
+    _sums(s, x, out, lambda v: v + c[s_i(s) * -1 + (N - 1)])
+    return s, 0
+
+
+WHAT = ["intermediate", "copy of a copy", "update in place", "update reads other elements", "old value read behind the update", "copied in another order", "part of a buffer",
+        "written twice", "copy of an input"]
+
+
+@pytest.mark.parametrize("what", WHAT)
+def test_which_copies_go(what, hiplib, monkeypatch, capfd):
+    monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
+    monkeypatch.setenv("POLY_HIP_DEBUG", "1")
+    s, n = _schedule(what)
+    assert hiplib.poly_hip_fused_groups(s.plan().schedule, -1, None, None) >= 0
+    said = [line for line in capfd.readouterr().err.splitlines() if "need no launch" in line]
+    assert [int(line.split(": ")[2].split()[0]) for line in said] == ([n] if n else [])
+
+
+def _run(plan, shared):
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    data, by = [None] * len(plan.slots), {}
+    for slot in plan.external_slots():
+        by[slot.name] = data[slot.index] = torch.rand(slot.numel, generator=g, device="cuda")
+    for small, large in shared:         # one buffer at the start of another
+        index = [s.index for s in plan.external_slots() if s.name == small][0]
+        data[index] = by[small] = by[large][:by[small].numel()]
+    for _ in range(3):
+        plan.run(data)
+    return {k: v.cpu().numpy().tobytes() for k, v in by.items()}, len(plan.kernel_info())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", WHAT)
+def test_same_bits_as_with_the_copies(what, monkeypatch):
+    s, n = _schedule(what)
+    got, launches = _run(s.plan(), [])
+    monkeypatch.setenv("POLY_HIP_NO_COPY_DROP", "1")
+    want, all_launches = _run(s.plan(), [])
+    assert got == want and launches == all_launches - min(n, 1)      # (two copies behind each other are one launch of two kernels)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [11, 33, 300])
+@pytest.mark.parametrize("shared", [[], [("logits", "X")], [("W2", "X")], [("b1", "b2")], [("loss", "Y")]])
+def test_training_step_on_buffers_that_share_memory(batch, shared, monkeypatch):
+    """The logits over the inputs they are made of, a parameter over the batch: the copies of the
+    schedule come late, so a step gives the same bits as with each of them launched."""
+    s = cases._mlp_schedule(dict(kind="mlp", batch=batch, d_in=50, d_hid=20, d_out=24))
+    got, launches = _run(s.plan(), shared)
+    monkeypatch.setenv("POLY_HIP_NO_COPY_DROP", "1")
+    want, all_launches = _run(s.plan(), shared)
+    assert got == want and launches <= all_launches - 5
