@@ -6,7 +6,8 @@
 //   POLY_TIN, POLY_F32  input element type, and 1 when it is float
 //   POLY_MFMA(a,b,c)    the 16x16x32 MFMA of a 16-bit type (fp32: 16x16x4)
 //   POLY_M/N/K/Z        problem sizes; no multiple of anything
-//   POLY_TM, POLY_TN    output tile of a workgroup in blocks of 16 rows / columns
+//   POLY_BLOCK          (optional) rows and columns of a block: 16, or 32 for fp32 (the 32x32x2 MFMA)
+//   POLY_TM, POLY_TN    output tile of a workgroup in blocks
 //   POLY_WAVES          waves of a workgroup: each has the whole tile and every
 //                       POLY_WAVES-th step of the depth
 //   POLY_DEPTH          steps of a wave whose loads are in flight at a time
@@ -68,17 +69,24 @@ __device__ __forceinline__ int poly_b_k(int k) { return k * POLY_N; }
 #undef POLY_MFMA
 #define POLY_MFMA(a, b, c) (c)
 #define POLY_MFMA_F32(a, b, c) (c)
+#elif defined(POLY_BLOCK) && POLY_BLOCK == 32
+#define POLY_MFMA_F32(a, b, c) __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0)
 #else
 #define POLY_MFMA_F32(a, b, c) __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0)
 #endif
+#ifndef POLY_BLOCK
+#define POLY_BLOCK 16
+#endif
+#define POLY_GROUPS (64 / POLY_BLOCK)              // of lanes: a group has a block's rows, each group its own k
+#define POLY_ACC (POLY_BLOCK * POLY_BLOCK / 64)    // registers of a block's sums
 
-typedef float poly_f32x4 __attribute__((ext_vector_type(4)));
+typedef float poly_acc __attribute__((ext_vector_type(POLY_ACC)));
 typedef POLY_TIN poly_in8 __attribute__((ext_vector_type(8)));
 typedef unsigned int poly_u32x4 __attribute__((ext_vector_type(4)));
 
 #define POLY_NTHREADS (64 * POLY_WAVES)
 #define POLY_KV (POLY_F32 ? 4 : 8)          // k per lane and step
-#define POLY_KSTEP (4 * POLY_KV)            // k per step
+#define POLY_KSTEP (POLY_GROUPS * POLY_KV)  // k per step
 #ifndef POLY_KSPLIT
 #define POLY_KSPLIT 1
 #endif
@@ -86,8 +94,8 @@ typedef unsigned int poly_u32x4 __attribute__((ext_vector_type(4)));
 #ifndef POLY_SUMS
 #define POLY_SUMS 1
 #endif
-#define POLY_BM (16 * POLY_TM)
-#define POLY_BN (16 * POLY_TN)
+#define POLY_BM (POLY_BLOCK * POLY_TM)
+#define POLY_BN (POLY_BLOCK * POLY_TN)
 
 // T consecutive elements of any alignment.
 template <int T> struct __attribute__((aligned(sizeof(POLY_TIN)))) PolyRow { POLY_TIN v[T]; };
@@ -161,11 +169,11 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
   constexpr int k_base = 0;
 #endif
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int col = lane & 15, grp = lane >> 4;
+  const int col = lane % POLY_BLOCK, grp = lane / POLY_BLOCK;
   const POLY_TIN *__restrict__ gA = POLY_A_PTR + poly_a_z(z);
   const POLY_TIN *__restrict__ gB = POLY_B_PTR + poly_b_z(z);
 
-  // Rows of A (columns of B) of a lane.  Along K: block t has row 16 t + col; rows past the
+  // Rows of A (columns of B) of a lane.  Along K: block t has row POLY_BLOCK t + col; rows past the
   // edge repeat the last one and are not stored.  Along the rows: rows T col .. T col + T - 1,
   // one of each block; a lane whose T rows cross the edge starts T rows before it, and its
   // block t then has row T col + t - (shift), which another lane's block has too unless
@@ -173,7 +181,7 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
 #if POLY_A_KC
   int a_row[POLY_TM];
 #pragma unroll
-  for (int t = 0; t < POLY_TM; t++) { const int m = m0 + 16 * t + col; a_row[t] = poly_a_row(m < POLY_M ? m : POLY_M - 1); }
+  for (int t = 0; t < POLY_TM; t++) { const int m = m0 + POLY_BLOCK * t + col; a_row[t] = poly_a_row(m < POLY_M ? m : POLY_M - 1); }
 #else
   int a_row[1];
   { const int m = m0 + POLY_TM * col; a_row[0] = poly_a_row(m <= POLY_M - POLY_TM ? m : POLY_M - POLY_TM); }
@@ -181,7 +189,7 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
 #if POLY_B_KC
   int b_row[POLY_TN];
 #pragma unroll
-  for (int t = 0; t < POLY_TN; t++) { const int n = n0 + 16 * t + col; b_row[t] = poly_b_row(n < POLY_N ? n : POLY_N - 1); }
+  for (int t = 0; t < POLY_TN; t++) { const int n = n0 + POLY_BLOCK * t + col; b_row[t] = poly_b_row(n < POLY_N ? n : POLY_N - 1); }
 #else
   int b_row[1];
   { const int n = n0 + POLY_TN * col; b_row[0] = poly_b_row(n <= POLY_N - POLY_TN ? n : POLY_N - POLY_TN); }
@@ -191,14 +199,16 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
   auto ka = [&](int k) { return poly_a_k(k_base + k); };
   auto kb = [&](int k) { return poly_b_k(k_base + k); };
 
-  poly_f32x4 sums[POLY_SUMS][POLY_TM][POLY_TN];
+  poly_acc sums[POLY_SUMS][POLY_TM][POLY_TN];
 #pragma unroll
   for (int s = 0; s < POLY_SUMS; s++)
 #pragma unroll
     for (int i = 0; i < POLY_TM; i++)
 #pragma unroll
-      for (int j = 0; j < POLY_TN; j++) sums[s][i][j] = poly_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  auto multiply = [&](const OpA &a, const OpB &b, poly_f32x4 (&acc)[POLY_TM][POLY_TN]) {
+      for (int j = 0; j < POLY_TN; j++)
+#pragma unroll
+        for (int r = 0; r < POLY_ACC; r++) sums[s][i][j][r] = 0.0f;
+  auto multiply = [&](const OpA &a, const OpB &b, poly_acc (&acc)[POLY_TM][POLY_TN]) {
 #if POLY_F32
 #pragma unroll
     for (int e = 0; e < POLY_KV; e++)
@@ -256,7 +266,7 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
     if (s + D < ALL) load(s % D, s + D);
   }
   static_assert(D % POLY_SUMS == 0, "a step of the unrolled loop has its sum");
-  poly_f32x4 (&acc)[POLY_TM][POLY_TN] = sums[0];
+  poly_acc (&acc)[POLY_TM][POLY_TN] = sums[0];
 #if POLY_SUMS == 2
 #pragma unroll
   for (int i = 0; i < POLY_TM; i++)
@@ -265,10 +275,11 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
 #endif
 
   // The partial tiles of the waves, CH blocks of rows at a time, in LDS as the MFMA leaves
-  // them (lane l, register r: row 4 (l / 16) + r, column l % 16 of a block): rows 20 floats
-  // apart and blocks 336, which keeps both the writes and the reads along n off each
-  // other's banks.  Each thread then adds up the elements it finishes, in wave order.
-  constexpr int RS = 20, BS = 336;
+  // them (lane l, register r of a block of 16: row 4 (l / 16) + r, column l % 16; of 32: row
+  // 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32): rows 20 (36) floats apart and blocks 336
+  // (1168), which keeps both the writes and the reads along n off each other's banks.  Each
+  // thread then adds up the elements it finishes, in wave order.
+  constexpr int RS = POLY_BLOCK + 4, BS = POLY_BLOCK * RS + 16;
   constexpr int CH = POLY_TM % 2 == 0 && POLY_WAVES * 2 * POLY_TN * BS * 4 <= 65536 ? 2 : 1;
   __shared__ float part[POLY_WAVES * CH * POLY_TN * BS];
 #pragma unroll
@@ -279,16 +290,17 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
 #pragma unroll
       for (int j = 0; j < POLY_TN; j++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) part[((wave * CH + i) * POLY_TN + j) * BS + (4 * grp + r) * RS + col] = acc[c + i][j][r];
+        for (int r = 0; r < POLY_ACC; r++)
+          part[((wave * CH + i) * POLY_TN + j) * BS + (4 * POLY_GROUPS * (r / 4) + 4 * grp + r % 4) * RS + col] = acc[c + i][j][r];
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < (CH * 16 * POLY_BN + POLY_NTHREADS - 1) / POLY_NTHREADS; q++) {
+    for (int q = 0; q < (CH * POLY_BLOCK * POLY_BN + POLY_NTHREADS - 1) / POLY_NTHREADS; q++) {
       const int id = q * POLY_NTHREADS + (int)threadIdx.x;
-      if (CH * 16 * POLY_BN % POLY_NTHREADS != 0 && id >= CH * 16 * POLY_BN) break;
-      const int x = id % POLY_BN, y = id / POLY_BN, row = y % 16, i = y / 16;
+      if (CH * POLY_BLOCK * POLY_BN % POLY_NTHREADS != 0 && id >= CH * POLY_BLOCK * POLY_BN) break;
+      const int x = id % POLY_BN, y = id / POLY_BN, row = y % POLY_BLOCK, i = y / POLY_BLOCK;
       const int n = n0 + x;
 #if POLY_A_KC
-      const int m = m0 + 16 * (c + i) + row;
+      const int m = m0 + POLY_BLOCK * (c + i) + row;
       const bool mine = m < POLY_M;
 #else
       const int first = m0 + POLY_TM * row, over = first - (POLY_M - POLY_TM), shift = over > 0 ? over : 0;
@@ -297,7 +309,7 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
 #endif
       if (!mine || n >= POLY_N) continue;
 #if POLY_B_KC
-      const int j = x / 16, cc = x % 16;
+      const int j = x / POLY_BLOCK, cc = x % POLY_BLOCK;
 #else
       const int cc = x / POLY_TN, nf = n0 + POLY_TN * cc - (POLY_N - POLY_TN), j = x % POLY_TN + (nf > 0 ? nf : 0);
 #endif

@@ -658,6 +658,18 @@ static void f32_variants(int64_t M, int64_t N, const F32Shape &chosen, const std
   if (out->variants.size() < 2) out->variants.clear();
 }
 
+// How many workgroups render_matmul_f32 deals the depth of a product to, and on which tile (0: its
+// usual one).
+static int f32_split(int64_t M, int64_t N, int64_t K, int64_t Z, int *tile) {
+  *tile = 0;
+  if (M <= 64 || N <= 64 || K < 2048 || K % 16 != 0) return 1;
+  const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128) * Z, t64 = ((M + 63) / 64) * ((N + 63) / 64) * Z;
+  const int s128 = ksplit_for(t128, K / 16, 32), s64 = ksplit_for(t64, K / 16, 32);
+  if (s128 > 1 && t128 * s128 >= 128) { *tile = 128; return s128; }
+  if (s64 > 1) { *tile = 64; return s64; }
+  return 1;
+}
+
 // Products of few or ragged tiles: kernels/matmul_wave.hip, the depth dealt to the waves of
 // a workgroup.  Where it is taken, and on which tile (all times: one launch, operands in the
 // memory-side cache, the other templates in brackets):
@@ -671,10 +683,14 @@ static void f32_variants(int64_t M, int64_t N, const F32Shape &chosen, const std
 //           (7473x219x188: 6.9 [17.7]; 410x7104x318: 13.5 [39.1]; 3001x2999x1003: 86 [53])
 //   fp32    up to 640 tiles of 32x64 (12x768x3072: 8.1 us [265]; 128x3072x768: 10.1 [22.3];
 //           1024^3: 21.6 [30.2]; 4096x512x784, 1024 tiles: 50.1 [38.9])
-//   From a depth of 4096 (fp32) or 8192 (16-bit) on, products of more than 64 rows and
-//   columns are left to the templates that deal the depth to several workgroups, which add
-//   up in a second kernel; of fewer, that is done here (100x50x4096 fp32: 5.6 us dealt to
-//   eight, 9.5 to one [277]; 40x700x5000: 13.2 to two [380]).
+//   From a depth of 4096 on the depth of an fp32 product goes to several workgroups as well,
+//   whose sums a second kernel adds (100x50x4096: 5.6 us dealt to eight, 9.5 to one [277];
+//   40x700x5000: 13.2 to two [380]).  More than 64 rows and columns run on 64x64 tiles of
+//   32x32 blocks there: the tile template puts one workgroup of four waves on a CU, whose
+//   matrix pipes idle at every barrier and load of a 16-deep K tile (53 TFLOP/s), where these
+//   waves meet once (512x784x4096: 41.9 us [69.9]; x4097: 70 [192]; 1024x1024x4096: 80 [106];
+//   128x1024x16384: 45 [105]; 200x300x8192: 25 [33]).  16-bit products of more than 64 rows and
+//   columns and a depth of 8192 are left to the templates that deal it to workgroups.
 // The smallest tile that does not need more workgroups than the chip runs at once: few rows
 // want many narrow workgroups (128x768x768 fp32: 16x32 4.9 us, 32x64 9.8), many rows tiles
 // that read each operand fewer times.
@@ -685,38 +701,41 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
   if (f32 && getenv("POLY_HIP_NO_F32_MFMA")) return false;
   const int kv = f32 ? 4 : 8;
   auto tiles_of = [&](int tm, int tn) { return (double)((M + 16 * tm - 1) / (16 * tm)) * (double)((N + 16 * tn - 1) / (16 * tn)) * (double)Z; };
-  struct Form { int tm, tn, waves, depth; };
-  Form f{1, 2, 8, 6};
+  struct Form { int tm, tn, waves, depth, block; };      // (tile in blocks of `block` rows and columns)
+  Form f{1, 2, 8, 6, 16};
   int S = 1;      // workgroups sharing the depth of a tile
   if (f32) {
     if (tiles_of(2, 4) > 640) return false;
-    if (tiles_of(1, 1) <= 192) f = Form{1, 1, 8, 6};
-    else if (tiles_of(1, 2) <= 288) f = Form{1, 2, 4, 6};
-    else f = Form{2, 4, 4, 6};
-    if (tiles_of(2, 4) > 256 && tiles_of(4, 4) <= 256 && M >= 64 && N >= 64) f = Form{4, 4, 4, 6};
+    if (tiles_of(1, 1) <= 192) f = Form{1, 1, 8, 6, 16};
+    else if (tiles_of(1, 2) <= 288) f = Form{1, 2, 4, 6, 16};
+    else f = Form{2, 4, 4, 6, 16};
+    if (tiles_of(2, 4) > 256 && tiles_of(4, 4) <= 256 && M >= 64 && N >= 64) f = Form{4, 4, 4, 6, 16};
     if (K >= 4096) {
-      if (M > 64 && N > 64) return false;
-      f = tiles_of(1, 1) <= 64 ? Form{1, 1, 8, 6} : Form{1, 2, 4, 6};
-      for (S = 8; S > 1 && (K % (S * kv) != 0 || tiles_of(f.tm, f.tn) * S > 256);) S /= 2;
+      if (M > 64 && N > 64) f = Form{2, 2, 4, 6, 32};
+      else f = tiles_of(1, 1) <= 64 ? Form{1, 1, 8, 6, 16} : Form{1, 2, 4, 6, 16};
+      for (S = M > 64 && N > 64 && K >= 8192 ? 16 : 8; S > 1 && (K % (S * kv) != 0 || tiles_of(f.tm * f.block / 16, f.tn * f.block / 16) * S > 256);) S /= 2;
     }
   } else {
     const bool few = M <= 16 || N <= 16 || tiles_of(4, 4) <= 64;
     if (!few && (whole_tiles || (double)M * (double)N * (double)K * (double)Z >= 1073741824.0)) return false;
-    if (tiles_of(1, 2) > 640 && M > 16) f = Form{2, 2, 8, 6};
-    if (f.tm == 2 && tiles_of(2, 2) > 640) f = Form{2, 4, 4, 6};
-    if (f.tn == 4 && tiles_of(2, 4) > 640) f = Form{4, 4, 4, 4};
+    if (tiles_of(1, 2) > 640 && M > 16) f = Form{2, 2, 8, 6, 16};
+    if (f.tm == 2 && tiles_of(2, 2) > 640) f = Form{2, 4, 4, 6, 16};
+    if (f.tn == 4 && tiles_of(2, 4) > 640) f = Form{4, 4, 4, 4, 16};
   }
-  if (K >= 8192 && M > 64 && N > 64) return false;
+  if (!f32 && K >= 8192 && M > 64 && N > 64) return false;
   if (K <= 256 && f.waves > 4) f.waves = 4;
   if (const char *ov = measurement_env("POLY_HIP_MM_WAVE")) {   // "TM,TN,WAVES,DEPTH": tuning experiments
-    if (sscanf(ov, "%d,%d,%d,%d,%d", &f.tm, &f.tn, &f.waves, &f.depth, &S) < 4) return false;
+    if (sscanf(ov, "%d,%d,%d,%d,%d,%d", &f.tm, &f.tn, &f.waves, &f.depth, &S, &f.block) < 4) return false;
   }
   if (S > 1 && (K % (S * kv) != 0 || !ep.scratch_type.empty() || Z * S > 65535 || getenv("POLY_HIP_NO_SPLIT_K"))) S = 1;
-  // From a depth of 2048 on the fp32 tile template deals it to as many as seven workgroups: no
+  // From a depth of 2048 on the fp32 tile template deals it to as many as sixteen workgroups: no
   // fewer partial sums here, or the sums get less exact (128x768x3072 against float64: 4.97e-7 with
   // four, 4.07e-7 there with six, 3.55e-7 with the eight of two sums a wave, whose time is within
   // 2 %).
-  const int sums = f32 && K >= 2048 && f.waves * S < 8 && f.depth % 2 == 0 ? 2 : 1;
+  int split_tile;
+  const int sums_there = f32 ? f32_split(M, N, K, Z, &split_tile) : 1;
+  const int sums = f32 && K >= 2048 && f.waves * S < std::max(8, sums_there) && f.depth % 2 == 0 ? 2 : 1;
+  if (f.block == 32 && f.waves * S * sums < sums_there) return false;
   // an operand is read along K where its steps are contiguous there, along its rows otherwise
   // (runs of as many rows as the tile has blocks)
   auto layout = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a, int64_t rows, int run, bool *kc) {
@@ -728,13 +747,15 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
   auto render = [&](const Form &f, RenderedKernel *out) {
     bool a_kc, b_kc;
     if (!layout(mm.ka, mm.md, true, M, f.tm, &a_kc) || !layout(mm.kb, mm.nd, false, N, f.tn, &b_kc)) return false;
-    const int64_t tiles = ((M + 16 * f.tm - 1) / (16 * f.tm)) * ((N + 16 * f.tn - 1) / (16 * f.tn));
+    const int bm = f.block * f.tm, bn = f.block * f.tn;
+    const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
     if (tiles > 2147483647LL / 2) return false;
     std::string cfg;
     cfg += strf("#define POLY_TIN %s\n#define POLY_F32 %d\n", dt_cname(mm.A.dt), f32 ? 1 : 0);
     if (!f32) cfg += strf("#define POLY_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_%s(a, b, c, 0, 0, 0)\n", mm.A.dt == DT_BF16 ? "bf16" : "f16");
     else cfg += "#define POLY_MFMA(a, b, c) (c)\n";
     cfg += strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_K %lld\n#define POLY_Z %lld\n", (long long)M, (long long)N, (long long)K, (long long)Z);
+    if (f.block != 16) cfg += strf("#define POLY_BLOCK %d\n", f.block);
     cfg += strf("#define POLY_TM %d\n#define POLY_TN %d\n#define POLY_WAVES %d\n#define POLY_DEPTH %d\n#define POLY_SUMS %d\n", f.tm, f.tn, f.waves, f.depth, sums);
     cfg += strf("#define POLY_A_KC %d\n#define POLY_B_KC %d\n#define POLY_A_PTR %s\n#define POLY_B_PTR %s\n", a_kc ? 1 : 0, b_kc ? 1 : 0, ep.a_ptr.c_str(), ep.b_ptr.c_str());
     cfg += offset_fn("poly_a_row", mm.md, true, 0) + offset_fn("poly_b_row", mm.nd, false, 0);
@@ -774,8 +795,8 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
     // weights ahead costs more than HBM does: GPT-2 small of 12 bf16 tokens 505 us [533 with it], of
     // 128 fp32 tokens, whose 500 MB of weights no cache holds, 967 [1015].
     out->reads_b_ahead = true;
-    out->strategy = strf("mfma %s M=%lld N=%lld K=%lld Z=%lld tile %dx%d, depth dealt to %d waves%s, A:%s B:%s", f32 ? "16x16x4 f32" : mm.A.dt == DT_BF16 ? "16x16x32 bf16" : "16x16x32 f16",
-                         (long long)M, (long long)N, (long long)K, (long long)Z, 16 * f.tm, 16 * f.tn, f.waves, sums == 2 ? " of two sums each" : "", a_kc ? "k-major" : "m-major", b_kc ? "k-major" : "n-major");
+    out->strategy = strf("mfma %s M=%lld N=%lld K=%lld Z=%lld tile %dx%d, depth dealt to %d waves%s, A:%s B:%s", f32 ? (f.block == 32 ? "32x32x2 f32" : "16x16x4 f32") : mm.A.dt == DT_BF16 ? "16x16x32 bf16" : "16x16x32 f16",
+                         (long long)M, (long long)N, (long long)K, (long long)Z, bm, bn, f.waves, sums == 2 ? " of two sums each" : "", a_kc ? "k-major" : "m-major", b_kc ? "k-major" : "n-major");
     if (S > 1) out->strategy += strf(", K dealt to %d workgroups per tile, partial results added by a second kernel", S);
     out->n_params = ep.n_params;
     out->n_vars = 0;
@@ -788,10 +809,11 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
   // adds up, and in what order, depends on the waves and sums alone, so these stay.
   if (matmul_tuning_enabled() && S == 1) {
     out->variants.push_back({"default", out->source, out->strategy, out->launch});
-    static const Form forms[] = {{1, 1, 0, 6}, {1, 2, 0, 6}, {2, 2, 0, 6}, {2, 4, 0, 6}, {4, 4, 0, 4}};
+    static const Form forms[] = {{1, 1, 0, 6, 16}, {1, 2, 0, 6, 16}, {2, 2, 0, 6, 16}, {2, 4, 0, 6, 16}, {4, 4, 0, 4, 16}};
     for (Form c : forms) {
       RenderedKernel v;
       c.waves = f.waves;
+      if (f.block != 16) break;
       if ((c.tm == f.tm && c.tn == f.tn) || M <= 8 * c.tm || N <= 8 * c.tn || !render(c, &v)) continue;      // (mostly padding)
       out->variants.push_back({strf(f32 ? "f32_%dx%dw%dx%d" : "%dx%dw%dx%dp1", 16 * c.tm, 16 * c.tn, c.waves, c.depth), v.source, v.strategy, v.launch});
     }
@@ -817,13 +839,9 @@ static bool render_matmul_f32(const MatmulMatch &mm, const MatmulEpilogue &ep, R
   int BM, BN, WVM, WVN;
   f32_tile(M, N, Z, &BM, &BN, &WVM, &WVN);
   // deep product on few tiles: larger tiles, K dealt to several workgroups each
-  int S = 1;
-  if (M > 64 && N > 64 && K >= 2048) {
-    const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128) * Z, t64 = ((M + 63) / 64) * ((N + 63) / 64) * Z;
-    const int s128 = ksplit_for(t128, K / 16, 32), s64 = ksplit_for(t64, K / 16, 32);
-    if (s128 > 1 && t128 * s128 >= 128) { BM = BN = 128; WVM = WVN = 2; S = s128; }
-    else if (s64 > 1) { BM = BN = 64; WVM = WVN = 2; S = s64; }
-  }
+  int split_tile;
+  const int S = f32_split(M, N, K, Z, &split_tile);
+  if (split_tile) { BM = BN = split_tile; WVM = WVN = 2; }
   if (((M + BM - 1) / BM) * ((N + BN - 1) / BN) > 2147483647LL / 2) return reject(__LINE__);
   std::string cfg;     // (all but the shape of the tile)
   cfg += strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_K %lld\n#define POLY_Z %lld\n", (long long)M, (long long)N, (long long)K, (long long)Z);
