@@ -774,6 +774,9 @@ static void collect_ref_loads(const Sched &sc, const Member &m, std::vector<std:
 // (set by find_fused_groups once it knows that the one reader of the buffer takes that)
 static thread_local int g_narrow_store_slot = -1;
 
+// Row chains on 1024 lanes of 128 registers: from how many elements a lane on each phase works its
+// positions out again, and how many registers' worth of kept elements stay out of LDS.
+constexpr int kRowChainLong1024 = 45, kRowChainKept1024 = 60;
 static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<char> &taken, FusedGroup *out, bool allow_rows, bool allow_side = false) {
   const PolySchedule *s = sc.s;
   const KernelGraph &gA = sc.graphs[(size_t)a_item];
@@ -1021,10 +1024,7 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
   // three or four: LayerNorm of 4097 x 1001 32.4 -> 11.4 us (5.8 TB/s), 2256 x 25472 462 -> 161,
   // 8000 x 8193 443 -> 183; softmax of 127 x 10278 22.1 -> 7.1, 38497 x 614 148 -> 66.
   // kept_values: what leaves the compiler registers for the loads in flight; 64 lanes x 16 and
-  // 256 x 32 keep four and two rows to a CU's SIMDs, 1024 x 52 is as far as it goes (above 45
-  // it spills some, and 1300 x 50257 still takes 341 us against 554 in three launches; what is
-  // kept is each operand of a computed row, and the six kernels of a cross-entropy's gradient over
-  // 4096 x 50257, three operands, take 1080 us against 1189 in three).
+  // 256 x 32 keep four and two rows to a CU's SIMDs, 1024 x 52 is as far as it goes.
   bool keeps_rows = false;
   for (const RowPhase &p : phases) keeps_rows = keeps_rows || p.keeps_row;
   if (getenv("POLY_HIP_NO_ROW_CHAIN_SIZES")) keeps_rows = false;
@@ -1086,19 +1086,21 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
       else row_decomp += strf("  const int r%d = (int)(t_ %% %lld); t_ /= %lld;\n", ord, (long long)e, (long long)e);
     }
   }
-  std::string code, calls, strat;
+  std::string code;
+  std::string calls, strat;
   std::string lead;   // results so far, as parameters
   std::string lead_call;
   // Short rows handled by one wave stay in registers between the phases: a vector load
   // that an earlier phase made from the same buffer at the same index is kept instead of
   // being repeated (the row is then read from memory once, not once per phase).
-  struct RowCache { std::string key, type; int nit; int V = 0; std::string what; };    // what: the key without the vector width
+  struct RowCache { std::string key, type; int nit; int V = 0; std::string what; int bytes = 0; size_t last = 0; };    // what: the key without the vector width; bytes: of a step; last: phase that takes it
   std::vector<RowCache> cache;
   int n_cached_uses = 0, n_exported = 0;
   bool narrow_stored = false;
   int n_walked_phases = 0;          // phases that walk their row from memory in a loop (nothing kept for the next one)
   int row_V = 0, row_nit = 0;       // vector width and step count of the rows kept between phases
-  std::string row_decls;             // their declarations in the kernel body
+  struct RowKept { std::string name, type; int bytes; size_t made; };
+  std::vector<RowKept> rows_kept;    // (bytes: of a step)
   for (size_t pi = 0; pi < phases.size(); pi++) {
     const RowPhase &ph = phases[pi];
     if (ph.is_copy) continue;        // (its value is the result before it, under the same name)
@@ -1201,12 +1203,16 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
       std::string key = strf("%d:%d:%d:%lld", sc.slot(ph.m.item, g.param_slot(ix.src[0])), V, (int)g.n(node).dt, (long long)a.c0);
       for (auto &kv : a.c) key += strf(",%d*%lld", kv.first, (long long)kv.second);
       for (size_t ci = 0; ci < cache.size(); ci++)
-        if (cache[ci].key == key && cache[ci].nit == nit) { n_cached_uses++; return strf("c%zu[it]", ci); }
+        if (cache[ci].key == key && cache[ci].nit == nit) { n_cached_uses++; cache[ci].last = pi; return strf("c%zu[it]", ci); }
+      // (what is the same for every row stays in the L2: the registers are for what comes from memory)
+      if (G == 1024 && std::all_of(a.c.begin(), a.c.end(), [&](const std::pair<const int, int64_t> &kv) { return kv.first == red_master; })) {
+        return ld;
+      }
       if (pi + 1 == phases.size()) return ld;   // nobody comes after the last phase
       {
         std::string what = strf("%d:%d:%lld", sc.slot(ph.m.item, g.param_slot(ix.src[0])), (int)g.n(node).dt, (long long)a.c0);
         for (auto &kv : a.c) what += strf(",%d*%lld", kv.first, (long long)kv.second);
-        cache.push_back({key, strf("poly_vec<%s,%d>", dt_cname(g.n(node).dt), V), nit, V, what});
+        cache.push_back({key, strf("poly_vec<%s,%d>", dt_cname(g.n(node).dt), V), nit, V, what, V * dt_size(g.n(node).dt)});
       }
       return strf("(c%zu[it] = %s)", cache.size() - 1, ld.c_str());
     };
@@ -1335,22 +1341,23 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
     if (em.failed() || em.uses_threefry) FA_REJECT();
     std::string cache_params, cache_args;
     for (size_t ci = 0; ci < cache.size(); ci++) {
-      cache_params += strf(", %s (&c%zu)[%d]", cache[ci].type.c_str(), ci, cache[ci].nit);
+      cache_params += strf(", kept_c%zu &c%zu", ci, ci);
       cache_args += strf(", c%zu", ci);
     }
-    code += strf("__device__ __forceinline__ %s %s(const long long row, const int lane%s%s, %s) {\n", ret.c_str(), fn.c_str(), lead.c_str(),
+    code += strf("__device__ __forceinline__ %s %s(const long long row, int lane%s%s, %s) {\n", ret.c_str(), fn.c_str(), lead.c_str(),
                  cache_params.c_str(), params_decl(g).c_str());
+    if (G == 1024 && pi) code += "  POLY_FRESH(lane);\n";
     code += row_decomp + loop + tail + "}\n";
     if (ph.keeps_row) {
       // the row it makes: an array the later phases receive by reference
       const std::string base = names[pi].substr(0, names[pi].find('['));
       const std::string type = strf("poly_vec<%s,%d>", dt_cname(g.n(g.stores[0].value).dt), V);
-      row_decls += strf("    %s %s[%d];\n", type.c_str(), base.c_str(), nit);
-      const std::string param = strf(", %s (&%s)[%d]", type.c_str(), base.c_str(), nit);
+      rows_kept.push_back({base, type, V * dt_size(g.n(g.stores[0].value).dt), pi});
+      const std::string param = strf(", kept_%s &%s", base.c_str(), base.c_str());
       // this phase's own signature needs it too: it was built above without it
-      const size_t sig_at = code.rfind(strf("%s(const long long row, const int lane%s", fn.c_str(), lead.c_str()));
+      const size_t sig_at = code.rfind(strf("%s(const long long row, int lane%s", fn.c_str(), lead.c_str()));
       if (sig_at == std::string::npos) FA_REJECT();
-      code.insert(sig_at + strf("%s(const long long row, const int lane%s", fn.c_str(), lead.c_str()).size(), param);
+      code.insert(sig_at + strf("%s(const long long row, int lane%s", fn.c_str(), lead.c_str()).size(), param);
       calls += strf("    %s(row, lane%s, %s%s, %s);\n", fn.c_str(), lead_call.c_str(), base.c_str(), cache_args.c_str(), call_args(ph.m.item).c_str());
       lead += param;
       lead_call += ", " + base;
@@ -1364,6 +1371,46 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
     }
     strat += strf("%s%s vec%d%s", pi ? ", " : "", ph.is_map ? "map" : "reduce", V, ragged ? " unaligned + tail" : "");
   }
+  // What the phases keep: registers.  On 1024 lanes rows of more than kRowChainLong1024 elements a
+  // lane spill: the compiler keeps the 64-bit address of every element from one phase to the next,
+  // twice what the elements take.  Each phase works its positions out again there (softmax of
+  // 1024 x 50257 249 -> 186 us, 1200 x 52001 310 -> 225; where nothing spilled no change: layernorm
+  // of 600 x 50000 90).  Of rows that are still needed together once the first of them is made, what
+  // kRowChainKept1024 registers do not hold is in LDS: the cross-entropy's gradient over
+  // 4096 x 50257 keeps the logits and a computed row, and the step it is part of takes 5977 us
+  // with 60 registers [5990 with 45, 5995 with 80, 6150 with all, 6640 before].  Not rows
+  // that only the first phases take: those in LDS cost 10 % (600 x 50000 90 -> 100).
+  std::string kept_types, kept_decls;
+  {
+    int dwords = 0, lds_left = 156 << 10, longest = row_nit * row_V;
+    for (const RowKept &k : rows_kept) dwords += row_nit * ((k.bytes + 3) / 4);
+    for (const RowCache &c : cache) {
+      longest = std::max(longest, c.nit * c.V);
+      // (operands that no phase takes after the first row is made are done with by then)
+      if (!rows_kept.empty() && c.last > rows_kept[0].made) dwords += c.nit * ((c.bytes + 3) / 4);
+    }
+    const bool over = G == 1024 && longest > kRowChainLong1024;
+    if (G == 1024 && !over) kept_types = "#define POLY_FRESH(lane)\n";
+    if (over)
+      kept_types = "#ifdef POLY_HOST_ADDRESS_CHECK\n#define POLY_FRESH(lane)\n#else\n#define POLY_FRESH(lane) asm volatile(\"\" : \"+v\"(lane)); lane &= 1023\n#endif\n"
+                   "// N steps of a row, the first L of them in LDS\ntemplate <typename T, int N, int L> struct poly_row_kept {\n"
+                   "  T reg[N > L ? N - L : 1];\n  T *lds;\n"
+                   "  __device__ __forceinline__ T &operator[](int i) { return i < L ? lds[i * 1024 + threadIdx.x] : reg[i - L]; }\n};\n";
+    auto declare = [&](const std::string &name, const std::string &type, int nit, int bytes) {
+      int in_lds = 0;
+      while (over && dwords > kRowChainKept1024 && in_lds < nit && lds_left >= 1024 * bytes) { in_lds++; lds_left -= 1024 * bytes; dwords -= (bytes + 3) / 4; }
+      if (in_lds) {
+        kept_types += strf("typedef poly_row_kept<%s, %d, %d> kept_%s;\n", type.c_str(), nit, in_lds, name.c_str());
+        kept_decls += strf("    __shared__ %s lds_%s[%d];\n    kept_%s %s;\n    %s.lds = lds_%s;\n", type.c_str(), name.c_str(), in_lds * 1024, name.c_str(), name.c_str(), name.c_str(), name.c_str());
+      } else {
+        kept_types += strf("typedef %s kept_%s[%d];\n", type.c_str(), name.c_str(), nit);
+        kept_decls += strf("    kept_%s %s;\n", name.c_str(), name.c_str());
+      }
+    };
+    for (const RowKept &k : rows_kept) declare(k.name, k.type, row_nit, k.bytes);
+    for (size_t ci = 0; ci < cache.size(); ci++) declare(strf("c%zu", ci), cache[ci].type, cache[ci].nit, cache[ci].bytes);
+    if (over) strat += ", kept rows partly in LDS";
+  }
   // (threads: the workgroup's size; a row per wave or half wave means threads / G rows per workgroup)
   auto body_for = [&](int threads) {
     std::string b = strf("extern \"C\" __global__ void __launch_bounds__(%d) poly_k(%s) {\n", threads, sig.c_str());
@@ -1376,8 +1423,7 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
     } else {
       b += "  const int lane = threadIdx.x;\n  const long long row = blockIdx.x;\n  {\n";
     }
-    for (size_t ci = 0; ci < cache.size(); ci++) b += strf("    %s c%zu[%d];\n", cache[ci].type.c_str(), ci, cache[ci].nit);
-    b += row_decls;
+    b += kept_decls;
     b += calls + "  }\n}\n";
     return b;
   };
@@ -1389,7 +1435,7 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
   out->arg_slots = arg_slots;
   RenderedKernel &rk = out->rk;
   rk = RenderedKernel();
-  rk.source = std::string(hip_prelude()) + code + body;
+  rk.source = std::string(hip_prelude()) + kept_types + code + body;
   rk.entry = "poly_k";
   rk.launch.grid[0] = (unsigned)(G >= 256 ? rows : G == 32 ? std::ceil(rows / 8) : std::ceil(rows / 4));
   rk.launch.block[0] = (unsigned)std::max(256, G);
@@ -1421,7 +1467,7 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
       LaunchSpec ls = rk.launch;
       ls.grid[0] = (unsigned)std::ceil(rows / (double)(threads / G));
       ls.block[0] = (unsigned)threads;
-      rk.variants.push_back({strf("rows_wg%d", threads), std::string(hip_prelude()) + code + body_for(threads),
+      rk.variants.push_back({strf("rows_wg%d", threads), std::string(hip_prelude()) + kept_types + code + body_for(threads),
                              rk.strategy + strf(", workgroups of %d threads", threads), ls});
     }
   }
