@@ -1164,6 +1164,21 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   // tile of 64 across) stay with the template that stages through registers.
   Dma chosen{0, 0, 0, 0, 0};
   bool dma_ok = !fixed_tile;
+  // A product whose depth is dealt to workgroups anyway: 256x256 tiles, one workgroup of 8 waves to a
+  // CU, dealt to as many as fill at least 13 of 16 CUs, where a part keeps a depth of 4096 and the
+  // edges pad little.  128x256 tiles dealt to half as many leave a CU one workgroup of 4
+  // waves, half of what it holds (4096x1024x100608, a vocabulary projection's gradient of two planes:
+  // 961 -> 730 us; more parts, so no less exact: 1.44e-6 -> 1.02e-6 against float64).  Shorter parts
+  // do not pay for twice the partial sums (4096x1024x8192 in four 101 us, in two 88).
+  if (S > 1 && dma_ok && BM * BN < 256 * 256 && !getenv("POLY_HIP_MM_TILE") && !measurement_env("POLY_HIP_MM_KSPLIT")) {
+    const int64_t t = ((M + 255) / 256) * ((N + 255) / 256);
+    Dma probe{0, 0, 0, 0, 0};
+    for (int s = 16; s > S && t * 65536 <= 1.1 * (double)M * (double)N; s--) {
+      if (t * Z * s > 256 || t * Z * s < 208 || (K / 32) % s != 0 || K / s < 4096 || !dma_for(256, 256, &probe)) continue;
+      S = s;
+      BM = BN = 256; WVM = 4; WVN = 2; pipe = 2;
+    }
+  }
   if (!fixed_tile && !getenv("POLY_HIP_MM_TILE") && BM * BN <= 128 * 256) {
     Dma probe{0, 0, 0, 0, 0};
     auto count = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * Z * S; };   // workgroups of the launch
@@ -1178,8 +1193,11 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     Dma small{0, 0, 0, 0, 0};
     const int64_t t64 = count(64, 64), t128 = count(64, 128);
     if (S == 1 && K >= 256 && !getenv("POLY_HIP_NO_SMALL_TILES")) {
+      // (on a depth of 2048 and more 128x128 tiles on three quarters of the CUs are ahead of two
+      // 64x128 to a CU: 3072x1024x4096 in every layout 37-40 us on the small ones, 30-32 on
+      // the large; 2048x1536x1024 12.8 on either)
       if (t64 <= 256) small = t64 > 192 ? Dma{64, 4, 2, 2, 2} : Dma{64, 6, 1, 2, 2};
-      else if (t128 <= 448) small = t128 > 256 ? Dma{64, 3, 2, 2, 2} : Dma{64, 4, 1, 2, 2};
+      else if (t128 <= 448 && !(K >= 2048 && count(128, 128) >= 192 && count(128, 128) <= 256)) small = t128 > 256 ? Dma{64, 3, 2, 2, 2} : Dma{64, 4, 1, 2, 2};
     }
     if (small.bk && dma_for(64, t64 <= 256 ? 64 : 128, &small)) { BM = 64; BN = t64 <= 256 ? 64 : 128; WVM = WVN = 2; chosen = small; }
     else if (dma_for(BM, BN, &probe)) {
