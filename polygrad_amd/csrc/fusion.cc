@@ -1071,6 +1071,7 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
   }
   // master row decomposition: fastest row range = smallest stride in the first result
   std::string row_decomp;
+  std::vector<int> row_ords;        // the row's ranges, the fastest first
   {
     std::vector<std::pair<int64_t, int>> keyed;
     for (int r : gA.stores[0].ranges) {
@@ -1078,6 +1079,7 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
       keyed.push_back({it == results[0].second.c.end() ? ((int64_t)1 << 50) : std::abs(it->second), r});
     }
     std::sort(keyed.begin(), keyed.end());
+    for (auto &k : keyed) row_ords.push_back(k.second);
     row_decomp += "  long long t_ = row;\n";
     for (size_t i = 0; i < keyed.size(); i++) {
       const int ord = keyed[i].second;
@@ -1451,6 +1453,44 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
   out->row_chain_from = a_item;
   {
     const KernelGraph &gl = sc.graphs[(size_t)phases.back().m.item];
+    // what a product that computes the rows itself takes: the last map's rows one after another
+    const RowPhase &last = phases.back();
+    Aff at;
+    bool dense = G <= 64 && last.is_map && n_exported == 0 && !narrow_stored && kept_types.find("poly_row_kept") == std::string::npos;
+    if (dense && last.m.range_expr.empty()) dense = store_aff(last.m, &at, true);
+    else if (dense) {       // (a flat map stores at the positions of the latest row)
+      dense = false;
+      for (size_t r = results.size(); r-- > 0 && !dense;) if (row_result[r]) { at = results[r].second; dense = true; }
+    }
+    int64_t stride = R;
+    dense = dense && at.c0 == 0 && at.c.count(red_master) && at.c[red_master] == 1;
+    if (dense) at.c.erase(red_master);
+    for (int ord : row_ords) {
+      const int64_t e = mext[(size_t)ord];
+      if (!dense || e == 1) { at.c.erase(ord); continue; }
+      dense = at.c.count(ord) && at.c[ord] == stride;
+      at.c.erase(ord);
+      stride *= e;
+    }
+    if (dense && at.c.empty()) {
+      // (its arguments under other names: the product's are fa<n>, too)
+      std::string text = kept_decls + calls;
+      for (size_t i = 0; (i = text.find("fa", i)) != std::string::npos; i++)
+        if ((i == 0 || !(isalnum((unsigned char)text[i - 1]) || text[i - 1] == '_')) && isdigit((unsigned char)text[i + 2])) text[i] = 'r';
+      for (size_t i = 0; (i = text.find('\n', i)) != std::string::npos;) text[i] = ' ';
+      std::string params;
+      for (size_t j = 1; j < arg_slots.size(); j++) {
+        const size_t name = sig.find(strf(" fa%zu", j)), from = sig.rfind(',', name) == std::string::npos ? 0 : sig.rfind(',', name) + 2;
+        params += (j > 1 ? ", " : "") + sig.substr(from, name - from) + strf(" ra%zu", j);
+      }
+      out->rows.code = kept_types + code;
+      out->rows.params = params;
+      out->rows.call = "{ " + strf("%s *const ra0 = poly_rows_out; ", dt_cname(gl.n(gl.stores[0].param).dt)) + text + "}";
+      out->rows.n_params = (int)arg_slots.size() - 1;
+      out->rows.lanes = G;
+      out->n_rows = (int64_t)rows;
+      out->row_len = R;
+    }
     out->row_chain_stores = phases.back().is_map ? sc.slot(phases.back().m.item, gl.param_slot(gl.stores[0].param)) : -1;
   }
   rk.n_params = (int)arg_slots.size();
@@ -3094,6 +3134,60 @@ void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &gr
     (*out)[gi] = std::move(attention);
     if (pj < n0) (*out)[pj] = std::move(product);
     else accept(product, taken);
+  }
+  // A row chain over up to 16 rows (the LayerNorms of a short prompt) in front of the one product that
+  // reads its rows: a launch of two workgroups, 2-3 us and as much as that between two launches that
+  // depend on each other.  The product's workgroups compute the rows themselves, each all of
+  // them, while the first loads of their weights are on the way.
+  for (size_t gi = 0; gi < out->size() && !getenv("POLY_HIP_NO_ROWS_IN_PRODUCT"); gi++) {
+    const FusedGroup &chain = (*out)[gi];
+    const int slot = chain.row_chain_stores;
+    if (chain.rows.code.empty() || chain.n_rows > 16 || chain.needs_group_at >= 0 || slot < 0 || !s->buf_slots[slot].is_intermediate) continue;
+    if (sc.writers[(size_t)slot].size() != 1 || sc.readers[(size_t)slot].size() != 1 || chain.arg_slots.empty() || chain.arg_slots[0] != slot) continue;
+    const int reader = sc.readers[(size_t)slot][0];
+    size_t pj = out->size();
+    for (size_t j = 0; j < out->size(); j++)
+      if (std::find((*out)[j].items.begin(), (*out)[j].items.end(), reader) != (*out)[j].items.end()) pj = j;
+    if (pj < out->size() && ((*out)[pj].matched_from != reader || (*out)[pj].rk.klass != KernelClass::MATMUL_MFMA || (*out)[pj].needs_group_at >= 0)) continue;
+    if (pj == out->size() && taken[(size_t)reader]) continue;
+    const KernelGraph &gr = graphs[(size_t)reader];
+    MatmulMatch mm;
+    if (!match_matmul(gr, &mm, nullptr) || sc.slot(reader, mm.A.param) != slot || mm.M != chain.n_rows || mm.K != chain.row_len || mm.Z != 1) continue;
+    int reads = 0;
+    for (const KNode &k : gr.nodes) reads += k.op == POLY_OP_LOAD && sc.slot(reader, gr.param_slot(gr.n(k.src[0]).src[0])) == slot;
+    if (reads != 1) continue;
+    FusedGroup product;
+    matmul_hint_a_rows(&chain.rows);
+    bool done;
+    if (pj < out->size()) {
+      std::vector<char> free_again = taken;
+      for (int it : (*out)[pj].items) free_again[(size_t)it] = 0;
+      done = match_matmul_tail(sc, reader, free_again, &product) && product.items == (*out)[pj].items && product.launch_item == (*out)[pj].launch_item;
+    } else {
+      const PolyExecItem &ri = s->items[reader];
+      std::string err;
+      done = render_kernel(gr, "poly_k", RenderOptions(), &product.rk, &err) && product.rk.guards.empty() && product.rk.n_vars == 0;
+      product.items = {reader};
+      product.launch_item = reader;
+      product.arg_slots.assign(ri.buf_slot_indices, ri.buf_slot_indices + ri.n_buf_slots);
+    }
+    matmul_hint_a_rows(nullptr);
+    const size_t a_at = (size_t)(std::find(product.arg_slots.begin(), product.arg_slots.end(), slot) - product.arg_slots.begin());
+    if (!done || !product.rk.computes_rows || !product.rk.pres.empty() || product.rk.scratch_bytes != 0 || a_at >= product.arg_slots.size()) continue;
+    product.arg_slots.erase(product.arg_slots.begin() + (long)a_at);
+    product.arg_slots.insert(product.arg_slots.begin() + (long)a_at, chain.arg_slots.begin() + 1, chain.arg_slots.end());
+    if (product.rk.n_params != (int)product.arg_slots.size()) continue;
+    product.items.insert(product.items.begin(), chain.items.begin(), chain.items.end());
+    product.internal_slots.insert(product.internal_slots.end(), chain.internal_slots.begin(), chain.internal_slots.end());
+    product.internal_slots.push_back(slot);
+    product.rk.strategy += strf(" (%s)", chain.rk.strategy.c_str());
+    std::vector<FusedGroup> with;
+    for (size_t j = 0; j < out->size(); j++) if (j != gi && j != pj) with.push_back((*out)[j]);
+    with.push_back(product);
+    if (!fused_groups_out_of_order(s, graphs, with).empty()) continue;
+    taken[(size_t)reader] = 1;
+    *out = std::move(with);
+    gi = (size_t)-1;       // (the groups have moved)
   }
   // every pair of items that share a buffer keeps its order; a group that breaks one is
   // dropped and its kernels launch one by one at their own places

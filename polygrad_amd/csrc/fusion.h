@@ -17,6 +17,11 @@ struct FusedGroup {
   RenderedKernel rk;
   // a row chain: the item it was grown from and the buffer its last kernel stores (-1: none)
   int row_chain_from = -1, row_chain_stores = -1;
+  // ... what a product that computes those rows itself needs of it (rows.code empty: its rows are not
+  // dealt to at most a wave each, or it stores more than them): `n_rows` rows of `row_len`
+  // elements, stored row after row; the arguments behind the first are its parameters
+  MatmulRows rows;
+  int64_t n_rows = 0, row_len = 0;
   // Two groups that only work together (a chain that stores bf16 values into an fp32 buffer
   // and the product that reads them as such) name each other's launch item here: dropping
   // one drops the other.

@@ -17,6 +17,10 @@
 //                       z * POLY_KSPLIT + part): each leaves its sum where POLY_EPILOGUE puts
 //                       it, which may use `poly_ks`, the part
 //   POLY_A_KC/B_KC      1: operand contiguous along K; 0: along M (resp. N)
+//   POLY_A_ROWS(row, lane, out)  (optional, one z, M <= 16, A contiguous along K in rows of K
+//                       elements) A is no buffer: this leaves element f of its row `row` at
+//                       out[row * K + f], called by POLY_A_ROW_LANES (32 or 64) lanes; and
+//                       POLY_A_UNREAD, which declares the pointer A would have had
 //   POLY_A_PTR/B_PTR, poly_a_row(m), poly_b_row(n), poly_a_z(z), poly_b_z(z),
 //   poly_a_k(k), poly_b_k(k), POLY_SIGNATURE, POLY_EPILOGUE(acc, m, n, z) and
 //   optionally POLY_EP_MID_VALUE / POLY_EP_MID_PTR: as in matmul_mfma.hip
@@ -151,6 +155,26 @@ template <int T> struct PolyOp<false, T> {
 #endif
 };
 
+#ifdef POLY_A_ROWS
+// Rows in LDS, 16 bytes further apart than they are long: the 16 lanes that read a chunk of 16
+// rows meet 16 different 16-byte slots of the banks.  K is a multiple of KV.
+#define POLY_ROW_PAD (16 / (int)sizeof(POLY_TIN))
+struct PolyOpRows {
+  PolyRow<POLY_KV> r[1];
+  template <class K> __device__ __forceinline__ void load(const POLY_TIN *base, const int (&row)[1], int k, K) {
+    r[0] = __builtin_bit_cast(PolyRow<POLY_KV>, *(const poly_u32x4 *)(base + row[0] + k));
+  }
+  template <class K> __device__ __forceinline__ void load_end(const POLY_TIN *base, const int (&row)[1], int k, K kofs) {
+    if (k < POLY_KPART) load(base, row, k, kofs);
+    else r[0] = PolyRow<POLY_KV>{};
+  }
+  __device__ __forceinline__ POLY_TIN at(int t, int e) const { return r[0].v[e]; }
+#if !POLY_F32
+  __device__ __forceinline__ poly_in8 frag(int t) const { return __builtin_bit_cast(poly_in8, r[0]); }
+#endif
+};
+#endif
+
 extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATURE) {
   // Workgroup ids congruent mod 8 run on one XCD (own L2): each XCD gets a contiguous run of
   // tiles, down the rows first, so that the workgroups that read one panel of B share an L2.
@@ -170,7 +194,13 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
 #endif
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int col = lane % POLY_BLOCK, grp = lane / POLY_BLOCK;
+#ifdef POLY_A_ROWS
+  POLY_A_UNREAD;
+  __shared__ __attribute__((aligned(16))) POLY_TIN gA[16 * (POLY_K + POLY_ROW_PAD)];
+  static_assert(POLY_TM == 1 && POLY_BLOCK == 16 && POLY_M <= 16 && POLY_KSPLIT == 1 && POLY_K % POLY_KV == 0, "one tile of whole rows");
+#else
   const POLY_TIN *__restrict__ gA = POLY_A_PTR + poly_a_z(z);
+#endif
   const POLY_TIN *__restrict__ gB = POLY_B_PTR + poly_b_z(z);
 
   // Rows of A (columns of B) of a lane.  Along K: block t has row POLY_BLOCK t + col; rows past the
@@ -178,7 +208,10 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
   // one of each block; a lane whose T rows cross the edge starts T rows before it, and its
   // block t then has row T col + t - (shift), which another lane's block has too unless
   // t >= shift: only that one is stored.
-#if POLY_A_KC
+#ifdef POLY_A_ROWS
+  int a_row[1];
+  a_row[0] = (col < POLY_M ? col : POLY_M - 1) * (POLY_K + POLY_ROW_PAD);
+#elif POLY_A_KC
   int a_row[POLY_TM];
 #pragma unroll
   for (int t = 0; t < POLY_TM; t++) { const int m = m0 + POLY_BLOCK * t + col; a_row[t] = poly_a_row(m < POLY_M ? m : POLY_M - 1); }
@@ -194,7 +227,11 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
   int b_row[1];
   { const int n = n0 + POLY_TN * col; b_row[0] = poly_b_row(n <= POLY_N - POLY_TN ? n : POLY_N - POLY_TN); }
 #endif
+#ifdef POLY_A_ROWS
+  typedef PolyOpRows OpA;
+#else
   typedef PolyOp<POLY_A_KC, POLY_TM> OpA;
+#endif
   typedef PolyOp<POLY_B_KC, POLY_TN> OpB;
   auto ka = [&](int k) { return poly_a_k(k_base + k); };
   auto kb = [&](int k) { return poly_b_k(k_base + k); };
@@ -239,21 +276,34 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
   OpB rb[D];
   const int kl = wave * POLY_KSTEP + grp * POLY_KV;
   // (fenced: the compiler would move every load down to its use)
-  auto load = [&](int d, int s) {
+  auto load = [&](int d, int s, bool a = true, bool b = true) {
     __builtin_amdgcn_sched_barrier(0);
     if (END && s == 0) {
       const int k = kl + STEPS * (POLY_KSTEP * POLY_WAVES);
-      ra[d].load_end(gA, a_row, k, ka);
-      rb[d].load_end(gB, b_row, k, kb);
+      if (a) ra[d].load_end(gA, a_row, k, ka);
+      if (b) rb[d].load_end(gB, b_row, k, kb);
     } else {
       const int k = kl + (s - END) * (POLY_KSTEP * POLY_WAVES);
-      ra[d].load(gA, a_row, k, ka);
-      rb[d].load(gB, b_row, k, kb);
+      if (a) ra[d].load(gA, a_row, k, ka);
+      if (b) rb[d].load(gB, b_row, k, kb);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
+#ifdef POLY_A_ROWS
+  // A's rows while B's first steps are on their way
+#pragma unroll
+  for (int s = 0; s < (ALL < D ? ALL : D); s++) load(s, s, false, true);
+  for (int row = wave * (64 / POLY_A_ROW_LANES) + lane / POLY_A_ROW_LANES; row < POLY_M; row += POLY_WAVES * (64 / POLY_A_ROW_LANES)) {
+    POLY_TIN *const to = gA + row * POLY_ROW_PAD;
+    POLY_A_ROWS((long long)row, lane % POLY_A_ROW_LANES, to);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < (ALL < D ? ALL : D); s++) load(s, s, true, false);
+#else
 #pragma unroll
   for (int s = 0; s < (ALL < D ? ALL : D); s++) load(s, s);
+#endif
   constexpr int STEADY = ALL > 2 * D ? (ALL - D) / D * D : 0;
 #pragma unroll 1
   for (int s = 0; s < STEADY; s += D) {

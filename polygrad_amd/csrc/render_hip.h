@@ -83,6 +83,7 @@ struct RenderedKernel {
   // own scratch memory, `scratch_offset` bytes in, and the plan hands this kernel that
   // address as its scratch pointer (`scratch_of_item`: the reader's launch item; -1: none).
   bool writes_block_maxima = false;
+  bool computes_rows = false;      // a product that computes the rows of its operand A (matmul_hint_a_rows)
   int scratch_of_item = -1;
   size_t scratch_offset = 0;
   // Kernels in two stages (reductions through partial results, matmuls whose operands are

@@ -534,6 +534,8 @@ static bool epilogue_from_graph(const KernelGraph &g, const MatmulMatch &mm, Mat
   return true;
 }
 
+static thread_local const MatmulRows *g_a_rows = nullptr;
+void matmul_hint_a_rows(const MatmulRows *rows) { g_a_rows = rows; }
 static thread_local MatmulEpilogue::BlockMaxima g_block_maxima;
 static thread_local int64_t g_block_maxima_rows = 0, g_block_maxima_pitch = 0;
 void matmul_hint_block_maxima(const MatmulEpilogue *e, int64_t rows, int64_t pitch) {
@@ -749,6 +751,20 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
     return (is_a ? dims.back().ca : dims.back().cb) == 1 && rows >= run && (dims.size() == 1 || dims.back().extent % run == 0);
   };
   if (Z > 65535 || M > 2147483647LL / 2 || N > 2147483647LL / 2 || K > 2147483647LL / 2) return false;
+  // Rows that the product computes itself: of all rows one tile, row-major, in LDS beside the
+  // partial sums, on no more workgroups than CUs (each computes the rows again).  Against a launch of their own:
+  // see there.
+  std::string signature = ep.signature;
+  if (g_a_rows) {
+    if (M > 16 || f.tm != 1 || f.block != 16 || S != 1 || mm.ka.s_lo != 1 || mm.ka.kb < K || mm.md.size() != 1 || mm.md[0].ca != K || mm.a_c0 != 0 || !mm.zd.empty() ||
+        K % kv != 0 || K * dt_size(mm.A.dt) > 4096 || tiles_of(f.tm, f.tn) > 256 || ep.a_ptr == ep.b_ptr)
+      return false;
+    // (A's parameter: from behind the comma in front of it to the one behind it)
+    const size_t name = (signature + ",").find(" " + ep.a_ptr + ",");
+    if (name == std::string::npos) return false;
+    const size_t from = signature.rfind(',', name) == std::string::npos ? 0 : signature.rfind(',', name) + 2;
+    signature.replace(from, name + 1 + ep.a_ptr.size() - from, g_a_rows->params);
+  }
   auto render = [&](const Form &f, RenderedKernel *out) {
     bool a_kc, b_kc;
     if (!layout(mm.ka, mm.md, true, M, f.tm, &a_kc) || !layout(mm.kb, mm.nd, false, N, f.tn, &b_kc)) return false;
@@ -771,8 +787,11 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
       cfg += offset_fn("poly_a_z", mm.zd, true, mm.a_c0) + offset_fn("poly_b_z", mm.zd, false, mm.b_c0);
     }
     cfg += matmul_k_fn("poly_a_k", mm.ka, K) + matmul_k_fn("poly_b_k", mm.kb, K);
-    const std::string shape = strf("#define POLY_SIGNATURE %s%s\n#define POLY_KSPLIT %d\n#define POLY_PARTIALS poly_scratch\n", ep.signature.c_str(), S > 1 ? ", float* poly_scratch" : "", S) + ep.code;
+    const std::string shape = strf("#define POLY_SIGNATURE %s%s\n#define POLY_KSPLIT %d\n#define POLY_PARTIALS poly_scratch\n", signature.c_str(), S > 1 ? ", float* poly_scratch" : "", S) + ep.code;
     cfg += shape;
+    if (g_a_rows)      // (the epilogue's functions take every parameter of their kernels: A's is not read)
+      cfg += g_a_rows->code + strf("#define POLY_A_ROWS(row, lane, poly_rows_out) %s\n#define POLY_A_ROW_LANES %d\n#define POLY_A_UNREAD const %s *const %s = nullptr; (void)%s\n",
+                                   g_a_rows->call.c_str(), g_a_rows->lanes, dt_cname(mm.A.dt), ep.a_ptr.c_str(), ep.a_ptr.c_str());
     // what the kernel that has an element's whole sum does with it
     std::string finish = strf("#define POLY_EPILOGUE(acc, m, n, z) %s\n", ep.call.c_str());
     if (!ep.mid_value_call.empty())
@@ -804,12 +823,19 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
                          (long long)M, (long long)N, (long long)K, (long long)Z, bm, bn, f.waves, sums == 2 ? " of two sums each" : "", a_kc ? "k-major" : "m-major", b_kc ? "k-major" : "n-major");
     if (S > 1) out->strategy += strf(", K dealt to %d workgroups per tile, partial results added by a second kernel", S);
     out->n_params = ep.n_params;
+    if (g_a_rows) {
+      if (!a_kc) return false;
+      out->computes_rows = true;
+      out->n_params += g_a_rows->n_params - 1;
+      out->strategy += ", which compute A's rows first";
+    }
     out->n_vars = 0;
     out->flops = 2.0 * (double)M * (double)N * (double)K * (double)Z;
     out->bytes = ep.bytes;
     return true;
   };
   if (!render(f, out)) return false;
+  if (g_a_rows) return true;
   // The other tiles and depths of loads as tuning candidates.  Which steps of the depth a wave
   // adds up, and in what order, depends on the waves and sums alone, so these stay.
   if (matmul_tuning_enabled() && S == 1) {

@@ -105,6 +105,16 @@ void matmul_hint_input_params(uint64_t mask);
 // that takes the buffer as a plain operand can read that, and render_kernel refuses every
 // other use.
 void matmul_hint_param_kinds(const std::vector<int> &kinds);
+// Also set around a lowering: operand A's rows, a buffer nothing else reads, are computed by the
+// product itself (a LayerNorm in front of it).  `call` leaves row `row` (`lane` of `lanes`, 32 or 64) at
+// poly_rows_out[row * K + f]; `params`, `n_params` of them, stand in A's place in the signature.
+// Products of up to 16 rows that the template whose waves deal the depth takes do that
+// (RenderedKernel::computes_rows says whether this one does).
+struct MatmulRows {
+  std::string code, params, call;
+  int n_params = 0, lanes = 64;
+};
+void matmul_hint_a_rows(const MatmulRows *rows);
 // Also set around a lowering: a later launch wants the block maxima of this product's
 // output, which it takes for a row-major matrix of `rows` x `pitch` elements from element 0
 // of the buffer (nullptr: no such wish).  The product grants it when its store is that.
