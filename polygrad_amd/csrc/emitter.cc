@@ -75,13 +75,13 @@ __device__ __forceinline__ void poly_vstore(T *p, const poly_vec<T, N> &r) {
 // 2^-149).  v_div_fixup gives a zero dividend the sign the quotient has.  Dividends beyond
 // 2^26, non-finite ones and every dividend of a divisor outside the range take the full
 // division.  Four instructions instead of eleven per quotient.
+__device__ __forceinline__ float poly_div_sure(float x, float d, float r) {
+  const float q = x * r;
+  const float e = __builtin_fmaf(-q, d, x);
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(e, r, q), d, x);
+}
 __device__ __forceinline__ float poly_div_shared(float x, float d, float r, bool ok) {
-  if (ok && __builtin_fabsf(x) <= 0x1p+26f) {
-    const float q = x * r;
-    const float e = __builtin_fmaf(-q, d, x);
-    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(e, r, q), d, x);
-  }
-  return x / d;
+  return ok && __builtin_fabsf(x) <= 0x1p+26f ? poly_div_sure(x, d, r) : x / d;
 }
 
 // ── wave64 reductions: DPP inside a row of 16 lanes, ds_swizzle across rows of

@@ -2326,8 +2326,10 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
     const int64_t units = f32 ? (mS.N + 15) / 16 : (mS.N + 31) / 32;
     int waves = units <= 1 ? 1 : units <= 2 ? 2 : units <= 16 ? 4 : 8;
     int qt = mS.Z * ((mS.M + 31) / 32) >= 512 ? 2 : 1;
+    bool near = true;
+    for (int sl : inputs) near = near && s->buf_slots[sl].nbytes <= (int64_t)1 << 32;
     if (const char *ov = measurement_env("POLY_HIP_FA_ROWS")) sscanf(ov, "%d,%d", &waves, &qt);   // "WAVES,QT": tuning experiments
-    fa_cfg = strf("#define POLY_F32 %d\n#define POLY_FA_WAVES %d\n#define POLY_FA_QT %d\n#define POLY_FA_PASS_ZEROS %d\n", f32 ? 1 : 0, waves, qt, whole_blocks ? 1 : 0) + cfg;
+    fa_cfg = strf("#define POLY_F32 %d\n#define POLY_FA_WAVES %d\n#define POLY_FA_QT %d\n#define POLY_FA_PASS_ZEROS %d\n#define POLY_FA_NEAR %d\n", f32 ? 1 : 0, waves, qt, whole_blocks ? 1 : 0, near ? 1 : 0) + cfg;
     rk.launch.grid[0] = (unsigned)(((mS.M + 16 * qt - 1) / (16 * qt)) * mS.Z);
     rk.launch.block[0] = (unsigned)(64 * waves);
     rk.strategy = strf("fused attention (%zu kernels): mfma %s Z=%lld M=%lld N=%lld D=64, one pass, scores of %d queries in registers, keys dealt to %d waves, exact roundings", all.size() + copy_items.size(),

@@ -18,6 +18,8 @@
 //                                      non-finite V under them does not propagate, as in the
 //                                      single-pass form of attention_mfma.hip, whose shapes
 //                                      these are); 0: it is, as in the unfused kernels
+//   POLY_FA_NEAR                       1: no byte of Q, K and V is 2^32 or more from its start
+//   POLY_FA_C                          POLY_FA_TERM(x, mx, ..) is exp2((x - mx) * C), C > 0
 //   POLY_Q_PTR, POLY_K_PTR, POLY_V_PTR, poly_q_off(z, m), poly_k_off(z, n), poly_v_off(z, n),
 //   POLY_FA_SCORE(acc, m, n, z), POLY_FA_MAXV(x, m, n, z), POLY_FA_TERM(x, mx, m, n, z),
 //   POLY_FA_OUT(acc, m, d, z), POLY_SIGNATURE: as in attention_mfma.hip
@@ -33,9 +35,11 @@
 // are read from the L2 by every query block.  One launch against the launches it replaces
 // (bf16, us): 12 heads of 12 queries and keys 4.1 against eight of 3 to 4 each, 36 of 345 16.3
 // [34.2 in three], 36 of 839 61.2 [146 in three]; GPT-2 small on 12 tokens 655 -> 502 us as a
-// whole.  What bounds it where rows are long is the arithmetic on the scores (some forty
-// vector instructions each), masked ones included, and what it keeps in registers: two
-// waves a SIMD.
+// whole.  What bounds it where rows are long is the arithmetic on the scores (some thirty
+// vector instructions each) and what it keeps in registers: two to four waves a SIMD.  The
+// scores of masked keys are computed, but not the terms and quotients of units that have no
+// other: with that, divisions that a wave decides on together and 32-bit addresses, 36 heads of 345
+// keys take 16.0 us inside GPT-2 small where they took 17.4.
 #ifdef POLY_TEMPLATE_STANDALONE
 #include <hip/hip_runtime.h>
 #define POLY_TIN __bf16
@@ -57,7 +61,10 @@ __device__ __forceinline__ int poly_v_off(int z, int n) { return (z / 12) * 7948
 #define POLY_FA_SCORE(acc, m, n, z) ((__bf16)((float)(__bf16)(acc) * 0.125f + (float)data2[(m) * 345 + (n)]))
 #define POLY_FA_MAXV(x, m, n, z) ((float)(x))
 #define POLY_FA_TERM(x, mx, m, n, z) __builtin_amdgcn_exp2f(((float)(x) - (mx)) * 0x1.715476p+0f)
+#define POLY_FA_C 0x1.715476p+0f
+#define POLY_FA_NEAR 1
 __device__ __forceinline__ float poly_div_shared(float x, float d, float r, bool ok) { return x / d; }
+__device__ __forceinline__ float poly_div_sure(float x, float d, float r) { return x * r; }
 #define POLY_FA_OUT(acc, m, d, z) data0[((z) / 12) * 264960 + ((z) % 12) * 22080 + (m) * 64 + (d)] = (__bf16)(acc)
 #endif
 
@@ -80,6 +87,14 @@ typedef unsigned int fr_u32x4 __attribute__((ext_vector_type(4)));
 #define FR_UW ((FR_UNITS + POLY_FA_WAVES - 1) / POLY_FA_WAVES)   // units of a wave: unit u of wave w is u * WAVES + w
 #define FR_DEPTH (FR_UW < 4 ? FR_UW : 4)          // units whose loads are in flight at a time
 #define FR_BM (16 * POLY_FA_QT)
+
+// Element `off` of a buffer: 32-bit byte offsets from its start where they reach all of it, which
+// the load instructions add to a scalar base themselves.
+#if POLY_FA_NEAR
+#define FR_AT(p, off) ((const POLY_TIN *)((const char *)(p) + (size_t)((unsigned)(off) * (unsigned)sizeof(POLY_TIN))))
+#else
+#define FR_AT(p, off) ((p) + (off))
+#endif
 
 // T consecutive elements of any alignment.
 template <int T> struct __attribute__((aligned(sizeof(POLY_TIN)))) FrRow { POLY_TIN v[T]; };
@@ -116,7 +131,7 @@ extern "C" __global__ void __launch_bounds__(64 * POLY_FA_WAVES) FR_BUDGET poly_
   for (int i = 0; i < POLY_FA_QT; i++) {
     const int m = m0 + 16 * i + col;
     mq[i] = m < POLY_FA_M ? m : POLY_FA_M - 1;
-    const POLY_TIN *p = POLY_Q_PTR + poly_q_off(z, mq[i]) + FR_KV * grp;
+    const POLY_TIN *p = FR_AT(POLY_Q_PTR, poly_q_off(z, mq[i]) + FR_KV * grp);
 #pragma unroll
     for (int s = 0; s < FR_STEPS; s++) q[i][s] = *(const FrRow<FR_KV> *)(p + 4 * FR_KV * s);
   }
@@ -141,7 +156,7 @@ extern "C" __global__ void __launch_bounds__(64 * POLY_FA_WAVES) FR_BUDGET poly_
 #pragma unroll
       for (int b = 0; b < FR_BU; b++) {
         const int n = block_at(u0 + d, b) + col;
-        const POLY_TIN *p = POLY_K_PTR + poly_k_off(z, key_for(u0 + d, n)) + FR_KV * grp;
+        const POLY_TIN *p = FR_AT(POLY_K_PTR, poly_k_off(z, key_for(u0 + d, n)) + FR_KV * grp);
 #pragma unroll
         for (int s = 0; s < FR_STEPS; s++) k[d][b][s] = *(const FrRow<FR_KV> *)(p + 4 * FR_KV * s);
       }
@@ -185,7 +200,7 @@ extern "C" __global__ void __launch_bounds__(64 * POLY_FA_WAVES) FR_BUDGET poly_
 #pragma unroll
       for (int e = 0; e < 4 * FR_BU; e++) {
         const int n = block_at(u0 + d, e / 4) + 4 * grp + e % 4;
-        v[d][e] = *(const FrRow<4> *)(POLY_V_PTR + poly_v_off(z, key_for(u0 + d, n)) + 4 * col);
+        v[d][e] = *(const FrRow<4> *)FR_AT(POLY_V_PTR, poly_v_off(z, key_for(u0 + d, n)) + 4 * col);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -202,16 +217,32 @@ extern "C" __global__ void __launch_bounds__(64 * POLY_FA_WAVES) FR_BUDGET poly_
   }
   __syncthreads();
   float sum[POLY_FA_QT], rcp[POLY_FA_QT];
-  bool rcp_ok[POLY_FA_QT];
+  bool rcp_ok[POLY_FA_QT], all_ok[POLY_FA_QT];
+  // units (a bit each) whose terms are 0 for all queries of the wave, which masked keys' are, and
+  // units whose terms are all small enough for poly_div_sure
+  unsigned long long dead[POLY_FA_QT], small[POLY_FA_QT];
 #pragma unroll
   for (int i = 0; i < POLY_FA_QT; i++) {
     float t = row_top[0][16 * i + col];
 #pragma unroll
     for (int w = 1; w < POLY_FA_WAVES; w++) t = __builtin_fmaxf(t, row_top[w][16 * i + col]);
     float acc = 0.0f;
+    dead[i] = small[i] = 0;
 #pragma unroll
     for (int u = 0; u < FR_UW; u++) {
       if (!has_unit(u)) continue;
+      // the unit's largest score, NaN if one is, bounds its terms; 2^-151 rounds to 0
+      float most = x[i][u][0][0];
+#pragma unroll
+      for (int e = 1; e < 4 * FR_BU; e++) most = __builtin_elementwise_maximum(most, x[i][u][e / 4][e % 4]);
+      const float power = (most - t) * POLY_FA_C;
+      if (__builtin_amdgcn_ballot_w64(!(power < -151.0f)) == 0) {
+        dead[i] |= 1ull << u;
+#pragma unroll
+        for (int e = 0; e < 4 * FR_BU; e++) x[i][u][e / 4][e % 4] = 0.0f;
+        continue;
+      }
+      if (__builtin_amdgcn_ballot_w64(!(power < 25.0f)) == 0) small[i] |= 1ull << u;
 #pragma unroll
       for (int b = 0; b < FR_BU; b++)
 #pragma unroll
@@ -234,6 +265,7 @@ extern "C" __global__ void __launch_bounds__(64 * POLY_FA_WAVES) FR_BUDGET poly_
     for (int w = 1; w < POLY_FA_WAVES; w++) sum[i] += row_sum[w][16 * i + col];
     rcp[i] = 1.0f / sum[i];
     rcp_ok[i] = __builtin_fabsf(sum[i]) >= 0x1p-100f && __builtin_fabsf(sum[i]) <= 0x1p+100f;
+    all_ok[i] = __builtin_amdgcn_ballot_w64(!rcp_ok[i]) == 0;
   }
 
   // ── P V over the wave's keys: tile t of the output has the features 4 col + t ────────────
@@ -283,10 +315,18 @@ extern "C" __global__ void __launch_bounds__(64 * POLY_FA_WAVES) FR_BUDGET poly_
 #pragma unroll
       for (int i = 0; i < POLY_FA_QT; i++) {
         POLY_TIN p[4 * FR_BU];
+        if (all_ok[i] && (dead[i] >> u & 1)) {
 #pragma unroll
-        for (int e = 0; e < 4 * FR_BU; e++) {
-          const POLY_TIN prob = (POLY_TIN)poly_div_shared(x[i][u][e / 4][e % 4], sum[i], rcp[i], rcp_ok[i]);
-          p[e] = has_key(u, block_at(u, e / 4) + 4 * grp + e % 4) ? prob : (POLY_TIN)0.0f;
+          for (int e = 0; e < 4 * FR_BU; e++) p[e] = (POLY_TIN)0.0f;
+        } else if (all_ok[i] && (small[i] >> u & 1)) {      // (a key that is not there has the term 0)
+#pragma unroll
+          for (int e = 0; e < 4 * FR_BU; e++) p[e] = (POLY_TIN)poly_div_sure(x[i][u][e / 4][e % 4], sum[i], rcp[i]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4 * FR_BU; e++) {
+            const POLY_TIN prob = (POLY_TIN)poly_div_shared(x[i][u][e / 4][e % 4], sum[i], rcp[i], rcp_ok[i]);
+            p[e] = has_key(u, block_at(u, e / 4) + 4 * grp + e % 4) ? prob : (POLY_TIN)0.0f;
+          }
         }
 #if POLY_F32
 #pragma unroll

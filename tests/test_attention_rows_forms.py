@@ -148,3 +148,28 @@ def test_probabilities_below_the_normal_floats(c):
     step = 2.0 ** -133 if w == "bfloat16" else 2.0 ** -149
     bound = (N * step * 1.5 * 2.0 ** 110) + want * (2.0 ** -16 + (2.0 ** -8 if w == "bfloat16" else N * 2.0 ** -24))
     assert float((got - want).abs().max()) <= bound < want / 4, (float(got.min()), float(got.max()), want, bound)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [(1, 2, 70, 100, "bfloat16"), (1, 2, 70, 100, "float16"), (1, 2, 70, 100, "float32"), (1, 16, 1023, 40, "bfloat16")], ids=_name)
+def test_non_finite_rows_and_values(c):
+    """Where a fused unit of keys has no terms but zeros, its values still meet them: an infinite value
+    under a masked key gives NaN as 0 * inf does; a row without any key, and one with a NaN score, are NaN
+    as a whole; rows beside them are what they are without these."""
+    import torch
+    B, H, M, N, w = c
+    D, dt = 64 * H, getattr(torch, w)
+    g = torch.Generator().manual_seed(N)
+    q, k, v = (torch.randn(B, n, D, generator=g).to(dt) for n in (M, N, N))
+    mask = torch.where(torch.arange(N)[None, :] > torch.arange(M)[:, None] % N, -6e4, 0.0)
+    clean = _run(c, q, k, v, mask.to(dt))
+    mask[3], mask[20, 5] = -math.inf, math.nan
+    v[:, N - 1, 7] = math.inf                    # of head 0: under a masked key for all but the rows that see it
+    got = _run(c, q, k, v, mask.to(dt))
+    assert bool(got[:, :, [3, 20]].isnan().all())
+    rows = [m for m in range(M) if m not in (3, 20)]
+    masked = [m for m in rows if m % N < N - 1]
+    assert bool(got[:, 0, masked, 7].isnan().all())
+    got, clean = got[:, :, rows].clone(), clean[:, :, rows].clone()
+    got[:, 0, :, 7] = clean[:, 0, :, 7] = 0.0
+    assert bool((got == clean).all())
