@@ -3137,14 +3137,15 @@ void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &gr
     if (pj < n0) (*out)[pj] = std::move(product);
     else accept(product, taken);
   }
-  // A row chain over up to 16 rows (the LayerNorms of a short prompt) in front of the one product that
-  // reads its rows: a launch of two workgroups, 2-3 us and as much as that between two launches that
-  // depend on each other.  The product's workgroups compute the rows themselves, each all of
-  // them, while the first loads of their weights are on the way.
+  // A row chain over up to 64 rows (the LayerNorms of a short prompt) in front of the one product that
+  // reads its rows: a launch of a few workgroups, 2-3 us and as much as that between two launches that
+  // depend on each other.  The product's workgroups compute the rows themselves, each those of
+  // its tile, while the first loads of their weights are on the way (render_matmul_wave says
+  // on which tiles that pays).
   for (size_t gi = 0; gi < out->size() && !getenv("POLY_HIP_NO_ROWS_IN_PRODUCT"); gi++) {
     const FusedGroup &chain = (*out)[gi];
     const int slot = chain.row_chain_stores;
-    if (chain.rows.code.empty() || chain.n_rows > 16 || chain.needs_group_at >= 0 || slot < 0 || !s->buf_slots[slot].is_intermediate) continue;
+    if (chain.rows.code.empty() || chain.n_rows > 64 || chain.needs_group_at >= 0 || slot < 0 || !s->buf_slots[slot].is_intermediate) continue;
     if (sc.writers[(size_t)slot].size() != 1 || sc.readers[(size_t)slot].size() != 1 || chain.arg_slots.empty() || chain.arg_slots[0] != slot) continue;
     const int reader = sc.readers[(size_t)slot][0];
     size_t pj = out->size();

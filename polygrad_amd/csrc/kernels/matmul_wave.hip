@@ -17,7 +17,7 @@
 //                       z * POLY_KSPLIT + part): each leaves its sum where POLY_EPILOGUE puts
 //                       it, which may use `poly_ks`, the part
 //   POLY_A_KC/B_KC      1: operand contiguous along K; 0: along M (resp. N)
-//   POLY_A_ROWS(row, lane, out)  (optional, one z, M <= 16, A contiguous along K in rows of K
+//   POLY_A_ROWS(row, lane, out)  (optional, one z, A contiguous along K in rows of K
 //                       elements) A is no buffer: this leaves element f of its row `row` at
 //                       out[row * K + f], called by POLY_A_ROW_LANES (32 or 64) lanes; and
 //                       POLY_A_UNREAD, which declares the pointer A would have had
@@ -160,17 +160,19 @@ template <int T> struct PolyOp<false, T> {
 // rows meet 16 different 16-byte slots of the banks.  K is a multiple of KV.
 #define POLY_ROW_PAD (16 / (int)sizeof(POLY_TIN))
 struct PolyOpRows {
-  PolyRow<POLY_KV> r[1];
-  template <class K> __device__ __forceinline__ void load(const POLY_TIN *base, const int (&row)[1], int k, K) {
-    r[0] = __builtin_bit_cast(PolyRow<POLY_KV>, *(const poly_u32x4 *)(base + row[0] + k));
+  PolyRow<POLY_KV> r[POLY_TM];
+  template <class K> __device__ __forceinline__ void load(const POLY_TIN *base, const int (&row)[POLY_TM], int k, K) {
+#pragma unroll
+    for (int t = 0; t < POLY_TM; t++) r[t] = __builtin_bit_cast(PolyRow<POLY_KV>, *(const poly_u32x4 *)(base + row[t] + k));
   }
-  template <class K> __device__ __forceinline__ void load_end(const POLY_TIN *base, const int (&row)[1], int k, K kofs) {
-    if (k < POLY_KPART) load(base, row, k, kofs);
-    else r[0] = PolyRow<POLY_KV>{};
+  template <class K> __device__ __forceinline__ void load_end(const POLY_TIN *base, const int (&row)[POLY_TM], int k, K kofs) {
+    if (k < POLY_KPART) { load(base, row, k, kofs); return; }
+#pragma unroll
+    for (int t = 0; t < POLY_TM; t++) r[t] = PolyRow<POLY_KV>{};
   }
-  __device__ __forceinline__ POLY_TIN at(int t, int e) const { return r[0].v[e]; }
+  __device__ __forceinline__ POLY_TIN at(int t, int e) const { return r[t].v[e]; }
 #if !POLY_F32
-  __device__ __forceinline__ poly_in8 frag(int t) const { return __builtin_bit_cast(poly_in8, r[0]); }
+  __device__ __forceinline__ poly_in8 frag(int t) const { return __builtin_bit_cast(poly_in8, r[t]); }
 #endif
 };
 #endif
@@ -196,8 +198,9 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
   const int col = lane % POLY_BLOCK, grp = lane / POLY_BLOCK;
 #ifdef POLY_A_ROWS
   POLY_A_UNREAD;
-  __shared__ __attribute__((aligned(16))) POLY_TIN gA[16 * (POLY_K + POLY_ROW_PAD)];
-  static_assert(POLY_TM == 1 && POLY_BLOCK == 16 && POLY_M <= 16 && POLY_KSPLIT == 1 && POLY_K % POLY_KV == 0, "one tile of whole rows");
+  __shared__ __attribute__((aligned(16))) POLY_TIN gA[POLY_BM * (POLY_K + POLY_ROW_PAD)];
+  const int n_rows = POLY_M - m0 < POLY_BM ? POLY_M - m0 : POLY_BM;
+  static_assert(POLY_BLOCK == 16 && POLY_KSPLIT == 1 && POLY_K % POLY_KV == 0, "a tile of whole rows");
 #else
   const POLY_TIN *__restrict__ gA = POLY_A_PTR + poly_a_z(z);
 #endif
@@ -209,8 +212,9 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
   // block t then has row T col + t - (shift), which another lane's block has too unless
   // t >= shift: only that one is stored.
 #ifdef POLY_A_ROWS
-  int a_row[1];
-  a_row[0] = (col < POLY_M ? col : POLY_M - 1) * (POLY_K + POLY_ROW_PAD);
+  int a_row[POLY_TM];
+#pragma unroll
+  for (int t = 0; t < POLY_TM; t++) a_row[t] = (16 * t + col < n_rows ? 16 * t + col : n_rows - 1) * (POLY_K + POLY_ROW_PAD);
 #elif POLY_A_KC
   int a_row[POLY_TM];
 #pragma unroll
@@ -293,9 +297,9 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
   // A's rows while B's first steps are on their way
 #pragma unroll
   for (int s = 0; s < (ALL < D ? ALL : D); s++) load(s, s, false, true);
-  for (int row = wave * (64 / POLY_A_ROW_LANES) + lane / POLY_A_ROW_LANES; row < POLY_M; row += POLY_WAVES * (64 / POLY_A_ROW_LANES)) {
-    POLY_TIN *const to = gA + row * POLY_ROW_PAD;
-    POLY_A_ROWS((long long)row, lane % POLY_A_ROW_LANES, to);
+  for (int row = wave * (64 / POLY_A_ROW_LANES) + lane / POLY_A_ROW_LANES; row < n_rows; row += POLY_WAVES * (64 / POLY_A_ROW_LANES)) {
+    POLY_TIN *const to = gA + row * POLY_ROW_PAD - (long long)m0 * POLY_K;
+    POLY_A_ROWS((long long)(m0 + row), lane % POLY_A_ROW_LANES, to);
   }
   __syncthreads();
 #pragma unroll

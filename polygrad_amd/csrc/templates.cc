@@ -751,13 +751,17 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
     return (is_a ? dims.back().ca : dims.back().cb) == 1 && rows >= run && (dims.size() == 1 || dims.back().extent % run == 0);
   };
   if (Z > 65535 || M > 2147483647LL / 2 || N > 2147483647LL / 2 || K > 2147483647LL / 2) return false;
-  // Rows that the product computes itself: of all rows one tile, row-major, in LDS beside the
-  // partial sums, on no more workgroups than CUs (each computes the rows again).  Against a launch of their own:
-  // see there.
+  // Rows that the product computes itself: the tile's, row-major, in LDS beside the partial sums,
+  // on no more workgroups than two to a CU (each computes its rows again), and no more than two rows
+  // one after another per wave: six layers of GPT-2 small on 17 bf16 tokens 224 -> 206 us, on 64 253
+  // -> 238 (one row after another), 12 fp32 342 -> 325 (two); 24 fp32 tokens 339 -> 342 with
+  // four, 128 512 -> 574 with eight.
   std::string signature = ep.signature;
   if (g_a_rows) {
-    if (M > 16 || f.tm != 1 || f.block != 16 || S != 1 || mm.ka.s_lo != 1 || mm.ka.kb < K || mm.md.size() != 1 || mm.md[0].ca != K || mm.a_c0 != 0 || !mm.zd.empty() ||
-        K % kv != 0 || K * dt_size(mm.A.dt) > 4096 || tiles_of(f.tm, f.tn) > 256 || ep.a_ptr == ep.b_ptr)
+    // (partial sums: of the waves, two blocks of rows at a time where 64 KiB hold them)
+    const int part = f.waves * f.tn * 336 * 4, lds = 16 * f.tm * (int)(K * dt_size(mm.A.dt) + 16) + (f.tm % 2 == 0 && 2 * part <= 65536 ? 2 * part : part);
+    if (lds > 160 << 10 || 16 * f.tm * g_a_rows->lanes > 2 * 64 * f.waves || f.block != 16 || S != 1 || mm.ka.s_lo != 1 || mm.ka.kb < K || mm.md.size() != 1 || mm.md[0].ca != K || mm.a_c0 != 0 || !mm.zd.empty() ||
+        K % kv != 0 || K * dt_size(mm.A.dt) > 4096 || tiles_of(f.tm, f.tn) > 256 * std::min(2, (160 << 10) / lds) || ep.a_ptr == ep.b_ptr)
       return false;
     // (A's parameter: from behind the comma in front of it to the one behind it)
     const size_t name = (signature + ",").find(" " + ep.a_ptr + ",");

@@ -1,6 +1,7 @@
-"""LayerNorms over up to 16 rows computed by the product behind them: whole models of one row, of
-odd numbers of rows and of 16, in bf16 (two rows to a wave) and fp32, give the bits they give with a
-launch for each LayerNorm; 17 rows keep the launches."""
+"""LayerNorms over up to 64 rows computed by the product behind them: whole models of one row, of
+odd numbers of rows, of whole tiles of 16 and of one row more, in bf16 (two rows to a wave) and fp32,
+give the bits they give with a launch for each LayerNorm; 65 rows, and fp32 tiles that would have four rows
+to a wave, keep the launches."""
 import ctypes as C
 import os
 import sys
@@ -14,7 +15,8 @@ sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), ".."
 import cases  # noqa: E402
 
 SIZES = [(1, 2, "bfloat16", 768, 4), (1, 12, "bfloat16", 768, 4), (3, 5, "bfloat16", 768, 4), (2, 8, "float32", 768, 4), (1, 7, "float32", 768, 4), (1, 16, "bfloat16", 768, 4),
-         (1, 11, "bfloat16", 256, 4), (1, 17, "bfloat16", 768, 0), (1, 5, "float32", 1024, 0)]
+         (1, 11, "bfloat16", 256, 4), (1, 17, "bfloat16", 768, 4), (3, 21, "bfloat16", 768, 4),
+         (1, 64, "bfloat16", 768, 4), (1, 65, "bfloat16", 768, 0), (1, 17, "float32", 768, 0), (1, 5, "float32", 1024, 0)]
 
 
 def _case(batch, ctx, dtype, d_model):
