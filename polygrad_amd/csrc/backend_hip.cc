@@ -152,8 +152,8 @@ HipRunner *runner_from_rendered(const RenderedKernel &rk, const char *fn_name, b
       if (!p) { runner_destroy(r); return nullptr; }
       r->guards.push_back(p);
     }
-    r->fallback = program_create(r->rk.fallback_source, r->rk.fallback_entry);
-    if (!r->fallback) { runner_destroy(r); return nullptr; }
+    if (!r->rk.fallback_source.empty()) r->fallback = program_create(r->rk.fallback_source, r->rk.fallback_entry);
+    if (!r->rk.fallback_source.empty() && !r->fallback) { runner_destroy(r); return nullptr; }
   }
   if (!r->rk.pres.empty()) {
     if (!r->rk.guards.empty()) { log_err("lower", "%s: a two-stage kernel cannot also be guarded", r->name.c_str()); runner_destroy(r); return nullptr; }
@@ -271,7 +271,7 @@ int runner_launch(HipRunner *r, void **args, int n_args, void *scratch_from_call
   }
   if (r->guards.empty()) return program_launch(r->main, r->arg_ptrs.data(), r->rk.launch);
   // The guard writes *flag (1 = fast path valid, 0 = not); the fast kernel and
-  // its generic twin both launch and exactly one of them does the work.
+  // its generic twin, in one launch or in two, look at it and exactly one of them does the work.
   r->ptr_store[(size_t)(np + nv + nt)] = r->flag;
   r->arg_ptrs[(size_t)(np + nv + nt)] = &r->ptr_store[(size_t)(np + nv + nt)];
   for (size_t gi = 0; gi < r->guards.size(); gi++) {
@@ -286,7 +286,7 @@ int runner_launch(HipRunner *r, void **args, int n_args, void *scratch_from_call
     if (program_launch(r->guards[gi], gargs, gd.launch) != 0) return -1;
   }
   if (program_launch(r->main, r->arg_ptrs.data(), r->rk.launch) != 0) return -1;
-  return program_launch(r->fallback, r->arg_ptrs.data(), r->rk.fallback_launch);
+  return r->fallback ? program_launch(r->fallback, r->arg_ptrs.data(), r->rk.fallback_launch) : 0;
 }
 
 }  // namespace polyhip

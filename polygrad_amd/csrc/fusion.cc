@@ -2794,21 +2794,6 @@ static bool match_ordered_sums_side_by_side(const Sched &sc, int a_item, const s
     members.push_back(std::move(ad));
   }
   if (members.size() < 2) return false;
-  // a kernel as a device function of its workgroup number
-  const std::string prelude = hip_prelude();
-  auto as_device_fn = [&](const std::string &src, const std::string &entry, const std::string &name, std::string *fn) {
-    if (src.compare(0, prelude.size(), prelude) != 0) return false;
-    std::string t = src.substr(prelude.size());
-    const std::string head = "extern \"C\" __global__ void __launch_bounds__(";
-    if (t.compare(0, head.size(), head) != 0) return false;        // (helpers of its own in front: names could clash)
-    const size_t open = t.find(entry + "(");
-    if (open == std::string::npos || open > 128) return false;
-    t = "__device__ __forceinline__ void " + name + "(const unsigned int poly_bid, " + t.substr(open + entry.size() + 1);
-    for (size_t at = t.find("blockIdx.x"); at != std::string::npos; at = t.find("blockIdx.x", at)) t.replace(at, 10, "poly_bid");
-    if (t.find("blockIdx") != std::string::npos || t.find("__shared__") != std::string::npos) return false;
-    *fn = t;
-    return true;
-  };
   std::vector<int> arg_slots;
   std::map<int, DT> slot_dt;
   std::set<int> written;
@@ -2823,6 +2808,7 @@ static bool match_ordered_sums_side_by_side(const Sched &sc, int a_item, const s
     }
   }
   auto arg_of = [&](int sl) { return (int)(std::find(arg_slots.begin(), arg_slots.end(), sl) - arg_slots.begin()); };
+  const std::string prelude = hip_prelude();
   std::string code, pre_body, main_body;
   size_t scratch = 0;
   unsigned pre_blocks = 0, main_blocks = 0;
@@ -2831,8 +2817,8 @@ static bool match_ordered_sums_side_by_side(const Sched &sc, int a_item, const s
     const Ad &m = members[mi];
     const KernelGraph &g = sc.graphs[(size_t)m.item];
     std::string f1, f2;
-    if (!as_device_fn(m.rk.pres[0].source, m.rk.pres[0].entry, strf("poly_terms_%zu", mi), &f1) ||
-        !as_device_fn(m.rk.source, m.rk.entry, strf("poly_adder_%zu", mi), &f2))
+    if (!kernel_as_device_fn(m.rk.pres[0].source, m.rk.pres[0].entry, strf("poly_terms_%zu", mi), &f1) ||
+        !kernel_as_device_fn(m.rk.source, m.rk.entry, strf("poly_adder_%zu", mi), &f2))
       return false;
     code += f1 + f2;
     std::string args;

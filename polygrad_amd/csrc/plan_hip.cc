@@ -838,7 +838,7 @@ static PolyHipPlan *compile_schedule(const PolySchedule *s, bool drop_copies) {
   for (int u = 0; u < n_units; u++) {
     const HipRunner *r = plan->units[(size_t)u].runner;
     plan->n_launches += (int)(plan->fills_before[(size_t)u].size() + plan->touch_at[(size_t)u].size() + (r->skip_pres ? 0 : r->pres.size()) + 1 +
-                              (r->guards.empty() ? 0 : r->guards.size() + 1));
+                              r->guards.size() + (r->fallback ? 1 : 0));
   }
   plan->kargs.resize((size_t)n_units);
   plan->var_vals.resize((size_t)n_units);

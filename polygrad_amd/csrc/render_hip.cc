@@ -1011,6 +1011,21 @@ class Generic {
 
 }  // namespace
 
+bool kernel_as_device_fn(const std::string &src, const std::string &entry, const std::string &name, std::string *fn) {
+  const std::string prelude = hip_prelude();
+  if (src.compare(0, prelude.size(), prelude) != 0) return false;
+  std::string t = src.substr(prelude.size());
+  const std::string head = "extern \"C\" __global__ void __launch_bounds__(";
+  if (t.compare(0, head.size(), head) != 0) return false;        // (helpers of its own in front: names could clash)
+  const size_t open = t.find(entry + "(");
+  if (open == std::string::npos || open > 128) return false;
+  t = "__device__ __forceinline__ void " + name + "(const unsigned int poly_bid, " + t.substr(open + entry.size() + 1);
+  for (size_t at = t.find("blockIdx.x"); at != std::string::npos; at = t.find("blockIdx.x", at)) t.replace(at, 10, "poly_bid");
+  if (t.find("blockIdx") != std::string::npos || t.find("__shared__") != std::string::npos) return false;
+  *fn = t;
+  return true;
+}
+
 static bool split_in_two(const KernelGraph &g, const std::string &fn_name, const RenderOptions &opt, int T, PolyOps top,
                          double rows, double per_output, int slice_range, int parts, RenderedKernel *out);
 
