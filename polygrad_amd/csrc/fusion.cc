@@ -1990,6 +1990,7 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
   cfg += strf("#define POLY_Q_PTR fa%d\n#define POLY_K_PTR fa%d\n#define POLY_V_PTR fa%d\n", operand_arg(0), operand_arg(1), operand_arg(2));
   // position in the operand's own buffer -> position in the buffer it was copied from
   const char *src_name[3] = {"poly_fa_qsrc", "poly_fa_ksrc", "poly_fa_vsrc"};
+  std::string src_text[3];
   for (int o = 0; o < 3; o++) {
     std::string f = strf("__device__ __forceinline__ int %s(int p) {\n", src_name[o]);
     if (folded[o].item < 0) f += "  return p;\n}\n";
@@ -1999,10 +2000,13 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
         f += strf("  off += ((p / %lld) %% %lld) * %lld;\n", (long long)d.stride, (long long)d.extent, (long long)d.coef);
       f += "  return off;\n}\n";
     }
+    src_text[o] = f;
     cfg += f;
   }
-  cfg += matmul_offset_fn("poly_fa_qz", mS.zd, true, mS.a_c0) + matmul_offset_fn("poly_fa_qm", mS.md, true, 0);
-  cfg += matmul_offset_fn("poly_fa_kz", mS.zd, false, mS.b_c0) + matmul_offset_fn("poly_fa_kn", mS.nd, false, 0);
+  // what the offsets of q, k and v are made of, as text
+  std::string raw_text[3] = {matmul_offset_fn("poly_fa_qz", mS.zd, true, mS.a_c0) + matmul_offset_fn("poly_fa_qm", mS.md, true, 0),
+                             matmul_offset_fn("poly_fa_kz", mS.zd, false, mS.b_c0) + matmul_offset_fn("poly_fa_kn", mS.nd, false, 0), ""};
+  cfg += raw_text[0] + raw_text[1];
   // Row offsets as the kernel sees them: source position of row x (query or key) of batch z.
   // When that is affine in x for every z -- the usual case -- the z part is evaluated once
   // and the row part is a multiplication; otherwise the general digit form is kept.
@@ -2033,11 +2037,19 @@ static bool match_attention(const Sched &sc, int s_item, const std::vector<char>
     const int64_t X = o == 0 ? mS.M : mS.N;
     bool affine = mS.Z * X <= (int64_t)1 << 24;
     const int64_t step = eval_src(o, raw_off(o, 0, 1)) - eval_src(o, raw_off(o, 0, 0));
-    for (int64_t z = 0; z < mS.Z && affine; z++) {
+    // (every z and x is looked at, 9 ms for three times 96 x 1024: once for all layers of a model, which
+    // differ in nothing that the texts say)
+    static thread_local std::map<std::string, bool> known;
+    if (known.size() > 64) known.clear();
+    const std::string key = strf("%d %lld %lld ", o, (long long)mS.Z, (long long)X) + src_text[o] + raw_text[o] + general[o];
+    const auto was = known.find(key);
+    if (was != known.end()) affine = was->second;
+    for (int64_t z = 0; z < mS.Z && affine && was == known.end(); z++) {
       const int64_t base = eval_src(o, raw_off(o, z, 0));
       for (int64_t x = 0; x < X; x++)
         if (eval_src(o, raw_off(o, z, x)) != base + x * step) { affine = false; break; }
     }
+    known[key] = affine;
     if (o == 1 && affine) k_pitch = step;
     if (affine)
       cfg += strf("__device__ __forceinline__ int %s(int z, int x) { return %s(%s(z, 0)) + x * %lld; }\n", off_name[o], src_name[o],
@@ -3170,13 +3182,17 @@ void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &gr
     product.internal_slots.insert(product.internal_slots.end(), chain.internal_slots.begin(), chain.internal_slots.end());
     product.internal_slots.push_back(slot);
     product.rk.strategy += strf(" (%s)", chain.rk.strategy.c_str());
-    std::vector<FusedGroup> with;
-    for (size_t j = 0; j < out->size(); j++) if (j != gi && j != pj) with.push_back((*out)[j]);
-    with.push_back(product);
+    std::vector<FusedGroup> with;      // (their items alone)
+    auto places = [&](const FusedGroup &g) { with.emplace_back(); with.back().items = g.items; with.back().launch_item = g.launch_item; };
+    for (size_t j = 0; j < out->size(); j++) if (j != gi && j != pj) places((*out)[j]);
+    places(product);
     if (!fused_groups_out_of_order(s, graphs, with).empty()) continue;
     taken[(size_t)reader] = 1;
-    *out = std::move(with);
-    gi = (size_t)-1;       // (the groups have moved)
+    const bool replaces = pj < out->size();
+    if (replaces) out->erase(out->begin() + (long)std::max(gi, pj));
+    out->erase(out->begin() + (long)(replaces ? std::min(gi, pj) : gi));
+    out->push_back(std::move(product));
+    gi -= replaces && pj < gi ? 2 : 1;      // (the next one has moved here)
   }
   // every pair of items that share a buffer keeps its order; a group that breaks one is
   // dropped and its kernels launch one by one at their own places
