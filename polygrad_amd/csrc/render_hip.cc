@@ -445,6 +445,29 @@ class Generic {
     return body;
   }
 
+  // Rows of fewer than 128 terms that a wave adds up all the same: few outputs, whose terms are reductions
+  // themselves (the loss of a small batch).  One thread walks all of such an output's elements, each load
+  // behind the last; with a term to a lane the chain is one term long (the loss over 33 rows of 10: the
+  // training step 37.9 -> 31.3 us).  With fewer than 16 terms or 128 elements the chain is no longer than the
+  // wave's own sum, with more than 64 outputs the chip has threads enough.
+  bool few_nested_terms(int64_t R, double rows) const {
+    if (R < 16 || rows > 64 || opt_.promote_reduce >= 0) return false;
+    std::vector<char> inside(g_.nodes.size(), 0);
+    for (int id : top_reduces_) mark_reachable(g_, g_.n(id).src[0], inside);
+    int64_t longest = 1;
+    for (int id : g_.reduces) {
+      if (!inside[(size_t)id]) continue;
+      int64_t n = 1;
+      for (size_t i = 1; i < g_.n(id).src.size(); i++) {
+        const int64_t e = g_.ranges[(size_t)g_.range_ord.at(g_.n(id).src[i])].extent;
+        if (e < 0) return false;
+        n = e == 0 ? 0 : n > 128 ? n : n * std::min<int64_t>(e, 128);
+      }
+      longest = std::max(longest, n);
+    }
+    return longest > 1 && R * longest >= 128;
+  }
+
   // ── cooperative row reduction ─────────────────────────────────────────────
   bool plan_coop() {
     if (top_reduces_.empty()) return false;
@@ -468,7 +491,7 @@ class Generic {
     for (int r : groups_[0].ranges) if (g_.ranges[(size_t)r].extent < 0) return false;
     double rows = 1;
     for (int r : groups_[0].ranges) rows *= (double)g_.ranges[(size_t)r].extent;
-    if (R < 128) return false;
+    if (R < 128 && !few_nested_terms(R, rows)) return false;
     // Lanes that walk along the reduce range only pay off when some operand is contiguous
     // along it.  When every load is strided there (X^T W forms: the reduce axis is the
     // outer axis of both operands) but contiguous along an output range, one thread per
