@@ -229,7 +229,7 @@ class Emitter {
  private:
   bool shared_division(DT dt, int num, int den, Scope *t, std::string *e);
   std::string emit_atom(int atom, Scope *s);
-  bool light_body(int root, int ord) const;
+  bool light_body(int root, int ord, int *n_loads = nullptr) const;
   std::string emit_raw(int node, Scope *s);
   Scope *place(uint64_t deps, Scope *s);
   const KernelGraph &g_;
