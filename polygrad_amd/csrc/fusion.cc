@@ -3157,6 +3157,18 @@ void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &gr
     int reads = 0;
     for (const KNode &k : gr.nodes) reads += k.op == POLY_OP_LOAD && sc.slot(reader, gr.param_slot(gr.n(k.src[0]).src[0])) == slot;
     if (reads != 1) continue;
+    // (every workgroup reads whole rows of the chain's operands, and stores columns of the product's
+    // outputs while others still read: none of these may be one of those)
+    bool in_place = false;
+    std::vector<int> writers = {reader};
+    if (pj < out->size()) writers = (*out)[pj].items;
+    for (int wi : writers)
+      for (size_t p = 0; p < graphs[(size_t)wi].params.size(); p++) {
+        if (!graphs[(size_t)wi].params[p].written) continue;
+        const int w = sc.slot(wi, (int)p);
+        in_place = in_place || std::find(chain.arg_slots.begin(), chain.arg_slots.end(), w) != chain.arg_slots.end();
+      }
+    if (in_place) continue;
     FusedGroup product;
     matmul_hint_a_rows(&chain.rows);
     bool done;
