@@ -157,7 +157,7 @@ int n_launches(const PolySchedule *s, const std::vector<FusedGroup> &groups) {
 
 }  // namespace
 
-bool plan_schedule(const PolySchedule *s, bool drop_copies, PlannedSchedule *out, std::string *err) {
+bool plan_schedule(const PolySchedule *s, bool buffers_apart, PlannedSchedule *out, std::string *err) {
   out->graphs.clear();
   out->graphs.resize((size_t)s->n_items);
   for (int k = 0; k < s->n_items; k++) {
@@ -167,9 +167,9 @@ bool plan_schedule(const PolySchedule *s, bool drop_copies, PlannedSchedule *out
   out->sched = *s;
   out->unused.assign((size_t)s->n_buf_slots, 0);
   out->written_early.clear();
-  find_fused_groups(s, out->graphs, &out->groups);
+  find_fused_groups(s, out->graphs, buffers_apart, &out->groups);
   // (a dropped copy is two buffers of the schedule in one place, which POLY_HIP_NO_ALIAS is about)
-  if (!drop_copies || getenv("POLY_HIP_NO_FUSION") || getenv("POLY_HIP_NO_COPY_DROP") || getenv("POLY_HIP_NO_ALIAS")) return true;
+  if (!buffers_apart || getenv("POLY_HIP_NO_FUSION") || getenv("POLY_HIP_NO_COPY_DROP") || getenv("POLY_HIP_NO_ALIAS")) return true;
 
   // (what a group has taken in costs no launch, and the matchers know those copies)
   std::vector<char> grouped((size_t)s->n_items, 0);
@@ -222,7 +222,7 @@ bool plan_schedule(const PolySchedule *s, bool drop_copies, PlannedSchedule *out
       for (int i = 0; i < s->items[k].n_buf_slots; i++) used_before = used_before || s->items[k].buf_slot_indices[i] == sl;
     if (!used_before || !s->buf_slots[sl].is_intermediate) p.unused[(size_t)sl] = 0;
   }
-  find_fused_groups(&p.sched, p.graphs, &p.groups);
+  find_fused_groups(&p.sched, p.graphs, buffers_apart, &p.groups);
   if (n_launches(&p.sched, p.groups) >= n_launches(s, out->groups)) return true;
   // (a kernel that reads the old contents of such a buffer is not in one launch with the one
   // that writes it: what one workgroup has stored, another might still have to read)

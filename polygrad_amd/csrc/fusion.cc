@@ -2959,7 +2959,7 @@ std::vector<int> fused_groups_out_of_order(const PolySchedule *s, const std::vec
   return std::vector<int>(bad.begin(), bad.end());
 }
 
-void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &graphs, std::vector<FusedGroup> *out) {
+void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &graphs, bool buffers_apart, std::vector<FusedGroup> *out) {
   out->clear();
   if (getenv("POLY_HIP_NO_FUSION")) return;
   Sched sc{s, graphs, {}, {}, {}, {}};
@@ -3140,7 +3140,7 @@ void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &gr
   // depend on each other.  The product's workgroups compute the rows themselves, each those of
   // its tile, while the first loads of their weights are on the way (render_matmul_wave says
   // on which tiles that pays).
-  for (size_t gi = 0; gi < out->size() && !getenv("POLY_HIP_NO_ROWS_IN_PRODUCT"); gi++) {
+  for (size_t gi = 0; gi < out->size() && buffers_apart && !getenv("POLY_HIP_NO_ROWS_IN_PRODUCT"); gi++) {
     const FusedGroup &chain = (*out)[gi];
     const int slot = chain.row_chain_stores;
     if (chain.rows.code.empty() || chain.n_rows > 64 || chain.needs_group_at >= 0 || slot < 0 || !s->buf_slots[slot].is_intermediate) continue;
@@ -3158,8 +3158,10 @@ void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &gr
     for (const KNode &k : gr.nodes) reads += k.op == POLY_OP_LOAD && sc.slot(reader, gr.param_slot(gr.n(k.src[0]).src[0])) == slot;
     if (reads != 1) continue;
     // (every workgroup reads whole rows of the chain's operands, and stores columns of the product's
-    // outputs while others still read: none of these may be one of those)
+    // outputs while others still read: none of these may be one of those, and the caller's ones
+    // may not be bound to the same memory)
     bool in_place = false;
+    std::vector<std::pair<int, int>> apart;
     std::vector<int> writers = {reader};
     if (pj < out->size()) writers = (*out)[pj].items;
     for (int wi : writers)
@@ -3167,6 +3169,8 @@ void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &gr
         if (!graphs[(size_t)wi].params[p].written) continue;
         const int w = sc.slot(wi, (int)p);
         in_place = in_place || std::find(chain.arg_slots.begin(), chain.arg_slots.end(), w) != chain.arg_slots.end();
+        for (int r : chain.arg_slots)
+          if (!s->buf_slots[w].is_intermediate && !s->buf_slots[r].is_intermediate) apart.push_back({w, r});
       }
     if (in_place) continue;
     FusedGroup product;
@@ -3193,6 +3197,7 @@ void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &gr
     product.items.insert(product.items.begin(), chain.items.begin(), chain.items.end());
     product.internal_slots.insert(product.internal_slots.end(), chain.internal_slots.begin(), chain.internal_slots.end());
     product.internal_slots.push_back(slot);
+    product.apart = apart;
     product.rk.strategy += strf(" (%s)", chain.rk.strategy.c_str());
     std::vector<FusedGroup> with;      // (their items alone)
     auto places = [&](const FusedGroup &g) { with.emplace_back(); with.back().items = g.items; with.back().launch_item = g.launch_item; };

@@ -22,6 +22,9 @@ struct FusedGroup {
   // elements, stored row after row; the arguments behind the first are its parameters
   MatmulRows rows;
   int64_t n_rows = 0, row_len = 0;
+  // a product that computes those rows itself: buffers of the caller's that it writes, each with
+  // one that its workgroups read whole rows of; where the two share memory the launches are two
+  std::vector<std::pair<int, int>> apart;
   // Two groups that only work together (a chain that stores bf16 values into an fp32 buffer
   // and the product that reads them as such) name each other's launch item here: dropping
   // one drops the other.
@@ -41,8 +44,9 @@ struct FusedGroup {
 };
 
 // Finds the fusable groups of a schedule.  graphs[k] is the analysed kernel of item k.
-// Setting POLY_HIP_NO_FUSION in the environment disables the search.
-void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &graphs, std::vector<FusedGroup> *out);
+// Setting POLY_HIP_NO_FUSION in the environment disables the search.  !buffers_apart: only groups
+// that do what their kernels do also where buffers of the caller's share memory (FusedGroup::apart).
+void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &graphs, bool buffers_apart, std::vector<FusedGroup> *out);
 // The groups (indices into `groups`) whose place of launch breaks the order of two kernels
 // of the schedule that share a buffer, one of them writing it; find_fused_groups drops such
 // groups itself, so that its result always passes.
@@ -70,7 +74,7 @@ struct PlannedSchedule {
   std::vector<int> order;
 };
 // Analyses and groups schedule `s` (POLY_HIP_NO_COPY_DROP in the environment, or
-// !drop_copies: every copy keeps its launch).  False with a message on a malformed kernel.
-bool plan_schedule(const PolySchedule *s, bool drop_copies, PlannedSchedule *out, std::string *err);
+// !buffers_apart: every copy keeps its launch).  False with a message on a malformed kernel.
+bool plan_schedule(const PolySchedule *s, bool buffers_apart, PlannedSchedule *out, std::string *err);
 
 }  // namespace polyhip

@@ -173,10 +173,12 @@ struct PolyHipPlan {
   // before launch u.
   std::vector<std::vector<int>> touch_at;
   Program *touch = nullptr;
-  // Buffers of the caller's that a launch writes before the schedule would (copies.cc).  Where
-  // one of them shares memory with another buffer bound beside it, `plain` runs instead: the
-  // schedule with all its copies, compiled when such a binding is first met.
+  // Buffers of the caller's that a launch writes before the schedule would (copies.cc), and pairs of
+  // them that a launch writes and reads whole rows of (FusedGroup::apart).  Where one of the former
+  // shares memory with another buffer bound beside it, or a pair does, `plain` runs instead: the
+  // schedule with all its copies and no such launches, compiled when such a binding is first met.
   std::vector<int> written_early;
+  std::vector<std::pair<int, int>> apart;
   std::vector<void *> last_bound;            // what `shares_memory` was worked out for
   bool shares_memory = false;
   PolyHipPlan *plain = nullptr;
@@ -323,16 +325,17 @@ int enqueue_captured(PolyHipPlan *plan) {
 
 extern "C" {
 
-static PolyHipPlan *compile_schedule(const PolySchedule *s, bool drop_copies);
+static PolyHipPlan *compile_schedule(const PolySchedule *s, bool buffers_apart);
 
 PolyHipPlan *poly_hip_compile_schedule(PolyCtx *ctx, const PolySchedule *s) {
   (void)ctx;
   return compile_schedule(s, true);
 }
 
-// The plan that runs on these buffers: `plan` itself, or the one that keeps every copy.
+// The plan that runs on these buffers: `plan` itself, or the one that does as the schedule says
+// also where they share memory.
 static PolyHipPlan *plan_for(PolyHipPlan *plan, void **slot_data, int n_slots) {
-  if (plan->written_early.empty() || !slot_data) return plan;
+  if ((plan->written_early.empty() && plan->apart.empty()) || !slot_data) return plan;
   const PolySchedule *s = plan->sched;
   const int n = std::min(n_slots, s->n_buf_slots);
   if (plan->last_bound.size() != (size_t)n || memcmp(plan->last_bound.data(), slot_data, (size_t)n * sizeof(void *)) != 0) {
@@ -353,6 +356,11 @@ static PolyHipPlan *plan_for(PolyHipPlan *plan, void **slot_data, int n_slots) {
       any_hi = std::max(any_hi, x.hi);
       if (x.early) early_hi = std::max(early_hi, x.hi);
     }
+    for (const auto &[w, r] : plan->apart) {
+      if (w >= n || r >= n || !slot_data[w] || !slot_data[r]) continue;
+      const uintptr_t a = (uintptr_t)slot_data[w], b = (uintptr_t)slot_data[r];
+      if (a < b + (uintptr_t)s->buf_slots[r].nbytes && b < a + (uintptr_t)s->buf_slots[w].nbytes) plan->shares_memory = true;
+    }
   }
   if (!plan->shares_memory) return plan;
   if (!plan->plain) {
@@ -364,7 +372,7 @@ static PolyHipPlan *plan_for(PolyHipPlan *plan, void **slot_data, int n_slots) {
   return plan->plain;
 }
 
-static PolyHipPlan *compile_schedule(const PolySchedule *s, bool drop_copies) {
+static PolyHipPlan *compile_schedule(const PolySchedule *s, bool buffers_apart) {
   if (!s) return nullptr;
   if (runtime_init() != 0) return nullptr;
   std::unique_ptr<PolyHipPlan> plan(new PolyHipPlan());
@@ -374,7 +382,7 @@ static PolyHipPlan *compile_schedule(const PolySchedule *s, bool drop_copies) {
   PlannedSchedule planned;
   {
     std::string err;
-    if (!plan_schedule(s, drop_copies, &planned, &err)) {
+    if (!plan_schedule(s, buffers_apart, &planned, &err)) {
       log_err("compile_schedule", "%s", err.c_str());
       return nullptr;
     }
@@ -383,6 +391,7 @@ static PolyHipPlan *compile_schedule(const PolySchedule *s, bool drop_copies) {
   const std::vector<KernelGraph> &graphs = planned.graphs;
   std::vector<FusedGroup> &groups = planned.groups;
   plan->written_early = planned.written_early;
+  for (const FusedGroup &fg : groups) plan->apart.insert(plan->apart.end(), fg.apart.begin(), fg.apart.end());
   std::vector<int> group_of((size_t)s->n_items, -1);
   std::vector<char> internal = planned.unused;
   for (size_t gi = 0; gi < groups.size(); gi++) {

@@ -105,3 +105,38 @@ def test_same_bits(rows, d, w, form, fused, monkeypatch):
     there, n_there = _run(rows, d, w, form)
     assert (n, n_there) == (int(fused), 0)
     assert here == there
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["out", "out plus", "copy beside"])
+@pytest.mark.parametrize("rows,d,w", SIZES)
+def test_output_bound_over_the_rows(rows, d, w, form, monkeypatch):
+    """The caller's own output over the rows that the LayerNorm reads, as a whole and from the middle on (not
+    where the rows are added to the result: that reads them where the output is written): the bits of
+    a plan that launches the LayerNorm by itself, before and after passes on buffers apart."""
+    import torch
+
+    def run():
+        plan = _schedule(rows, d, w, form).plan()
+        g = torch.Generator(device="cuda").manual_seed(rows)
+        by, data = {}, [None] * len(plan.slots)
+        for slot in plan.external_slots():
+            scale = dict(weight=d ** -0.5, bias=0.02, beta=0.02).get(slot.name, 1.0)
+            n = slot.numel + (slot.numel // 2 if slot.name == "x" else 0)
+            by[slot.name] = (torch.randn(n, generator=g, device="cuda") * scale).to(getattr(torch, w))
+            data[slot.index] = by[slot.name][:slot.numel]
+        out, n = [s.index for s in plan.external_slots() if s.name == "out"][0], rows * d
+        seen = []
+        middle = [] if form == "out plus" else [by["x"][n // 2:]]
+        for bound in [data[out], by["x"][:n], data[out]] + middle + [by["x"][:n], data[out]]:
+            data[out] = bound
+            plan.run(data)
+            seen += [v.cpu().view(torch.uint8).numpy().tobytes() for v in (by["x"], bound)]
+        return seen, sum("compute A's rows" in k["desc"] for k in plan.kernel_info())
+
+    here, n = run()
+    monkeypatch.setenv("POLY_HIP_NO_ROWS_IN_PRODUCT", "1")
+    monkeypatch.setenv("POLY_HIP_NO_COPY_DROP", "1")
+    there, n_there = run()
+    assert (n, n_there) == (1, 0)
+    assert here == there
