@@ -172,7 +172,9 @@ int poly_hip_plan_kernel_info(const PolyHipPlan *plan, int cap, int *klass, doub
  * (hipExtModuleLaunchKernel): ms_out[k], k in execution order, is the sum over the
  * kernels of launch k (a fill or first stage in front of it included) -- what a
  * profiler's kernel trace reports, without the waits between launches.  Returns
- * the number of launches or <0. */
+ * the number of launches or <0: poly_hip_plan_n_kernels of them, or, on buffers whose sharing
+ * of memory takes other launches (poly_hip_plan_run), as many as that form has, never more than
+ * the schedule has kernels; at most cap of them are in ms_out. */
 int poly_hip_plan_profile(PolyHipPlan *plan, void **slot_data, int n_slots, float *ms_out, int cap);
 /* Malloc'd description ("lower0_k3 matmul-mfma ...") of kernel k; free with
  * poly_hip_free_string. */

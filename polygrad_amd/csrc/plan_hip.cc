@@ -1214,7 +1214,8 @@ int poly_hip_plan_kernel_info(const PolyHipPlan *plan, int cap, int *klass, doub
 }
 
 int poly_hip_plan_profile(PolyHipPlan *plan, void **slot_data, int n_slots, float *ms_out, int cap) {
-  if (!plan) return -1;
+  if (!plan || !plan->sched) return -1;
+  if (!(plan = plan_for(plan, slot_data, n_slots))) return -1;
   uint64_t key;
   if (bind_args(plan, slot_data, n_slots, nullptr, 0, &key) != 0) return -1;
   if (!plan->tuned) {

@@ -137,11 +137,14 @@ class HipPlan:
         """Per-launch milliseconds of one eager pass: the durations of each launch's kernels,
         from the HIP events that their dispatches stamp at start and end."""
         arr = self._ptr_array(slot_data)
-        ms = (C.c_float * self.n_kernels)()
-        rc = self.lib.poly_hip_plan_profile(self.handle, arr, len(self.slots), ms, self.n_kernels)
+        # (buffers that share memory may take more launches than n_kernels, but no more than the
+        # schedule has kernels)
+        cap = C.cast(self.schedule, C.POINTER(_ffi.PolySchedule)).contents.n_items
+        ms = (C.c_float * cap)()
+        rc = self.lib.poly_hip_plan_profile(self.handle, arr, len(self.slots), ms, cap)
         if rc < 0:
             raise RuntimeError("poly_hip_plan_profile failed")
-        return list(ms)
+        return list(ms[:rc])
 
     def workspace_bytes(self):
         return int(self.lib.poly_hip_plan_workspace_bytes(self.handle))

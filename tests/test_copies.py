@@ -142,3 +142,30 @@ def test_training_step_on_buffers_that_share_memory(batch, shared, monkeypatch):
     monkeypatch.setenv("POLY_HIP_NO_COPY_DROP", "1")
     want, all_launches = _run(s.plan(), shared)
     assert got == want and launches <= all_launches - 5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shared", [[], [("logits", "X")], [("b1", "b2")]])
+def test_profile_leaves_what_a_run_leaves(shared):
+    """A timed pass, launch by launch, is a pass: on buffers that share memory, too."""
+    import torch
+    seen = []
+    for timed in (False, True):
+        plan = cases._mlp_schedule(dict(kind="mlp", batch=33, d_in=50, d_hid=20, d_out=24)).plan()
+        g = torch.Generator(device="cuda")
+        g.manual_seed(3)
+        data, by = [None] * len(plan.slots), {}
+        for slot in plan.external_slots():
+            by[slot.name] = data[slot.index] = torch.rand(slot.numel, generator=g, device="cuda")
+        for small, large in shared:
+            index = [s.index for s in plan.external_slots() if s.name == small][0]
+            data[index] = by[small] = by[large][:by[small].numel()]
+        for _ in range(2):
+            if timed:
+                times = plan.profile(data)
+                assert len(times) == plan.n_kernels if not shared else len(times) > plan.n_kernels
+                assert all(t > 0 for t in times)
+            else:
+                plan.run(data)
+        seen.append({k: v.cpu().numpy().tobytes() for k, v in by.items()})
+    assert seen[0] == seen[1]
