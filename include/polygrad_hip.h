@@ -127,6 +127,13 @@ typedef struct PolyHipPlan PolyHipPlan;
 PolyHipPlan *poly_hip_compile_schedule(PolyCtx *ctx, const PolySchedule *schedule);
 /* slot_data[i]: device pointer for every external slot (ignored for
  * intermediates).  Returns after enqueueing; poly_hip_sync() waits.
+ * A kernel that copies a whole intermediate into a buffer of the caller's need not be launched: the
+ * kernel that makes the values writes that buffer, earlier in the pass than the schedule says.
+ * Buffers of the caller's may share memory: where one of them would see that, or a launch would
+ * store into what it still reads, the pass takes the launches that keep the schedule's
+ * order.  These are compiled, and their workspace is allocated, by the first pass on such
+ * buffers; poly_hip_plan_workspace_bytes and poly_hip_plan_graph_counts count them in from then
+ * on, the other introspection calls speak of the usual form.
  * With POLY_BEAM > 0 in the environment at compile and run time (the switch of
  * the reference's kernel search, src/render_c.c:839; its timing loop and disk
  * cache are src/codegen.c:1012-1195), the first run goes through the launches
@@ -179,7 +186,9 @@ int poly_hip_plan_profile(PolyHipPlan *plan, void **slot_data, int n_slots, floa
 /* Malloc'd description ("lower0_k3 matmul-mfma ...") of kernel k; free with
  * poly_hip_free_string. */
 char *poly_hip_plan_kernel_desc(const PolyHipPlan *plan, int k);
-/* Device address of an intermediate slot (tests compare intermediates). */
+/* Device address of the buffer that the latest pass left an intermediate slot's value in: its own,
+ * or that of the slot it is a copy of or is copied to, where the copy takes no launch.  NULL
+ * where the value never leaves a launch. */
 void *poly_hip_plan_slot_ptr(const PolyHipPlan *plan, int slot);
 /* Replay this plan from a hipGraph (1), or never (0).  A plan that neither was said of does
  * so unless it has only a few launches, which take the host less time one by one. */

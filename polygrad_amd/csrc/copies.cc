@@ -82,6 +82,7 @@ struct Rewrite {
   std::vector<char> dropped;                // items without a launch
   std::vector<int> step;
   std::vector<int> early;                   // the caller's buffers that are written before their copy's place
+  std::vector<int> held_by;                 // per slot: the one that has its value, -1: itself
 
   bool uses(int item, int slot, bool written) const {
     const KernelGraph &g = graphs[(size_t)item];
@@ -101,6 +102,8 @@ struct Rewrite {
   }
   void rename(int from, int to) {
     for (auto &a : args) std::replace(a.begin(), a.end(), from, to);
+    std::replace(held_by.begin(), held_by.end(), from, to);
+    held_by[(size_t)from] = to;
   }
 
   bool drop(int c) {
@@ -167,6 +170,7 @@ bool plan_schedule(const PolySchedule *s, bool buffers_apart, PlannedSchedule *o
   out->sched = *s;
   out->unused.assign((size_t)s->n_buf_slots, 0);
   out->written_early.clear();
+  out->held_by.clear();
   find_fused_groups(s, out->graphs, buffers_apart, &out->groups);
   // (a dropped copy is two buffers of the schedule in one place, which POLY_HIP_NO_ALIAS is about)
   if (!buffers_apart || getenv("POLY_HIP_NO_FUSION") || getenv("POLY_HIP_NO_COPY_DROP") || getenv("POLY_HIP_NO_ALIAS")) return true;
@@ -179,7 +183,8 @@ bool plan_schedule(const PolySchedule *s, bool buffers_apart, PlannedSchedule *o
     for (int it : fg.items) copies = copies && is_identity(out->graphs[(size_t)it], &pd, &ps);
     if (!copies) for (int it : fg.items) grouped[(size_t)it] = 1;
   }
-  Rewrite rw{s, out->graphs, {}, {}, {}, {}};
+  Rewrite rw{s, out->graphs, {}, {}, {}, {}, {}};
+  rw.held_by.assign((size_t)s->n_buf_slots, -1);
   rw.dropped.assign((size_t)s->n_items, 0);
   rw.step.assign((size_t)s->n_items, 0);
   for (int st = 0; st < s->n_items; st++) rw.step[(size_t)s->exec_order[st]] = st;
@@ -214,6 +219,7 @@ bool plan_schedule(const PolySchedule *s, bool buffers_apart, PlannedSchedule *o
   p.sched.n_items = (int)p.items.size();
   p.sched.exec_order = p.order.data();
   p.written_early = rw.early;
+  p.held_by = rw.held_by;
   p.unused.assign((size_t)s->n_buf_slots, 1);
   for (const auto &a : p.args) for (int sl : a) p.unused[(size_t)sl] = 0;
   for (int sl = 0; sl < s->n_buf_slots; sl++) {

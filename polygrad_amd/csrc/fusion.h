@@ -66,6 +66,7 @@ struct PlannedSchedule {
   std::vector<FusedGroup> groups;
   std::vector<char> unused;                 // per slot: an intermediate that no kernel touches any more
   std::vector<int> written_early;           // the caller's buffers that are written before their copy's place
+  std::vector<int> held_by;                 // per slot: the one that has its value, -1: itself (empty: all themselves)
   PlannedSchedule() = default;
   PlannedSchedule(const PlannedSchedule &) = delete;
   PlannedSchedule &operator=(PlannedSchedule &&) = default;

@@ -182,6 +182,8 @@ struct PolyHipPlan {
   std::vector<void *> last_bound;            // what `shares_memory` was worked out for
   bool shares_memory = false;
   PolyHipPlan *plain = nullptr;
+  bool ran_plain = false;                    // the latest pass was one of `plain`
+  std::vector<int> held_by;                  // PlannedSchedule::held_by
   bool use_graph = true;
   bool graph_asked = false;      // by poly_hip_plan_set_graph, however few launches there are
   // Kernel launches of one pass.  A plan of a few of them is launched kernel by kernel unless
@@ -335,6 +337,7 @@ PolyHipPlan *poly_hip_compile_schedule(PolyCtx *ctx, const PolySchedule *s) {
 // The plan that runs on these buffers: `plan` itself, or the one that does as the schedule says
 // also where they share memory.
 static PolyHipPlan *plan_for(PolyHipPlan *plan, void **slot_data, int n_slots) {
+  plan->ran_plain = false;
   if ((plan->written_early.empty() && plan->apart.empty()) || !slot_data) return plan;
   const PolySchedule *s = plan->sched;
   const int n = std::min(n_slots, s->n_buf_slots);
@@ -369,6 +372,7 @@ static PolyHipPlan *plan_for(PolyHipPlan *plan, void **slot_data, int n_slots) {
   }
   plan->plain->use_graph = plan->use_graph;
   plan->plain->graph_asked = plan->graph_asked;
+  plan->ran_plain = true;
   return plan->plain;
 }
 
@@ -391,6 +395,7 @@ static PolyHipPlan *compile_schedule(const PolySchedule *s, bool buffers_apart) 
   const std::vector<KernelGraph> &graphs = planned.graphs;
   std::vector<FusedGroup> &groups = planned.groups;
   plan->written_early = planned.written_early;
+  plan->held_by = planned.held_by;
   for (const FusedGroup &fg : groups) plan->apart.insert(plan->apart.end(), fg.apart.begin(), fg.apart.end());
   std::vector<int> group_of((size_t)s->n_items, -1);
   std::vector<char> internal = planned.unused;
@@ -1268,7 +1273,9 @@ char *poly_hip_plan_kernel_desc(const PolyHipPlan *plan, int step) {
 
 void *poly_hip_plan_slot_ptr(const PolyHipPlan *plan, int slot) {
   if (!plan || slot < 0 || slot >= (int)plan->slot_ptr.size()) return nullptr;
-  return plan->slot_ptr[(size_t)slot];
+  if (plan->ran_plain) plan = plan->plain;
+  const int held = plan->held_by.empty() ? -1 : plan->held_by[(size_t)slot];
+  return plan->slot_ptr[(size_t)(held >= 0 ? held : slot)];
 }
 
 void poly_hip_plan_set_graph(PolyHipPlan *plan, int enabled) { if (plan) plan->use_graph = plan->graph_asked = enabled != 0; }
@@ -1279,10 +1286,12 @@ int poly_hip_plan_side_launches(const PolyHipPlan *plan) {
 }
 
 void poly_hip_plan_graph_counts(const PolyHipPlan *plan, long long *captures, long long *rebinds) {
-  if (captures) *captures = plan ? plan->n_captures : 0;
-  if (rebinds) *rebinds = plan ? plan->n_rebinds : 0;
+  if (captures) *captures = plan ? plan->n_captures + (plan->plain ? plan->plain->n_captures : 0) : 0;
+  if (rebinds) *rebinds = plan ? plan->n_rebinds + (plan->plain ? plan->plain->n_rebinds : 0) : 0;
 }
 
-size_t poly_hip_plan_workspace_bytes(const PolyHipPlan *plan) { return plan ? plan->arena_bytes + plan->scratch_bytes + plan->kept_scratch_bytes : 0; }
+size_t poly_hip_plan_workspace_bytes(const PolyHipPlan *plan) {
+  return plan ? plan->arena_bytes + plan->scratch_bytes + plan->kept_scratch_bytes + poly_hip_plan_workspace_bytes(plan->plain) : 0;
+}
 
 }  // extern "C"

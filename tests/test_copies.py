@@ -169,3 +169,41 @@ def test_profile_leaves_what_a_run_leaves(shared):
                 plan.run(data)
         seen.append({k: v.cpu().numpy().tobytes() for k, v in by.items()})
     assert seen[0] == seen[1]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what,held,by", [("intermediate", [4], 3), ("copy of a copy", [4, 5], 3), ("update in place", [3], "p")])
+def test_where_a_slots_value_is(what, held, by):
+    """poly_hip_plan_slot_ptr of a slot whose copy takes no launch: the buffer that holds its value; on buffers
+    that share memory, where every kernel is launched, its own again.  The workspace of both forms counts."""
+    import ctypes as C
+
+    import torch
+    s, _ = _schedule(what)
+    plan = s.plan()
+    data, index = [None] * len(plan.slots), {}
+    for slot in plan.external_slots():
+        data[slot.index] = torch.rand(slot.numel, device="cuda")
+        index[slot.name] = slot.index
+
+    def value(slot):
+        plan.sync()
+        host = (C.c_float * N)()
+        assert plan.lib.poly_hip_copy_dtoh(host, plan.slot_ptr(slot), 4 * N) == 0
+        return list(host)
+
+    plan.run(data)
+    at = data[index["p"]].data_ptr() if by == "p" else plan.slot_ptr(by)
+    assert at and all(plan.slot_ptr(h) == at for h in held)
+    if by == "p":
+        small = plan.workspace_bytes()
+        data[index["p"]] = data[index["x"]][:N]
+        plan.run(data)
+        assert plan.slot_ptr(held[0]) not in (None, data[index["p"]].data_ptr()) and value(held[0]) == data[index["p"]].tolist()
+        assert plan.workspace_bytes() > small
+        data[index["p"]] = torch.rand(N, device="cuda")
+        plan.run(data)
+        assert plan.slot_ptr(held[0]) == data[index["p"]].data_ptr()
+    else:
+        want = data[index["x"]].double().reshape(N, K).sum(1)
+        assert all(abs(v - w) <= K * 2.0 ** -24 * w for v, w in zip(value(held[0]), want.tolist()))      # (a rounding per term)
