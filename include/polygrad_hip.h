@@ -46,7 +46,8 @@ int poly_hip_execute(PolyRunner *runner, void **args, int n_args);
  * allocates on its first poly_hip_execute.  Calls no hipMalloc/hipFree once
  * poly_hip_init() (or a first call on the device) has looked the array up.  Returns -1
  * with a "polygrad: execute_static:" message when the kernel needs more scratch than the
- * array holds; a one-stage kernel is simply launched.  Every call on a GPU uses the
+ * array holds (poly_hip_lower_item takes a form that fits where a kernel has one, and a plan the
+ * fastest); a one-stage kernel is simply launched.  Every call on a GPU uses the
  * same array: calls that overlap on one GPU (other streams, other threads) race. */
 #define POLY_HIP_STATIC_SCRATCH_BYTES (32u << 20)
 int poly_hip_execute_static(PolyRunner *runner, void **args, int n_args);

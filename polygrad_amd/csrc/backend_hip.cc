@@ -71,10 +71,17 @@ static bool render_root(const PolyUOp *root, const char *fn_name, int flags, Ren
   return true;
 }
 
-HipRunner *runner_create(const PolyUOp *root, const char *fn_name, int flags) {
+HipRunner *runner_create(const PolyUOp *root, const char *fn_name, int flags, size_t scratch_limit) {
   if (runtime_init() != 0) return nullptr;
   RenderedKernel rk;
   if (!render_root(root, fn_name ? fn_name : "kernel", flags, &rk)) return nullptr;
+  if (scratch_limit && rk.scratch_bytes > scratch_limit) {
+    RenderedKernel small;
+    matmul_hint_scratch_limit(scratch_limit);
+    const bool ok = render_root(root, fn_name ? fn_name : "kernel", flags, &small);
+    matmul_hint_scratch_limit(0);
+    if (ok && small.scratch_bytes <= scratch_limit) rk = std::move(small);
+  }
   return runner_from_rendered(rk, fn_name, true);
 }
 
@@ -365,7 +372,9 @@ void poly_hip_program_destroy(PolyHipProgram *prog) {
 int poly_hip_lower_item(PolyCtx *ctx, PolyUOp *scheduled_root, const char *fn_name, PolyRunner *out) {
   (void)ctx;  // the lowering only reads the graph; it creates no UOps
   if (!scheduled_root || !out) return -1;
-  HipRunner *r = runner_create(scheduled_root, fn_name, 0);
+  // (poly_hip_execute_static may be asked for any of them: a product whose fastest form leaves more
+  // partial sums than the static array holds takes the form that fits, if it has one)
+  HipRunner *r = runner_create(scheduled_root, fn_name, 0, POLY_HIP_STATIC_SCRATCH_BYTES);
   if (!r) return -1;
   out->kind = POLY_RUNNER_COMPILED;
   out->handle = r;

@@ -82,7 +82,7 @@ struct HipRunner {
   std::vector<void *> arg_ptrs;
 };
 
-HipRunner *runner_create(const PolyUOp *root, const char *fn_name, int flags);
+HipRunner *runner_create(const PolyUOp *root, const char *fn_name, int flags, size_t scratch_limit = 0);
 // From a kernel rendered elsewhere (fused groups); `named` false: the entry is still the
 // placeholder poly_k and gets its descriptive symbol here.
 HipRunner *runner_from_rendered(const RenderedKernel &rk, const char *fn_name, bool named);

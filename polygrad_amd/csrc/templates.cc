@@ -536,6 +536,8 @@ static bool epilogue_from_graph(const KernelGraph &g, const MatmulMatch &mm, Mat
 
 static thread_local const MatmulRows *g_a_rows = nullptr;
 void matmul_hint_a_rows(const MatmulRows *rows) { g_a_rows = rows; }
+static thread_local size_t g_scratch_limit = 0;
+void matmul_hint_scratch_limit(size_t bytes) { g_scratch_limit = bytes; }
 static thread_local MatmulEpilogue::BlockMaxima g_block_maxima;
 static thread_local int64_t g_block_maxima_rows = 0, g_block_maxima_pitch = 0;
 void matmul_hint_block_maxima(const MatmulEpilogue *e, int64_t rows, int64_t pitch) {
@@ -1205,6 +1207,7 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     Dma probe{0, 0, 0, 0, 0};
     for (int s = 16; s > S && t * 65536 <= 1.1 * (double)M * (double)N; s--) {
       if (t * Z * s > 256 || t * Z * s < 208 || (K / 32) % s != 0 || K / s < 4096 || !dma_for(256, 256, &probe)) continue;
+      if (g_scratch_limit && (double)part_off + (double)s * (double)Z * (double)M * (double)N * 4.0 > (double)g_scratch_limit) continue;
       S = s;
       BM = BN = 256; WVM = 4; WVN = 2; pipe = 2;
     }
