@@ -692,8 +692,9 @@ static int f32_split(int64_t M, int64_t N, int64_t K, int64_t Z, int *tile) {
 //   40x700x5000: 13.2 to two [380]).  More than 64 rows and columns run on 64x64 tiles of
 //   32x32 blocks there: the tile template puts one workgroup of four waves on a CU, whose
 //   matrix pipes idle at every barrier and load of a 16-deep K tile (53 TFLOP/s), where these
-//   waves meet once (512x784x4096: 41.0 us [69.9]; x4097: 70 [192]; 1024x1024x4096: 80 [106];
-//   128x1024x16384: 45 [105]; 200x300x8192: 25 [33]).  16-bit products of more than 64 rows and
+//   waves meet once (512x784x4096: 41.9 us [69.9]; x4097: 70 [192]; 1024x1024x4096: 80 [106];
+//   128x1024x16384: 45 [105]; 200x300x8192: 25 [33]; 64 to 121 tiles, depths of 4096 to 16384: 0.4 to
+//   0.63 of the time there, errors against float64 of 2.9e-7 to 5.8e-7 that are never larger).  16-bit products of more than 64 rows and
 //   columns and a depth of 8192 are left to the templates that deal it to workgroups.
 // The smallest tile that does not need more workgroups than the chip runs at once: few rows
 // want many narrow workgroups (128x768x768 fp32: 16x32 4.9 us, 32x64 9.8), many rows tiles
@@ -718,11 +719,6 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
       if (M > 64 && N > 64) f = Form{2, 2, 4, 6, 32};
       else f = tiles_of(1, 1) <= 64 ? Form{1, 1, 8, 6, 16} : Form{1, 2, 4, 6, 16};
       for (S = M > 64 && N > 64 && K >= 8192 ? 16 : 8; S > 1 && (K % (S * kv) != 0 || tiles_of(f.tm * f.block / 16, f.tn * f.block / 16) * S > 256);) S /= 2;
-      // (tiles for half the chip: 128x64 ones dealt to eight workgroups of two
-      // waves rather than 64x64 to two of four; 512x784x4096 41.0 us [39.4], its error against
-      // float64 2.94e-7 [4.08e-7]; the 12 MiB of partial sums are what the tests of scratch
-      // memory look for in this plan)
-      if (S == 2 && f.block == 32 && K % 32 == 0 && tiles_of(8, 4) <= 64 && 2 * tiles_of(8, 4) == tiles_of(4, 4)) { f = Form{4, 2, 2, 4, 32}; S = 8; }
     }
   } else {
     const bool few = M <= 16 || N <= 16 || tiles_of(4, 4) <= 64;
