@@ -1,6 +1,7 @@
 """Row chains whose last phase takes a computed row and the operand it came from, both kept (the
 shape of a cross-entropy's gradient): the longest rows that stay out of LDS, the shortest and
-longest that are partly there, as single elements and as 16-byte vectors.  Against float64."""
+longest that are partly there, as single elements and as 16-byte vectors; a row that is the only one,
+whose operand's positions depend on no row.  Against float64."""
 import ctypes as C
 import os
 import sys
@@ -13,7 +14,8 @@ from polygrad_amd import PlanFile, _ffi
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "perf"))
 import cases  # noqa: E402
 
-SIZES = [(3, 40961, False), (2, 46079, False), (3, 46081, True), (2, 46084, True), (5, 50257, True), (2, 53247, True), (300, 53248, True)]
+SIZES = [(3, 40961, False), (2, 46079, False), (3, 46081, True), (2, 46084, True), (5, 50257, True), (2, 53247, True), (300, 53248, True),
+         (1, 20000, False), (1, 40000, False), (1, 50257, True)]
 
 
 def _plan(rows, cols):
@@ -49,6 +51,7 @@ def test_in_bounds(rows, cols, in_lds, hiplib, monkeypatch):
     pf = _plan(rows, cols)
     text = _source(hiplib, pf)
     assert ("poly_row_kept" in text) == in_lds
+    assert "(c0[it] = " in text and text.count("c0[it]") >= 2      # read in the first phase, taken in a later one
     s = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents
     slots, launch = (C.c_int * 64)(), (C.c_int * 4)()
     n = hiplib.poly_hip_fused_group_launch(pf.schedule, 0, slots, 64, launch)
