@@ -1473,7 +1473,10 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
       at.c.erase(ord);
       stride *= e;
     }
-    if (dense && at.c.empty()) {
+    // (the last map's output is no buffer there: the product says where each of its positions is)
+    const std::string out_param = strf(", %s* data0", dt_cname(gl.n(gl.stores[0].param).dt));
+    const size_t out_at = code.rfind(out_param);
+    if (dense && at.c.empty() && out_at != std::string::npos) {
       // (its arguments under other names: the product's are fa<n>, too)
       std::string text = kept_decls + calls;
       for (size_t i = 0; (i = text.find("fa", i)) != std::string::npos; i++)
@@ -1484,9 +1487,9 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
         const size_t name = sig.find(strf(" fa%zu", j)), from = sig.rfind(',', name) == std::string::npos ? 0 : sig.rfind(',', name) + 2;
         params += (j > 1 ? ", " : "") + sig.substr(from, name - from) + strf(" ra%zu", j);
       }
-      out->rows.code = kept_types + code;
+      out->rows.code = kept_types + std::string(code).replace(out_at, out_param.size(), ", const PolyRowsOut data0");
       out->rows.params = params;
-      out->rows.call = "{ " + strf("%s *const ra0 = poly_rows_out; ", dt_cname(gl.n(gl.stores[0].param).dt)) + text + "}";
+      out->rows.call = "{ const PolyRowsOut ra0 = poly_rows_out; " + text + "}";
       out->rows.n_params = (int)arg_slots.size() - 1;
       out->rows.lanes = G;
       out->n_rows = (int64_t)rows;

@@ -18,9 +18,11 @@
 //                       it, which may use `poly_ks`, the part
 //   POLY_A_KC/B_KC      1: operand contiguous along K; 0: along M (resp. N)
 //   POLY_A_ROWS(row, lane, out)  (optional, one z, A contiguous along K in rows of K
-//                       elements) A is no buffer: this leaves element f of its row `row` at
-//                       out[row * K + f], called by POLY_A_ROW_LANES (32 or 64) lanes; and
-//                       POLY_A_UNREAD, which declares the pointer A would have had
+//                       elements) A is no buffer: this stores element f of its row `row` at
+//                       position row * K + f of `out`, called by POLY_A_ROW_LANES (32 or 64)
+//                       lanes; PolyRowsOut{place, first}, what `out` is: the rows from position
+//                       `first` on, in LDS at `place`; and POLY_A_UNREAD, which declares the
+//                       pointer A would have had
 //   POLY_A_PTR/B_PTR, poly_a_row(m), poly_b_row(n), poly_a_z(z), poly_b_z(z),
 //   poly_a_k(k), poly_b_k(k), POLY_SIGNATURE, POLY_EPILOGUE(acc, m, n, z) and
 //   optionally POLY_EP_MID_VALUE / POLY_EP_MID_PTR: as in matmul_mfma.hip
@@ -298,7 +300,7 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
 #pragma unroll
   for (int s = 0; s < (ALL < D ? ALL : D); s++) load(s, s, false, true);
   for (int row = wave * (64 / POLY_A_ROW_LANES) + lane / POLY_A_ROW_LANES; row < n_rows; row += POLY_WAVES * (64 / POLY_A_ROW_LANES)) {
-    POLY_TIN *const to = gA + row * POLY_ROW_PAD - (long long)m0 * POLY_K;
+    const PolyRowsOut to{gA + row * (POLY_K + POLY_ROW_PAD), (m0 + row) * POLY_K};
     POLY_A_ROWS((long long)(m0 + row), lane % POLY_A_ROW_LANES, to);
   }
   __syncthreads();

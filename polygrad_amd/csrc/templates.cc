@@ -792,7 +792,10 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
     const std::string shape = strf("#define POLY_SIGNATURE %s%s\n#define POLY_KSPLIT %d\n#define POLY_PARTIALS poly_scratch\n", signature.c_str(), S > 1 ? ", float* poly_scratch" : "", S) + ep.code;
     cfg += shape;
     if (g_a_rows)      // (the epilogue's functions take every parameter of their kernels: A's is not read)
-      cfg += g_a_rows->code + strf("#define POLY_A_ROWS(row, lane, poly_rows_out) %s\n#define POLY_A_ROW_LANES %d\n#define POLY_A_UNREAD const %s *const %s = nullptr; (void)%s\n",
+      cfg += "struct PolyRowsOut {\n  POLY_TIN *place;\n  int first;\n"
+             "  template <class I> __device__ __forceinline__ POLY_TIN *operator+(I i) const { return place + ((int)i - first); }\n"
+             "  template <class I> __device__ __forceinline__ POLY_TIN &operator[](I i) const { return place[(int)i - first]; }\n};\n" +
+             g_a_rows->code + strf("#define POLY_A_ROWS(row, lane, poly_rows_out) %s\n#define POLY_A_ROW_LANES %d\n#define POLY_A_UNREAD const %s *const %s = nullptr; (void)%s\n",
                                    g_a_rows->call.c_str(), g_a_rows->lanes, dt_cname(mm.A.dt), ep.a_ptr.c_str(), ep.a_ptr.c_str());
     // what the kernel that has an element's whole sum does with it
     std::string finish = strf("#define POLY_EPILOGUE(acc, m, n, z) %s\n", ep.call.c_str());

@@ -106,10 +106,11 @@ void matmul_hint_input_params(uint64_t mask);
 // other use.
 void matmul_hint_param_kinds(const std::vector<int> &kinds);
 // Also set around a lowering: operand A's rows, a buffer nothing else reads, are computed by the
-// product itself (a LayerNorm in front of it).  `call` leaves row `row` (`lane` of `lanes`, 32 or 64) at
-// poly_rows_out[row * K + f]; `params`, `n_params` of them, stand in A's place in the signature.
-// Products of up to 16 rows that the template whose waves deal the depth takes do that
-// (RenderedKernel::computes_rows says whether this one does).
+// product itself (a LayerNorm in front of it).  `call` stores row `row` (`lane` of `lanes`, 32 or 64) at
+// the positions row * K + f of poly_rows_out, a PolyRowsOut (kernels/matmul_wave.hip); `params`,
+// `n_params` of them, stand in A's place in the signature.  Products of up to 64 rows that the template
+// whose waves deal the depth takes do that where its tile's rows have room in LDS and are no more than
+// two to a wave, one after another (RenderedKernel::computes_rows says whether this one does).
 struct MatmulRows {
   std::string code, params, call;
   int n_params = 0, lanes = 64;

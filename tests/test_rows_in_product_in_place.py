@@ -72,9 +72,13 @@ def test_grouping(rows, d, w, form, fused, hiplib, monkeypatch):
     for gi in range(hiplib.poly_hip_fused_groups(pf.schedule, -1, None, None)):
         src = C.c_void_p()
         hiplib.poly_hip_fused_groups(pf.schedule, gi, C.byref(src), None)
-        if "#define POLY_A_ROWS(" not in _ffi.take_string(src.value):
+        text = _ffi.take_string(src.value)
+        if "#define POLY_A_ROWS(" not in text:
             continue
         found += 1
+        # (positions in the rows' own array, never a pointer in front of it)
+        assert text.count("const PolyRowsOut data0") == 1
+        assert hiplib.poly_hip_compile_check(text.split("\n// ---- ")[0].encode()) == 0
         slots = (C.c_int * 64)()
         n = hiplib.poly_hip_fused_group_launch(pf.schedule, gi, slots, 64, None)
         assert slots[0] not in list(slots[1:n]), list(slots[:n])
