@@ -171,9 +171,13 @@ bool plan_schedule(const PolySchedule *s, bool buffers_apart, PlannedSchedule *o
   out->unused.assign((size_t)s->n_buf_slots, 0);
   out->written_early.clear();
   out->held_by.clear();
-  find_fused_groups(s, out->graphs, buffers_apart, &out->groups);
+  find_fused_groups(s, out->graphs, &out->groups);
+  auto as_it_is = [&]() {
+    refine_fused_groups(s, out->graphs, buffers_apart, &out->groups);
+    return true;
+  };
   // (a dropped copy is two buffers of the schedule in one place, which POLY_HIP_NO_ALIAS is about)
-  if (!buffers_apart || getenv("POLY_HIP_NO_FUSION") || getenv("POLY_HIP_NO_COPY_DROP") || getenv("POLY_HIP_NO_ALIAS")) return true;
+  if (!buffers_apart || getenv("POLY_HIP_NO_FUSION") || getenv("POLY_HIP_NO_COPY_DROP") || getenv("POLY_HIP_NO_ALIAS")) return as_it_is();
 
   // (what a group has taken in costs no launch, and the matchers know those copies)
   std::vector<char> grouped((size_t)s->n_items, 0);
@@ -190,9 +194,9 @@ bool plan_schedule(const PolySchedule *s, bool buffers_apart, PlannedSchedule *o
   for (int st = 0; st < s->n_items; st++) rw.step[(size_t)s->exec_order[st]] = st;
   for (int k = 0; k < s->n_items; k++) {
     const PolyExecItem &it = s->items[k];
-    if ((int)out->graphs[(size_t)k].params.size() != it.n_buf_slots) return true;
+    if ((int)out->graphs[(size_t)k].params.size() != it.n_buf_slots) return as_it_is();
     for (int i = 0; i < it.n_buf_slots; i++)
-      if (it.buf_slot_indices[i] < 0 || it.buf_slot_indices[i] >= s->n_buf_slots) return true;
+      if (it.buf_slot_indices[i] < 0 || it.buf_slot_indices[i] >= s->n_buf_slots) return as_it_is();
     rw.args.push_back(std::vector<int>(it.buf_slot_indices, it.buf_slot_indices + it.n_buf_slots));
   }
   int n_dropped = 0;
@@ -200,17 +204,22 @@ bool plan_schedule(const PolySchedule *s, bool buffers_apart, PlannedSchedule *o
     const int k = s->exec_order[st];
     if (!grouped[(size_t)k] && out->graphs[(size_t)k].reduces.empty() && rw.drop(k)) n_dropped++;
   }
-  if (n_dropped == 0) return true;
+  if (n_dropped == 0) return as_it_is();
 
   PlannedSchedule p;
   p.sched = *s;
   std::vector<int> number((size_t)s->n_items, -1);
+  auto keep_copies = [&]() {
+    for (int k = 0; k < s->n_items; k++)
+      if (number[(size_t)k] >= 0) out->graphs[(size_t)k] = std::move(p.graphs[(size_t)number[(size_t)k]]);
+    return as_it_is();
+  };
   for (int k = 0; k < s->n_items; k++) {
     if (rw.dropped[(size_t)k]) continue;
     number[(size_t)k] = (int)p.items.size();
     p.items.push_back(s->items[k]);
     p.args.push_back(rw.args[(size_t)k]);
-    p.graphs.push_back(out->graphs[(size_t)k]);
+    p.graphs.push_back(std::move(out->graphs[(size_t)k]));
   }
   for (size_t i = 0; i < p.items.size(); i++) p.items[i].buf_slot_indices = p.args[i].data();
   for (int st = 0; st < s->n_items; st++)
@@ -222,14 +231,13 @@ bool plan_schedule(const PolySchedule *s, bool buffers_apart, PlannedSchedule *o
   p.held_by = rw.held_by;
   p.unused.assign((size_t)s->n_buf_slots, 1);
   for (const auto &a : p.args) for (int sl : a) p.unused[(size_t)sl] = 0;
-  for (int sl = 0; sl < s->n_buf_slots; sl++) {
-    bool used_before = false;
-    for (int k = 0; k < s->n_items && !used_before; k++)
-      for (int i = 0; i < s->items[k].n_buf_slots; i++) used_before = used_before || s->items[k].buf_slot_indices[i] == sl;
-    if (!used_before || !s->buf_slots[sl].is_intermediate) p.unused[(size_t)sl] = 0;
-  }
-  find_fused_groups(&p.sched, p.graphs, buffers_apart, &p.groups);
-  if (n_launches(&p.sched, p.groups) >= n_launches(s, out->groups)) return true;
+  std::vector<char> used_before((size_t)s->n_buf_slots, 0);
+  for (int k = 0; k < s->n_items; k++)
+    for (int i = 0; i < s->items[k].n_buf_slots; i++) used_before[(size_t)s->items[k].buf_slot_indices[i]] = 1;
+  for (int sl = 0; sl < s->n_buf_slots; sl++)
+    if (!used_before[(size_t)sl] || !s->buf_slots[sl].is_intermediate) p.unused[(size_t)sl] = 0;
+  find_fused_groups(&p.sched, p.graphs, &p.groups);
+  if (n_launches(&p.sched, p.groups) >= n_launches(s, out->groups)) return keep_copies();
   // (a kernel that reads the old contents of such a buffer is not in one launch with the one
   // that writes it: what one workgroup has stored, another might still have to read)
   for (const FusedGroup &fg : p.groups)
@@ -239,9 +247,10 @@ bool plan_schedule(const PolySchedule *s, bool buffers_apart, PlannedSchedule *o
           bool writes = false, reads = false;
           for (size_t i = 0; i < p.args[(size_t)a].size(); i++) writes = writes || (p.args[(size_t)a][i] == sl && p.graphs[(size_t)a].params[i].written);
           for (size_t i = 0; i < p.args[(size_t)b].size(); i++) reads = reads || (p.args[(size_t)b][i] == sl && p.graphs[(size_t)b].params[i].read);
-          if (writes && reads && std::find(p.order.begin(), p.order.end(), b) < std::find(p.order.begin(), p.order.end(), a)) return true;
+          if (writes && reads && std::find(p.order.begin(), p.order.end(), b) < std::find(p.order.begin(), p.order.end(), a)) return keep_copies();
         }
   if (getenv("POLY_HIP_DEBUG")) fprintf(stderr, "polygrad: compile_schedule: %d copies need no launch, %zu buffers of the caller are written by the kernel in front\n", n_dropped, p.written_early.size());
+  refine_fused_groups(&p.sched, p.graphs, buffers_apart, &p.groups);
   *out = std::move(p);
   return true;
 }

@@ -2963,31 +2963,43 @@ std::vector<int> fused_groups_out_of_order(const PolySchedule *s, const std::vec
   return std::vector<int>(bad.begin(), bad.end());
 }
 
-void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &graphs, bool buffers_apart, std::vector<FusedGroup> *out) {
+// Who reads and who writes each buffer, and when; false where the schedule is not one to look at.
+static bool index_schedule(Sched *sc) {
+  const PolySchedule *s = sc->s;
+  sc->step_of.assign((size_t)s->n_items, 0);
+  for (int st = 0; st < s->n_items; st++) sc->step_of[(size_t)s->exec_order[st]] = st;
+  sc->launch_step = sc->step_of;
+  sc->readers.assign((size_t)s->n_buf_slots, {});
+  sc->writers.assign((size_t)s->n_buf_slots, {});
+  for (int k = 0; k < s->n_items; k++) {
+    const PolyExecItem &it = s->items[k];
+    const KernelGraph &g = sc->graphs[(size_t)k];
+    if ((int)g.params.size() != it.n_buf_slots) return false;
+    for (int i = 0; i < it.n_buf_slots; i++) {
+      const int sl = it.buf_slot_indices[i];
+      if (sl < 0 || sl >= s->n_buf_slots) return false;
+      if (g.params[(size_t)i].read) sc->readers[(size_t)sl].push_back(k);
+      if (g.params[(size_t)i].written) sc->writers[(size_t)sl].push_back(k);
+    }
+  }
+  for (auto &v : sc->readers) { std::sort(v.begin(), v.end()); v.erase(std::unique(v.begin(), v.end()), v.end()); }
+  return true;
+}
+
+// `fg` takes its kernels.
+static void take_items(Sched *sc, const FusedGroup &fg, std::vector<char> *taken) {
+  for (int it : fg.items) { (*taken)[(size_t)it] = 1; sc->launch_step[(size_t)it] = sc->step_of[(size_t)fg.launch_item]; }
+}
+
+void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &graphs, std::vector<FusedGroup> *out) {
   out->clear();
   if (getenv("POLY_HIP_NO_FUSION")) return;
   Sched sc{s, graphs, {}, {}, {}, {}};
-  sc.step_of.assign((size_t)s->n_items, 0);
-  for (int st = 0; st < s->n_items; st++) sc.step_of[(size_t)s->exec_order[st]] = st;
-  sc.launch_step = sc.step_of;
+  if (!index_schedule(&sc)) return;
   auto accept = [&](FusedGroup &fg, std::vector<char> &taken) {
-    for (int it : fg.items) { taken[(size_t)it] = 1; sc.launch_step[(size_t)it] = sc.step_of[(size_t)fg.launch_item]; }
+    take_items(&sc, fg, &taken);
     out->push_back(std::move(fg));
   };
-  sc.readers.assign((size_t)s->n_buf_slots, {});
-  sc.writers.assign((size_t)s->n_buf_slots, {});
-  for (int k = 0; k < s->n_items; k++) {
-    const PolyExecItem &it = s->items[k];
-    const KernelGraph &g = graphs[(size_t)k];
-    if ((int)g.params.size() != it.n_buf_slots) return;
-    for (int i = 0; i < it.n_buf_slots; i++) {
-      const int sl = it.buf_slot_indices[i];
-      if (sl < 0 || sl >= s->n_buf_slots) return;
-      if (g.params[(size_t)i].read) sc.readers[(size_t)sl].push_back(k);
-      if (g.params[(size_t)i].written) sc.writers[(size_t)sl].push_back(k);
-    }
-  }
-  for (auto &v : sc.readers) { std::sort(v.begin(), v.end()); v.erase(std::unique(v.begin(), v.end()), v.end()); }
   std::vector<char> taken((size_t)s->n_items, 0);
   for (int st = 0; st < s->n_items; st++) {
     const int k = s->exec_order[st];
@@ -3021,6 +3033,18 @@ void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &gr
     if (!match_side_by_side(sc, k, taken, &fg)) continue;
     accept(fg, taken);
   }
+}
+
+void refine_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &graphs, bool buffers_apart, std::vector<FusedGroup> *out) {
+  if (out->empty()) return;
+  Sched sc{s, graphs, {}, {}, {}, {}};
+  if (!index_schedule(&sc)) return;
+  std::vector<char> taken((size_t)s->n_items, 0);
+  for (const FusedGroup &fg : *out) take_items(&sc, fg, &taken);
+  auto accept = [&](FusedGroup &fg, std::vector<char> &taken) {
+    take_items(&sc, fg, &taken);
+    out->push_back(std::move(fg));
+  };
   // A row chain whose result is an fp32 buffer of bf16 values (the derivative of the scores
   // of attention: a cast of a bf16 product), read by one product that can take it as a
   // 16-bit operand where it lies: the chain stores the bf16 values, the product reads them,

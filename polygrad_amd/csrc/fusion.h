@@ -44,11 +44,14 @@ struct FusedGroup {
 };
 
 // Finds the fusable groups of a schedule.  graphs[k] is the analysed kernel of item k.
-// Setting POLY_HIP_NO_FUSION in the environment disables the search.  !buffers_apart: only groups
-// that do what their kernels do also where buffers of the caller's share memory (FusedGroup::apart).
-void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &graphs, bool buffers_apart, std::vector<FusedGroup> *out);
+// Setting POLY_HIP_NO_FUSION in the environment disables the search.
+void find_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &graphs, std::vector<FusedGroup> *out);
+// What is done with the groups once they are known: pairs that work together are rendered again,
+// and groups that would launch out of order are dropped.  !buffers_apart: only what does as the
+// kernels do also where buffers of the caller's share memory (FusedGroup::apart).
+void refine_fused_groups(const PolySchedule *s, const std::vector<KernelGraph> &graphs, bool buffers_apart, std::vector<FusedGroup> *out);
 // The groups (indices into `groups`) whose place of launch breaks the order of two kernels
-// of the schedule that share a buffer, one of them writing it; find_fused_groups drops such
+// of the schedule that share a buffer, one of them writing it; refine_fused_groups drops such
 // groups itself, so that its result always passes.
 std::vector<int> fused_groups_out_of_order(const PolySchedule *s, const std::vector<KernelGraph> &graphs, const std::vector<FusedGroup> &groups);
 

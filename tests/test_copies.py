@@ -106,6 +106,16 @@ def test_which_copies_go(what, hiplib, monkeypatch, capfd):
     assert [int(line.split(": ")[2].split()[0]) for line in said] == ([n] if n else [])
 
 
+def test_groups_are_refined_once(hiplib, monkeypatch, capfd):
+    """Which copies go is found out with the groups as they are first; those that work in pairs (attention and
+    the product its keys come from, one in each of 12 layers) are rendered for each other once."""
+    monkeypatch.setenv("POLY_HIP_DEBUG", "1")
+    pf = PlanFile(os.path.join(cases.PLANS, "gpt2_small_bf16_b8_t1024.polyplan"))
+    assert hiplib.poly_hip_fused_groups(pf.schedule, -1, None, None) > 12
+    err = capfd.readouterr().err
+    assert err.count("leaves the block maxima of the keys") == 12 and err.count("need no launch") == 1
+
+
 def _run(plan, shared):
     import torch
     g = torch.Generator(device="cuda")
