@@ -1164,12 +1164,14 @@ static bool split_in_two(const KernelGraph &g, const std::string &fn_name, const
   o2.allow_vectorize = false;       // thread id == flat output index, which is what the terms are filed under
   const long long RT = (long long)rt;
   // Promoted terms (at most 64 outputs of 64 terms and more): a wave per output adds them up side
-  // by side, where one thread did it term after term (the loss over 4096 tokens 83 -> 4 us)
-  // and with a rounding of the whole sum for each.
+  // by side, four outputs to a workgroup, where one thread did it term after term and with a rounding of
+  // the whole sum for each (the loss over 4096 tokens 83 -> 4 us; both stages, terms of 300 elements, by
+  // one thread per output and by waves: 1 output of 4096 70 -> 19 us, 5 of 1000 18.6 -> 9.5, 33 of 1000
+  // 23.6 -> 14.1, 64 of 4096 138 -> 85, where one workgroup's four waves for all 64 took 310).
   const bool by_waves = slice_range < 0;
   o2.reduce_override[T] = [T, RT, top, by_waves](Emitter &em, Scope *s) {
     (void)em;
-    if (by_waves) return std::string("poly_sums[gid]");
+    if (by_waves) return std::string("poly_sums[threadIdx.x]");
     const std::string acc = strf("acc%d", T);
     std::string pad((size_t)s->indent * 2, ' ');
     s->code += pad + strf("float %s = %s;\n", acc.c_str(), Emitter::reduce_identity(top, DT_F32).c_str());
@@ -1183,12 +1185,15 @@ static bool split_in_two(const KernelGraph &g, const std::string &fn_name, const
     const size_t body = out->source.find("  const long long gid = ", out->source.rfind("__global__"));
     const unsigned waves = out->launch.block[0] / 64;
     if (body == std::string::npos || out->launch.grid[0] != 1 || waves == 0) return false;
-    out->source.insert(body, strf("  __shared__ float poly_sums[%d];\n", (int)rows) +
-                             strf("  for (int o_ = threadIdx.x >> 6; o_ < %d; o_ += %u) {\n    float acc = %s;\n", (int)rows, waves, Emitter::reduce_identity(top, DT_F32).c_str()) +
-                             strf("    for (int q_ = threadIdx.x & 63; q_ < %lld; q_ += 64) acc = %s;\n", RT,
-                                  Emitter::reduce_combine(top, DT_F32, "acc", strf("poly_scratch[o_ * %lldll + q_]", RT)).c_str()) +
-                             strf("    acc = %s;\n", wave_reduce_call(top, DT_F32, "acc").c_str()) +
-                             "    if ((threadIdx.x & 63) == 0) poly_sums[o_] = acc;\n  }\n  __syncthreads();\n");
+    out->source.replace(body, out->source.find('\n', body) - body,
+                        strf("  __shared__ float poly_sums[%u];\n  const long long o_ = (long long)blockIdx.x * %u + (threadIdx.x >> 6);\n", waves, waves) +
+                            strf("  if (o_ < %d) {\n    float acc = %s;\n", (int)rows, Emitter::reduce_identity(top, DT_F32).c_str()) +
+                            strf("    for (int q_ = threadIdx.x & 63; q_ < %lld; q_ += 64) acc = %s;\n", RT,
+                                 Emitter::reduce_combine(top, DT_F32, "acc", strf("poly_scratch[o_ * %lldll + q_]", RT)).c_str()) +
+                            strf("    acc = %s;\n", wave_reduce_call(top, DT_F32, "acc").c_str()) +
+                            "    if ((threadIdx.x & 63) == 0) poly_sums[threadIdx.x >> 6] = acc;\n  }\n  __syncthreads();\n" +
+                            strf("  const long long gid = threadIdx.x < %u ? (long long)blockIdx.x * %u + threadIdx.x : %dll;", waves, waves, (int)rows));
+    out->launch.grid[0] = ((unsigned)rows + waves - 1) / waves;
   }
   out->pres.push_back({pre.source, pre.entry, pre.launch});
   out->scratch_bytes = (size_t)(rows * rt) * sizeof(float);

@@ -1,5 +1,5 @@
 """Reductions of reductions to few outputs in two stages, the second a wave per output: the fewest and
-most outputs, the fewest terms, one more, and many.  Against float64 on the host."""
+most outputs, the fewest terms, one more, and many; every output on a wave of its own.  Against float64 on the host."""
 import ctypes as C
 import os
 import sys
@@ -12,7 +12,7 @@ from polygrad_amd import PlanFile, _ffi
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "perf"))
 import cases  # noqa: E402
 
-SIZES = [(1, 64, 256), (1, 65, 300), (3, 127, 257), (5, 4096, 256), (64, 70, 256)]
+SIZES = [(1, 64, 256), (1, 65, 300), (3, 127, 257), (5, 4096, 256), (64, 70, 256), (33, 1000, 256)]
 
 
 def _plan(op, rows, terms, inner):
@@ -35,6 +35,9 @@ def test_in_bounds(op, rows, terms, inner, hiplib, monkeypatch):
     pf = _plan(op, rows, terms, inner)
     s = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents
     assert "two stages" in _ffi.take_string(hiplib.poly_hip_describe(s.items[0].root, 0))
+    launch = (C.c_int * 8)()
+    _ffi.take_string(hiplib.poly_hip_render(s.items[0].root, b"k", 0, launch))
+    assert launch[0] == (rows + 3) // 4 and launch[3] == 256      # of the second stage: four waves to a workgroup
     assert hostcheck.check_schedule(hiplib, pf.schedule) == 2
 
 
