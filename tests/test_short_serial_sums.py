@@ -1,5 +1,5 @@
-"""Sums that one thread adds up term by term, about the extents where all loads of a loop or those of eight
-terms are in flight: column sums and sums of products, few and many outputs.  Against float64 on the host."""
+"""Sums that one thread adds up term by term, about the extents where all loads of a loop, those of as many
+terms as divide it, of sixteen or of eight are in flight: column sums and sums of products, few and many outputs.  Against float64 on the host."""
 import ctypes as C
 import os
 
@@ -10,8 +10,9 @@ from polygrad_amd import PlanFile, _ffi
 from test_promoted_reduce import cases
 
 # columns, terms, whether two operands are read a term, how the loop is unrolled
-SIZES = [(100, 15, False, ""), (100, 16, False, "unroll"), (1290, 33, True, "unroll"), (70, 36, True, "unroll"), (70, 37, True, "unroll 8"),
-         (257, 63, False, "unroll"), (257, 64, False, "unroll 8"), (70001, 17, True, "unroll")]
+SIZES = [(100, 15, False, ""), (100, 16, False, "unroll"), (1290, 33, True, "unroll 11"), (70, 36, True, "unroll 12"), (70, 37, True, "unroll 16"), (70, 28, True, "unroll"),
+         (70, 29, True, "unroll 16"), (100000, 32, True, "unroll 16"), (257, 56, False, "unroll"), (257, 57, False, "unroll 16"), (257, 63, False, "unroll 9"), (257, 64, False, "unroll 8"),
+         (70001, 17, True, "unroll")]
 
 
 def _plan(cols, terms, two):
