@@ -674,6 +674,15 @@ static int f32_split(int64_t M, int64_t N, int64_t K, int64_t Z, int *tile) {
   return 1;
 }
 
+// How render_matmul_f32 reads an operand, in 16-byte pieces along K (*kc) or along the operand's row axis;
+// false where it cannot.
+static bool f32_layout(const KSplit &ks, const std::vector<Dim> &dims, bool is_a, int64_t rows, int64_t K, bool *kc) {
+  const int64_t inner_c = is_a ? dims.back().ca : dims.back().cb;
+  const bool along_k = ks.s_lo == 1 && ks.kb % 16 == 0;
+  if (kc) *kc = along_k;
+  return K % 16 == 0 && (along_k || (inner_c == 1 && dims.back().extent % 4 == 0 && rows % 4 == 0));
+}
+
 // Products of few or ragged tiles: kernels/matmul_wave.hip, the depth dealt to the waves of
 // a workgroup.  Where it is taken, and on which tile (all times: one launch, operands in the
 // memory-side cache, the other templates in brackets):
@@ -740,7 +749,19 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
   int split_tile;
   const int sums_there = f32 ? f32_split(M, N, K, Z, &split_tile) : 1;
   const int sums = f32 && K >= 2048 && f.waves * S < std::max(8, sums_there) && f.depth % 2 == 0 ? 2 : 1;
-  if (f.block == 32 && f.waves * S * sums < sums_there) return false;
+  const bool tiled = f32 && ep.mid_value_call.empty() && f32_layout(mm.ka, mm.md, true, M, K, nullptr) && f32_layout(mm.kb, mm.nd, false, N, K, nullptr);
+  if (f.block == 32 && tiled && f.waves * S * sums < sums_there) return false;
+  // ... nor fewer workgroups than pay: the depth is dealt here to 1, 2, 4, 8 or 16 as S * 4 divides it, there to as
+  // many as its steps of 16 divide into.  By rounds over the chip, depth of a part and area of a tile this
+  // template takes some 0.6 of the time for the same work (0.5 with a few tiles): 344x136x21424 93 us dealt to
+  // 4 [65 to 13], 910x1108x12960 434 on 270 tiles [330, 128x128 dealt to 6], 466x524x15648 145 [130];
+  // 719x352x4800 and 80x1092x5856, 1.5 times the work, the same either way.
+  if (f.block == 32 && tiled && sums_there > 1) {
+    const double t = tiles_of(4, 4), st = split_tile;
+    const double there = std::ceil((double)((M + split_tile - 1) / split_tile) * (double)((N + split_tile - 1) / split_tile) * (double)Z * sums_there / 256.0) / sums_there * st * st;
+    const double here = std::ceil(t * S / 256.0) / S * 64.0 * 64.0;
+    if (here > (t >= 30 ? 1.45 : 2.0) * there) return false;
+  }
   // an operand is read along K where its steps are contiguous there, along its rows otherwise
   // (runs of as many rows as the tile has blocks)
   auto layout = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a, int64_t rows, int run, bool *kc) {
@@ -862,16 +883,8 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
 static bool render_matmul_f32(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKernel *out) {
   const int64_t K = mm.K, M = mm.M, N = mm.N, Z = mm.Z;
   if (getenv("POLY_HIP_NO_F32_MFMA")) return reject(__LINE__);
-  // operand layout: 16-byte pieces along K, or along the operand's row axis
-  auto layout = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a, int64_t rows, bool *kc) {
-    const int64_t inner_c = is_a ? dims.back().ca : dims.back().cb;
-    if (K % 16 != 0) return reject(__LINE__);
-    if (ks.s_lo == 1 && ks.kb % 16 == 0) { *kc = true; return true; }
-    if (inner_c == 1 && dims.back().extent % 4 == 0 && rows % 4 == 0) { *kc = false; return true; }
-    return reject(__LINE__);
-  };
   bool a_kc, b_kc;
-  if (!layout(mm.ka, mm.md, true, M, &a_kc) || !layout(mm.kb, mm.nd, false, N, &b_kc)) return reject(__LINE__);
+  if (!f32_layout(mm.ka, mm.md, true, M, K, &a_kc) || !f32_layout(mm.kb, mm.nd, false, N, K, &b_kc)) return reject(__LINE__);
   int BM, BN, WVM, WVN;
   f32_tile(M, N, Z, &BM, &BN, &WVM, &WVN);
   // deep product on few tiles: larger tiles, K dealt to several workgroups each

@@ -13,7 +13,7 @@ from polygrad_amd import PlanFile, _ffi
 from test_small_matmul import _case, _name, cases
 
 DEEP = [(65, 65, 4096, "nn", 8), (128, 66, 4100, "nt", 1), (129, 191, 4097, "tn", 1), (512, 784, 4096, "tn", 2), (384, 900, 4128, "nn", 2), (70, 130, 8192, "nn", 16), (192, 193, 5000, "nt", 2),
-        (700, 700, 4112, "tn", 2), (1000, 1024, 4104, "nn", 1)]
+        (700, 700, 4112, "tn", 2), (1000, 1024, 4104, "nn", 1), (829, 863, 18832, "tn", 1)]
 
 
 def _form(split):
@@ -29,6 +29,18 @@ def test_stays_in_bounds(c, hiplib, monkeypatch):
     desc = _ffi.take_string(hiplib.poly_hip_describe(s.items[0].root, 0))
     assert "mfma 32x32x2 f32" in desc and "depth dealt to 4 waves" in desc and _form(c[4]) in desc
     assert hostcheck.check_schedule(hiplib, pf.schedule) >= 1
+
+
+@pytest.mark.parametrize("m,n,k,layout,here", [(344, 136, 21424, "tn", False), (344, 136, 21504, "tn", True), (910, 1108, 12960, "nt", False), (910, 1108, 12961, "nt", True),
+                                               (466, 524, 15648, "nt", False), (466, 524, 15360, "nt", True), (126, 108, 15840, "nt", True), (147, 315, 5808, "nn", True),
+                                               (829, 863, 18832, "tn", True)])
+def test_which_template(m, n, k, layout, here, hiplib, monkeypatch):
+    """A depth that 16 and 32 do not divide well goes to the tile template where that deals it to several times
+    as many workgroups; one that it cannot deal at all, or rows that it cannot read, stay."""
+    monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
+    pf = cases._matmul_schedule(_case(m, n, k, "float32", layout)).plan()
+    s = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents
+    assert ("depth dealt to" in _ffi.take_string(hiplib.poly_hip_describe(s.items[0].root, 0))) == here
 
 
 @pytest.mark.gpu
