@@ -1381,18 +1381,22 @@ static bool match_row_chain_impl(const Sched &sc, int a_item, const std::vector<
   // of 600 x 50000 90).  Of rows that are still needed together once the first of them is made, what
   // kRowChainKept1024 registers do not hold is in LDS: the cross-entropy's gradient over
   // 4096 x 50257 keeps the logits and a computed row, and the step it is part of takes 5977 us
-  // with 60 registers [5990 with 45, 5995 with 80, 6150 with all, 6640 before].  Not rows
+  // with 60 registers [5990 with 45, 5995 with 80, 6150 with all, 6640 before].  Vectors of four have an address
+  // for four elements: 300 rows of 46084 to 48000 gain 6 to 9 % all the same, of 49152 to 53248 within 2 %, but
+  // one row alone does not (softmax of 1 x 53248 13.6 us, 16.7 so) unless registers do not hold what is
+  // kept.  Not rows
   // that only the first phases take: those in LDS cost 10 % (600 x 50000 90 -> 100).
   std::string kept_types, kept_decls;
   {
-    int dwords = 0, lds_left = 156 << 10, longest = row_nit * row_V;
+    int dwords = 0, lds_left = 156 << 10, longest = row_nit * row_V, wide = row_V;
     for (const RowKept &k : rows_kept) dwords += row_nit * ((k.bytes + 3) / 4);
     for (const RowCache &c : cache) {
       longest = std::max(longest, c.nit * c.V);
+      wide = std::max(wide, c.V);
       // (operands that no phase takes after the first row is made are done with by then)
       if (!rows_kept.empty() && c.last > rows_kept[0].made) dwords += c.nit * ((c.bytes + 3) / 4);
     }
-    const bool over = G == 1024 && longest > kRowChainLong1024;
+    const bool over = G == 1024 && longest > kRowChainLong1024 && (wide == 1 || rows > 1 || dwords > kRowChainKept1024);
     if (G == 1024 && !over) kept_types = "#define POLY_FRESH(lane)\n";
     if (over)
       kept_types = "#ifdef POLY_HOST_ADDRESS_CHECK\n#define POLY_FRESH(lane)\n#else\n#define POLY_FRESH(lane) asm volatile(\"\" : \"+v\"(lane)); lane &= 1023\n#endif\n"
