@@ -15,7 +15,7 @@ sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), ".."
 import cases  # noqa: E402
 
 SIZES = [(5, 8), (9, 31), (70, 32), (3, 33), (33, 127), (1, 128), (2049, 1001), (5, 1023), (2050, 1024), (2049, 1025), (2048, 2050), (3, 4095), (7, 8191), (3, 8193), (2, 8194),
-         (2, 16388), (2, 50257), (2, 53248)]
+         (2, 16388), (2, 50257), (2, 53248), (1, 50257), (1, 53248)]
 TOO_LONG = [(2, 53249)]
 
 
@@ -35,6 +35,8 @@ def test_one_launch_in_bounds(op, rows, cols, hiplib, monkeypatch):
     hiplib.poly_hip_fused_groups(pf.schedule, 0, C.byref(src), C.byref(n_items))
     text = _ffi.take_string(src.value)
     assert n_items.value == (2 if (rows, cols) in TOO_LONG else s.n_items)
+    # (positions worked out again in each phase: where elements have an address each, or rows are many)
+    assert ("asm volatile" in text) == (cols in (50257, 53248) and (rows, cols) != (1, 53248))
     slots, launch = (C.c_int * 64)(), (C.c_int * 4)()
     n = hiplib.poly_hip_fused_group_launch(pf.schedule, 0, slots, 64, launch)
     sizes = [int(s.buf_slots[slots[i]].nbytes) for i in range(n)]
