@@ -163,10 +163,10 @@ struct RenderOptions {
   const RenderedKernel::OperandPlanes *planes_before = nullptr;
 };
 
-// Returns false and sets *err on unsupported graphs (never falls back to a
-// host path).
 // A rendered kernel without helpers or LDS of its own as a device function `name` of its workgroup number.
 bool kernel_as_device_fn(const std::string &src, const std::string &entry, const std::string &name, std::string *fn);
+// Returns false and sets *err on unsupported graphs (never falls back to a
+// host path).
 bool render_kernel(const KernelGraph &g, const std::string &fn_name, const RenderOptions &opt,
                    RenderedKernel *out, std::string *err);
 

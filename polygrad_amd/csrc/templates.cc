@@ -2185,8 +2185,9 @@ extern "C" __global__ void __launch_bounds__(1024) poly_guard(int* flag, const %
   // One launch for the gather and the walk over all V that replaces it where the check fails, each a
   // branch on workgroups of its own count (the walk's dealt to at most 4096, more than the
   // chip holds at once); and none for the check where every workgroup can make it on the way, eight
-  // elements a thread.  GPT-2 small, two tables, three launches fewer: 8 x 1024 bf16 tokens 2888 ->
-  // 2871 us (the walk's 24576 workgroups that left at once), 128 fp32 tokens 888.5 -> 883.3.
+  // elements a thread.  GPT-2 small, two tables, three launches fewer: their kernels 38 -> 25 us on
+  // 8 x 1024 bf16 tokens (the walk's 24576 workgroups that left at once) and 24 -> 13 on 128 fp32 tokens,
+  // the whole forward 3138 -> 3130 and 896 -> 888 us.
   std::string f1, f2;
   const std::string f_exit = "  if (*poly_flag == 0) return;\n", s_exit = "  if (*poly_flag != 0) return;\n";
   auto alone = [](const LaunchSpec &l) { return l.grid[1] == 1 && l.grid[2] == 1 && l.block[0] == 256 && l.block[1] == 1 && l.block[2] == 1; };
