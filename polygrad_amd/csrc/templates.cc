@@ -760,7 +760,8 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
     const double t = tiles_of(4, 4), st = split_tile;
     const double there = std::ceil((double)((M + split_tile - 1) / split_tile) * (double)((N + split_tile - 1) / split_tile) * (double)Z * sums_there / 256.0) / sums_there * st * st;
     const double here = std::ceil(t * S / 256.0) / S * 64.0 * 64.0;
-    if (here > (t >= 30 ? 1.45 : 2.0) * there) return false;
+    const bool fits = !g_scratch_limit || (double)sums_there * (double)Z * (double)M * (double)N * 4.0 <= (double)g_scratch_limit;
+    if (fits && here > (t >= 30 ? 1.45 : 2.0) * there) return false;
   }
   // an operand is read along K where its steps are contiguous there, along its rows otherwise
   // (runs of as many rows as the tile has blocks)
