@@ -16,6 +16,9 @@
 //   POLY_KSPLIT         (optional) workgroups that share the depth of a tile (blockIdx.y =
 //                       z * POLY_KSPLIT + part): each leaves its sum where POLY_EPILOGUE puts
 //                       it, which may use `poly_ks`, the part
+//   POLY_TOUCH_WGS      (optional, one z, no POLY_KSPLIT) that many extra workgroups at the front of
+//                       the grid, a multiple of 8, which multiply nothing: they read one element of every
+//                       64 bytes of B and leave, each the columns that the tiles of its own XCD have
 //   POLY_A_KC/B_KC      1: operand contiguous along K; 0: along M (resp. N)
 //   POLY_A_ROWS(row, lane, out)  (optional, one z, A contiguous along K in rows of K
 //                       elements) A is no buffer: this stores element f of its row `row` at
@@ -43,7 +46,10 @@
 // fp32 128 x 3072 x 768 22.3 -> 10.1 (60 TFLOP/s of the 157 of the fp32 MFMAs),
 // 33 x 129 x 784 30.6 -> 3.8.  What bounds it where there are
 // many rows is the address path: 16 lanes of a load along K read 16 different rows, 64 bytes
-// of each (1035 x 768 x 3072 takes 20 us where tiles in LDS take 12).
+// of each (1035 x 768 x 3072 takes 20 us where tiles in LDS take 12).  Where B comes from HBM
+// it is its latency: the waves have some 50 KB a CU on their way, which at 2 us is half of what
+// they take.  CUs without a tile read ahead then (POLY_TOUCH_WGS: fp32 128 x 768 x 3072
+// 17.3 -> 14.1 us, 13.0 with B in the caches; bf16 12 x 768 x 3072 7.6 -> 6.5).
 #ifdef POLY_TEMPLATE_STANDALONE
 #include <hip/hip_runtime.h>
 #define POLY_TIN __bf16
@@ -183,7 +189,43 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) poly_k(POLY_SIGNATUR
   // Workgroup ids congruent mod 8 run on one XCD (own L2): each XCD gets a contiguous run of
   // tiles, down the rows first, so that the workgroups that read one panel of B share an L2.
   constexpr int TILES_M = (POLY_M + POLY_BM - 1) / POLY_BM, NT = TILES_M * ((POLY_N + POLY_BN - 1) / POLY_BN);
+#ifdef POLY_TOUCH_WGS
+  static_assert(POLY_TOUCH_WGS % 8 == 0, "the workgroups behind keep their XCDs");
+  if (blockIdx.x < POLY_TOUCH_WGS) {
+    // this XCD's tiles, and their columns of B: one element of every 64 bytes
+    constexpr int PER = NT / 8, REM = NT % 8, EL = 64 / (int)sizeof(POLY_TIN);
+    const int xcd = blockIdx.x & 7, first = xcd < REM ? xcd * (PER + 1) : REM * (PER + 1) + (xcd - REM) * PER, last = first + PER + (xcd < REM) - 1;
+    const int n_lo = first / TILES_M * POLY_BN, n_end = (last / TILES_M + 1) * POLY_BN, n_hi = n_end < POLY_N ? n_end : POLY_N;
+    if (last < first) return;
+    const POLY_TIN *__restrict__ const p = POLY_B_PTR + poly_b_z(0);
+    constexpr int STEP = POLY_TOUCH_WGS / 8 * POLY_NTHREADS;
+    unsigned int seen = 0;
+#if POLY_B_KC
+    const int per_row = (POLY_K + EL - 1) / EL, lines = (n_hi - n_lo) * per_row;
+#else
+    const int per_row = (n_hi - n_lo + EL - 1) / EL, lines = POLY_K * per_row;
+#endif
+#pragma unroll 8
+    for (int i = (blockIdx.x >> 3) * POLY_NTHREADS + threadIdx.x; i < lines; i += STEP) {
+      const int r = i / per_row, x = (i - r * per_row) * EL;
+#if POLY_B_KC
+      const POLY_TIN v = p[poly_b_row(n_lo + r) + poly_b_k(x)];
+#else
+      const POLY_TIN v = p[poly_b_row(n_lo + x) + poly_b_k(r)];
+#endif
+#if POLY_F32
+      seen ^= __builtin_bit_cast(unsigned int, v);
+#else
+      seen ^= __builtin_bit_cast(unsigned short, v);
+#endif
+    }
+    asm volatile("" ::"v"(seen));
+    return;
+  }
+  int bid = blockIdx.x - POLY_TOUCH_WGS;
+#else
   int bid = blockIdx.x;
+#endif
   {
     constexpr int PER = NT / 8, REM = NT % 8;
     const int xcd = bid & 7, idx = bid >> 3;

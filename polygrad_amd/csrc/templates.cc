@@ -801,6 +801,17 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
     else cfg += "#define POLY_MFMA(a, b, c) (c)\n";
     cfg += strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_K %lld\n#define POLY_Z %lld\n", (long long)M, (long long)N, (long long)K, (long long)Z);
     if (f.block != 16) cfg += strf("#define POLY_BLOCK %d\n", f.block);
+    // Weights of 2 MiB and more that come from HBM: workgroups on CUs that have no tile read them into
+    // the L2s that want them, ahead of the waves, whose loads in flight are too few for HBM's latency.
+    // GPT-2 small, per launch: 12x768x3072 bf16 7.6 -> 6.5 us, 12x3072x768 5.4 -> 4.7, 128x768x3072 fp32
+    // 17.3 -> 14.1, 128x768x768 5.7 -> 5.1; less is on its way at once as it is (12x768x768 bf16, 1.1 MiB:
+    // 3.9 us and 4.0 with them).  Never more workgroups than CUs: the head of 12 tokens, 1571 tiles,
+    // takes 14.9 us, and 19.9 behind 64 of these.
+    int touch_wgs = 0;
+    if (ep.b_from_hbm && S == 1 && Z == 1 && mm.zd.empty() && mm.nd.size() == 1 && mm.kb.kb >= K && !getenv("POLY_HIP_NO_PREFETCH") &&
+        K * N * dt_size(mm.A.dt) >= (2 << 20) && tiles <= 248)
+      touch_wgs = (int)std::min<int64_t>(64, (256 - tiles) / 8 * 8);
+    if (touch_wgs) cfg += strf("#define POLY_TOUCH_WGS %d\n", touch_wgs);
     cfg += strf("#define POLY_TM %d\n#define POLY_TN %d\n#define POLY_WAVES %d\n#define POLY_DEPTH %d\n#define POLY_SUMS %d\n", f.tm, f.tn, f.waves, f.depth, sums);
     cfg += strf("#define POLY_A_KC %d\n#define POLY_B_KC %d\n#define POLY_A_PTR %s\n#define POLY_B_PTR %s\n", a_kc ? 1 : 0, b_kc ? 1 : 0, ep.a_ptr.c_str(), ep.b_ptr.c_str());
     cfg += offset_fn("poly_a_row", mm.md, true, 0) + offset_fn("poly_b_row", mm.nd, false, 0);
@@ -828,7 +839,7 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
     *out = RenderedKernel();
     out->source = std::string(hip_prelude()) + cfg + kMatmulWaveTemplate;
     out->entry = "poly_k";
-    out->launch.grid[0] = (unsigned)tiles;
+    out->launch.grid[0] = (unsigned)(tiles + touch_wgs);
     out->launch.grid[1] = (unsigned)(Z * S);
     out->launch.block[0] = (unsigned)(64 * f.waves);
     if (S > 1) {
@@ -848,6 +859,7 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
     out->reads_b_ahead = true;
     out->strategy = strf("mfma %s M=%lld N=%lld K=%lld Z=%lld tile %dx%d, depth dealt to %d waves%s, A:%s B:%s", f32 ? (f.block == 32 ? "32x32x2 f32" : "16x16x4 f32") : mm.A.dt == DT_BF16 ? "16x16x32 bf16" : "16x16x32 f16",
                          (long long)M, (long long)N, (long long)K, (long long)Z, bm, bn, f.waves, sums == 2 ? " of two sums each" : "", a_kc ? "k-major" : "m-major", b_kc ? "k-major" : "n-major");
+    if (touch_wgs) out->strategy += strf(", %d workgroups read B ahead", touch_wgs);
     if (S > 1) out->strategy += strf(", K dealt to %d workgroups per tile, partial results added by a second kernel", S);
     out->n_params = ep.n_params;
     if (g_a_rows) {
