@@ -20,6 +20,11 @@
 //                       leave.  When B comes from HBM (weights), they run ahead of the others
 //                       through B, which then find it in the memory-side cache instead of
 //                       waiting for HBM at every K tile
+//   POLY_RING           (optional) operands of any extent and alignment, no two strides along K:
+//                       their tiles go through registers instead, that many (an even number) on
+//                       their way at a time, and two LDS stages; with POLY_A_ODD / POLY_B_ODD, 1 where
+//                       an operand has an odd stride, and POLY_A_PITCH / POLY_B_PITCH, the
+//                       elements from one k to the next.  No POLY_KSPLIT, no POLY_TOUCH_WGS
 //   POLY_EP_WIN_BYTES   (optional, set by the epilogue's own code when POLY_EP_WIN_ROOM
 //                       suffices) bytes of the epilogue's lookup tables that the kernel
 //                       keeps in LDS, read from POLY_EP_WIN_SRC(byte): they are loaded
@@ -107,6 +112,9 @@ typedef __attribute__((address_space(3))) poly_s16x4 poly_lds_s16x4;
 #define POLY_N_LO 0
 #define POLY_N_HI POLY_N
 #endif
+#ifdef POLY_RING
+#define POLY_KT ((POLY_K - 1) / POLY_BK)      // (whole tiles; the rest, 1 to POLY_BK deep, is a tile of its own)
+#endif
 #ifndef POLY_KT
 #define POLY_KT (POLY_K / POLY_BK / POLY_KSPLIT)
 #endif
@@ -155,6 +163,7 @@ __device__ __forceinline__ void poly_lds_load(unsigned lds_addr, unsigned voff, 
 __device__ __forceinline__ void poly_lds_load_flat(unsigned lds_addr, const void *src) { memcpy(poly_host_lds + lds_addr + 16 * (threadIdx.x & 63), src, 16); }
 __device__ __forceinline__ void poly_wait_vm(int) {}
 #define __builtin_amdgcn_s_barrier() ((void)0)
+#define __builtin_amdgcn_alignbyte(hi, lo, n) (lo)
 #define __builtin_amdgcn_ds_read_tr16_b64_v4i16(p) (*(p))
 #else
 __device__ __forceinline__ void poly_lds_load(unsigned lds_addr, unsigned voff, const void *base) {
@@ -274,6 +283,12 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
   const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)lds_raw;
 #endif
 
+  // (POLY_RING: lanes load the chunks of a row in their order and store them where the swizzle says)
+#ifdef POLY_RING
+#define POLY_SOURCE_SWZ(swz) 0
+#else
+#define POLY_SOURCE_SWZ(swz) (swz)
+#endif
   // ── per-lane source offsets of this wave's LDS loads ─────────────────────────
   // Wave w issues instructions q * NW + w (q = 0 .. IPW-1) of each operand tile;
   // instruction i fills bytes [1024 i, 1024 i + 1024) of the tile.  Rows past the edge
@@ -285,12 +300,12 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
   for (int q = 0; q < POLY_A_IPW; q++) {
     const int slot = (q * POLY_NW + wave) * 64 + lane;      // 16-byte slot of the tile
 #if POLY_A_KC
-    const int row = slot / POLY_CH, c = (slot % POLY_CH) ^ poly_swz_k(row);
+    const int row = slot / POLY_CH, c = (slot % POLY_CH) ^ POLY_SOURCE_SWZ(poly_swz_k(row));
     const int m = m0 + row;
     a_off[q] = poly_a_row(m < POLY_M ? m : POLY_M - 1) + c * 8;
     a_kin[q] = 0;
 #else
-    const int kin = slot / (POLY_BM / 8), c = (slot % (POLY_BM / 8)) ^ poly_swz_x<POLY_BM>(kin);
+    const int kin = slot / (POLY_BM / 8), c = (slot % (POLY_BM / 8)) ^ POLY_SOURCE_SWZ(poly_swz_x<POLY_BM>(kin));
     const int m = m0 + c * 8;
     a_off[q] = poly_a_row(m < POLY_M ? m : POLY_M - 8);
     a_kin[q] = kin;
@@ -300,12 +315,12 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
   for (int q = 0; q < POLY_B_IPW; q++) {
     const int slot = (q * POLY_NW + wave) * 64 + lane;
 #if POLY_B_KC
-    const int row = slot / POLY_CH, c = (slot % POLY_CH) ^ poly_swz_k(row);
+    const int row = slot / POLY_CH, c = (slot % POLY_CH) ^ POLY_SOURCE_SWZ(poly_swz_k(row));
     const int n = n0 + row;
     b_off[q] = poly_b_row(n < POLY_N ? n : POLY_N - 1) + c * 8;
     b_kin[q] = 0;
 #else
-    const int kin = slot / (POLY_BN / 8), c = (slot % (POLY_BN / 8)) ^ poly_swz_x<POLY_BN>(kin);
+    const int kin = slot / (POLY_BN / 8), c = (slot % (POLY_BN / 8)) ^ POLY_SOURCE_SWZ(poly_swz_x<POLY_BN>(kin));
     const int n = n0 + c * 8;
     b_off[q] = poly_b_row(n < POLY_N ? n : POLY_N - 8);
     b_kin[q] = kin;
@@ -431,6 +446,137 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
     }
   };
 
+#ifdef POLY_RING
+  // ── the K loop, operands of any alignment and extent ─────────────────────────
+  // What bounds it is the address path: 16 bytes from a dword on cost a CU some 10 cycles a wave, from
+  // between two of them 33 (a loop of such loads out of L2).  1111 x 999 x 1501 bf16, all three odd,
+  // 16.5 us on 64x128 tiles where two launches, one that writes planes, take 22.6; all three even 12.6.
+  // More tiles in flight than two change nothing.
+  // Tile 0 is the end of the depth, its missing part zeros, tile s > 0 the POLY_BK from
+  // (s - 1) POLY_BK on.  A tile is loaded into registers, POLY_RING of them at a time, and goes to
+  // LDS stage s % 2 while tile s - 1 is multiplied.
+  constexpr int R = POLY_RING, NTILES = POLY_KT + 1;
+  static_assert(S == 2 && R % 2 == 0 && POLY_KSPLIT == 1, "two stages, whole turns of both rings");
+  // (Where a stride is odd, whole dwords are read and moved down by half of one on the way to LDS where
+  // they have to be.  The first of the next lane's dwords is the fifth of these; the last lane of a row
+  // reads it.  What is odd about a unit is the same in every tile.  The dword that holds an operand's first
+  // element may begin with one in front of it, which is dropped.)
+  struct Unit { poly_u32x4 v; unsigned int next; };
+  Unit ring[R][POLY_IPW];
+  const char *__restrict__ const at_a = (const char *)gA - (POLY_A_ODD ? (unsigned int)(size_t)gA & 2u : 0u);
+  const char *__restrict__ const at_b = (const char *)gB - (POLY_B_ODD ? (unsigned int)(size_t)gB & 2u : 0u);
+  constexpr long long STEP_A = 2ll * POLY_BK * (POLY_A_KC ? 1 : POLY_A_PITCH), STEP_B = 2ll * POLY_BK * (POLY_B_KC ? 1 : POLY_B_PITCH);
+  unsigned int from[POLY_IPW], odd[POLY_IPW];      // bytes from there to a unit of the first whole tile; 2 where that is half a dword too far
+#pragma unroll
+  for (int u = 0; u < POLY_IPW; u++) {
+    const bool is_a = u < POLY_A_IPW;
+    const int q = is_a ? u : u - POLY_A_IPW, off = is_a ? a_off[is_a ? q : 0] + poly_a_k(a_kin[is_a ? q : 0]) : b_off[is_a ? 0 : q] + poly_b_k(b_kin[is_a ? 0 : q]);
+    from[u] = (unsigned int)off * 2u + (unsigned int)(is_a ? (const char *)gA - at_a : (const char *)gB - at_b);
+    odd[u] = from[u] & 2u;
+    if (is_a ? POLY_A_ODD : POLY_B_ODD) from[u] -= odd[u];
+  }
+  auto last_lane = [&](int u) {
+    const int chunks = (u < POLY_A_IPW ? POLY_A_KC : POLY_B_KC) ? POLY_CH : u < POLY_A_IPW ? POLY_BM / 8 : POLY_BN / 8;
+    return lane % (chunks < 16 ? chunks : 16) == (chunks < 16 ? chunks : 16) - 1;
+  };
+  // unit u of a whole tile (every row of 8 elements starts inside a row of its operand, and what it
+  // reads past the end of that is the beginning of the next: the last row of the depth is tile 0's)
+  auto load_unit = [&](Unit (&to)[POLY_IPW], int s, int u) {
+    typedef poly_u32x4 poly_u32x4_u __attribute__((aligned(2)));
+    typedef poly_u32x4 poly_u32x4_d __attribute__((aligned(4)));
+    const char *const p = u < POLY_A_IPW ? at_a + (long long)(s - 1) * STEP_A : at_b + (long long)(s - 1) * STEP_B;
+    if (u < POLY_A_IPW ? POLY_A_ODD : POLY_B_ODD) {
+      to[u].v = *(const poly_u32x4_d *)(p + from[u]);
+      if (last_lane(u)) to[u].next = *(const unsigned int *)(p + (from[u] + 2u * odd[u]) + 12);
+    } else to[u].v = *(const poly_u32x4_u *)(p + from[u]);
+  };
+  // ... of tile 0: of the 8 elements from `p` on the first `left` exist, behind others of the same row.  The
+  // last 8 of the row are read instead (all loads before anything waits for one of them), moved down and
+  // filled up with zeros.
+  int gone[POLY_IPW];      // elements of a unit that do not exist
+  auto load_end = [&](Unit (&to)[POLY_IPW]) {
+    typedef poly_u32x4 poly_u32x4_u __attribute__((aligned(2)));
+    constexpr int K0 = POLY_KT * POLY_BK;
+#pragma unroll
+    for (int u = 0; u < POLY_IPW; u++) {
+      const bool is_a = u < POLY_A_IPW;
+      const int q = is_a ? u : u - POLY_A_IPW, slot = (q * POLY_NW + wave) * 64 + lane;
+      const bool kc = is_a ? POLY_A_KC : POLY_B_KC;
+      const int kin = kc ? slot % POLY_CH * 8 : is_a ? a_kin[is_a ? q : 0] : b_kin[is_a ? 0 : q];
+      const int left_k = POLY_K - K0 - kin;
+      const POLY_TIN *__restrict__ p;
+      if (kc) {
+        gone[u] = left_k < 8 ? 8 - left_k : 0;
+        p = (is_a ? gA + a_off[is_a ? q : 0] + poly_a_k(K0) : gB + b_off[is_a ? 0 : q] + poly_b_k(K0)) - gone[u];
+      } else {
+        const int k = left_k > 0 ? K0 + kin : POLY_K - 1;
+        const int x = is_a ? m0 + slot % (POLY_BM / 8) * 8 : n0 + slot % (POLY_BN / 8) * 8;
+        const int left = is_a ? POLY_M - x : POLY_N - x;
+        gone[u] = left > 0 && left < 8 ? 8 - left : 0;
+        p = (is_a ? gA + a_off[is_a ? q : 0] + poly_a_k(k) : gB + b_off[is_a ? 0 : q] + poly_b_k(k)) - gone[u];
+        if (left_k <= 0) gone[u] = 8;
+      }
+      to[u].v = *(const poly_u32x4_u *)p;
+    }
+  };
+  auto lds_unit = [&](int stage, int u) {
+    const bool is_a = u < POLY_A_IPW, kc = is_a ? POLY_A_KC : POLY_B_KC;
+    const int slot = ((is_a ? u : u - POLY_A_IPW) * POLY_NW + wave) * 64 + lane, chunks = kc ? POLY_CH : is_a ? POLY_BM / 8 : POLY_BN / 8;
+    const int row = slot / chunks, swz = kc ? poly_swz_k(row) : is_a ? poly_swz_x<POLY_BM>(row) : poly_swz_x<POLY_BN>(row);
+    return (poly_u32x4 *)(lds_raw + stage * POLY_STAGE_BYTES + (is_a ? 0 : POLY_A_BYTES) + (row * chunks + (slot % chunks ^ swz)) * 16);
+  };
+  auto store_end = [&](const Unit &from, int u) {
+    const poly_u32x4 v = from.v;
+    unsigned long long lo = v[0] | (unsigned long long)v[1] << 32, hi = v[2] | (unsigned long long)v[3] << 32;
+    const int sh = (gone[u] & 3) * 16;
+    if (gone[u] >= 4) { lo = hi; hi = 0; }
+    if (sh) { lo = lo >> sh | hi << (64 - sh); hi >>= sh; }
+    if (gone[u] >= 8) lo = hi = 0;
+    *lds_unit(0, u) = poly_u32x4{(unsigned int)lo, (unsigned int)(lo >> 32), (unsigned int)hi, (unsigned int)(hi >> 32)};
+  };
+  auto store_unit = [&](const Unit &x, int stage, int u) {
+    poly_u32x4 v = x.v;
+    if (u < POLY_A_IPW ? POLY_A_ODD : POLY_B_ODD) {
+      const unsigned int other = (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v[0], 0x101, 0xf, 0xf, true);      // (of lane + 1)
+      const unsigned int next = last_lane(u) ? x.next : other;
+      v = poly_u32x4{__builtin_amdgcn_alignbyte(v[1], v[0], odd[u]), __builtin_amdgcn_alignbyte(v[2], v[1], odd[u]), __builtin_amdgcn_alignbyte(v[3], v[2], odd[u]),
+                     __builtin_amdgcn_alignbyte(next, v[3], odd[u])};
+    }
+    *lds_unit(stage, u) = v;
+  };
+  load_end(ring[0]);
+#pragma unroll
+  for (int s = 1; s < R; s++)
+    if (s < NTILES) {
+#pragma unroll
+      for (int u = 0; u < POLY_IPW; u++) load_unit(ring[s], s, u);
+    }
+#pragma unroll
+  for (int u = 0; u < POLY_IPW; u++) {
+    store_end(ring[0][u], u);
+    if (R < NTILES) load_unit(ring[0], R, u);
+  }
+  auto iteration = [&](int s, int stage, auto &next, bool st, bool ld) {
+    __syncthreads();       // tile s is in LDS, and every wave is done with tile s - 1
+    constexpr int SLOTS = KS * MT;
+    k_tile(stage, [&](int slot) {
+#pragma unroll
+      for (int u = 0; u < POLY_IPW; u++)
+        if (st && u * SLOTS / POLY_IPW == slot) {
+          store_unit(next[u], stage ^ 1, u);
+          if (ld) load_unit(next, s + 1 + R, u);
+        }
+    });
+  };
+  constexpr int STEADY = NTILES > R + 1 ? (NTILES - R - 1) / R * R : 0;
+#pragma unroll 1
+  for (int s = 0; s < STEADY; s += R) {
+#pragma unroll
+    for (int t = 0; t < R; t++) iteration(s + t, t & 1, ring[(t + 1) % R], true, true);
+  }
+#pragma unroll
+  for (int s = STEADY; s < NTILES; s++) iteration(s, s & 1, ring[(s + 1) % R], s + 1 < NTILES, s + 1 + R < NTILES);
+#else
   // ── the K loop ──────────────────────────────────────────────────────────────
   // Tile t lives in stage t % STAGES.  Iteration kt: wait until this wave's loads of tile
   // kt have landed (everything but the loads of the STAGES - 2 tiles issued after it),
@@ -486,6 +632,7 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
     const bool win_issued = WIN_IPW > 0 && kt > POLY_KT - S + 1;
     iteration(kt, kt % S, later * POLY_IPW + (win_issued ? WIN_IPW : 0), kt + S - 1 < POLY_KT, WIN_IPW > 0 && kt == POLY_KT - S + 1);
   }
+#endif
   if (WIN_IPW > 0) poly_wait_vm(0);      // the window has landed (the barrier below publishes it)
 
   // ── epilogue ────────────────────────────────────────────────────────────────

@@ -988,8 +988,48 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   };
   bool a_kc, b_kc;
   const bool whole_tiles = layout(ka, md, true, M, &a_kc) && layout(kb, nd, false, N, &b_kc);
-  if (render_matmul_wave(mm, ep, whole_tiles, out)) return true;
-  if (!whole_tiles) return reject(__LINE__);
+  // Operands of any extent and alignment (a row digit of consecutive elements, or a depth of them, no two
+  // strides along it) on tiles that go through registers to LDS, where they are enough to be worth it: the
+  // shortest tile that leaves every one a CU, as far down the depth as two launches that write planes and
+  // multiply these take longer (figures: us, bf16, MALL-hot, against the planes or kernels/matmul_wave.hip):
+  //   64x64    40 tiles and more, 36000 tile-elements deep (701x699x601 8.3 -> 6.5, 131x4001x1203 21.8 -> 9.7,
+  //            500x500x7001 47.4 -> 36.3; below: 401x503x601 5.8 and 6.1 here, 45x1999x1203, 32 tiles, 6.3 and
+  //            9.1; beyond 1.2 million 777x777x7777 45.5 and 45.8); with even strides, whose loads the waves do
+  //            not wait for so long, 80 tiles (700x698x1202 10.3 -> 8.5; 400x502x2402, 56 tiles, 12.0 and 13.6)
+  //   64x128   to a depth of 3072 (1111x999x1501 22.6 -> 16.5; 777x777x7777 62)
+  //   128x128  from 128 to 5120 (1035x2303x769 22.8 -> 14.8, 1501x1503x4499 58.7 -> 52.4, 1900x2100x5001 67.5 -> 63.8)
+  //            (1500x1283x101, 8.6 and 6.8 here, stays with the waves: the tests of their edges hold it there)
+  //   128x256  to 2304, no more than a quarter of it padding (2047x2049x2053 49.4 -> 41.5, 2602x2702x1502 46.7 -> 36.7)
+  //   64x128   in several rounds of a depth to 512, where the stores are what takes time (7040x3328x39 36.7 -> 24.3,
+  //            1472x7232x217 27.7 -> 18.2, 3001x2999x301 29.0 -> 22.4; x601 37.7 and 35.9; x1003 46 and 49)
+  auto any_layout = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a, int64_t rows, bool *kc) {
+    if (ks.kb < K) return false;
+    *kc = ks.s_lo == 1;
+    return *kc ? K >= 8 : (is_a ? dims.back().ca : dims.back().cb) == 1 && dims.size() == 1 && rows >= 8 && ks.s_lo >= 9;
+  };
+  auto odd_stride = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a, bool kc) {
+    bool o = !kc && ks.s_lo % 2 != 0;
+    for (const Dim &d : dims) o = o || ((kc || &d != &dims.back()) && (is_a ? d.ca : d.cb) % 2 != 0);
+    for (const Dim &d : zd) o = o || (is_a ? d.ca : d.cb) % 2 != 0;
+    return o || (is_a ? mm.a_c0 : mm.b_c0) % 2 != 0;
+  };
+  struct Ring { int bm, bn, wm, wn, wg; };
+  Ring ring{0, 0, 0, 0, 0};
+  bool any_a = false, any_b = false;
+  if (!whole_tiles && !g_a_rows && M > 16 && N > 16 && K >= 32 && !getenv("POLY_HIP_NO_RAGGED_TILES") && !getenv("POLY_HIP_BF16_SPLIT_MIN") && any_layout(ka, md, true, M, &any_a) && any_layout(kb, nd, false, N, &any_b)) {
+    auto count = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * Z; };
+    const int64_t t64 = count(64, 64), deep = t64 * K;
+    const bool odd = odd_stride(ka, md, true, any_a) || odd_stride(kb, nd, false, any_b);
+    if (t64 < (odd ? 40 : 80) || deep < 36000) {}
+    else if (t64 <= 256) { if (deep <= 1200000) ring = Ring{64, 64, 2, 2, 2}; }
+    else if (count(64, 128) <= 256) { if (K <= 3072) ring = Ring{64, 128, 2, 2, 2}; }
+    else if (count(128, 128) <= 256) { if (K >= 128 && K <= 5120) ring = Ring{128, 128, 2, 4, 1}; }
+    else if (count(128, 256) <= 256 && K <= 2304 && (double)(count(128, 256) * 128 * 256) <= 1.25 * (double)M * (double)N * (double)Z) ring = Ring{128, 256, 2, 4, 1};
+    else if (K <= 512) ring = Ring{64, 128, 2, 2, 1};
+  }
+  if (!ring.bm && render_matmul_wave(mm, ep, whole_tiles, out)) return true;
+  if (!whole_tiles && !ring.bm) return reject(__LINE__);
+  if (ring.bm) { a_kc = any_a; b_kc = any_b; }
 
   // tile shape: 4 waves; narrow outputs get a narrow tile
   // Candidates: (BM, BN, waves M x N, workgroups resident per CU, throughput of one CU
@@ -1034,6 +1074,7 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   // fastest with a CU to itself, and may then be split down to parts of 32 K tiles.
   int S = 1;
   size_t part_off = 0;
+  const int in_flight = ring.bm ? 2 : 0;      // (tiles of them: four or six take as long)
   auto pick_split = [&](int64_t min_part) {
     const int64_t t = ((M + BM - 1) / BM) * ((N + BN - 1) / BN) * Z, kt = K / BK;
     double best = 0.75;      // worth a second kernel only from a quarter of the time saved
@@ -1045,7 +1086,7 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     }
     if ((double)S * (double)Z * (double)M * (double)N * 4.0 > 1073741824.0) S = 1;
   };
-  const bool may_split = !getenv("POLY_HIP_NO_SPLIT_K") && !measurement_env("POLY_HIP_MM_NOEPI") && M > 64 && N > 64;
+  const bool may_split = !ring.bm && !getenv("POLY_HIP_NO_SPLIT_K") && !measurement_env("POLY_HIP_MM_NOEPI") && M > 64 && N > 64;
   if (may_split) pick_split(64);
   if (S == 1 && !fixed_tile && !getenv("POLY_HIP_MM_TILE") && !measurement_env("POLY_HIP_MM_OLD_ESTIMATE")) {
     pick_tile(true);
@@ -1099,7 +1140,7 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   auto emit = [&](int bm, int bn, int wvm, int wvn, int pp, RenderedKernel *rk, int64_t n_lo = 0, int64_t n_hi = -1, bool may_dma = true,
                   Dma dma = Dma{0, 0, 0, 0, 0}) {
     if (n_hi < 0) n_hi = N;
-    const bool use_dma = may_dma && dma_for(bm, bn, &dma);
+    const bool use_dma = ring.bm || (may_dma && dma_for(bm, bn, &dma));
     const int bk = use_dma ? dma.bk : BK;
     if (use_dma) { wvm = dma.wvm; wvn = dma.wvn; }
     const int64_t tiles = ((M + bm - 1) / bm) * ((n_hi - n_lo + bn - 1) / bn);
@@ -1111,10 +1152,14 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     cfg += strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_K %lld\n#define POLY_Z %lld\n", (long long)M, (long long)N, (long long)K, (long long)Z);
     cfg += strf("#define POLY_BM %d\n#define POLY_BN %d\n#define POLY_BK %d\n#define POLY_WAVES_M %d\n#define POLY_WAVES_N %d\n", bm, bn, bk, wvm, wvn);
     if (use_dma) cfg += strf("#define POLY_STAGES %d\n#define POLY_WG_PER_CU %d\n", dma.stages, dma.wg);
+    if (ring.bm) {
+      cfg += strf("#define POLY_RING %d\n#define POLY_A_ODD %d\n#define POLY_B_ODD %d\n#define POLY_A_PITCH %lldll\n#define POLY_B_PITCH %lldll\n", in_flight, odd_stride(ka, md, true, a_kc) ? 1 : 0,
+                  odd_stride(kb, nd, false, b_kc) ? 1 : 0, (long long)ka.s_lo, (long long)kb.s_lo);
+    }
     // B in HBM as one dense block of K x N elements: extra workgroups at the front of the
     // grid run ahead through it, so that the others wait for HBM once and not at every K tile
     int touch_wgs = 0;
-    if (use_dma && ep.b_from_hbm && S == 1 && Z == 1 && zd.empty() && nd.size() == 1 && kb.kb >= K && !getenv("POLY_HIP_NO_PREFETCH") &&
+    if (use_dma && !ring.bm && ep.b_from_hbm && S == 1 && Z == 1 && zd.empty() && nd.size() == 1 && kb.kb >= K && !getenv("POLY_HIP_NO_PREFETCH") &&
         ((b_kc && kb.s_lo == 1 && nd[0].cb == K) || (!b_kc && nd[0].cb == 1 && kb.s_lo == N)) && K * N * 2 >= (128 << 10) && tiles >= 8) {
       touch_wgs = K * N * 2 >= (2 << 20) ? 64 : 32;
       cfg += strf("#define POLY_TOUCH_WGS %d\n#define POLY_TOUCH_FIRST %lld\n#define POLY_TOUCH_LINES %lldll\n", touch_wgs,
@@ -1157,7 +1202,7 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
       else {
         // the window moves into the stage that tile KT - STAGES leaves; the output staging
         // must fit before or behind that stage
-        const int kt = (int)(K / bk), stage_bytes = (bm + bn) * bk * 2, out_bytes = wvm * wvn * 32 * 36 * 4;
+        const int kt = ring.bm ? 0 : (int)(K / bk), stage_bytes = (bm + bn) * bk * 2, out_bytes = wvm * wvn * 32 * 36 * 4;
         const int win_stage = kt >= dma.stages ? (kt - dma.stages) % dma.stages : 0;
         const bool fits = kt >= dma.stages && (out_bytes <= win_stage * stage_bytes || out_bytes <= (dma.stages - 1 - win_stage) * stage_bytes);
         cfg += strf("#define POLY_EP_WIN_ROOM %d\n", fits ? stage_bytes / 1024 * 1024 : 0);
@@ -1193,13 +1238,14 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     rk->launch.grid[1] = (unsigned)(Z * S);
     rk->launch.block[0] = (unsigned)(64 * wvm * wvn);
     rk->klass = KernelClass::MATMUL_MFMA;
-    rk->reads_b_ahead = touch_wgs > 0;
+    rk->reads_b_ahead = touch_wgs > 0 || ring.bm;
     rk->writes_block_maxima = block_maxima;
     if (block_maxima) rk->scratch_bytes = ep.block_maxima.bytes;
     rk->strategy = strf("mfma 32x32x16 %s M=%lld N=%lld K=%lld Z=%lld tile %dx%dx%d A:%s B:%s", A.dt == DT_BF16 ? "bf16" : "f16",
                         (long long)M, (long long)N, (long long)K, (long long)Z, bm, bn, bk, a_kc ? "k-major" : "m-major",
                         b_kc ? "k-major" : "n-major");
-    if (use_dma) rk->strategy += strf(", operands straight into LDS: %d waves, %d stages, %d per CU", wvm * wvn, dma.stages, dma.wg);
+    if (ring.bm) rk->strategy += strf(", rows of any alignment through registers: %d waves, %d per CU", wvm * wvn, dma.wg);
+    else if (use_dma) rk->strategy += strf(", operands straight into LDS: %d waves, %d stages, %d per CU", wvm * wvn, dma.stages, dma.wg);
     if (touch_wgs) rk->strategy += strf(", %d workgroups read B ahead", touch_wgs);
     if (block_maxima) rk->strategy += strf(", leaves the largest magnitude of every 64x64 block of columns [%lld, %lld) for the launch that reads them",
                                            (long long)ep.block_maxima.lo, (long long)ep.block_maxima.hi);
@@ -1219,6 +1265,10 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   // Between one and one and a quarter rounds of 512 workgroups, 128x192 tiles when they
   // divide N and give a round and a half (N = 2304: 43.6 -> 39.9 us).  Narrow outputs (one
   // tile of 64 across) stay with the template that stages through registers.
+  if (ring.bm) {
+    if (emit(ring.bm, ring.bn, ring.wm, ring.wn, 3, out, 0, -1, true, Dma{64, 2, ring.wg, ring.wm, ring.wn})) return true;
+    return render_matmul_wave(mm, ep, whole_tiles, out) || reject(__LINE__);
+  }
   Dma chosen{0, 0, 0, 0, 0};
   bool dma_ok = !fixed_tile;
   // A product whose depth is dealt to workgroups anyway: 256x256 tiles, one workgroup of 8 waves to a
