@@ -6,6 +6,7 @@
 
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 
 #include "polygrad_hip.h"
 #include "runtime_hip.h"
@@ -432,6 +433,7 @@ static char *dup_string(const std::string &s) {
 
 char *poly_hip_render(PolyUOp *scheduled_root, const char *fn_name, int flags, int *launch_out) {
   RenderedKernel rk;
+  const std::unique_ptr<MatmulsOfPlan> of_plan(flags & 8 ? new MatmulsOfPlan : nullptr);
   if (!scheduled_root || !render_root(scheduled_root, fn_name ? fn_name : "kernel", flags, &rk)) return nullptr;
   if (launch_out) {
     for (int i = 0; i < 3; i++) { launch_out[i] = (int)rk.launch.grid[i]; launch_out[3 + i] = (int)rk.launch.block[i]; }
@@ -448,6 +450,7 @@ char *poly_hip_render(PolyUOp *scheduled_root, const char *fn_name, int flags, i
 
 char *poly_hip_describe(PolyUOp *scheduled_root, int flags) {
   RenderedKernel rk;
+  const std::unique_ptr<MatmulsOfPlan> of_plan(flags & 8 ? new MatmulsOfPlan : nullptr);
   if (!scheduled_root || !render_root(scheduled_root, "kernel", flags, &rk)) return nullptr;
   return dup_string(strf("%s: %s bytes=%.0f flops=%.0f grid=%u,%u,%u block=%u", kernel_class_name(rk.klass),
                          rk.strategy.c_str(), rk.bytes, rk.flops, rk.launch.grid[0], rk.launch.grid[1],

@@ -21,6 +21,7 @@
 #include <cstdlib>
 
 #include "fusion.h"
+#include "templates.h"
 
 namespace polyhip {
 
@@ -161,6 +162,7 @@ int n_launches(const PolySchedule *s, const std::vector<FusedGroup> &groups) {
 }  // namespace
 
 bool plan_schedule(const PolySchedule *s, bool buffers_apart, PlannedSchedule *out, std::string *err) {
+  MatmulsOfPlan of_plan;
   out->graphs.clear();
   out->graphs.resize((size_t)s->n_items);
   for (int k = 0; k < s->n_items; k++) {

@@ -430,6 +430,7 @@ static PolyHipPlan *compile_schedule(const PolySchedule *s, bool buffers_apart) 
           }
           if (!written) mask |= (uint64_t)1 << p;
         }
+        MatmulsOfPlan of_plan;
         matmul_hint_input_params(mask);
         matmul_hint_param_kinds(matmul_param_kinds_of(s, graphs, k, {}));
         u.runner = runner_create(it.root, name.c_str(), 0);

@@ -20,6 +20,9 @@ namespace {
 const char *const kMatmulTemplate =
 #include "matmul_mfma.hip.inc"
     ;
+const char *const kMatmulF32SplitTemplate =
+#include "matmul_f32_split.hip.inc"
+    ;
 const char *const kMatmulDmaTemplate =
 #include "matmul_dma.hip.inc"
     ;
@@ -538,6 +541,9 @@ static thread_local const MatmulRows *g_a_rows = nullptr;
 void matmul_hint_a_rows(const MatmulRows *rows) { g_a_rows = rows; }
 static thread_local size_t g_scratch_limit = 0;
 void matmul_hint_scratch_limit(size_t bytes) { g_scratch_limit = bytes; }
+static thread_local int g_in_plan = 0;
+MatmulsOfPlan::MatmulsOfPlan() { g_in_plan++; }
+MatmulsOfPlan::~MatmulsOfPlan() { g_in_plan--; }
 static thread_local MatmulEpilogue::BlockMaxima g_block_maxima;
 static thread_local int64_t g_block_maxima_rows = 0, g_block_maxima_pitch = 0;
 void matmul_hint_block_maxima(const MatmulEpilogue *e, int64_t rows, int64_t pitch) {
@@ -975,8 +981,47 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   const KSplit &ka = mm.ka, &kb = mm.kb;
   const std::vector<Dim> &md = mm.md, &nd = mm.nd, &zd = mm.zd;
   if (M > 2147483647LL || N > 2147483647LL || Z > 65535) return reject(__LINE__);
-  if (A.dt == DT_F32 && render_matmul_wave(mm, ep, false, out)) return true;
-  if (A.dt == DT_F32) return ep.mid_value_call.empty() ? render_matmul_f32(mm, ep, out) : false;     // (no second output in the fp32 template)
+  auto any_layout = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a, int64_t rows, bool *kc) {
+    if (ks.kb < K) return false;
+    *kc = ks.s_lo == 1;
+    return *kc ? K >= 8 : (is_a ? dims.back().ca : dims.back().cb) == 1 && dims.size() == 1 && rows >= 8 && ks.s_lo >= 9;
+  };
+  struct Ring { int bm, bn, wm, wn, wg, bk, parts; };
+  Ring ring{0, 0, 0, 0, 0, 64, 1};
+  bool any_a = false, any_b = false;
+  const bool f32 = A.dt == DT_F32;
+  if (f32) {
+    // Three bf16 planes of each value on the bf16 matrix pipes (kernels/matmul_f32_split.hip).  A 128x128 tile
+    // takes 1.1 us for 32 of its depth by itself on a CU and 1.55 where every CU has one, a 64x64 tile 0.64:
+    //   128x128  where the last round over the chip leaves no more than three in ten CUs idle (2048^3
+    //            183 us -> 100, 4096x1024x1024 88 -> 53, 2047x2039x1201 168 -> 112, 128x50257x768 115 -> 80;
+    //            1500x1500x1504, 144 tiles, 94 and 120 here)
+    //   128x128  of a depth dealt to two or four workgroups, 384 or more each, on as many CUs, from 1.2e9
+    //            multiply-adds on (1024x1024x4096 77 -> 60, 512x3072x768 37 -> 26; 1024^3 22.5 and 24.0,
+    //            704x704x2048 22.6 and 28.0; to eight 512x784x4096 41.5 and 34.2, which the tests of deep
+    //            products hold where it is)
+    //   64x64    from 257 tiles, where the waves that share a depth need several rounds, to 512, two on a CU
+    //            (4096x512x784 37.6 -> 31.0, 512x2304x768 48.4 -> 27.2, 2048x1024x64 9.4 -> 5.9; 1024^3, 256 tiles, 22.5 and
+    //            25.7; a depth of 4096 and more stays with the templates for that)
+    // The latter two only where the rows of an operand that lies along them begin on 64 bytes (1001x1503x777 61
+    // either way, 1500x1500x1504 94 and 186).  Errors against float64 are a half to a third of those
+    // of the fp32 MFMA templates, that deal the depth to waves and workgroups or not.  A kernel lowered by itself,
+    // outside a plan, keeps those.
+    if (g_in_plan && !g_a_rows && Z == 1 && zd.empty() && ep.scratch_type.empty() && !getenv("POLY_HIP_NO_F32_MFMA") && !getenv("POLY_HIP_NO_F32_SPLIT") &&
+        any_layout(ka, md, true, M, &any_a) && any_layout(kb, nd, false, N, &any_b)) {
+      const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128), t64 = ((M + 63) / 64) * ((N + 63) / 64);
+      const bool lines = (any_a || ka.s_lo % 16 == 0) && (any_b || kb.s_lo % 16 == 0);
+      const double work = (double)M * (double)N * (double)K;
+      if (K >= 128 && t128 >= 176 && 10 * t128 >= 7 * ((t128 + 255) / 256 * 256) - 32) ring = Ring{128, 128, 2, 4, 1, 32, 1};
+      else if (lines && t64 > 256 && t64 <= 512 && K >= 64 && K < 4096) ring = Ring{64, 64, 2, 2, 2, 32, 1};
+      if (ring.bm != 128 && lines && work >= 1.2e9 && (double)M * (double)N >= 0.85 * (double)(t128 * 16384) && !getenv("POLY_HIP_NO_SPLIT_K") && ep.mid_value_call.empty())
+        for (int parts = 2; parts <= 4; parts *= 2)
+          if (t128 * parts >= 176 && t128 * parts <= 256 && K % (32 * parts) == 0 && K / parts >= 384 && (!g_scratch_limit || (double)parts * (double)M * (double)N * 4.0 <= (double)g_scratch_limit))
+            ring = Ring{128, 128, 2, 4, 1, 32, parts};
+    }
+    if (!ring.bm && render_matmul_wave(mm, ep, false, out)) return true;
+    if (!ring.bm) return ep.mid_value_call.empty() ? render_matmul_f32(mm, ep, out) : false;     // (no second output in the fp32 template)
+  }
   int BK = 64;
   if (const char *e = measurement_env("POLY_HIP_MM_BK")) BK = atoi(e) == 32 ? 32 : 64;
   // operand layout: contiguous along K, or along its row axis
@@ -1002,30 +1047,22 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   //   128x256  to 2304, no more than a quarter of it padding (2047x2049x2053 49.4 -> 41.5, 2602x2702x1502 46.7 -> 36.7)
   //   64x128   in several rounds of a depth to 512, where the stores are what takes time (7040x3328x39 36.7 -> 24.3,
   //            1472x7232x217 27.7 -> 18.2, 3001x2999x301 29.0 -> 22.4; x601 37.7 and 35.9; x1003 46 and 49)
-  auto any_layout = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a, int64_t rows, bool *kc) {
-    if (ks.kb < K) return false;
-    *kc = ks.s_lo == 1;
-    return *kc ? K >= 8 : (is_a ? dims.back().ca : dims.back().cb) == 1 && dims.size() == 1 && rows >= 8 && ks.s_lo >= 9;
-  };
   auto odd_stride = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a, bool kc) {
     bool o = !kc && ks.s_lo % 2 != 0;
     for (const Dim &d : dims) o = o || ((kc || &d != &dims.back()) && (is_a ? d.ca : d.cb) % 2 != 0);
     for (const Dim &d : zd) o = o || (is_a ? d.ca : d.cb) % 2 != 0;
     return o || (is_a ? mm.a_c0 : mm.b_c0) % 2 != 0;
   };
-  struct Ring { int bm, bn, wm, wn, wg; };
-  Ring ring{0, 0, 0, 0, 0};
-  bool any_a = false, any_b = false;
-  if (!whole_tiles && !g_a_rows && M > 16 && N > 16 && K >= 32 && !getenv("POLY_HIP_NO_RAGGED_TILES") && !getenv("POLY_HIP_BF16_SPLIT_MIN") && any_layout(ka, md, true, M, &any_a) && any_layout(kb, nd, false, N, &any_b)) {
+  if (!f32 && !whole_tiles && !g_a_rows && M > 16 && N > 16 && K >= 32 && !getenv("POLY_HIP_NO_RAGGED_TILES") && !getenv("POLY_HIP_BF16_SPLIT_MIN") && any_layout(ka, md, true, M, &any_a) && any_layout(kb, nd, false, N, &any_b)) {
     auto count = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * Z; };
     const int64_t t64 = count(64, 64), deep = t64 * K;
     const bool odd = odd_stride(ka, md, true, any_a) || odd_stride(kb, nd, false, any_b);
     if (t64 < (odd ? 40 : 80) || deep < 36000) {}
-    else if (t64 <= 256) { if (deep <= 1200000) ring = Ring{64, 64, 2, 2, 2}; }
-    else if (count(64, 128) <= 256) { if (K <= 3072) ring = Ring{64, 128, 2, 2, 2}; }
-    else if (count(128, 128) <= 256) { if (K >= 128 && K <= 5120) ring = Ring{128, 128, 2, 4, 1}; }
-    else if (count(128, 256) <= 256 && K <= 2304 && (double)(count(128, 256) * 128 * 256) <= 1.25 * (double)M * (double)N * (double)Z) ring = Ring{128, 256, 2, 4, 1};
-    else if (K <= 512) ring = Ring{64, 128, 2, 2, 1};
+    else if (t64 <= 256) { if (deep <= 1200000) ring = Ring{64, 64, 2, 2, 2, 64, 1}; }
+    else if (count(64, 128) <= 256) { if (K <= 3072) ring = Ring{64, 128, 2, 2, 2, 64, 1}; }
+    else if (count(128, 128) <= 256) { if (K >= 128 && K <= 5120) ring = Ring{128, 128, 2, 4, 1, 64, 1}; }
+    else if (count(128, 256) <= 256 && K <= 2304 && (double)(count(128, 256) * 128 * 256) <= 1.25 * (double)M * (double)N * (double)Z) ring = Ring{128, 256, 2, 4, 1, 64, 1};
+    else if (K <= 512) ring = Ring{64, 128, 2, 2, 1, 64, 1};
   }
   if (!ring.bm && render_matmul_wave(mm, ep, whole_tiles, out)) return true;
   if (!whole_tiles && !ring.bm) return reject(__LINE__);
@@ -1074,6 +1111,7 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   // fastest with a CU to itself, and may then be split down to parts of 32 K tiles.
   int S = 1;
   size_t part_off = 0;
+  if (ring.bm) S = ring.parts;
   const int in_flight = ring.bm ? 2 : 0;      // (tiles of them: four or six take as long)
   auto pick_split = [&](int64_t min_part) {
     const int64_t t = ((M + BM - 1) / BM) * ((N + BN - 1) / BN) * Z, kt = K / BK;
@@ -1148,7 +1186,7 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     // ── configuration block ─────────────────────────────────────────────────
     std::string cfg;
     cfg += strf("#define POLY_TIN %s\n", dt_cname(A.dt));
-    cfg += strf("#define POLY_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_%s(a, b, c, 0, 0, 0)\n", A.dt == DT_BF16 ? "bf16" : "f16");
+    cfg += strf("#define POLY_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_%s(a, b, c, 0, 0, 0)\n", A.dt == DT_F16 ? "f16" : "bf16");
     cfg += strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_K %lld\n#define POLY_Z %lld\n", (long long)M, (long long)N, (long long)K, (long long)Z);
     cfg += strf("#define POLY_BM %d\n#define POLY_BN %d\n#define POLY_BK %d\n#define POLY_WAVES_M %d\n#define POLY_WAVES_N %d\n", bm, bn, bk, wvm, wvn);
     if (use_dma) cfg += strf("#define POLY_STAGES %d\n#define POLY_WG_PER_CU %d\n", dma.stages, dma.wg);
@@ -1232,7 +1270,7 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     }
 
     *rk = RenderedKernel();
-    rk->source = std::string(hip_prelude()) + cfg + (use_dma ? kMatmulDmaTemplate : kMatmulTemplate);
+    rk->source = std::string(hip_prelude()) + cfg + (f32 ? kMatmulF32SplitTemplate : use_dma ? kMatmulDmaTemplate : kMatmulTemplate);
     rk->entry = "poly_k";
     rk->launch.grid[0] = (unsigned)(tiles + touch_wgs);
     rk->launch.grid[1] = (unsigned)(Z * S);
@@ -1244,7 +1282,9 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     rk->strategy = strf("mfma 32x32x16 %s M=%lld N=%lld K=%lld Z=%lld tile %dx%dx%d A:%s B:%s", A.dt == DT_BF16 ? "bf16" : "f16",
                         (long long)M, (long long)N, (long long)K, (long long)Z, bm, bn, bk, a_kc ? "k-major" : "m-major",
                         b_kc ? "k-major" : "n-major");
-    if (ring.bm) rk->strategy += strf(", rows of any alignment through registers: %d waves, %d per CU", wvm * wvn, dma.wg);
+    if (f32) rk->strategy = strf("mfma 32x32x16 bf16, three planes of each f32 value, M=%lld N=%lld K=%lld Z=%lld tile %dx%dx%d A:%s B:%s, %d waves, %d per CU", (long long)M, (long long)N, (long long)K,
+                                 (long long)Z, bm, bn, bk, a_kc ? "k-major" : "m-major", b_kc ? "k-major" : "n-major", wvm * wvn, dma.wg);
+    else if (ring.bm) rk->strategy += strf(", rows of any alignment through registers: %d waves, %d per CU", wvm * wvn, dma.wg);
     else if (use_dma) rk->strategy += strf(", operands straight into LDS: %d waves, %d stages, %d per CU", wvm * wvn, dma.stages, dma.wg);
     if (touch_wgs) rk->strategy += strf(", %d workgroups read B ahead", touch_wgs);
     if (block_maxima) rk->strategy += strf(", leaves the largest magnitude of every 64x64 block of columns [%lld, %lld) for the launch that reads them",
@@ -1265,9 +1305,29 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   // Between one and one and a quarter rounds of 512 workgroups, 128x192 tiles when they
   // divide N and give a round and a half (N = 2304: 43.6 -> 39.9 us).  Narrow outputs (one
   // tile of 64 across) stay with the template that stages through registers.
+  auto add_parts = [&]() {
+    // the template becomes a first stage; the kernel proper adds the partial results up
+    RenderedKernel::Pre pre{out->source, out->entry, out->launch};
+    out->pres.push_back(pre);
+    out->scratch_bytes = part_off + (size_t)S * (size_t)Z * (size_t)M * (size_t)N * sizeof(float);
+    std::string cfg;
+    cfg += strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_Z %lld\n#define POLY_KSPLIT %d\n", (long long)M, (long long)N, (long long)Z, S);
+    cfg += strf("#define POLY_PARTIALS %s\n#define POLY_SIGNATURE %s\n", partials.c_str(), signature.c_str());
+    cfg += ep.code;
+    cfg += strf("#define POLY_EPILOGUE(acc, m, n, z) %s\n", ep.call.c_str());
+    if (f32 && !ep.mid_value_call.empty())
+      cfg += strf("#define POLY_EP_MID_VALUE(acc, m, n, z) %s\n#define POLY_EP_MID_PTR(m, n, z) %s\n", ep.mid_value_call.c_str(), ep.mid_ptr_call.c_str());
+    out->source = std::string(hip_prelude()) + cfg + kSplitKCombine;
+    out->launch = LaunchSpec();
+    out->launch.grid[0] = (unsigned)(((double)Z * M * N + 255) / 256);
+    out->launch.block[0] = 256;
+    out->strategy += strf(", K dealt to %d workgroups per tile, partial results added by a second kernel", S);
+    return true;
+  };
   if (ring.bm) {
-    if (emit(ring.bm, ring.bn, ring.wm, ring.wn, 3, out, 0, -1, true, Dma{64, 2, ring.wg, ring.wm, ring.wn})) return true;
-    return render_matmul_wave(mm, ep, whole_tiles, out) || reject(__LINE__);
+    if (emit(ring.bm, ring.bn, ring.wm, ring.wn, 3, out, 0, -1, true, Dma{ring.bk, 2, ring.wg, ring.wm, ring.wn})) return S > 1 ? add_parts() : true;
+    if (render_matmul_wave(mm, ep, whole_tiles, out)) return true;
+    return f32 && ep.mid_value_call.empty() ? render_matmul_f32(mm, ep, out) : reject(__LINE__);
   }
   Dma chosen{0, 0, 0, 0, 0};
   bool dma_ok = !fixed_tile;
@@ -1349,23 +1409,7 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     if (dma_for(128, 256, &d)) { BM = 128; BN = 256; WVM = WVN = 2; chosen = d; pipe = 3; }
   }
   if (!emit(BM, BN, WVM, WVN, pipe, out, 0, -1, dma_ok, chosen)) return false;
-  if (S > 1) {
-    // the template becomes a first stage; the kernel proper adds the partial results up
-    RenderedKernel::Pre pre{out->source, out->entry, out->launch};
-    out->pres.push_back(pre);
-    out->scratch_bytes = part_off + (size_t)S * (size_t)Z * (size_t)M * (size_t)N * sizeof(float);
-    std::string cfg;
-    cfg += strf("#define POLY_M %lld\n#define POLY_N %lld\n#define POLY_Z %lld\n#define POLY_KSPLIT %d\n", (long long)M, (long long)N, (long long)Z, S);
-    cfg += strf("#define POLY_PARTIALS %s\n#define POLY_SIGNATURE %s\n", partials.c_str(), signature.c_str());
-    cfg += ep.code;
-    cfg += strf("#define POLY_EPILOGUE(acc, m, n, z) %s\n", ep.call.c_str());
-    out->source = std::string(hip_prelude()) + cfg + kSplitKCombine;
-    out->launch = LaunchSpec();
-    out->launch.grid[0] = (unsigned)(((double)Z * M * N + 255) / 256);
-    out->launch.block[0] = 256;
-    out->strategy += strf(", K dealt to %d workgroups per tile, partial results added by a second kernel", S);
-    return true;
-  }
+  if (S > 1) return add_parts();
   // A last round over the chip that is at most half full (8192 x 2304 in 128 x 256 tiles:
   // 576 tiles, two rounds and a quarter) costs a whole round.  The launch then keeps the
   // columns whose tiles make whole rounds, and the columns left over go to a launch of

@@ -119,6 +119,12 @@ void matmul_hint_a_rows(const MatmulRows *rows);
 // Also set around a lowering: bytes of scratch memory that a product may take, where it has a form of
 // no more (0: no limit).
 void matmul_hint_scratch_limit(size_t bytes);
+// While one lives, kernels are lowered for a plan: its fp32 products may take the bf16 matrix pipes
+// (kernels/matmul_f32_split.hip).
+struct MatmulsOfPlan {
+  MatmulsOfPlan();
+  ~MatmulsOfPlan();
+};
 // Also set around a lowering: a later launch wants the block maxima of this product's
 // output, which it takes for a row-major matrix of `rows` x `pitch` elements from element 0
 // of the buffer (nullptr: no such wish).  The product grants it when its store is that.

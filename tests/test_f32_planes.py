@@ -1,0 +1,111 @@
+"""kernels/matmul_f32_split.hip, the fp32 products of a plan on the bf16 matrix pipes: ragged and whole rows,
+columns and depths (its end 1, 31 and 32 deep), every layout, 64x64 and 128x128 tiles, a depth dealt to
+workgroups.  Against the product in float64, element by element, within the rounding of K fp32
+additions and products (K * 2^-24 * sum of |a b|); no further off than the fp32 MFMA; infinities, NaN and values too
+small for three bf16 planes to hold as the fp32 MFMA has them."""
+import os
+import re
+import sys
+
+import pytest
+
+import hostcheck
+from polygrad_amd import PlanFile, _ffi
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "perf"))
+import cases  # noqa: E402
+
+PLAN = 8      # poly_hip_render and poly_hip_describe: as a kernel of a plan
+SHAPES = [(1025, 1024, 64, "nt", "64x64"), (1030, 1040, 97, "nn", "64x64"), (1088, 992, 127, "tn", "64x64"), (1056, 1000, 65, "tt", "64x64"),
+          (1793, 1664, 129, "nn", "128x128"), (1801, 1700, 160, "tn", "128x128"), (1665, 1793, 191, "nt", "128x128"), (1700, 1799, 128, "tt", "128x128"),
+          (1024, 1024, 2048, "nn", "128x128"), (1008, 1008, 3072, "tn", "128x128"), (512, 3070, 768, "nt", "128x128")]
+
+
+def _case(c):
+    return dict(kind="matmul", m=c[0], n=c[1], k=c[2], dtype="float32", layout=c[3])
+
+
+def _is_it(desc, c):
+    dealt = re.search(r"K dealt to (\d+)", desc)
+    return "three planes of each f32 value" in desc and f"tile {c[4]}x32" in desc and (dealt is not None) == (c[2] >= 768)
+
+
+@pytest.mark.skipif(not os.path.exists(hostcheck.CLANG), reason="no host clang with AddressSanitizer")
+@pytest.mark.parametrize("c", SHAPES, ids=lambda c: "-".join(map(str, c)))
+def test_stays_in_bounds(c, hiplib, monkeypatch):
+    import ctypes as C
+    monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
+    pf = cases._matmul_schedule(_case(c)).plan()
+    s = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents
+    it, launch = s.items[0], (C.c_int * 7)()
+    assert _is_it(_ffi.take_string(hiplib.poly_hip_describe(it.root, PLAN)), c)
+    assert "three planes" not in _ffi.take_string(hiplib.poly_hip_describe(it.root, 0))
+    units = _ffi.take_string(hiplib.poly_hip_render(it.root, b"k", PLAN, launch)).split("\n// ---- ")
+    sizes, scratch = [s.buf_slots[it.buf_slot_indices[p]].nbytes for p in range(it.n_buf_slots)], 0
+    jobs = [(units[0], (launch[0], launch[1], launch[2]), launch[3])]
+    for u in units[1:]:
+        m = re.match(r"first stage ---- grid=(\d+),(\d+) block=(\d+) scratch=(\d+)\n", u)
+        scratch = int(m.group(4))
+        jobs.append((u[m.end():], (int(m.group(1)), int(m.group(2)), 1), int(m.group(3))))
+    for source, grid, block in jobs:
+        hostcheck.check_kernel(source, hostcheck._entry_name(source), grid, block, sizes, block_stride=max(1, grid[0] * grid[1] * block // (1 << 17)), scratch_bytes=scratch)
+
+
+def _product(c, change=None):
+    state = cases.prepare(_case(c), 9)
+    by = {s.name: state["data"][s.index] for s in state["plan"].external_slots()}
+    if change:
+        change(by["A"], by["B"])
+    got = cases.run(state)["C"]
+    state["plan"].sync()
+    m, n, k, layout = c[:4]
+    a = by["A"].reshape(k, m).T if layout[0] == "t" else by["A"].reshape(m, k)
+    b = by["B"].reshape(n, k).T if layout[1] == "t" else by["B"].reshape(k, n)
+    return state["plan"].kernel_info()[0]["desc"], got.reshape(m, n).cpu(), a.double().cpu(), b.double().cpu()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", SHAPES, ids=lambda c: "-".join(map(str, c)))
+def test_against_float64(c, monkeypatch):
+    desc, got, a, b = _product(c)
+    assert _is_it(desc, c)
+    want = a @ b
+    err = (got.double() - want).abs()
+    assert bool((err <= c[2] * 2.0 ** -24 * (a.abs() @ b.abs())).all())
+    monkeypatch.setenv("POLY_HIP_NO_F32_SPLIT", "1")
+    desc, there, _, _ = _product(c)
+    assert "three planes" not in desc
+    assert float(err.norm()) <= float((there.double() - want).norm())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["inf", "nan", "largest", "tiny", "overflow"])
+@pytest.mark.parametrize("c", [SHAPES[1], SHAPES[4], SHAPES[8]], ids=lambda c: "-".join(map(str, c)))
+def test_values_that_planes_do_not_hold(c, what, monkeypatch):
+    """The same infinities and NaN as the fp32 MFMA, and finite values within the rounding of both."""
+    import torch
+
+    def change(a, b):
+        if what == "inf":
+            a[5], a[4000], b[77] = float("inf"), -float("inf"), float("inf")
+        elif what == "nan":
+            a[5], b[77] = float("nan"), float("nan")
+        elif what == "largest":
+            a[5] = torch.finfo(torch.float32).max
+            b.mul_(2.0 ** -30)
+        elif what == "tiny":
+            a.mul_(2.0 ** -118)
+        else:
+            a[5] = 3e38
+            b[77] = 3e38
+    desc, got, a, b = _product(c, change)
+    assert _is_it(desc, c)
+    monkeypatch.setenv("POLY_HIP_NO_F32_SPLIT", "1")
+    _, want, _, _ = _product(c, change)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    finite = want.isfinite()
+    assert torch.equal(got[~finite & ~want.isnan()], want[~finite & ~want.isnan()])
+    a, b = a.nan_to_num(0.0, 0.0, 0.0), b.nan_to_num(0.0, 0.0, 0.0)
+    # (below the smallest normal number a product's rounding is absolute)
+    bound = 2 * c[2] * (2.0 ** -24 * (a.abs() @ b.abs()) + 2.0 ** -149)
+    assert bool(((got.double() - want.double()).abs() <= bound)[finite].all())
