@@ -7,7 +7,7 @@
 // instantiates it by prepending the same configuration block as for matmul_mfma.hip
 // (POLY_TIN, POLY_MFMA, POLY_M/N/K/Z, POLY_BM/BN/BK, POLY_WAVES_M/N, POLY_A_KC/B_KC,
 // POLY_A_PTR/B_PTR, poly_a_row/poly_b_row/poly_a_z/poly_b_z/poly_a_k/poly_b_k,
-// POLY_SIGNATURE, the POLY_EP* epilogue macros, POLY_KSPLIT, POLY_N_LO/HI, POLY_GROUP_M,
+// POLY_SIGNATURE, the POLY_EP* epilogue macros, POLY_KSPLIT, POLY_N_LO/HI, POLY_M_LO/HI, POLY_GROUP_M,
 // POLY_GROUP_ALONG_N) plus
 //
 //   POLY_STAGES         LDS stages of one K tile (POLY_BK deep) each; loads run
@@ -111,6 +111,11 @@ typedef __attribute__((address_space(3))) poly_s16x4 poly_lds_s16x4;
 #ifndef POLY_N_LO
 #define POLY_N_LO 0
 #define POLY_N_HI POLY_N
+#endif
+// (and rows [POLY_M_LO, POLY_M_HI) likewise)
+#ifndef POLY_M_LO
+#define POLY_M_LO 0
+#define POLY_M_HI POLY_M
 #endif
 #ifdef POLY_RING
 #define POLY_KT ((POLY_K - 1) / POLY_BK)      // (whole tiles; the rest, 1 to POLY_BK deep, is a tile of its own)
@@ -216,7 +221,7 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
 
   // Tile coordinates: ids congruent mod 8 (one XCD, one L2) form a contiguous run of
   // tiles; within a run, bands of POLY_GROUP_M tile rows (or tile columns).
-  constexpr int TILES_M = (POLY_M + POLY_BM - 1) / POLY_BM;
+  constexpr int TILES_M = (POLY_M_HI - POLY_M_LO + POLY_BM - 1) / POLY_BM;
   constexpr int TILES_N = (POLY_N_HI - POLY_N_LO + POLY_BN - 1) / POLY_BN;
   constexpr int NT = TILES_M * TILES_N;
 #ifdef POLY_TOUCH_WGS
@@ -271,7 +276,7 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
   const int z = blockIdx.y;
   constexpr int k_base = 0;
 #endif
-  const int m0 = tile_m * POLY_BM, n0 = POLY_N_LO + tile_n * POLY_BN;
+  const int m0 = POLY_M_LO + tile_m * POLY_BM, n0 = POLY_N_LO + tile_n * POLY_BN;
   const POLY_TIN *__restrict__ gA = POLY_A_PTR + poly_a_z(z);
   const POLY_TIN *__restrict__ gB = POLY_B_PTR + poly_b_z(z);
 

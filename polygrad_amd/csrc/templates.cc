@@ -1176,12 +1176,14 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     return true;
   };
   auto emit = [&](int bm, int bn, int wvm, int wvn, int pp, RenderedKernel *rk, int64_t n_lo = 0, int64_t n_hi = -1, bool may_dma = true,
-                  Dma dma = Dma{0, 0, 0, 0, 0}) {
+                  Dma dma = Dma{0, 0, 0, 0, 0}, int64_t m_lo = 0, int64_t m_hi = -1) {
     if (n_hi < 0) n_hi = N;
+    if (m_hi < 0) m_hi = M;
     const bool use_dma = ring.bm || (may_dma && dma_for(bm, bn, &dma));
     const int bk = use_dma ? dma.bk : BK;
     if (use_dma) { wvm = dma.wvm; wvn = dma.wvn; }
-    const int64_t tiles = ((M + bm - 1) / bm) * ((n_hi - n_lo + bn - 1) / bn);
+    if ((m_lo != 0 || m_hi != M) && !use_dma) return false;      // (only that template knows of a launch of some rows)
+    const int64_t tiles = ((m_hi - m_lo + bm - 1) / bm) * ((n_hi - n_lo + bn - 1) / bn);
     if (tiles > 2147483647LL / 2) return reject(__LINE__);
     // ── configuration block ─────────────────────────────────────────────────
     std::string cfg;
@@ -1204,6 +1206,7 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
                   (long long)(mm.b_c0 & ~1ll), (long long)((K * N * 2 - 64) / 64));
     }
     if (n_lo != 0 || n_hi != N) cfg += strf("#define POLY_N_LO %lld\n#define POLY_N_HI %lld\n", (long long)n_lo, (long long)n_hi);
+    if (m_lo != 0 || m_hi != M) cfg += strf("#define POLY_M_LO %lld\n#define POLY_M_HI %lld\n", (long long)m_lo, (long long)m_hi);
     // each XCD (own L2) works on a contiguous run of tiles: let it re-read the smaller operand
     const bool along_n = N > 2 * M && !measurement_env("POLY_HIP_MM_GROUP_M");
     // (bands of 8 tile columns for the wide product: the 50257-wide head 727 -> 710 us against bands of 4)
@@ -1451,6 +1454,28 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
         out->strategy = strategy + strf(", columns from %lld on by a launch of %dx%d tiles ahead of it", (long long)n_lo, pick->bm, pick->bn);
         return true;
       }
+    }
+  }
+  // The same along the rows where there are too many of them for whole columns to be left out: a last round
+  // that at most a quarter of the CUs take part in costs nearly a whole one of 256x256 tiles.  The launch keeps the rows
+  // whose tiles make whole rounds, and those left over go to 64x128 tiles that each have a CU, if a
+  // depth of 512 and more is worth the launch: 50257x1024x12288 (788 tiles, a vocabulary projection's
+  // gradient in three planes) 1233 us -> 1018 + 72, the same bits, the training block 5726 -> 5562.
+  if (Z == 1 && S == 1 && BM == 256 && BN == 256 && K >= 512 && !matmul_tuning_enabled() && !getenv("POLY_HIP_NO_TAIL_LAUNCH") && !getenv("POLY_HIP_MM_TILE") &&
+      !measurement_env("POLY_HIP_MM_NOEPI")) {
+    const int64_t tn = (N + 255) / 256, T = ((M + 255) / 256) * tn, whole = T / 256, rest = T % 256;
+    const int64_t m_lo = tn > 0 ? whole * 256 / tn * 256 : 0;
+    Dma small{64, 4, 1, 2, 2};
+    RenderedKernel main, tail;
+    if (whole >= 1 && rest > 0 && rest <= 64 && m_lo > 0 && m_lo < M && ((M - m_lo + 63) / 64) * ((N + 127) / 128) <= 256 && (a_kc || m_lo % 8 == 0) &&
+        dma_for(64, 128, &small) && emit(BM, BN, WVM, WVN, pipe, &main, 0, -1, dma_ok, chosen, 0, m_lo) && emit(64, 128, 2, 2, 3, &tail, 0, -1, true, small, m_lo, M) &&
+        main.writes_block_maxima == out->writes_block_maxima && tail.writes_block_maxima == out->writes_block_maxima) {
+      const std::string strategy = out->strategy;
+      *out = main;
+      out->pres.push_back({tail.source, tail.entry, tail.launch});
+      out->scratch_bytes = std::max<size_t>(256, main.scratch_bytes);      // (a kernel with a first stage owns scratch memory)
+      out->strategy = strategy + strf(", rows from %lld on by a launch of 64x128 tiles ahead of it", (long long)m_lo);
+      return true;
     }
   }
   // Candidates for on-device tuning: the same kernel in the other tile shapes and
