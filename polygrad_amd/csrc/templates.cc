@@ -1047,13 +1047,14 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   //   128x256  to 2304, no more than a quarter of it padding (2047x2049x2053 49.4 -> 41.5, 2602x2702x1502 46.7 -> 36.7)
   //   64x128   in several rounds of a depth to 512, where the stores are what takes time (7040x3328x39 36.7 -> 24.3,
   //            1472x7232x217 27.7 -> 18.2, 3001x2999x301 29.0 -> 22.4; x601 37.7 and 35.9; x1003 46 and 49)
+  // A kernel lowered by itself, outside a plan, keeps its planes or waves.
   auto odd_stride = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a, bool kc) {
     bool o = !kc && ks.s_lo % 2 != 0;
     for (const Dim &d : dims) o = o || ((kc || &d != &dims.back()) && (is_a ? d.ca : d.cb) % 2 != 0);
     for (const Dim &d : zd) o = o || (is_a ? d.ca : d.cb) % 2 != 0;
     return o || (is_a ? mm.a_c0 : mm.b_c0) % 2 != 0;
   };
-  if (!f32 && !whole_tiles && !g_a_rows && M > 16 && N > 16 && K >= 32 && !getenv("POLY_HIP_NO_RAGGED_TILES") && !getenv("POLY_HIP_BF16_SPLIT_MIN") && any_layout(ka, md, true, M, &any_a) && any_layout(kb, nd, false, N, &any_b)) {
+  if (g_in_plan && !f32 && !whole_tiles && !g_a_rows && M > 16 && N > 16 && K >= 32 && !getenv("POLY_HIP_NO_RAGGED_TILES") && !getenv("POLY_HIP_BF16_SPLIT_MIN") && any_layout(ka, md, true, M, &any_a) && any_layout(kb, nd, false, N, &any_b)) {
     auto count = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * Z; };
     const int64_t t64 = count(64, 64), deep = t64 * K;
     const bool odd = odd_stride(ka, md, true, any_a) || odd_stride(kb, nd, false, any_b);

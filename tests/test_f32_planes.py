@@ -3,6 +3,7 @@ columns and depths (its end 1, 31 and 32 deep), every layout, 64x64 and 128x128 
 workgroups.  Against the product in float64, element by element, within the rounding of K fp32
 additions and products (K * 2^-24 * sum of |a b|); no further off than the fp32 MFMA; infinities, NaN and values too
 small for three bf16 planes to hold as the fp32 MFMA has them."""
+import ctypes as C
 import os
 import re
 import sys
@@ -30,18 +31,11 @@ def _is_it(desc, c):
     return "three planes of each f32 value" in desc and f"tile {c[4]}x32" in desc and (dealt is not None) == (c[2] >= 768)
 
 
-@pytest.mark.skipif(not os.path.exists(hostcheck.CLANG), reason="no host clang with AddressSanitizer")
-@pytest.mark.parametrize("c", SHAPES, ids=lambda c: "-".join(map(str, c)))
-def test_stays_in_bounds(c, hiplib, monkeypatch):
-    import ctypes as C
-    monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
-    pf = cases._matmul_schedule(_case(c)).plan()
-    s = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents
-    it, launch = s.items[0], (C.c_int * 7)()
-    assert _is_it(_ffi.take_string(hiplib.poly_hip_describe(it.root, PLAN)), c)
-    assert "three planes" not in _ffi.take_string(hiplib.poly_hip_describe(it.root, 0))
-    units = _ffi.take_string(hiplib.poly_hip_render(it.root, b"k", PLAN, launch)).split("\n// ---- ")
-    sizes, scratch = [s.buf_slots[it.buf_slot_indices[p]].nbytes for p in range(it.n_buf_slots)], 0
+def check_as_of_a_plan(hiplib, schedule, item):
+    """The kernel of `item` as a plan has it, and its first stages, on the host with buffers of their exact size."""
+    launch = (C.c_int * 7)()
+    units = _ffi.take_string(hiplib.poly_hip_render(item.root, b"k", PLAN, launch)).split("\n// ---- ")
+    sizes, scratch = [schedule.buf_slots[item.buf_slot_indices[p]].nbytes for p in range(item.n_buf_slots)], 0
     jobs = [(units[0], (launch[0], launch[1], launch[2]), launch[3])]
     for u in units[1:]:
         m = re.match(r"first stage ---- grid=(\d+),(\d+) block=(\d+) scratch=(\d+)\n", u)
@@ -49,6 +43,18 @@ def test_stays_in_bounds(c, hiplib, monkeypatch):
         jobs.append((u[m.end():], (int(m.group(1)), int(m.group(2)), 1), int(m.group(3))))
     for source, grid, block in jobs:
         hostcheck.check_kernel(source, hostcheck._entry_name(source), grid, block, sizes, block_stride=max(1, grid[0] * grid[1] * block // (1 << 17)), scratch_bytes=scratch)
+
+
+@pytest.mark.skipif(not os.path.exists(hostcheck.CLANG), reason="no host clang with AddressSanitizer")
+@pytest.mark.parametrize("c", SHAPES, ids=lambda c: "-".join(map(str, c)))
+def test_stays_in_bounds(c, hiplib, monkeypatch):
+    monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
+    pf = cases._matmul_schedule(_case(c)).plan()
+    s = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents
+    it = s.items[0]
+    assert _is_it(_ffi.take_string(hiplib.poly_hip_describe(it.root, PLAN)), c)
+    assert "three planes" not in _ffi.take_string(hiplib.poly_hip_describe(it.root, 0))
+    check_as_of_a_plan(hiplib, s, it)
 
 
 def _product(c, change=None):

@@ -10,6 +10,7 @@ import pytest
 
 import hostcheck
 from polygrad_amd import PlanFile, _ffi
+from test_f32_planes import PLAN, check_as_of_a_plan
 
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "perf"))
 import cases  # noqa: E402
@@ -35,8 +36,10 @@ def test_stays_in_bounds(c, hiplib, monkeypatch):
     monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
     pf = cases._matmul_schedule(_case(*c)).plan()
     s = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents
-    assert _is_it(_ffi.take_string(hiplib.poly_hip_describe(s.items[0].root, 0)), c[5])
-    assert hostcheck.check_schedule(hiplib, pf.schedule) >= 1
+    it = s.items[0]
+    assert _is_it(_ffi.take_string(hiplib.poly_hip_describe(it.root, PLAN)), c[5])
+    assert "rows of any alignment" not in _ffi.take_string(hiplib.poly_hip_describe(it.root, 0))
+    check_as_of_a_plan(hiplib, s, it)
 
 
 @pytest.mark.gpu
