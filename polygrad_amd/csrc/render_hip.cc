@@ -527,6 +527,10 @@ class Generic {
     // Long rows, or too few rows to fill the chip with one wave each: a whole
     // workgroup per row.
     if (R >= 4096 || (rows < 2048 && R >= 1024)) coop_G_ = 256; else coop_G_ = 64;
+    // ... of sixteen waves where four would be all that a CU has, or two of them eight: their loads in flight
+    // are too few (sums of 6 x 31855 8.2 -> 4.2 us, 64 x 50257 21.5 -> 8.8, 200 x 50000 35.2 -> 21.8, 400 x 20001 17.1 ->
+    // 16.2; 512 x 50257 46.9 and 48.7, 512 x 8192 8.6 either way)
+    if (R >= 4096 && rows <= 400 && opt_.promote_reduce < 0 && opt_.block == 256) coop_G_ = opt_.block = 1024;
     coop_R_ = R;
     coop_ranges_ = rr;
     return true;
@@ -673,7 +677,7 @@ class Generic {
       const KNode &k = g_.n(id);
       line(red, 2, strf("acc%d = %s;", id, wave_reduce_call(reduce_op(k), k.dt, strf("acc%d", id)).c_str()));
     }
-    if (G == 256) {
+    if (G >= 256) {
       int ri = 0;
       for (int id : top_reduces_) {
         const KNode &k = g_.n(id);
@@ -686,9 +690,16 @@ class Generic {
       for (int id : top_reduces_) {
         const KNode &k = g_.n(id);
         PolyOps op = reduce_op(k);
-        std::string e = strf("red%d[0]", ri);
-        for (int w = 1; w < 4; w++) e = Emitter::reduce_combine(op, k.dt, e, strf("red%d[%d]", ri, w));
-        line(red, 2, strf("acc%d = %s;", id, e.c_str()));
+        // (sixteen waves pairwise: one after the other the last additions, of nearly whole sums, would
+        // round twice as often as those of four waves do)
+        std::vector<std::string> e;
+        for (int w = 0; w < G / 64; w++) e.push_back(strf("red%d[%d]", ri, w));
+        while (e.size() > 4) {
+          for (size_t w = 0; w < e.size() / 2; w++) e[w] = Emitter::reduce_combine(op, k.dt, e[2 * w], e[2 * w + 1]);
+          e.resize(e.size() / 2);
+        }
+        for (size_t w = 1; w < e.size(); w++) e[0] = Emitter::reduce_combine(op, k.dt, e[0], e[w]);
+        line(red, 2, strf("acc%d = %s;", id, e[0].c_str()));
         ri++;
       }
     }
@@ -710,10 +721,10 @@ class Generic {
     }
     std::string tail = S0.code + tail_stores;
 
-    if (G == 256) {
+    if (G >= 256) {
       int ri = 0;
       for (int id : top_reduces_) {
-        line(body, 1, strf("__shared__ %s red%d[4];", dt_cname(g_.n(id).dt), ri));
+        line(body, 1, strf("__shared__ %s red%d[%d];", dt_cname(g_.n(id).dt), ri, G / 64));
         ri++;
       }
       line(body, 1, "{");
@@ -728,7 +739,7 @@ class Generic {
     line(body, 1, "}");
     (void)nred;
 
-    double blocks = G == 256 ? rows : std::ceil(rows / rows_per_block);
+    double blocks = G >= 256 ? rows : std::ceil(rows / rows_per_block);
     if (blocks > 2147483647.0) { error_ = "grid too large"; return body; }
     out->launch.grid[0] = (unsigned)std::max(1.0, blocks);
     out->launch.block[0] = (unsigned)opt_.block;

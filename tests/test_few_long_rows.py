@@ -1,0 +1,44 @@
+"""Sums and maxima over a few long rows, sixteen waves to a row: one vector a lane and many, ragged ends, rows that begin on
+no vector, the most and one more than the most rows that are dealt out so.  Sums against float64 within the rounding of
+the additions on the way of a term (its lane's, six across the lanes of a wave, four across the waves) and the chain's."""
+import ctypes as C
+import os
+import sys
+
+import pytest
+
+import hostcheck
+from polygrad_amd import PlanFile, _ffi
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "perf"))
+import cases  # noqa: E402
+
+SHAPES = [(1, 4096, True), (2, 4097, True), (3, 16387, True), (7, 50257, True), (400, 4100, True), (401, 4100, False), (5, 4095, False)]
+
+
+@pytest.mark.skipif(not os.path.exists(hostcheck.CLANG), reason="no host clang with AddressSanitizer")
+@pytest.mark.parametrize("op", ["sum", "max"])
+@pytest.mark.parametrize("rows,cols,wide", SHAPES)
+def test_stays_in_bounds(rows, cols, wide, op, hiplib, monkeypatch):
+    monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
+    pf = cases._rows_schedule(dict(kind="rows", op=op, rows=rows, cols=cols)).plan()
+    s = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents
+    assert ("G=1024" in _ffi.take_string(hiplib.poly_hip_describe(s.items[0].root, 0))) == wide
+    assert hostcheck.check_schedule(hiplib, pf.schedule) >= 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", ["sum", "max"])
+@pytest.mark.parametrize("rows,cols,wide", SHAPES)
+def test_against_float64(rows, cols, wide, op):
+    state = cases.prepare(dict(kind="rows", op=op, rows=rows, cols=cols), 3)
+    assert ("G=1024" in state["plan"].kernel_info()[0]["desc"]) == wide
+    got = cases.run(state)["out"]
+    state["plan"].sync()
+    by = {s.name: state["data"][s.index].double().reshape(rows, cols) for s in state["plan"].external_slots() if s.name != "out"}
+    y = (by["a"] * by["b"] + by["c"]).exp2().clamp(-4, 4)
+    want = y.sum(1) if op == "sum" else y.max(1).values
+    steps = (cols + 255) // 256 + 12 if op == "sum" else 0
+    # (the elements: two roundings of at most 3 in front of exp2, whose own error is within 2 units)
+    bound = (steps + 8) * 2.0 ** -24 * (y.abs().sum(1) if op == "sum" else y.abs().max(1).values)
+    assert bool(((got.double() - want).abs() <= bound).all())
