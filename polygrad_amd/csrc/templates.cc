@@ -738,6 +738,12 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
   } else {
     const bool few = M <= 16 || N <= 16 || tiles_of(4, 4) <= 64;
     if (!few && (whole_tiles || (double)M * (double)N * (double)K * (double)Z >= 1073741824.0)) return false;
+    // (a deep one's time is a wave's: where each 16x16 tile has a CU, that tile (12x768x3072 6.8 -> 6.4 us, 64x512x4096 with both
+    // operands along the depth 12.6 -> 9.3); where 16x32 tiles share CUs and 32x32 would not, that one (300x768x3072 14.7 ->
+    // 12.1, both along the depth 18.1 -> 12.9, 156x1024x4096 15.8 -> 14.3, 200x1000x2048 10.0 -> 7.9, 300x768x1500 7.5 ->
+    // 6.3; 100x1024x4096, 224 tiles of 16x32, 8.9 and 12.1).  The same waves: the same order of additions)
+    if (!g_a_rows && K >= 2048 && tiles_of(1, 1) <= 256) f = Form{1, 1, 8, 6, 16};
+    else if (!g_a_rows && K >= 1024 && M > 16 && tiles_of(1, 2) > 256 && tiles_of(2, 2) <= 256) f = Form{2, 2, 8, 6, 16};
     if (tiles_of(1, 2) > 640 && M > 16) f = Form{2, 2, 8, 6, 16};
     if (f.tm == 2 && tiles_of(2, 2) > 640) f = Form{2, 4, 4, 6, 16};
     if (f.tn == 4 && tiles_of(2, 4) > 640) f = Form{4, 4, 4, 4, 16};
