@@ -1042,17 +1042,25 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   // Operands of any extent and alignment (a row digit of consecutive elements, or a depth of them, no two
   // strides along it) on tiles that go through registers to LDS, where they are enough to be worth it: the
   // shortest tile that leaves every one a CU, as far down the depth as two launches that write planes and
-  // multiply these take longer (figures: us, bf16, MALL-hot, against the planes or kernels/matmul_wave.hip):
-  //   64x64    40 tiles and more, 36000 tile-elements deep (701x699x601 8.3 -> 6.5, 131x4001x1203 21.8 -> 9.7,
-  //            500x500x7001 47.4 -> 36.3; below: 401x503x601 5.8 and 6.1 here, 45x1999x1203, 32 tiles, 6.3 and
-  //            9.1; beyond 1.2 million 777x777x7777 45.5 and 45.8); with even strides, whose loads the waves do
-  //            not wait for so long, 80 tiles (700x698x1202 10.3 -> 8.5; 400x502x2402, 56 tiles, 12.0 and 13.6)
-  //   64x128   to a depth of 3072 (1111x999x1501 22.6 -> 16.5; 777x777x7777 62)
-  //   128x128  from 128 to 5120 (1035x2303x769 22.8 -> 14.8, 1501x1503x4499 58.7 -> 52.4, 1900x2100x5001 67.5 -> 63.8)
+  // multiply these take longer.  Figures: us, bf16, operands from HBM, planes or kernels/matmul_wave.hip and here.
+  //   64x64    at least 36000 tile-elements deep (401x503x601 5.8 and 6.1) and 1024 tiles of 16x16: fewer are a wave
+  //            on every SIMD, each of which reads its own operands (17x4701x605 5.7 and 6.6, 49x3501x1505 11.0 and
+  //            15.0; above, 17x9001x1505 17.9 -> 14.9, 131x2001x1505 17.9 -> 14.2).  With both operands read along
+  //            the depth, which waves wait longest for, and more than 64 of both rows and columns 500
+  //            (129x901x1505 14.8 -> 10.5, 70x1901x3001 30.5 -> 25.9; 70x1301x3001, 410 of them, 23.2 and 25.7).
+  //            With neither and a depth below 1024, not between 1280 and 1900, which are one round of 32x32
+  //            (514x642x603 5.7 and 6.2, 513x901x603 6.4 and 6.7; 1001x261x603 7.3 -> 6.4, 700x698x602 6.4 -> 5.8).
+  //            With even strides, whose loads the waves do not wait for so long, 80 tiles that are no more than a
+  //            tenth padding (700x698x1506 12.0 -> 9.8; 130x2600x1506 11.7 and 12.7, 400x502x2402 12.0 and 13.6).
+  //            To a depth of 2560 (601x701x1505 19.4 -> 11.0, 900x1000x2401 24.5 -> 20.1; 601x701x3501 25.4 and 30.8)
+  //   64x128   to 2304 (1111x999x1501 24.0 -> 17.6, 2001x900x2001 27.9 -> 20.3; 1111x999x3001 28.1 and 31.4)
+  //   128x128  from 128 to 4096 (1500x1501x1501 31.8 -> 25.3, x4001 58.7 -> 55.6), with both operands read along the
+  //            depth to 2304 (2001x1801x1501 31.2 -> 28.4, x4001 56.5 and 61.0)
   //            (1500x1283x101, 8.6 and 6.8 here, stays with the waves: the tests of their edges hold it there)
-  //   128x256  to 2304, no more than a quarter of it padding (2047x2049x2053 49.4 -> 41.5, 2602x2702x1502 46.7 -> 36.7)
+  //   128x256  to 2304, no more than a quarter of it padding (3001x2501x2201 67 -> 54); with both operands read
+  //            along the depth and fewer than 200 tiles to 1024 (2049x2501x601 30.9 -> 27.6, x1501 42.1 and 45.5)
   //   64x128   in several rounds of a depth to 512, where the stores are what takes time (7040x3328x39 36.7 -> 24.3,
-  //            1472x7232x217 27.7 -> 18.2, 3001x2999x301 29.0 -> 22.4; x601 37.7 and 35.9; x1003 46 and 49)
+  //            1472x7232x217 27.7 -> 18.2, 3001x2999x301 29.0 -> 22.4 MALL-hot; x601 37.7 and 35.9; x1003 46 and 49)
   // A kernel lowered by itself, outside a plan, keeps its planes or waves.
   auto odd_stride = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a, bool kc) {
     bool o = !kc && ks.s_lo % 2 != 0;
@@ -1064,11 +1072,15 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     auto count = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * Z; };
     const int64_t t64 = count(64, 64), deep = t64 * K;
     const bool odd = odd_stride(ka, md, true, any_a) || odd_stride(kb, nd, false, any_b);
-    if (t64 < (odd ? 40 : 80) || deep < 36000) {}
-    else if (t64 <= 256) { if (deep <= 1200000) ring = Ring{64, 64, 2, 2, 2, 64, 1}; }
-    else if (count(64, 128) <= 256) { if (K <= 3072) ring = Ring{64, 128, 2, 2, 2, 64, 1}; }
-    else if (count(128, 128) <= 256) { if (K >= 128 && K <= 5120) ring = Ring{128, 128, 2, 4, 1, 64, 1}; }
-    else if (count(128, 256) <= 256 && K <= 2304 && (double)(count(128, 256) * 128 * 256) <= 1.25 * (double)M * (double)N * (double)Z) ring = Ring{128, 256, 2, 4, 1, 64, 1};
+    const int64_t t16 = count(16, 16);
+    const bool along_k = any_a && any_b, one_round = !any_a && !any_b && K < 1024 && t16 > 1280 && t16 < 1900;
+    const bool waves = t16 < (along_k && M > 64 && N > 64 ? 500 : 1024) || one_round;
+    auto padded = [&](int64_t bm, int64_t bn) { return (double)(count(bm, bn) * bm * bn) / ((double)M * (double)N * (double)Z); };
+    if (t64 < (odd ? 40 : 80) || deep < 36000 || waves || (!odd && t64 <= 256 && padded(64, 64) > 1.1)) {}
+    else if (t64 <= 256) { if (K <= 2560) ring = Ring{64, 64, 2, 2, 2, 64, 1}; }
+    else if (count(64, 128) <= 256) { if (K <= 2304) ring = Ring{64, 128, 2, 2, 2, 64, 1}; }
+    else if (count(128, 128) <= 256) { if (K >= 128 && K <= (along_k ? 2304 : 4096)) ring = Ring{128, 128, 2, 4, 1, 64, 1}; }
+    else if (count(128, 256) <= 256 && K <= (along_k && count(128, 256) < 200 ? 1024 : 2304) && padded(128, 256) <= 1.25) ring = Ring{128, 256, 2, 4, 1, 64, 1};
     else if (K <= 512) ring = Ring{64, 128, 2, 2, 1, 64, 1};
   }
   if (!ring.bm && render_matmul_wave(mm, ep, whole_tiles, out)) return true;
