@@ -1010,7 +1010,7 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     //            (4096x512x784 37.6 -> 31.0, 512x2304x768 48.4 -> 27.2, 2048x1024x64 9.4 -> 5.9; 1024^3, 256 tiles, 22.5 and
     //            25.7; a depth of 4096 and more stays with the templates for that)
     // The latter two only where the rows of an operand that lies along them begin on 64 bytes (1001x1503x777 61
-    // either way, 1500x1500x1504 94 and 186).  Errors against float64 are a half to a third of those
+    // either way, 1500x1500x1504 94 and 186).  Errors against float64 are a third to two thirds of those
     // of the fp32 MFMA templates, that deal the depth to waves and workgroups or not.  A kernel lowered by itself,
     // outside a plan, keeps those.
     if (g_in_plan && !g_a_rows && Z == 1 && zd.empty() && ep.scratch_type.empty() && !getenv("POLY_HIP_NO_F32_MFMA") && !getenv("POLY_HIP_NO_F32_SPLIT") &&
@@ -1347,7 +1347,15 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     return true;
   };
   if (ring.bm) {
-    if (emit(ring.bm, ring.bn, ring.wm, ring.wn, 3, out, 0, -1, true, Dma{ring.bk, 2, ring.wg, ring.wm, ring.wn})) return S > 1 ? add_parts() : true;
+    if (emit(ring.bm, ring.bn, ring.wm, ring.wn, 3, out, 0, -1, true, Dma{ring.bk, 2, ring.wg, ring.wm, ring.wn})) {
+      if (S > 1) return add_parts();
+      RenderedKernel alone;      // a candidate for on-device tuning: the registers of a workgroup that has a CU to itself
+      if (f32 && ring.wg > 1 && matmul_tuning_enabled() && emit(ring.bm, ring.bn, ring.wm, ring.wn, 3, &alone, 0, -1, true, Dma{ring.bk, 2, 1, ring.wm, ring.wn})) {
+        out->variants.push_back({"default", out->source, out->strategy, out->launch});
+        out->variants.push_back({strf("f32_%dx%dw%dx%d", ring.bm, ring.bn, ring.wm, ring.wn), alone.source, alone.strategy, alone.launch});
+      }
+      return true;
+    }
     if (render_matmul_wave(mm, ep, whole_tiles, out)) return true;
     return f32 && ep.mid_value_call.empty() ? render_matmul_f32(mm, ep, out) : reject(__LINE__);
   }
