@@ -1236,14 +1236,22 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     if (const char *e = measurement_env("POLY_HIP_MM_KT")) if (atoi(e) > 0 && atoi(e) <= K / bk) cfg += strf("#define POLY_KT %d\n", atoi(e));
     cfg += strf("#define POLY_A_KC %d\n#define POLY_B_KC %d\n", a_kc ? 1 : 0, b_kc ? 1 : 0);
     cfg += strf("#define POLY_A_PTR %s\n#define POLY_B_PTR %s\n", ep.a_ptr.c_str(), ep.b_ptr.c_str());
-    cfg += offset_fn("poly_a_row", md, true, 0);
-    cfg += offset_fn("poly_b_row", nd, false, 0);
+    // (the templates of the LDS tiles add a row's and a depth's offset to a 64-bit pointer as one unsigned number: where
+    // an operand is read in reverse order, its pointer begins at its lowest element)
+    auto lowest = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a) {
+      int64_t low = ks.kb >= K ? std::min<int64_t>(0, (K - 1) * ks.s_lo) : std::min<int64_t>(0, (K - 1) / ks.kb * ks.s_hi) + std::min<int64_t>(0, (ks.kb - 1) * ks.s_lo);
+      for (const Dim &d : dims) low += std::min<int64_t>(0, (d.extent - 1) * (is_a ? d.ca : d.cb));
+      return low;
+    };
+    const int64_t a_low = lowest(ka, md, true), b_low = lowest(kb, nd, false);
+    cfg += offset_fn("poly_a_row", md, true, -a_low);
+    cfg += offset_fn("poly_b_row", nd, false, -b_low);
     if (zd.empty()) {
-      cfg += strf("__device__ __forceinline__ int poly_a_z(int) { return %lld; }\n", (long long)mm.a_c0);
-      cfg += strf("__device__ __forceinline__ int poly_b_z(int) { return %lld; }\n", (long long)mm.b_c0);
+      cfg += strf("__device__ __forceinline__ int poly_a_z(int) { return %lld; }\n", (long long)(mm.a_c0 + a_low));
+      cfg += strf("__device__ __forceinline__ int poly_b_z(int) { return %lld; }\n", (long long)(mm.b_c0 + b_low));
     } else {
-      cfg += offset_fn("poly_a_z", zd, true, mm.a_c0);
-      cfg += offset_fn("poly_b_z", zd, false, mm.b_c0);
+      cfg += offset_fn("poly_a_z", zd, true, mm.a_c0 + a_low);
+      cfg += offset_fn("poly_b_z", zd, false, mm.b_c0 + b_low);
     }
     cfg += matmul_k_fn("poly_a_k", ka, K);
     cfg += matmul_k_fn("poly_b_k", kb, K);

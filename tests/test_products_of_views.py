@@ -1,0 +1,96 @@
+"""Products whose operands are views, on every template a plan's products run on, both operands and both ways they can
+lie: rows or the depth in reverse order, which an operand's offsets run down.  On the host with buffers of their exact
+size, and against the product in float64, element by element, within the rounding of K fp32 additions and products
+(K * 2^-24 * sum of |a b|)."""
+import ctypes as C
+import os
+import re
+import sys
+
+import pytest
+
+import hostcheck
+from polygrad_amd import PlanFile, _ffi
+from test_f32_planes import PLAN, check_as_of_a_plan
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "perf"))
+import cases  # noqa: E402
+
+F32_PLANES, RING, DMA, REGISTERS, WAVES = "three planes of each f32 value", "rows of any alignment", "straight into LDS", "32x32x16", "depth dealt to"
+REVERSED = [(1793, 1664, 129, "float32", "nn", "A rows", F32_PLANES), (1665, 1793, 191, "float32", "nt", "B rows", F32_PLANES), (1665, 1793, 191, "float32", "nt", "A rows B rows", F32_PLANES),
+            (1025, 1024, 65, "float32", "nt", "A rows B rows", F32_PLANES), (1024, 1024, 2048, "float32", "nt", "A rows B rows", F32_PLANES),
+            (513, 511, 1001, "bfloat16", "nn", "A rows", RING), (1091, 1030, 161, "float16", "nt", "A rows B rows", RING), (1502, 1400, 130, "bfloat16", "nt", "A rows B rows", RING),
+            (1152, 1024, 1536, "bfloat16", "nn", "A rows", DMA), (1152, 1024, 1536, "bfloat16", "tn", "A depth", DMA), (1152, 1024, 1536, "bfloat16", "nn", "B depth", DMA),
+            (4096, 4096, 512, "float16", "nt", "A rows B rows", DMA), (2304, 512, 1536, "bfloat16", "nt", "B rows", DMA), (512, 512, 16384, "bfloat16", "nt", "A rows B rows", DMA),
+            (49452, 1000, 512, "bfloat16", "nt", "A rows B rows", DMA), (16384, 64, 512, "bfloat16", "nt", "A rows B rows", REGISTERS),
+            (40, 768, 512, "bfloat16", "nt", "A rows B rows", WAVES), (40, 768, 512, "float32", "nt", "A rows B rows", WAVES)]
+
+
+def _is_it(desc, template):
+    return template in desc and (template != REGISTERS or not any(t in desc for t in (F32_PLANES, RING, DMA)))
+
+
+def _slice(name, view, rows, k, along_k):
+    """Outer extent, inner extent, elements from one outer index to the next and the first element."""
+    outer, inner = (rows, k) if along_k else (k, rows)
+    given = re.search(name + r" (\d+) (\d+)", view)
+    pitch, first = (int(given.group(1)), int(given.group(2))) if given else (inner, 0)
+    return outer, inner, pitch, first
+
+
+def schedule(m, n, k, dtype, layout, view):
+    """C = A B, A and B buffers that end with their last element, read as `view` says."""
+    s = cases.Schedule()
+
+    def buf(name, rows, along_k):
+        outer, inner, pitch, first = _slice(name, view, rows, k, along_k)
+        return s.buf(name, first + (outer - 1) * pitch + inner, dtype)
+
+    out, a, b = s.buf("C", m * n), buf("A", m, layout[0] == "n"), buf("B", n, layout[1] == "t")
+    (r,) = s.ranges(m * n)
+    x = s.rrange(k)
+
+    def at(name, row, rows, along_k):
+        row = row * -1 + (rows - 1) if name + " rows" in view else row
+        d = x * -1 + (k - 1) if name + " depth" in view else x
+        _, _, pitch, first = _slice(name, view, rows, k, along_k)
+        return (row * pitch + d if along_k else d * pitch + row) + first
+
+    s.store(out, r, s.reduce("ADD", a[at("A", r // n, m, layout[0] == "n")].cast(cases.F32) * b[at("B", r % n, n, layout[1] == "t")].cast(cases.F32), x), r)
+    return s
+
+
+@pytest.mark.skipif(not os.path.exists(hostcheck.CLANG), reason="no host clang with AddressSanitizer")
+@pytest.mark.parametrize("c", REVERSED, ids=lambda c: "-".join(map(str, c)))
+def test_stays_in_bounds(c, hiplib, monkeypatch):
+    monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
+    pf = schedule(*c[:6]).plan()
+    s = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents
+    assert _is_it(_ffi.take_string(hiplib.poly_hip_describe(s.items[0].root, PLAN)), c[6])
+    check_as_of_a_plan(hiplib, s, s.items[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", REVERSED, ids=lambda c: "-".join(map(str, c)))
+def test_against_float64(c):
+    import torch
+    from polygrad_amd.inputs import torch_dtype
+    m, n, k, dtype, layout, view, template = c
+    plan, g = schedule(*c[:6]).plan(), torch.Generator(device="cuda")
+    g.manual_seed(6)
+    assert _is_it(plan.kernel_info()[0]["desc"], template)
+    data, by = [None] * len(plan.slots), {}
+    for slot in plan.external_slots():
+        data[slot.index] = by[slot.name] = torch.randn(slot.numel, generator=g, device="cuda").to(torch_dtype(slot.dtype))
+
+    def operand(name, rows, along_k):
+        outer, inner, pitch, first = _slice(name, view, rows, k, along_k)
+        t = torch.as_strided(by[name], (outer, inner), (pitch, 1), first).double()
+        t = t if along_k else t.T
+        return t.flip([d for d, axis in enumerate(("rows", "depth")) if f"{name} {axis}" in view])
+
+    plan.run(data)
+    plan.sync()
+    a, b = operand("A", m, layout[0] == "n"), operand("B", n, layout[1] == "t").T
+    err = (by["C"].double().reshape(m, n) - a @ b).abs()
+    assert bool((err <= k * 2.0 ** -24 * (a.abs() @ b.abs())).all())
