@@ -8,6 +8,7 @@
 //
 //   POLY_A_PITCH/B_PITCH   elements from one k of the operand to the next
 //   POLY_WG_PER_CU         workgroups meant to share a CU (sets the register budget)
+//   POLY_FAR               1: an operand is read further than 4 GiB behind its beginning
 //   POLY_KSPLIT            (optional) workgroups that share the depth of a tile, a multiple of POLY_BK each
 //
 // An fp32 value is the sum of three bf16 values, hi + mid + lo (each the rounding of what the ones before
@@ -49,6 +50,7 @@
 #define POLY_B_KC 0
 #define POLY_A_PITCH 1ll
 #define POLY_B_PITCH 1023ll
+#define POLY_FAR 0
 #define POLY_A_PTR data1
 #define POLY_B_PTR data2
 __device__ __forceinline__ int poly_a_row(int m) { return m * POLY_K; }
@@ -116,6 +118,11 @@ __device__ __forceinline__ int poly_swz_x(int k) { return (ROWS % 128 == 0) ? ((
 #endif
 
 struct PolyUnit { float v[8]; };
+#if POLY_FAR
+typedef unsigned long long poly_bytes;
+#else
+typedef unsigned int poly_bytes;
+#endif
 
 extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly_k(POLY_SIGNATURE) {
   __shared__ __attribute__((aligned(1024))) unsigned char lds_raw[2 * POLY_STAGE_BYTES];
@@ -167,11 +174,11 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
   auto first_row = [&](int u) { return (is_a(u) ? m0 : n0) + (along_k(u) ? slot_of(u) / POLY_CH : slot_of(u) % chunks_of(u) * 8); };
   auto k_of = [&](int u) { return along_k(u) ? slot_of(u) % POLY_CH * 8 : slot_of(u) / chunks_of(u); };
   // (Two halves of 4 elements half a tile apart, which lanes side by side load side by side, change nothing.)
-  unsigned int from[POLY_UNITS];      // bytes to it in the first whole tile
+  poly_bytes from[POLY_UNITS];      // bytes to it in the first whole tile
 #pragma unroll
   for (int u = 0; u < POLY_UNITS; u++) {
     const int r = first_row(u), row = r < rows_of(u) ? r : rows_of(u) - (along_k(u) ? 1 : 8);
-    from[u] = 4u * (unsigned int)(is_a(u) ? poly_a_row(row) + poly_a_k(k_of(u)) : poly_b_row(row) + poly_b_k(k_of(u)));
+    from[u] = (poly_bytes)4 * (unsigned int)(is_a(u) ? poly_a_row(row) + poly_a_k(k_of(u)) : poly_b_row(row) + poly_b_k(k_of(u)));
   }
   constexpr long long STEP_A = 4ll * POLY_BK * (POLY_A_KC ? 1 : POLY_A_PITCH), STEP_B = 4ll * POLY_BK * (POLY_B_KC ? 1 : POLY_B_PITCH);
   // Tile s > 0 is the depth from (s - 1) POLY_BK on.  (What 8 elements along the rows read past their end is

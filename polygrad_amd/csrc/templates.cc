@@ -1244,6 +1244,15 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
       return low;
     };
     const int64_t a_low = lowest(ka, md, true), b_low = lowest(kb, nd, false);
+    if (f32) {
+      // (buffers have fewer than 2^31 elements: 16-bit ones fit)
+      auto reach = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a) {
+        int64_t far = (K - 1) * ks.s_lo;
+        for (const Dim &d : dims) far += (d.extent - 1) * std::llabs(is_a ? d.ca : d.cb);
+        return far;
+      };
+      cfg += strf("#define POLY_FAR %d\n", std::max(reach(ka, md, true), reach(kb, nd, false)) >= ((int64_t)1 << 30) - 8 ? 1 : 0);
+    }
     cfg += offset_fn("poly_a_row", md, true, -a_low);
     cfg += offset_fn("poly_b_row", nd, false, -b_low);
     if (zd.empty()) {

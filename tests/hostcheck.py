@@ -23,6 +23,17 @@ SHIM = r"""
 #include <cstdlib>
 #include <cstring>
 #include <cstdint>
+#include <sys/mman.h>
+// address space of `size` bytes in which only the pages of `count` pieces can be touched, `step` bytes from one to the next
+static void *poly_pieces(size_t size, size_t first, size_t bytes, size_t step, size_t count) {
+  char *const p = (char *)mmap(0, size, PROT_NONE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+  if (p == MAP_FAILED) abort();
+  for (size_t i = 0; i < count; i++) {
+    const size_t lo = (first + i * step) & ~(size_t)4095, hi = (first + i * step + bytes + 4095) & ~(size_t)4095;
+    if (mprotect(p + lo, hi - lo, PROT_READ | PROT_WRITE)) abort();
+  }
+  return p;
+}
 struct poly_dim3 { unsigned x, y, z; };
 static poly_dim3 threadIdx, blockIdx, blockDim, gridDim;
 #define POLY_HOST_ADDRESS_CHECK 1
@@ -60,8 +71,11 @@ int main() {
   gridDim = {GX, GY, GZ};
   blockDim = {BX, 1, 1};
   void *bufs[NBUF + 1];
+  bool whole[NBUF + 1];
   static const size_t sizes[NBUF + 1] = {SIZES 0};
   for (int i = 0; i < NBUF; i++) {
+    whole[i] = !(PIECES);
+    if (!whole[i]) continue;
     bufs[i] = malloc(sizes[i]);          // exact size: ASan guards both ends
     memset(bufs[i], 1, sizes[i]);        // (no zeros: integer kernels divide by their inputs)
   }
@@ -73,7 +87,7 @@ int main() {
           threadIdx = {tx, 0, 0};
           ENTRY(ARGS);
         }
-  for (int i = 0; i < NBUF; i++) free(bufs[i]);
+  for (int i = 0; i < NBUF; i++) if (whole[i]) free(bufs[i]);
   puts("ok");
   return 0;
 }
@@ -110,10 +124,11 @@ def _entry_name(source):
     return [m for m in re.findall(r"(\w+)\s*\(", line) if m.startswith("poly_")][-1]
 
 
-def check_kernel(source, entry, grid, block, buf_sizes, block_stride=1, timeout=600, scratch_bytes=0):
+def check_kernel(source, entry, grid, block, buf_sizes, block_stride=1, timeout=600, scratch_bytes=0, pieces=None):
     """Compiles `source` for the host and runs kernel `entry` over its whole launch (or
     every `block_stride`-th workgroup along x) with exact-size buffers.  Raises with the
-    sanitizer's report on an out-of-bounds access."""
+    sanitizer's report on an out-of-bounds access.  `pieces` = {buffer: (first byte, bytes, step, count)}: of that
+    buffer, which takes no memory, the kernel may touch those pieces alone."""
     types = _arg_types(source, entry)
     assert len(types) >= len(buf_sizes), (entry, types, buf_sizes)
     # what follows the buffers: DEFINE_VAR ints (passed as 0) and lookup tables (65536 entries of at most 16 bytes)
@@ -123,6 +138,7 @@ def check_kernel(source, entry, grid, block, buf_sizes, block_stride=1, timeout=
     args = ", ".join(f"({t})bufs[{i}]" if "*" in t else "0" for i, t in enumerate(types))
     tail = (DRIVER_TAIL.replace("GX", str(grid[0])).replace("GY", str(grid[1])).replace("GZ", str(grid[2]))
             .replace("BX", str(block)).replace("NBUF", str(len(buf_sizes))).replace("STRIDE", str(block_stride))
+            .replace("PIECES", " || ".join(f"(i == {i} && (bufs[i] = poly_pieces(sizes[i], {', '.join(map(str, piece))})))" for i, piece in (pieces or {}).items()) or "0")
             .replace("SIZES", "".join(f"{int(s)}, " for s in buf_sizes)).replace("ENTRY", entry).replace("ARGS", args))
     with tempfile.TemporaryDirectory() as d:
         src = os.path.join(d, "k.cc")

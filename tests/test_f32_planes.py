@@ -31,8 +31,9 @@ def _is_it(desc, c):
     return "three planes of each f32 value" in desc and f"tile {c[4]}x32" in desc and (dealt is not None) == (c[2] >= 768)
 
 
-def check_as_of_a_plan(hiplib, schedule, item):
-    """The kernel of `item` as a plan has it, and its first stages, on the host with buffers of their exact size."""
+def check_as_of_a_plan(hiplib, schedule, item, pieces=None):
+    """The kernel of `item` as a plan has it, and its first stages, on the host with buffers of their exact size, or
+    of some of them only the pieces that there are (hostcheck.check_kernel)."""
     launch = (C.c_int * 7)()
     units = _ffi.take_string(hiplib.poly_hip_render(item.root, b"k", PLAN, launch)).split("\n// ---- ")
     sizes, scratch = [schedule.buf_slots[item.buf_slot_indices[p]].nbytes for p in range(item.n_buf_slots)], 0
@@ -42,7 +43,7 @@ def check_as_of_a_plan(hiplib, schedule, item):
         scratch = int(m.group(4))
         jobs.append((u[m.end():], (int(m.group(1)), int(m.group(2)), 1), int(m.group(3))))
     for source, grid, block in jobs:
-        hostcheck.check_kernel(source, hostcheck._entry_name(source), grid, block, sizes, block_stride=max(1, grid[0] * grid[1] * block // (1 << 17)), scratch_bytes=scratch)
+        hostcheck.check_kernel(source, hostcheck._entry_name(source), grid, block, sizes, block_stride=max(1, grid[0] * grid[1] * block // (1 << 17)), scratch_bytes=scratch, pieces=pieces)
 
 
 @pytest.mark.skipif(not os.path.exists(hostcheck.CLANG), reason="no host clang with AddressSanitizer")

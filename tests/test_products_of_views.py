@@ -1,5 +1,6 @@
 """Products whose operands are views, on every template a plan's products run on, both operands and both ways they can
-lie: rows or the depth in reverse order, which an operand's offsets run down.  On the host with buffers of their exact
+lie: rows or the depth in reverse order, which an operand's offsets run down; rows far
+apart, in buffers of 4 GiB and more.  On the host with buffers of their exact
 size, and against the product in float64, element by element, within the rounding of K fp32 additions and products
 (K * 2^-24 * sum of |a b|)."""
 import ctypes as C
@@ -24,6 +25,9 @@ REVERSED = [(1793, 1664, 129, "float32", "nn", "A rows", F32_PLANES), (1665, 179
             (4096, 4096, 512, "float16", "nt", "A rows B rows", DMA), (2304, 512, 1536, "bfloat16", "nt", "B rows", DMA), (512, 512, 16384, "bfloat16", "nt", "A rows B rows", DMA),
             (49452, 1000, 512, "bfloat16", "nt", "A rows B rows", DMA), (16384, 64, 512, "bfloat16", "nt", "A rows B rows", REGISTERS),
             (40, 768, 512, "bfloat16", "nt", "A rows B rows", WAVES), (40, 768, 512, "float32", "nt", "A rows B rows", WAVES)]
+# (of 2^30 elements and more, in 1.1 million from one row to the next)
+FAR = [(1793, 1664, 129, "float32", "nn", "A 1100000 1", F32_PLANES), (1665, 1921, 191, "float32", "nt", "B 1100003 2", F32_PLANES), (1025, 1024, 65, "float32", "nn", "A 1100000 0", F32_PLANES),
+       (1001, 1696, 1930, "float32", "tn", "A 1100000 0", F32_PLANES), (1090, 1941, 161, "bfloat16", "nt", "B 1100001 1", RING), (1152, 1024, 1920, "bfloat16", "nn", "B 1100000 0", DMA)]
 
 
 def _is_it(desc, template):
@@ -70,8 +74,22 @@ def test_stays_in_bounds(c, hiplib, monkeypatch):
     check_as_of_a_plan(hiplib, s, s.items[0])
 
 
+@pytest.mark.skipif(not os.path.exists(hostcheck.CLANG), reason="no host clang with AddressSanitizer")
+@pytest.mark.parametrize("c", FAR, ids=lambda c: "-".join(map(str, c)))
+def test_far_rows_are_those_read(c, hiplib, monkeypatch):
+    monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
+    m, n, k, dtype, layout, view, template = c
+    pf = schedule(*c[:6]).plan()
+    s = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents
+    assert _is_it(_ffi.take_string(hiplib.poly_hip_describe(s.items[0].root, PLAN)), template)
+    name = view[0]
+    outer, inner, pitch, first = _slice(name, view, *((m, k, layout[0] == "n") if name == "A" else (n, k, layout[1] == "t")))
+    size = 4 if dtype == "float32" else 2
+    check_as_of_a_plan(hiplib, s, s.items[0], pieces={1 if name == "A" else 2: (first * size, inner * size, pitch * size, outer)})
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("c", REVERSED, ids=lambda c: "-".join(map(str, c)))
+@pytest.mark.parametrize("c", REVERSED + FAR, ids=lambda c: "-".join(map(str, c)))
 def test_against_float64(c):
     import torch
     from polygrad_amd.inputs import torch_dtype
@@ -81,16 +99,21 @@ def test_against_float64(c):
     assert _is_it(plan.kernel_info()[0]["desc"], template)
     data, by = [None] * len(plan.slots), {}
     for slot in plan.external_slots():
-        data[slot.index] = by[slot.name] = torch.randn(slot.numel, generator=g, device="cuda").to(torch_dtype(slot.dtype))
+        t = torch.zeros(slot.numel, dtype=torch_dtype(slot.dtype), device="cuda")
+        data[slot.index] = by[slot.name] = t if slot.numel > 1 << 28 else t.copy_(torch.randn(slot.numel, generator=g, device="cuda"))
 
     def operand(name, rows, along_k):
         outer, inner, pitch, first = _slice(name, view, rows, k, along_k)
-        t = torch.as_strided(by[name], (outer, inner), (pitch, 1), first).double()
+        t = torch.as_strided(by[name], (outer, inner), (pitch, 1), first)
+        if by[name].numel() > 1 << 28:      # (a few elements of it are all that is random)
+            t.copy_(torch.randn((outer, inner), generator=g, device="cuda"))
+        t = t.double()
         t = t if along_k else t.T
         return t.flip([d for d, axis in enumerate(("rows", "depth")) if f"{name} {axis}" in view])
 
+    a, b = operand("A", m, layout[0] == "n"), operand("B", n, layout[1] == "t").T
+    torch.cuda.synchronize()
     plan.run(data)
     plan.sync()
-    a, b = operand("A", m, layout[0] == "n"), operand("B", n, layout[1] == "t").T
     err = (by["C"].double().reshape(m, n) - a @ b).abs()
     assert bool((err <= k * 2.0 ** -24 * (a.abs() @ b.abs())).all())
