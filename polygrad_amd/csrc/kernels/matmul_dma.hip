@@ -463,8 +463,8 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
   constexpr int R = POLY_RING, NTILES = POLY_KT + 1;
   static_assert(S == 2 && R % 2 == 0 && POLY_KSPLIT == 1, "two stages, whole turns of both rings");
   // (Where a stride is odd, whole dwords are read and moved down by half of one on the way to LDS where
-  // they have to be.  The first of the next lane's dwords is the fifth of these; the last lane of a row
-  // reads it.  What is odd about a unit is the same in every tile.  The dword that holds an operand's first
+  // they have to be.  The first of the next lane's dwords is the fifth of these; the last lane of a row of the tile or
+  // of the operand reads it.  What is odd about a unit is the same in every tile.  The dword that holds an operand's first
   // element may begin with one in front of it, which is dropped.)
   struct Unit { poly_u32x4 v; unsigned int next; };
   Unit ring[R][POLY_IPW];
@@ -481,8 +481,12 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
     if (is_a ? POLY_A_ODD : POLY_B_ODD) from[u] -= odd[u];
   }
   auto last_lane = [&](int u) {
-    const int chunks = (u < POLY_A_IPW ? POLY_A_KC : POLY_B_KC) ? POLY_CH : u < POLY_A_IPW ? POLY_BM / 8 : POLY_BN / 8;
-    return lane % (chunks < 16 ? chunks : 16) == (chunks < 16 ? chunks : 16) - 1;
+    const bool is_a = u < POLY_A_IPW, kc = is_a ? POLY_A_KC : POLY_B_KC;
+    const int chunks = kc ? POLY_CH : is_a ? POLY_BM / 8 : POLY_BN / 8, slot = ((is_a ? u : u - POLY_A_IPW) * POLY_NW + wave) * 64 + lane;
+    // (along rows of whole 8 also the last chunk that exists: the lane behind it repeats an earlier one)
+    const int end = is_a ? POLY_M : POLY_N;
+    const bool edge = !kc && end % 8 == 0 && end - (is_a ? m0 : n0) == slot % chunks * 8 + 8;
+    return edge || lane % (chunks < 16 ? chunks : 16) == (chunks < 16 ? chunks : 16) - 1;
   };
   // unit u of a whole tile (every row of 8 elements starts inside a row of its operand, and what it
   // reads past the end of that is the beginning of the next: the last row of the depth is tile 0's)

@@ -1,8 +1,8 @@
 """Products whose operands are views, on every template a plan's products run on, both operands and both ways they can
-lie: rows or the depth in reverse order, which an operand's offsets run down; rows far
-apart, in buffers of 4 GiB and more.  On the host with buffers of their exact
-size, and against the product in float64, element by element, within the rounding of K fp32 additions and products
-(K * 2^-24 * sum of |a b|)."""
+lie: rows or the depth in reverse order, which an operand's offsets run down; slices of wider buffers, whose rows begin
+between two dwords or 16 bytes and end inside a tile, behind whole 8 elements or not; rows far apart, in buffers
+of 4 GiB and more.  On the host with buffers of their exact size, and against the product in float64, element by
+element, within the rounding of K fp32 additions and products (K * 2^-24 * sum of |a b|)."""
 import ctypes as C
 import os
 import re
@@ -25,6 +25,12 @@ REVERSED = [(1793, 1664, 129, "float32", "nn", "A rows", F32_PLANES), (1665, 179
             (4096, 4096, 512, "float16", "nt", "A rows B rows", DMA), (2304, 512, 1536, "bfloat16", "nt", "B rows", DMA), (512, 512, 16384, "bfloat16", "nt", "A rows B rows", DMA),
             (49452, 1000, 512, "bfloat16", "nt", "A rows B rows", DMA), (16384, 64, 512, "bfloat16", "nt", "A rows B rows", REGISTERS),
             (40, 768, 512, "bfloat16", "nt", "A rows B rows", WAVES), (40, 768, 512, "float32", "nt", "A rows B rows", WAVES)]
+# ("A 1003 1": rows of A, or where it lies along its rows depths of it, are 1003 elements apart, the first at 1)
+SLICED = [(513, 520, 1001, "bfloat16", "nn", "B 521 0", RING), (513, 520, 1001, "bfloat16", "nn", "B 522 1", RING), (520, 513, 1001, "float16", "tn", "A 521 1", RING),
+          (520, 504, 769, "bfloat16", "tt", "A 521 3 B 771 1", RING), (1096, 1032, 161, "bfloat16", "tn", "A 1099 0 B 1033 0", RING), (1111, 1000, 1501, "bfloat16", "nn", "B 1001 1", RING),
+          (1400, 1504, 129, "bfloat16", "tn", "A 1401 5 B 1506 1", RING), (2056, 2104, 130, "float16", "tn", "A 2057 0 B 2106 1", RING), (3000, 3008, 33, "bfloat16", "nn", "A 35 1 B 3009 0", RING),
+          (512, 514, 1001, "bfloat16", "nn", "B 515 1", RING), (1030, 1040, 97, "float32", "nn", "A 99 1 B 1056 3", F32_PLANES), (1801, 1700, 160, "float32", "tn", "A 1805 2 B 1701 1", F32_PLANES),
+          (1152, 1024, 1536, "bfloat16", "nt", "A 1538 2 B 1544 8", DMA), (1152, 1024, 1536, "bfloat16", "tn", "A 1156 4 B 1026 2", DMA)]
 # (of 2^30 elements and more, in 1.1 million from one row to the next)
 FAR = [(1793, 1664, 129, "float32", "nn", "A 1100000 1", F32_PLANES), (1665, 1921, 191, "float32", "nt", "B 1100003 2", F32_PLANES), (1025, 1024, 65, "float32", "nn", "A 1100000 0", F32_PLANES),
        (1001, 1696, 1930, "float32", "tn", "A 1100000 0", F32_PLANES), (1090, 1941, 161, "bfloat16", "nt", "B 1100001 1", RING), (1152, 1024, 1920, "bfloat16", "nn", "B 1100000 0", DMA)]
@@ -65,7 +71,7 @@ def schedule(m, n, k, dtype, layout, view):
 
 
 @pytest.mark.skipif(not os.path.exists(hostcheck.CLANG), reason="no host clang with AddressSanitizer")
-@pytest.mark.parametrize("c", REVERSED, ids=lambda c: "-".join(map(str, c)))
+@pytest.mark.parametrize("c", REVERSED + SLICED, ids=lambda c: "-".join(map(str, c)))
 def test_stays_in_bounds(c, hiplib, monkeypatch):
     monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
     pf = schedule(*c[:6]).plan()
@@ -89,7 +95,7 @@ def test_far_rows_are_those_read(c, hiplib, monkeypatch):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("c", REVERSED + FAR, ids=lambda c: "-".join(map(str, c)))
+@pytest.mark.parametrize("c", REVERSED + SLICED + FAR, ids=lambda c: "-".join(map(str, c)))
 def test_against_float64(c):
     import torch
     from polygrad_amd.inputs import torch_dtype
