@@ -6,7 +6,9 @@ small for three bf16 planes to hold as the fp32 MFMA has them."""
 import ctypes as C
 import os
 import re
+import subprocess
 import sys
+import tempfile
 
 import pytest
 
@@ -56,6 +58,35 @@ def test_stays_in_bounds(c, hiplib, monkeypatch):
     assert _is_it(_ffi.take_string(hiplib.poly_hip_describe(it.root, PLAN)), c)
     assert "three planes" not in _ffi.take_string(hiplib.poly_hip_describe(it.root, 0))
     check_as_of_a_plan(hiplib, s, it)
+
+
+def _scratch_bytes(source):
+    """Of scratch memory to a lane, in the code object that the run-time compiler makes of `source`."""
+    rtc, prog, size = C.CDLL("/opt/rocm/lib/libhiprtc.so"), C.c_void_p(), C.c_size_t()
+    options = (C.c_char_p * 8)(*b"--offload-arch=gfx950 -O3 -std=c++17 -ffp-contract=off -Xclang -target-feature -Xclang -packed-fp32-ops".split())
+    assert rtc.hiprtcCreateProgram(C.byref(prog), source.encode(), b"k.hip", 0, None, None) == 0
+    assert rtc.hiprtcCompileProgram(prog, 8, options) == 0
+    rtc.hiprtcGetCodeSize(prog, C.byref(size))
+    code = C.create_string_buffer(size.value)
+    rtc.hiprtcGetCode(prog, code)
+    rtc.hiprtcDestroyProgram(C.byref(prog))
+    with tempfile.NamedTemporaryFile() as f:
+        f.write(code.raw)
+        f.flush()
+        notes = subprocess.run(["/opt/rocm/llvm/bin/llvm-readelf", "--notes", f.name], capture_output=True, text=True, check=True).stdout
+    return int(re.search(r"\.private_segment_fixed_size: +(\d+)", notes).group(1))
+
+
+@pytest.mark.skipif(not os.path.exists("/opt/rocm/llvm/bin/llvm-readelf"), reason="no reader of code objects")
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("m,n,ks", [(320, 3776, (74, 82, 90, 372)), (1793, 1664, (129, 138, 148, 157))])
+def test_ends_of_the_depth_stay_in_registers(m, n, ks, layout, hiplib, monkeypatch):
+    monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
+    for k in ks:
+        pf = cases._matmul_schedule(dict(kind="matmul", m=m, n=n, k=k, dtype="float32", layout=layout)).plan()
+        it = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents.items[0]
+        if "three planes" in _ffi.take_string(hiplib.poly_hip_describe(it.root, PLAN)):      # (rows of an odd number of lines are another template's)
+            assert _scratch_bytes(_ffi.take_string(hiplib.poly_hip_render(it.root, b"k", PLAN, None)).split("\n// ---- ")[0]) == 0
 
 
 def _product(c, change=None):
