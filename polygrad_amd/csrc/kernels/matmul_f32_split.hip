@@ -12,12 +12,14 @@
 //   POLY_KSPLIT            (optional) workgroups that share the depth of a tile, a multiple of POLY_BK each
 //
 // An fp32 value is the sum of three bf16 values, hi + mid + lo (each the rounding of what the ones before
-// leave; the differences are exact).  Products of bf16 values are exact in fp32, and of the nine of two such
-// sums the six down to 2^-18 of the value are added up; what is left out is 2^-26 of it, a quarter of
-// what one rounding of an fp32 addition may be.  The products of the leading planes have sums of their
-// own: one rounding at the size of the result for 16 products, where the fp32 MFMA has eight.  Errors
-// against float64: 4096 x 512 x 784 1.6e-7 [fp32 MFMA 5.0e-7], 2048^3 2.7e-7 [8.1e-7],
-// 1024 x 1024 x 4096 1.9e-7 [4.1e-7].
+// leave; the differences are exact), as in G. Henry, P. T. P. Tang, A. Heinecke, "Leveraging the bfloat16 Artificial
+// Intelligence Datatype For Higher-Precision Computations" (ARITH 2019).  Products of bf16 values are exact in
+// fp32, and of the nine of two such sums all but lo lo are added up, which is 2^-34 of the value at most (mid is up to
+// 2^-8 of it, lo 2^-17: without mid lo and lo mid a sum of one term is off by up to 1.8 roundings).  The products of the
+// leading planes have sums of their own: one rounding at the size of the result for 16 products, where the fp32 MFMA has
+// eight, and one more of each product's 2^-7 for those behind.  Errors against float64: 4096 x 512 x 784 1.6e-7 [fp32
+// MFMA 5.0e-7], 2048^3 2.7e-7 [8.1e-7], 1024 x 1024 x 4096 1.9e-7 [4.1e-7]; sums of one term 1.01 x 2^-24 [1.00], one in
+// a thousand of them not the nearest value.
 //
 // That holds for finite values of 2^-110 and more, below which bf16 has no 24 bits left, and zeros.
 // Operands are looked over for smaller ones on the way, results for infinities and NaN (an
@@ -28,8 +30,8 @@
 // contiguous along K and [plane][k][rows] for one along its rows, swizzled as in matmul_dma.hip, two
 // stages; one barrier per K tile.  The end of the depth is a tile of its own, the first, filled up
 // with zeros.  What bounds it: 64x64 tiles the first loads and the split, seven vector instructions per
-// element (4096 x 512 x 784 37.6 -> 31.0 us; its kernel 27.1, 20.3 without the loads of its K loop), larger ones
-// the matrix pipes, 6 MFMAs of 32 cycles where fp32 has 8 of 64 (2048^3 183 -> 100 us).
+// element (4096 x 512 x 784 45 -> 34 us), larger ones the matrix pipes, 8 MFMAs of 32 cycles where fp32 has 8 of 64
+// (2048^3 200 -> 117 us, 97 without the products mid lo and lo mid).
 #ifdef POLY_TEMPLATE_STANDALONE
 #include <hip/hip_runtime.h>
 #define POLY_TIN float
@@ -215,7 +217,7 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
     }
   };
   // (Each of the two is read whether it is taken or not: a choice between two places keeps the array in scratch memory,
-  // which for one depth in three took 12.5 us in place of 6.4 for 320x3776x82.)
+  // which at depths of 9 to 12, 17 to 20 and 25 to 28 modulo 32 took 12.5 us in place of 6.4 for 320x3776x82.)
   auto move_down = [&](PolyUnit &x, int by) {
 #pragma unroll
     for (int step = 4; step > 0; step /= 2)
@@ -296,7 +298,7 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
 
   // Iteration s: tile s is in LDS; the registers of tile s + 1 are split and stored into the other stage, a
   // pair of elements behind each MFMA or so, and refilled from tile s + 3, while it is multiplied.
-  constexpr int KS = POLY_BK / 16, SLOTS = KS * 6 * POLY_TM * POLY_TN, PAIRS = 4 * POLY_UNITS;
+  constexpr int KS = POLY_BK / 16, SLOTS = KS * 8 * POLY_TM * POLY_TN, PAIRS = 4 * POLY_UNITS;
   PolyUnit ring[2][POLY_UNITS];
   load_end(ring[0]);
   if (POLY_NTILES > 1) {
@@ -331,15 +333,15 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
       if (ks + 1 < KS) read_step(ks + 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int c = 0; c < 6; c++) {
-        constexpr int PA[6] = {0, 0, 1, 1, 0, 2}, PB[6] = {0, 1, 0, 1, 2, 0};
+      for (int c = 0; c < 8; c++) {
+        constexpr int PA[8] = {0, 0, 1, 1, 0, 2, 1, 2}, PB[8] = {0, 1, 0, 1, 2, 0, 2, 1};
 #pragma unroll
         for (int i = 0; i < POLY_TM; i++)
 #pragma unroll
           for (int j = 0; j < POLY_TN; j++) {
             poly_acc16 &to = c == 0 ? acc[i][j] : low[i][j];
             to = POLY_MFMA(fa[ks & 1][PA[c]][i], fb[ks & 1][PB[c]][j], to);
-            const int slot = ((ks * 6 + c) * POLY_TM + i) * POLY_TN + j;
+            const int slot = ((ks * 8 + c) * POLY_TM + i) * POLY_TN + j;
             if (st) {
 #pragma unroll
               for (int q = 0; q < PAIRS; q++)

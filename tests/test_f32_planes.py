@@ -147,3 +147,28 @@ def test_values_that_planes_do_not_hold(c, what, monkeypatch):
     # (below the smallest normal number a product's rounding is absolute)
     bound = 2 * c[2] * (2.0 ** -24 * (a.abs() @ b.abs()) + 2.0 ** -149)
     assert bool(((got.double() - want.double()).abs() <= bound)[finite].all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["whole", "smallest"])
+@pytest.mark.parametrize("c", SHAPES, ids=lambda c: "-".join(map(str, c)))
+def test_rows_of_one_term(c, what):
+    """One rounding of the one product of each sum: of the nine products of planes eight are there (the ninth is 2^-34
+    of it), and the sums of the seven behind the leading one, 2^-7 of it at most, are rounded seven times.  Also of the smallest
+    values that planes hold, 2^-110 to 2^-104, the last plane of which is below the smallest normal number."""
+    import torch
+    m, n, k = c[:3]
+
+    def change(a, b):
+        a2 = a.view(k, m).T if c[3][0] == "t" else a.view(m, k)
+        at = (torch.arange(m, device="cuda"), torch.randint(0, k, (m,), device="cuda"))
+        one = a2[at].sign() * (a2[at].abs().fmod(1.0) + 1.0)
+        if what == "smallest":
+            one *= 2.0 ** torch.randint(-110, -104, (m,), device="cuda").double()
+            b.mul_(2.0 ** 60)
+        a2.zero_()
+        a2[at] = one
+    desc, got, a, b = _product(c, change)
+    assert _is_it(desc, c)
+    want = a @ b
+    assert bool(((got.double() - want).abs() <= 2.0 ** -24 * (1 + 2.0 ** -4) * want.abs()).all())
