@@ -230,6 +230,12 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
 #pragma unroll
     for (int e = 0; e < 8; e++) x.v[e] = by >= 8 ? 0.0f : x.v[e];
   };
+  // elements of a unit along rows of its operand that exist, where not all may: what lies behind a row is nothing
+  // that the product is made of
+  auto cut = [&](int u) { return !along_k(u) && rows_of(u) % 8 != 0; };
+  int exist[POLY_UNITS];
+#pragma unroll
+  for (int u = 0; u < POLY_UNITS; u++) exist[u] = rows_of(u) - first_row(u) > 0 ? rows_of(u) - first_row(u) : 8;
   // smallest magnitude met that is not 0, as twice the bits of the float less 1
   unsigned int least = 0xffffffffu;
   // elements 2 p and 2 p + 1 of a row of 8, as words p of its three planes
@@ -346,6 +352,9 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
 #pragma unroll
               for (int q = 0; q < PAIRS; q++)
                 if (q * SLOTS / PAIRS == slot) {
+                  if (cut(q / 4))
+#pragma unroll
+                    for (int e = q % 4 * 2; e < q % 4 * 2 + 2; e++) next[q / 4].v[e] = e < exist[q / 4] ? next[q / 4].v[e] : 0.0f;
                   split_pair(next[q / 4], planes, q % 4);
                   if (q % 4 == 3) {
                     store_unit(planes, stage ^ 1, q / 4);

@@ -123,3 +123,28 @@ def test_against_float64(c):
     plan.sync()
     err = (by["C"].double().reshape(m, n) - a @ b).abs()
     assert bool((err <= k * 2.0 ** -24 * (a.abs() @ b.abs())).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [(1030, 1041, 97, "float32", "nn", "A 99 1 B 1056 3", F32_PLANES), (1801, 1703, 160, "float32", "tn", "A 1805 2 B 1709 1", F32_PLANES)],
+                         ids=lambda c: "-".join(map(str, c)))
+def test_what_lies_between_rows_changes_no_bit(c):
+    """Not the values that three planes do not hold either, which send a tile another way."""
+    import torch
+    m, n, k, dtype, layout, view, template = c
+    plan, g, outputs = schedule(*c[:6]).plan(), torch.Generator(device="cuda"), []
+    assert _is_it(plan.kernel_info()[0]["desc"], template)
+    for between in (0.0, 1e-40, float("nan"), float("inf")):
+        g.manual_seed(7)
+        data = [None] * len(plan.slots)
+        for slot in plan.external_slots():
+            data[slot.index] = t = torch.full((slot.numel,), between, device="cuda")
+            if slot.name != "C":
+                outer, inner, pitch, first = _slice(slot.name, view, m if slot.name == "A" else n, k, layout[0] == "n" if slot.name == "A" else layout[1] == "t")
+                torch.as_strided(t, (outer, inner), (pitch, 1), first).copy_(torch.randn((outer, inner), generator=g, device="cuda"))
+            else:
+                outputs.append(t)
+        torch.cuda.synchronize()
+        plan.run(data)
+        plan.sync()
+    assert all(torch.equal(outputs[0], o) for o in outputs[1:])
