@@ -24,7 +24,9 @@
 // That holds for finite values of 2^-110 and more, below which bf16 has no 24 bits left, and zeros.
 // Operands are looked over for smaller ones on the way, results for infinities and NaN (an
 // infinity leaves NaN behind: inf - inf), and a workgroup that met one computes its tile again
-// with the fp32 MFMA from operands in memory.
+// with the fp32 MFMA from operands in memory.  That takes what the fp32 templates take and some of the time up to
+// there: 2048^3 is 117 us without such values, 253 with one in every row, 295 with a single one in the middle of a row
+// [fp32 MFMA 200], 4096 x 512 x 784 34, 53 and 60 [45], 128 x 50257 x 768 86, 165 and 207 [120].
 //
 // Data path: global --16-byte loads--> registers, split there, --> LDS, [plane][row][BK] for an operand
 // contiguous along K and [plane][k][rows] for one along its rows, swizzled as in matmul_dma.hip, two
@@ -368,13 +370,23 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
     }
   };
   constexpr int STEADY = POLY_NTILES > 3 ? (POLY_NTILES - 3) / 2 * 2 : 0;
+  constexpr unsigned int LEAST = 2u * ((127u - 110u) << 23) - 1u;
+  // (a workgroup that has met a value below 2^-110 stops: one iteration's barrier lies between what it writes here and
+  // what every wave reads)
+  bool stopped = false;
 #pragma unroll 1
-  for (int s = 0; s < STEADY; s += 2) {
+  for (int s = 0; s < STEADY && !stopped; s += 2) {
     iteration(s, 0, ring[1], true, true);
-    iteration(s + 1, 1, ring[0], true, true);
+#ifndef POLY_HOST_ADDRESS_CHECK
+    stopped = poly_again != 0;
+#endif
+    if (!stopped) iteration(s + 1, 1, ring[0], true, true);
+    if (least < LEAST) poly_again = 1;
   }
+  if (!stopped) {
 #pragma unroll
-  for (int s = STEADY; s < POLY_NTILES; s++) iteration(s, s & 1, ring[(s + 1) & 1], s + 1 < POLY_NTILES, s + 3 < POLY_NTILES);
+    for (int s = STEADY; s < POLY_NTILES; s++) iteration(s, s & 1, ring[(s + 1) & 1], s + 1 < POLY_NTILES, s + 3 < POLY_NTILES);
+  }
 
 #pragma unroll
   for (int i = 0; i < POLY_TM; i++)
@@ -383,7 +395,7 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
 
   // Values that three planes do not hold: the tile again in fp32.
   {
-    bool again = least < 2u * ((127u - 110u) << 23) - 1u;
+    bool again = least < LEAST;
 #pragma unroll
     for (int i = 0; i < POLY_TM; i++)
 #pragma unroll
@@ -393,31 +405,85 @@ extern "C" __global__ void __launch_bounds__(POLY_NTHREADS) POLY_WAVES_ATTR poly
     if (again) poly_again = 1;
     __syncthreads();
     if (poly_again) {
+      poly_acc16 third[POLY_TM][POLY_TN], fourth[POLY_TM][POLY_TN];
 #pragma unroll
       for (int i = 0; i < POLY_TM; i++)
 #pragma unroll
         for (int j = 0; j < POLY_TN; j++)
 #pragma unroll
-          for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+          for (int r = 0; r < 16; r++) acc[i][j][r] = low[i][j][r] = third[i][j][r] = fourth[i][j][r] = 0.0f;
+      // 16 of the depth at a time, 8 to each half of the lanes, which is read while the 16 before are multiplied, into
+      // four sums of each result, as many as the fp32 templates have of products of these sizes
+      const float *pa[POLY_TM], *pb[POLY_TN];
+#pragma unroll
+      for (int i = 0; i < POLY_TM; i++) {
+        const int m = m0 + wm + i * 32 + (lane & 31);
+        pa[i] = gA + poly_a_row(m < POLY_M ? m : POLY_M - 1);
+      }
+#pragma unroll
+      for (int j = 0; j < POLY_TN; j++) {
+        const int n = n0 + wn + j * 32 + (lane & 31);
+        pb[j] = gB + poly_b_row(n < POLY_N ? n : POLY_N - 1);
+      }
+      auto load_16 = [&](PolyUnit (&a)[POLY_TM], PolyUnit (&b)[POLY_TN], int k0) {
+        const int k = k0 + 8 * (lane >> 5);
+        auto load_8 = [&](PolyUnit &to, const float *row, bool kc, auto &&at) {
+          if (kc) {
+            const poly_f32x4 lo = *(const poly_f32x4_u *)(row + at(k)), hi = *(const poly_f32x4_u *)(row + at(k) + 4);
+#pragma unroll
+            for (int e = 0; e < 4; e++) { to.v[e] = lo[e]; to.v[4 + e] = hi[e]; }
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; e++) to.v[e] = row[at(k + e)];
+          }
+        };
+#pragma unroll
+        for (int i = 0; i < POLY_TM; i++) load_8(a[i], pa[i], POLY_A_KC, [](int x) { return poly_a_k(x); });
+#pragma unroll
+        for (int j = 0; j < POLY_TN; j++) load_8(b[j], pb[j], POLY_B_KC, [](int x) { return poly_b_k(x); });
+      };
+      auto multiply_16 = [&](const PolyUnit (&a)[POLY_TM], const PolyUnit (&b)[POLY_TN]) {
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+#pragma unroll
+          for (int i = 0; i < POLY_TM; i++)
+#pragma unroll
+            for (int j = 0; j < POLY_TN; j++) {
+              poly_acc16 &to = e % 4 == 0 ? acc[i][j] : e % 4 == 1 ? low[i][j] : e % 4 == 2 ? third[i][j] : fourth[i][j];
+              to = POLY_MFMA_F32(a[i].v[e], b[j].v[e], to);
+            }
+      };
+      constexpr int WHOLE = POLY_KP / 16 * 16;
+      PolyUnit a0[POLY_TM], b0[POLY_TN], a1[POLY_TM], b1[POLY_TN];
+      if (WHOLE > 0) load_16(a0, b0, 0);
 #pragma unroll 1
-      for (int k0 = 0; k0 < POLY_KP; k0 += 2) {
+      for (int k0 = 0; k0 < WHOLE; k0 += 32) {
+        if (k0 + 16 < WHOLE) load_16(a1, b1, k0 + 16);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply_16(a0, b0);
+        if (k0 + 16 < WHOLE) {
+          if (k0 + 32 < WHOLE) load_16(a0, b0, k0 + 32);
+          __builtin_amdgcn_sched_barrier(0);
+          multiply_16(a1, b1);
+        }
+      }
+#pragma unroll 1
+      for (int k0 = WHOLE; k0 < POLY_KP; k0 += 2) {
         const int k = k0 + (lane >> 5);
         float fa[POLY_TM], fb[POLY_TN];
 #pragma unroll
-        for (int i = 0; i < POLY_TM; i++) {
-          const int m = m0 + wm + i * 32 + (lane & 31);
-          fa[i] = k < POLY_KP ? gA[poly_a_row(m < POLY_M ? m : POLY_M - 1) + poly_a_k(k)] : 0.0f;
-        }
+        for (int i = 0; i < POLY_TM; i++) fa[i] = k < POLY_KP ? pa[i][poly_a_k(k)] : 0.0f;
 #pragma unroll
-        for (int j = 0; j < POLY_TN; j++) {
-          const int n = n0 + wn + j * 32 + (lane & 31);
-          fb[j] = k < POLY_KP ? gB[poly_b_row(n < POLY_N ? n : POLY_N - 1) + poly_b_k(k)] : 0.0f;
-        }
+        for (int j = 0; j < POLY_TN; j++) fb[j] = k < POLY_KP ? pb[j][poly_b_k(k)] : 0.0f;
 #pragma unroll
         for (int i = 0; i < POLY_TM; i++)
 #pragma unroll
           for (int j = 0; j < POLY_TN; j++) acc[i][j] = POLY_MFMA_F32(fa[i], fb[j], acc[i][j]);
       }
+#pragma unroll
+      for (int i = 0; i < POLY_TM; i++)
+#pragma unroll
+        for (int j = 0; j < POLY_TN; j++) acc[i][j] = (acc[i][j] + low[i][j]) + (third[i][j] + fourth[i][j]);
     }
   }
 

@@ -172,3 +172,39 @@ def test_rows_of_one_term(c, what):
     assert _is_it(desc, c)
     want = a @ b
     assert bool(((got.double() - want).abs() <= 2.0 ** -24 * (1 + 2.0 ** -4) * want.abs()).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [2.0 ** -108, 2.0 ** -66])
+@pytest.mark.parametrize("c", [SHAPES[1], SHAPES[4], SHAPES[8]], ids=lambda c: "-".join(map(str, c)))
+def test_small_values_beside_ones_that_planes_do_not_hold(c, scale):
+    """Values about the smallest that planes hold, times large ones, one of them below it, and values whose products are
+    about the smallest normal number: within the rounding of K additions and products, of a product below that number
+    an absolute one."""
+    def change(a, b):
+        a.mul_(scale)
+        a[4000] = 2.0 ** -111
+        b.mul_(2.0 ** 60 if scale < 2.0 ** -100 else scale)
+    desc, got, a, b = _product(c, change)
+    assert _is_it(desc, c)
+    err = (got.double() - a @ b).abs()
+    assert bool((err <= c[2] * (2.0 ** -24 * (a.abs() @ b.abs()) + 2.0 ** -149)).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", SHAPES, ids=lambda c: "-".join(map(str, c)))
+def test_tiles_that_are_computed_again_against_float64(c, monkeypatch):
+    """A value below 2^-110 in every row sends every tile to the fp32 MFMA: within the rounding of K additions and
+    products, and no further off than the fp32 templates are (whose sums are as many, of other terms: a twentieth for
+    that)."""
+    def change(a, b):
+        (a.view(c[2], c[0])[c[2] // 2] if c[3][0] == "t" else a.view(c[0], c[2])[:, c[2] // 2]).fill_(2.0 ** -112)
+    desc, got, a, b = _product(c, change)
+    assert _is_it(desc, c)
+    want = a @ b
+    err = (got.double() - want).abs()
+    assert bool((err <= c[2] * 2.0 ** -24 * (a.abs() @ b.abs())).all())
+    monkeypatch.setenv("POLY_HIP_NO_F32_SPLIT", "1")
+    desc, there, _, _ = _product(c, change)
+    assert "three planes" not in desc
+    assert float(err.norm()) <= 1.05 * float((there.double() - want).norm())
