@@ -27,6 +27,23 @@ def test_stays_in_bounds(rows, cols, wide, op, hiplib, monkeypatch):
     assert hostcheck.check_schedule(hiplib, pf.schedule) >= 1
 
 
+@pytest.mark.parametrize("rows,operands,wide", [(256, 4, True), (257, 3, True), (257, 4, False), (400, 3, True), (400, 6, False)])
+def test_rows_of_many_operands(rows, operands, wide, hiplib, monkeypatch):
+    """More rows than CUs go to sixteen waves each only where a few operands are read."""
+    monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
+    s = cases.Schedule()
+    out, bufs = s.buf("out", rows), [s.buf(f"b{i}", rows * 4096) for i in range(operands)]
+    (r,) = s.ranges(rows)
+    k = s.rrange(4096)
+    value = bufs[0][r * 4096 + k]
+    for b in bufs[1:]:
+        value = value * b[r * 4096 + k]
+    s.store(out, r, s.reduce("ADD", value, k), r)
+    pf = s.plan()
+    item = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents.items[0]
+    assert ("G=1024" in _ffi.take_string(hiplib.poly_hip_describe(item.root, 0))) == wide
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("op", ["sum", "max"])
 @pytest.mark.parametrize("rows,cols,wide", SHAPES)
