@@ -1366,10 +1366,21 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   if (ring.bm) {
     if (emit(ring.bm, ring.bn, ring.wm, ring.wn, 3, out, 0, -1, true, Dma{ring.bk, 2, ring.wg, ring.wm, ring.wn})) {
       if (S > 1) return add_parts();
-      RenderedKernel alone;      // a candidate for on-device tuning: the registers of a workgroup that has a CU to itself
-      if (f32 && ring.wg > 1 && matmul_tuning_enabled() && emit(ring.bm, ring.bn, ring.wm, ring.wn, 3, &alone, 0, -1, true, Dma{ring.bk, 2, 1, ring.wm, ring.wn})) {
+      if (matmul_tuning_enabled()) {
+        // candidates for on-device tuning, the same order of additions in all of them; of fp32 values, whose tiles are
+        // computed again as a whole, the same tile with other waves or with the registers of a workgroup that has a CU to itself
+        struct Shape { int bm, bn, wm, wn, wg; };
+        static const Shape shapes16[] = {{64, 64, 2, 2, 2}, {64, 128, 2, 2, 2}, {64, 128, 2, 2, 1}, {128, 128, 2, 4, 1}, {128, 256, 2, 4, 1}};
+        static const Shape shapes32[] = {{64, 64, 2, 2, 1}, {128, 128, 4, 2, 1}};
+        auto label = [&](const Shape &c) { return f32 ? strf("f32_%dx%dw%dx%d", c.bm, c.bn, c.wm, c.wn) : strf("%dx%dx%dw%dx%ds2g%d", c.bm, c.bn, ring.bk, c.wm, c.wn, c.wg); };
         out->variants.push_back({"default", out->source, out->strategy, out->launch});
-        out->variants.push_back({strf("f32_%dx%dw%dx%d", ring.bm, ring.bn, ring.wm, ring.wn), alone.source, alone.strategy, alone.launch});
+        auto add = [&](const Shape &c) {
+          RenderedKernel v;
+          if ((!f32 || (c.bm == ring.bm && c.bn == ring.bn)) && emit(c.bm, c.bn, c.wm, c.wn, 3, &v, 0, -1, true, Dma{ring.bk, 2, c.wg, c.wm, c.wn}) && v.source != out->source)
+            out->variants.push_back({label(c), v.source, v.strategy, v.launch});
+        };
+        if (f32) for (const Shape &c : shapes32) add(c);
+        else for (const Shape &c : shapes16) add(c);
       }
       return true;
     }

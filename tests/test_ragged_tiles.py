@@ -4,6 +4,7 @@ layout, operands that begin between two dwords.  Against the product in float64,
 rounding of K fp32 additions (K * 2^-24 * sum of |a b|; the products of 16-bit values are exact)."""
 import ctypes as C
 import os
+import re
 import sys
 
 import pytest
@@ -40,6 +41,25 @@ def test_stays_in_bounds(c, hiplib, monkeypatch):
     assert _is_it(_ffi.take_string(hiplib.poly_hip_describe(it.root, PLAN)), c[5])
     assert "rows of any alignment" not in _ffi.take_string(hiplib.poly_hip_describe(it.root, 0))
     check_as_of_a_plan(hiplib, s, it)
+
+
+@pytest.mark.skipif(not os.path.exists(hostcheck.CLANG), reason="no host clang with AddressSanitizer")
+@pytest.mark.parametrize("c", [SHAPES[0][:5], SHAPES[9][:5], (1030, 1040, 97, "float32", "nn"), (1801, 1700, 160, "float32", "tn")], ids=lambda c: "-".join(map(str, c)))
+def test_candidates_for_tuning_stay_in_bounds(c, hiplib, monkeypatch):
+    """The other tiles that the on-device search times."""
+    monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
+    monkeypatch.setenv("POLY_BEAM", "1")
+    pf = cases._matmul_schedule(_case(*c, None)).plan()
+    s = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents
+    it = s.items[0]
+    variants = _ffi.take_string(hiplib.poly_hip_render(it.root, b"k", PLAN, None)).split("\n// ---- variant ")[1:]
+    assert len(variants) >= (1 if c[3] == "float32" else 3)
+    sizes = [s.buf_slots[it.buf_slot_indices[p]].nbytes for p in range(it.n_buf_slots)]
+    for v in variants:
+        label, source = v.split("\n", 1)
+        bm, bn, wm, wn = map(int, re.match(r"(?:f32_)?(\d+)x(\d+)\w*?w(\d)x(\d)", label).groups())
+        grid = (-(-c[0] // bm) * -(-c[1] // bn), 1, 1)
+        hostcheck.check_kernel(source, hostcheck._entry_name(source), grid, 64 * wm * wn, sizes, block_stride=max(1, grid[0] * 64 * wm * wn // (1 << 16)))
 
 
 @pytest.mark.gpu

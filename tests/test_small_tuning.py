@@ -1,4 +1,4 @@
-"""The on-device search (POLY_BEAM) over products of few or ragged tiles and attention of few,
+"""The on-device search (POLY_BEAM) over products of few or ragged tiles, fp32 ones on bf16 planes and attention of few,
 ragged or fp32 queries and keys: they bring candidates, each of which runs, and what the
 search decides changes no bit."""
 import os
@@ -13,6 +13,8 @@ pytestmark = pytest.mark.gpu
 # case, kernels that have candidates: what their descriptions say, and the label of one
 CASES = [(_case(100, 300, 515, "bfloat16", "nn"), "depth dealt to", "32x32w8x6p1"), (_case(12, 770, 1000, "float16", "tn"), "depth dealt to", "16x16w8x6p1"),
          (_case(128, 768, 768, "float32", "nt"), "depth dealt to", "f32_32x32w4x6"), (_case(345, 776, 2304, "float32", "nn"), "of two sums each", "f32_64x64w4x4"),
+         (_case(1111, 999, 601, "bfloat16", "nn"), "rows of any alignment", "128x128x64w2x4s2g1"), (_case(1500, 1401, 130, "float16", "tn"), "rows of any alignment", "64x64x64w2x2s2g2"),
+         (_case(1030, 1040, 97, "float32", "nn"), "three planes", "f32_64x64w2x2"), (_case(1801, 1700, 160, "float32", "tn"), "three planes", "f32_128x128w4x2"),
          (cases._gpt2(3, 40, "bfloat16", layers=1), "scores of", "attn_occ2"), (cases._gpt2(1, 130, "float32", layers=1), "scores of", "attn_occ4")]
 
 
