@@ -161,23 +161,24 @@ def _jobs(lib, schedule, max_threads, only, groups):
         if only is not None and step not in only:
             continue
         it = s.items[s.exec_order[step]]
-        launch = (C.c_int * 7)()
-        text = _ffi.take_string(lib.poly_hip_render(it.root, b"k", 0, launch))
-        if "\n// ---- guard" in text:
-            continue                    # guarded fast path: its arguments include a flag set by another kernel
-        main = text.split("\n// ---- ")[0]
-        sizes = tuple(max(int(s.buf_slots[it.buf_slot_indices[p]].nbytes), 4) for p in range(it.n_buf_slots))
-        if (main, sizes) in seen:
-            continue
-        seen.add((main, sizes))
-        grid = (launch[0], launch[1], launch[2])
-        scratch = 0
-        for unit in text.split("\n// ---- ")[1:]:
-            m = re.match(r"first stage ---- grid=(\d+),(\d+) block=(\d+) scratch=(\d+)\n", unit)
-            if m:       # first stage of a two-stage kernel: same arguments plus the scratch, its own launch
-                scratch = int(m.group(4))
-                yield f"step {step} (first stage)", unit[m.end():], (int(m.group(1)), int(m.group(2)), 1), int(m.group(3)), sizes, scratch
-        yield f"step {step}", main, grid, launch[3], sizes, scratch
+        for flags in (0, 8):                # by itself, and as a kernel of a plan
+            launch = (C.c_int * 7)()
+            text = _ffi.take_string(lib.poly_hip_render(it.root, b"k", flags, launch))
+            if "\n// ---- guard" in text:
+                continue                    # guarded fast path: its arguments include a flag set by another kernel
+            main = text.split("\n// ---- ")[0]
+            sizes = tuple(max(int(s.buf_slots[it.buf_slot_indices[p]].nbytes), 4) for p in range(it.n_buf_slots))
+            if (main, sizes) in seen:
+                continue
+            seen.add((main, sizes))
+            grid = (launch[0], launch[1], launch[2])
+            scratch = 0
+            for unit in text.split("\n// ---- ")[1:]:
+                m = re.match(r"first stage ---- grid=(\d+),(\d+) block=(\d+) scratch=(\d+)\n", unit)
+                if m:       # first stage of a two-stage kernel: same arguments plus the scratch, its own launch
+                    scratch = int(m.group(4))
+                    yield f"step {step} (flags {flags}, first stage)", unit[m.end():], (int(m.group(1)), int(m.group(2)), 1), int(m.group(3)), sizes, scratch
+            yield f"step {step} (flags {flags})", main, grid, launch[3], sizes, scratch
     if not groups or only is not None:
         return
     for gi in range(lib.poly_hip_fused_groups(schedule, -1, None, None)):
@@ -207,7 +208,7 @@ def _jobs(lib, schedule, max_threads, only, groups):
 
 def check_schedule(lib, schedule, max_threads=1 << 21, only=None, groups=True, workers=6):
     """Host-checks every distinct kernel of `schedule`: each scheduled kernel as the
-    per-kernel lowering renders it (guarded fast paths aside) and each fused group of the
+    per-kernel lowering and as a plan has it (guarded fast paths aside) and each fused group of the
     plan-level lowering.  Launches larger than `max_threads` threads are sampled by
     workgroup.  Returns the number of kernels checked; raises on the first failure."""
     from concurrent.futures import ThreadPoolExecutor
