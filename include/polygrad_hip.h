@@ -100,8 +100,8 @@ void poly_hip_program_destroy(PolyHipProgram *prog);
  * poly_render_cuda (src/render_cuda.c:196) in the reference's tests.
  * launch_out, when non-NULL, receives grid[3], block[3], lds bytes (7 ints).
  * flags: bit0 disable templates, bit1 disable vectorisation, bit2 disable
- * cooperative reductions, bit3 as a kernel of a plan (whose fp32 products have
- * a template of their own). */
+ * cooperative reductions, bit3 as a kernel of a plan (whose large fp32 and ragged
+ * 16-bit products have templates of their own). */
 char *poly_hip_render(PolyUOp *scheduled_root, const char *fn_name, int flags, int *launch_out);
 /* One-line description of how the kernel was lowered ("row-reduce G=64 ..."). */
 char *poly_hip_describe(PolyUOp *scheduled_root, int flags);

@@ -834,7 +834,7 @@ static PolyHipPlan *compile_schedule(const PolySchedule *s, bool buffers_apart) 
     bool any = false;
     for (int t = 0; t < n_units; t++) {
       const Unit &u = plan->units[(size_t)t];
-      if (u.runner->rk.klass != KernelClass::MATMUL_MFMA || plan->on_side[(size_t)t] || u.runner->rk.reads_b_ahead) continue;
+      if (u.runner->rk.klass != KernelClass::MATMUL_MFMA || plan->on_side[(size_t)t] || u.runner->rk.wants_no_reader) continue;
       for (int sl : u.slots) {
         const PolyScheduleBufSlot &b = s->buf_slots[sl];
         if (b.is_intermediate || written[(size_t)sl] || b.nbytes < (128 << 10) || b.nbytes > most) continue;

@@ -76,7 +76,7 @@ struct RenderedKernel {
   // A matrix product that the plan launches nothing ahead of to read operand B into the
   // memory-side cache: its own first workgroups do that, its first stage reads both operands, or
   // its loads are far enough ahead for what such a launch costs to be more than it gives.
-  bool reads_b_ahead = false;
+  bool wants_no_reader = false;
   // A product that leaves the largest magnitude of every 64 x 64 block of some of its output
   // columns in its scratch memory (MatmulEpilogue::block_maxima) -- and, set by the plan-level
   // fusion, whose scratch memory that is: the launch that reads the bounds keeps them in its

@@ -868,7 +868,7 @@ static bool render_matmul_wave(const MatmulMatch &mm, const MatmulEpilogue &ep, 
     // Its waves have four to six steps of loads in flight, and a launch of its own that reads the
     // weights ahead costs more than HBM does: GPT-2 small of 12 bf16 tokens 505 us [533 with it], of
     // 128 fp32 tokens, whose 500 MB of weights no cache holds, 967 [1015].
-    out->reads_b_ahead = true;
+    out->wants_no_reader = true;
     out->strategy = strf("mfma %s M=%lld N=%lld K=%lld Z=%lld tile %dx%d, depth dealt to %d waves%s, A:%s B:%s", f32 ? (f.block == 32 ? "32x32x2 f32" : "16x16x4 f32") : mm.A.dt == DT_BF16 ? "16x16x32 bf16" : "16x16x32 f16",
                          (long long)M, (long long)N, (long long)K, (long long)Z, bm, bn, f.waves, sums == 2 ? " of two sums each" : "", a_kc ? "k-major" : "m-major", b_kc ? "k-major" : "n-major");
     if (touch_wgs) out->strategy += strf(", %d workgroups read B ahead", touch_wgs);
@@ -1315,7 +1315,7 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     rk->launch.grid[1] = (unsigned)(Z * S);
     rk->launch.block[0] = (unsigned)(64 * wvm * wvn);
     rk->klass = KernelClass::MATMUL_MFMA;
-    rk->reads_b_ahead = touch_wgs > 0 || ring.bm;
+    rk->wants_no_reader = touch_wgs > 0 || ring.bm;
     rk->writes_block_maxima = block_maxima;
     if (block_maxima) rk->scratch_bytes = ep.block_maxima.bytes;
     rk->strategy = strf("mfma 32x32x16 %s M=%lld N=%lld K=%lld Z=%lld tile %dx%dx%d A:%s B:%s", A.dt == DT_BF16 ? "bf16" : "f16",
@@ -1354,8 +1354,6 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
     cfg += strf("#define POLY_PARTIALS %s\n#define POLY_SIGNATURE %s\n", partials.c_str(), signature.c_str());
     cfg += ep.code;
     cfg += strf("#define POLY_EPILOGUE(acc, m, n, z) %s\n", ep.call.c_str());
-    if (f32 && !ep.mid_value_call.empty())
-      cfg += strf("#define POLY_EP_MID_VALUE(acc, m, n, z) %s\n#define POLY_EP_MID_PTR(m, n, z) %s\n", ep.mid_value_call.c_str(), ep.mid_ptr_call.c_str());
     out->source = std::string(hip_prelude()) + cfg + kSplitKCombine;
     out->launch = LaunchSpec();
     out->launch.grid[0] = (unsigned)(((double)Z * M * N + 255) / 256);
@@ -1515,14 +1513,16 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   // that at most a quarter of the CUs take part in costs nearly a whole one of 256x256 tiles.  The launch keeps the rows
   // whose tiles make whole rounds, and those left over go to 64x128 tiles that each have a CU, if a
   // depth of 512 and more is worth the launch: 50257x1024x12288 (788 tiles, a vocabulary projection's
-  // gradient in three planes) 1233 us -> 1018 + 72, the same bits, the training block 5726 -> 5562.
+  // gradient in three planes) 1233 us -> 1018 + 72, the same bits, the training block 5726 -> 5562; 51200x1024x1024 147 -> 133,
+  // x512 98 -> 88, 102400x512x512 103 -> 95, 198656x256x512 108 -> 101, behind six whole rounds 100000x1000x512 220 -> 214.
+  // (Before three whole rounds other tiles are the faster ones.)
   if (Z == 1 && S == 1 && BM == 256 && BN == 256 && K >= 512 && !matmul_tuning_enabled() && !getenv("POLY_HIP_NO_TAIL_LAUNCH") && !getenv("POLY_HIP_MM_TILE") &&
       !measurement_env("POLY_HIP_MM_NOEPI")) {
     const int64_t tn = (N + 255) / 256, T = ((M + 255) / 256) * tn, whole = T / 256, rest = T % 256;
     const int64_t m_lo = tn > 0 ? whole * 256 / tn * 256 : 0;
     Dma small{64, 4, 1, 2, 2};
     RenderedKernel main, tail;
-    if (whole >= 1 && rest > 0 && rest <= 64 && m_lo > 0 && m_lo < M && ((M - m_lo + 63) / 64) * ((N + 127) / 128) <= 256 && (a_kc || m_lo % 8 == 0) &&
+    if (whole >= 1 && rest > 0 && rest <= 64 && m_lo > 0 && m_lo < M && ((M - m_lo + 63) / 64) * ((N + 127) / 128) <= 256 &&
         dma_for(64, 128, &small) && emit(BM, BN, WVM, WVN, pipe, &main, 0, -1, dma_ok, chosen, 0, m_lo) && emit(64, 128, 2, 2, 3, &tail, 0, -1, true, small, m_lo, M) &&
         main.writes_block_maxima == out->writes_block_maxima && tail.writes_block_maxima == out->writes_block_maxima) {
       const std::string strategy = out->strategy;
@@ -2162,7 +2162,7 @@ bool try_render_matmul_generic(const KernelGraph &g, const std::string &fn, cons
         if (write_a || write_b) out->pres.insert(out->pres.begin(), plane_writer(write_a, write_b));
         // (what writes the planes streams both operands once: a launch that reads them before it
         // only costs its own time)
-        if (write_a && write_b) out->reads_b_ahead = true;
+        if (write_a && write_b) out->wants_no_reader = true;
         out->scratch_bytes = std::max(planes_bytes, main.scratch_bytes);
         out->flops = 2.0 * (double)M * (double)N * (double)K * (double)Z;
         out->strategy = strf("operands as expressions, written as %s planes first (%d + %d planes of K=%lld, %.0f MB%s): ", plane_dt == DT_F16 ? "fp16" : "bf16", parts[0], parts[1],

@@ -120,7 +120,9 @@ void matmul_hint_a_rows(const MatmulRows *rows);
 // no more (0: no limit).
 void matmul_hint_scratch_limit(size_t bytes);
 // While one lives, kernels are lowered for a plan: its fp32 products may take the bf16 matrix pipes
-// (kernels/matmul_f32_split.hip).
+// (kernels/matmul_f32_split.hip), its ragged 16-bit ones tiles that go through registers
+// (kernels/matmul_dma.hip, POLY_RING).  A kernel that its caller launches by itself keeps the templates
+// and the scratch memory that the caller has planned for.
 struct MatmulsOfPlan {
   MatmulsOfPlan();
   ~MatmulsOfPlan();
