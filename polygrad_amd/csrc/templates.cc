@@ -998,21 +998,22 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   const bool f32 = A.dt == DT_F32;
   if (f32) {
     // Three bf16 planes of each value on the bf16 matrix pipes (kernels/matmul_f32_split.hip).  A 128x128 tile
-    // takes 1.1 us for 32 of its depth by itself on a CU and 1.55 where every CU has one, a 64x64 tile 0.64:
+    // takes 1.35 us for 32 of its depth by itself on a CU and 1.9 where every CU has one, a 64x64 tile 0.7.  Figures: us,
+    // operands from HBM, the fp32 templates and here.
     //   128x128  where the last round over the chip leaves no more than three in ten CUs idle (2048^3
-    //            183 us -> 100, 4096x1024x1024 88 -> 53, 2047x2039x1201 168 -> 112, 128x50257x768 115 -> 80;
-    //            1500x1500x1504, 144 tiles, 94 and 120 here)
+    //            202 -> 137, 4096x1024x1024 109 -> 64, 2047x2039x1201 183 -> 76, 128x50257x768 127 -> 90)
     //   128x128  of a depth dealt to two or four workgroups, 384 or more each, on as many CUs, from 1.2e9
-    //            multiply-adds on (1024x1024x4096 77 -> 60, 512x3072x768 37 -> 26; 1024^3 22.5 and 24.0,
-    //            704x704x2048 22.6 and 28.0; to eight 512x784x4096 41.5 and 34.2, which the tests of deep
+    //            multiply-adds on (1024x1024x4096 82 -> 69, 512x3072x768 42 -> 30; 1024^3 24.4 and 25.7,
+    //            704x704x2048 23 and 34; to eight 512x784x4096 47 and 38, which the tests of deep
     //            products hold where it is)
     //   64x64    from 257 tiles, where the waves that share a depth need several rounds, to 512, two on a CU
-    //            (4096x512x784 37.6 -> 31.0, 512x2304x768 48.4 -> 27.2, 2048x1024x64 9.4 -> 5.9; 1024^3, 256 tiles, 22.5 and
-    //            25.7; a depth of 4096 and more stays with the templates for that)
-    // The latter two only where the rows of an operand that lies along them begin on 64 bytes (1001x1503x777 61
-    // either way, 1500x1500x1504 94 and 186).  Errors against float64 are a third to two thirds of those
-    // of the fp32 MFMA templates, that deal the depth to waves and workgroups or not.  A kernel lowered by itself,
-    // outside a plan, keeps those.
+    //            (4096x512x784 46 -> 35, 512x2304x768 50 -> 29, 2048x1024x64 14.2 -> 6.1, with few tiles more than
+    //            CUs no gain: 192x5760x128 6.8 and 7.9, 320x3776x81 6.2 and 6.6; 1024^3, 256 tiles, 24.4 and 27.4;
+    //            a depth of 4096 and more stays with the templates for that)
+    // The latter two only where the rows of an operand that lies along them begin on 64 bytes.  (That line and the share
+    // of idle CUs were drawn while ends of the depth went through scratch memory; both could be wider: 1001x1503x777 69
+    // and 33 on 64x64, 1500x1500x1504, 144 tiles of 128x128, 103 and 79.)  Errors against float64 are a third to two thirds
+    // of those of the fp32 MFMA templates, that deal the depth to waves and workgroups or not.
     if (g_in_plan && !g_a_rows && Z == 1 && zd.empty() && ep.scratch_type.empty() && !getenv("POLY_HIP_NO_F32_MFMA") && !getenv("POLY_HIP_NO_F32_SPLIT") &&
         any_layout(ka, md, true, M, &any_a) && any_layout(kb, nd, false, N, &any_b)) {
       const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128), t64 = ((M + 63) / 64) * ((N + 63) / 64);
@@ -1056,12 +1057,12 @@ bool render_matmul(const MatmulMatch &mm, const MatmulEpilogue &ep, RenderedKern
   //   64x128   to 2304 (1111x999x1501 24.0 -> 17.6, 2001x900x2001 27.9 -> 20.3; 1111x999x3001 28.1 and 31.4)
   //   128x128  from 128 to 4096 (1500x1501x1501 31.8 -> 25.3, x4001 58.7 -> 55.6), with both operands read along the
   //            depth to 2304 (2001x1801x1501 31.2 -> 28.4, x4001 56.5 and 61.0)
-  //            (1500x1283x101, 8.6 and 6.8 here, stays with the waves: the tests of their edges hold it there)
+  //            (1500x1283x101, 7.5 and 6.6 here, stays with the waves: the tests of their edges hold it there)
   //   128x256  to 2304, no more than a quarter of it padding (3001x2501x2201 67 -> 54); with both operands read
   //            along the depth and fewer than 200 tiles to 1024 (2049x2501x601 30.9 -> 27.6, x1501 42.1 and 45.5)
   //   64x128   in several rounds of a depth to 512, where the stores are what takes time (7040x3328x39 36.7 -> 24.3,
   //            1472x7232x217 27.7 -> 18.2, 3001x2999x301 29.0 -> 22.4 MALL-hot; x601 37.7 and 35.9; x1003 46 and 49)
-  // A kernel lowered by itself, outside a plan, keeps its planes or waves.
+  // POLY_HIP_BF16_SPLIT_MIN asks for planes, which leaves none for these.
   auto odd_stride = [&](const KSplit &ks, const std::vector<Dim> &dims, bool is_a, bool kc) {
     bool o = !kc && ks.s_lo % 2 != 0;
     for (const Dim &d : dims) o = o || ((kc || &d != &dims.back()) && (is_a ? d.ca : d.cb) % 2 != 0);
