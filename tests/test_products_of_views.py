@@ -30,7 +30,9 @@ SLICED = [(513, 520, 1001, "bfloat16", "nn", "B 521 0", RING), (513, 520, 1001, 
           (520, 504, 769, "bfloat16", "tt", "A 521 3 B 771 1", RING), (1096, 1032, 161, "bfloat16", "tn", "A 1099 0 B 1033 0", RING), (1111, 1000, 1501, "bfloat16", "nn", "B 1001 1", RING),
           (1400, 1504, 129, "bfloat16", "tn", "A 1401 5 B 1506 1", RING), (2056, 2104, 130, "float16", "tn", "A 2057 0 B 2106 1", RING), (3000, 3008, 33, "bfloat16", "nn", "A 35 1 B 3009 0", RING),
           (512, 514, 1001, "bfloat16", "nn", "B 515 1", RING), (1030, 1040, 97, "float32", "nn", "A 99 1 B 1056 3", F32_PLANES), (1801, 1700, 160, "float32", "tn", "A 1805 2 B 1701 1", F32_PLANES),
-          (1152, 1024, 1536, "bfloat16", "nt", "A 1538 2 B 1544 8", DMA), (1152, 1024, 1536, "bfloat16", "tn", "A 1156 4 B 1026 2", DMA)]
+          (1152, 1024, 1536, "bfloat16", "nt", "A 1538 2 B 1544 8", DMA), (1152, 1024, 1536, "bfloat16", "tn", "A 1156 4 B 1026 2", DMA),
+          (1152, 1024, 1536, "bfloat16", "nn", "A 1537 1 B 1025 0", DMA), (1152, 1024, 1536, "float16", "tn", "A 1153 0 B 1024 1", DMA), (4096, 4096, 512, "bfloat16", "nt", "A 513 1 B 515 2", DMA),
+          (2304, 512, 1536, "bfloat16", "nt", "A 1537 0 B 1539 3", DMA), (512, 512, 16384, "bfloat16", "nn", "B 513 1", DMA), (16384, 64, 512, "bfloat16", "nn", "A 513 1 B 65 1", REGISTERS)]
 # (of 2^30 elements and more, in 1.1 million from one row to the next)
 FAR = [(1793, 1664, 129, "float32", "nn", "A 1100000 1", F32_PLANES), (1665, 1921, 191, "float32", "nt", "B 1100003 2", F32_PLANES), (1025, 1024, 65, "float32", "nn", "A 1100000 0", F32_PLANES),
        (1001, 1696, 1930, "float32", "tn", "A 1100000 0", F32_PLANES), (1090, 1941, 161, "bfloat16", "nt", "B 1100001 1", RING), (1152, 1024, 1920, "bfloat16", "nn", "B 1100000 0", DMA)]
