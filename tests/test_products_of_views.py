@@ -1,7 +1,7 @@
 """Products whose operands are views, on every template a plan's products run on, both operands and both ways they can
 lie: rows or the depth in reverse order, which an operand's offsets run down; slices of wider buffers, whose rows begin
 between two dwords or 16 bytes and end inside a tile, behind whole 8 elements or not; rows far apart, in buffers
-of 4 GiB and more.  On the host with buffers of their exact size, and against the product in float64, element by
+of 4 GiB and more; batches of matrices.  On the host with buffers of their exact size, and against the product in float64, element by
 element, within the rounding of K fp32 additions and products (K * 2^-24 * sum of |a b|)."""
 import ctypes as C
 import os
@@ -150,3 +150,58 @@ def test_what_lies_between_rows_changes_no_bit(c):
         plan.run(data)
         plan.sync()
     assert all(torch.equal(outputs[0], o) for o in outputs[1:])
+
+
+# (batch, rows, columns, depth, dtype, layout, elements from one matrix of A to the next and of B, template; 0: the same for
+# the whole batch, below 0: the batch in reverse order)
+BATCHED = [(3, 400, 501, 601, "bfloat16", "nn", 400 * 601 + 1, 601 * 501 + 3, RING), (3, 400, 504, 601, "bfloat16", "nn", -400 * 601, 601 * 504 + 1, RING), (2, 520, 520, 769, "float16", "tt", 520 * 769 + 1, -520 * 769, RING),
+           (3, 401, 1031, 161, "bfloat16", "nn", 401 * 161 + 7, 0, RING), (3, 385, 1031, 161, "bfloat16", "nt", -385 * 161 - 1, 0, RING), (3, 384, 512, 1024, "bfloat16", "nn", -384 * 1024, 1024 * 512 + 2, DMA),
+           (4, 512, 512, 1024, "bfloat16", "nt", -512 * 1024, 0, DMA), (3, 600, 1664, 160, "float32", "nn", 600 * 160 + 3, 0, F32_PLANES), (3, 600, 1664, 161, "float32", "nt", -600 * 161, 0, F32_PLANES)]
+
+
+def _batched_schedule(z, m, n, k, dtype, layout, za, zb, template):
+    s = cases.Schedule()
+    out, a, b = s.buf("C", z * m * n), s.buf("A", (z - 1) * abs(za) + m * k, dtype), s.buf("B", (z - 1) * abs(zb) + k * n, dtype)
+    q, r = s.ranges(z, m * n)
+    x = s.rrange(k)
+
+    def at(row, rows, along_k, step):
+        first = q * step + (1 - z) * step if step < 0 else q * step
+        return first + (row * k + x if along_k else x * rows + row)
+
+    s.store(out, q * (m * n) + r, s.reduce("ADD", a[at(r // n, m, layout[0] == "n", za)].cast(cases.F32) * b[at(r % n, n, layout[1] == "t", zb)].cast(cases.F32), x), q, r)
+    return s
+
+
+@pytest.mark.skipif(not os.path.exists(hostcheck.CLANG), reason="no host clang with AddressSanitizer")
+@pytest.mark.parametrize("c", BATCHED, ids=lambda c: "-".join(map(str, c)))
+def test_batched_stays_in_bounds(c, hiplib, monkeypatch):
+    monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
+    pf = _batched_schedule(*c).plan()
+    s = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents
+    assert _is_it(_ffi.take_string(hiplib.poly_hip_describe(s.items[0].root, PLAN)), c[8])
+    check_as_of_a_plan(hiplib, s, s.items[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", BATCHED, ids=lambda c: "-".join(map(str, c)))
+def test_batched_against_float64(c):
+    import torch
+    from polygrad_amd.inputs import torch_dtype
+    z, m, n, k, dtype, layout, za, zb, template = c
+    plan, g = _batched_schedule(*c).plan(), torch.Generator(device="cuda")
+    g.manual_seed(8)
+    assert _is_it(plan.kernel_info()[0]["desc"], template)
+    data, by = [None] * len(plan.slots), {}
+    for slot in plan.external_slots():
+        data[slot.index] = by[slot.name] = torch.randn(slot.numel, generator=g, device="cuda").to(torch_dtype(slot.dtype))
+    torch.cuda.synchronize()
+    plan.run(data)
+    plan.sync()
+    for i in range(z):
+        def matrix(name, rows, cols, step):
+            return torch.as_strided(by[name], (rows, cols), (cols, 1), (z - 1 - i if step < 0 else i) * abs(step)).double()
+        a = matrix("A", m, k, za) if layout[0] == "n" else matrix("A", k, m, za).T
+        b = matrix("B", k, n, zb) if layout[1] == "n" else matrix("B", n, k, zb).T
+        err = (by["C"].double().reshape(z, m, n)[i] - a @ b).abs()
+        assert bool((err <= k * 2.0 ** -24 * (a.abs() @ b.abs())).all())
