@@ -27,9 +27,10 @@ def test_stays_in_bounds(rows, cols, wide, op, hiplib, monkeypatch):
     assert hostcheck.check_schedule(hiplib, pf.schedule) >= 1
 
 
-@pytest.mark.parametrize("rows,operands,wide", [(256, 4, True), (257, 3, True), (257, 4, False), (400, 3, True), (400, 6, False)])
+@pytest.mark.parametrize("rows,operands,wide", [(256, 4, True), (257, 3, True), (257, 4, False), (400, 3, True), (400, 6, False), (64, 16, True), (64, 17, False)])
 def test_rows_of_many_operands(rows, operands, wide, hiplib, monkeypatch):
-    """More rows than CUs go to sixteen waves each only where a few operands are read."""
+    """More rows than CUs go to sixteen waves each only where a few operands are read, and none where a lane's registers
+    would not hold what it reads."""
     monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
     s = cases.Schedule()
     out, bufs = s.buf("out", rows), [s.buf(f"b{i}", rows * 4096) for i in range(operands)]
