@@ -533,12 +533,16 @@ class Generic {
     // 48.7, 512 x 8192 8.6 either way): with more the loads of four waves are enough, and the CUs with two rows are
     // what takes time (257 x 16384 of four 14.4 and 16.8, 300 x 6001 of six 9.9 and 11.7).  Never of more than 16 operands: a
     // lane of sixteen waves has 128 registers (256 x 8192 of 20 29.7 and 34.5, of 24 35.8 and 57.3, of 32 40.9 and 105;
-    // of 16 24.0 and 24.4, 64 x 8192 8.5 -> 7.6).
-    int loads = 0;
+    // of 16 24.0 and 24.4, 64 x 8192 8.5 -> 7.6).  A sine counts as four more: three of them leave nothing in scratch
+    // memory, eight 160 bytes a lane (exponentials, logarithms, roots and quotients add nothing).
+    int loads = 0, sines = 0;
     std::vector<char> mark(g_.nodes.size(), 0);
     for (int id : top_reduces_) mark_reachable(g_, g_.n(id).src[0], mark);
-    for (int i = 0; i < (int)g_.nodes.size(); i++) loads += mark[(size_t)i] && g_.n(i).op == POLY_OP_LOAD;
-    if (R >= 4096 && rows <= (loads <= 3 ? 400 : loads <= 16 ? 256 : 0) && opt_.promote_reduce < 0 && opt_.block == 256) coop_G_ = opt_.block = 1024;
+    for (int i = 0; i < (int)g_.nodes.size(); i++) {
+      loads += mark[(size_t)i] && g_.n(i).op == POLY_OP_LOAD;
+      sines += mark[(size_t)i] && g_.n(i).op == POLY_OP_SIN;
+    }
+    if (R >= 4096 && rows <= (loads + 4 * sines > 16 ? 0 : loads <= 3 ? 400 : 256) && opt_.promote_reduce < 0 && opt_.block == 256) coop_G_ = opt_.block = 1024;
     coop_R_ = R;
     coop_ranges_ = rr;
     return true;

@@ -27,8 +27,9 @@ def test_stays_in_bounds(rows, cols, wide, op, hiplib, monkeypatch):
     assert hostcheck.check_schedule(hiplib, pf.schedule) >= 1
 
 
-@pytest.mark.parametrize("rows,operands,wide", [(256, 4, True), (257, 3, True), (257, 4, False), (400, 3, True), (400, 6, False), (64, 16, True), (64, 17, False)])
-def test_rows_of_many_operands(rows, operands, wide, hiplib, monkeypatch):
+@pytest.mark.parametrize("rows,operands,sines,wide", [(256, 4, 0, True), (257, 3, 0, True), (257, 4, 0, False), (400, 3, 0, True), (400, 6, 0, False), (64, 16, 0, True), (64, 17, 0, False), (64, 3, 3, True),
+                                                      (64, 4, 4, False)])
+def test_rows_of_many_operands(rows, operands, sines, wide, hiplib, monkeypatch):
     """More rows than CUs go to sixteen waves each only where a few operands are read, and none where a lane's registers
     would not hold what it reads."""
     monkeypatch.setattr(cases, "HipPlan", type("Loader", (), {"from_file": staticmethod(PlanFile)}))
@@ -36,9 +37,11 @@ def test_rows_of_many_operands(rows, operands, wide, hiplib, monkeypatch):
     out, bufs = s.buf("out", rows), [s.buf(f"b{i}", rows * 4096) for i in range(operands)]
     (r,) = s.ranges(rows)
     k = s.rrange(4096)
-    value = bufs[0][r * 4096 + k]
-    for b in bufs[1:]:
-        value = value * b[r * 4096 + k]
+    monkeypatch.setitem(cases._OPS, "SIN", 27)
+    values = [b[r * 4096 + k].un("SIN") if i < sines else b[r * 4096 + k] for i, b in enumerate(bufs)]
+    value = values[0]
+    for v in values[1:]:
+        value = value * v
     s.store(out, r, s.reduce("ADD", value, k), r)
     pf = s.plan()
     item = C.cast(pf.schedule, C.POINTER(_ffi.PolySchedule)).contents.items[0]
